@@ -6,27 +6,170 @@
 namespace tf {
 namespace {
 
-// ---- router: logits[m, e] = x[m] . rows[e], bf16 MFMA, K in steps of 32 in order ------------------------------------
+// ---- router: logits[m, e] = x[m] . rows[e] on the bf16 matrix cores -----------------------------------------------------
+//
+// K is cut into ROUTER_SLICES slices of whole 32-input chunks (by the hidden size alone); a slice is one MFMA chain in
+// order and the slices' fp32 sums are added in slice order, so a logit's bits depend on its row and expert only.  A
+// single chain of 64 to 84 dependent chunks a wave, 8 to 33 waves on the whole chip at decode, was what the first
+// form spent its time on (11 us at 1 to 8 rows x 128 experts x 2688, 131 us at 4,096 x 513 x 2048).
 
-__global__ void __launch_bounds__(64)
+constexpr int ROUTER_SLICES = 8;
+constexpr int64_t ROUTER_WIDE_TILES = 2048;      // more 16 x 16 tiles than this: the wide kernel
+
+__device__ __forceinline__ int router_chunk(int s, int chunks) { return s * chunks / ROUTER_SLICES; }
+
+// Few tiles: a workgroup takes 16 RM rows x 16 RN experts, a wave a slice, all of a slice's operands (or UNR chunks
+// of them) requested together, the slices added through LDS.
+template <int RM, int RN, int UNR>
+__global__ void __launch_bounds__(64 * ROUTER_SLICES)
     router_kernel(const uint16_t* __restrict__ X, int64_t ldx, const uint16_t* __restrict__ R, float* __restrict__ out,
                   int M, int D, int NE) {
-  const int lane = threadIdx.x, r = lane & 15, kq = lane >> 4;
-  const int m0 = blockIdx.x * 16, e0 = blockIdx.y * 16;
-  const uint16_t* xa = X + (size_t)min(m0 + r, M - 1) * ldx + kq * 8;
-  const uint16_t* wb = R + (size_t)min(e0 + r, NE - 1) * D + kq * 8;
-  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < D; k0 += 32) {
-    const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(xa + k0);
-    const bf16x8_t b = *reinterpret_cast<const bf16x8_t*>(wb + k0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-  }
-  const int col = e0 + r;
+  __shared__ f32x4_t part[ROUTER_SLICES][RM * RN][64];
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m0 = blockIdx.x * 16 * RM, e0 = blockIdx.y * 16 * RN;
+  const uint16_t* xa[RM];
+  const uint16_t* wb[RN];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = m0 + 4 * kq + i;
-    if (row < M && col < NE) out[(size_t)row * NE + col] = acc[i];
+  for (int i = 0; i < RM; ++i) xa[i] = X + (size_t)min(m0 + 16 * i + r, M - 1) * ldx + kq * 8;
+#pragma unroll
+  for (int j = 0; j < RN; ++j) wb[j] = R + (size_t)min(e0 + 16 * j + r, NE - 1) * D + kq * 8;
+  f32x4_t acc[RM][RN];
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int j = 0; j < RN; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  const int c0 = router_chunk(wave, D / 32), c1 = router_chunk(wave + 1, D / 32);
+  for (int c = c0; c < c1; c += UNR) {
+    bf16x8_t a[UNR][RM], b[UNR][RN];
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+      const int k0 = 32 * min(c + u, c1 - 1);
+#pragma unroll
+      for (int i = 0; i < RM; ++i) a[u][i] = *reinterpret_cast<const bf16x8_t*>(xa[i] + k0);
+#pragma unroll
+      for (int j = 0; j < RN; ++j) b[u][j] = *reinterpret_cast<const bf16x8_t*>(wb[j] + k0);
+    }
+#pragma unroll
+    for (int u = 0; u < UNR; ++u)
+      if (c + u < c1)
+#pragma unroll
+        for (int i = 0; i < RM; ++i)
+#pragma unroll
+          for (int j = 0; j < RN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][i], b[u][j], acc[i][j], 0, 0, 0);
   }
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int j = 0; j < RN; ++j) part[wave][i * RN + j][lane] = acc[i][j];
+  __syncthreads();
+  for (int t = wave; t < RM * RN; t += ROUTER_SLICES) {
+    f32x4_t s = part[0][t][lane];
+#pragma unroll
+    for (int q = 1; q < ROUTER_SLICES; ++q) {
+      const f32x4_t v = part[q][t][lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[i] = __fadd_rn(s[i], v[i]);
+    }
+    const int row = m0 + 16 * (t / RN) + 4 * kq, col = e0 + 16 * (t % RN) + r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (row + i < M && col < NE) out[(size_t)(row + i) * NE + col] = s[i];
+  }
+}
+
+// Many tiles: four waves on 64 rows x 128 experts, both operands through LDS (whole 128-byte lines from memory, 64
+// inputs a step, two steps in flight in registers), a wave on 32 x 64 walking the slices itself.  Column tiles past the
+// last expert are not computed (a shared expert's gate leaves a workgroup with one of eight).
+constexpr int RW_M = 64, RW_N = 128, RW_STEP = 64, RW_ROW = RW_STEP * 2 + 16;      // bytes of an LDS row, padded
+
+__global__ void __launch_bounds__(256)
+    router_wide_kernel(const uint16_t* __restrict__ X, int64_t ldx, const uint16_t* __restrict__ R,
+                       float* __restrict__ out, int M, int D, int NE) {
+  __shared__ __align__(16) unsigned char lds[2][(RW_M + RW_N) * RW_ROW];
+  constexpr int PIECES = (RW_M + RW_N) * 8 / 256;
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m0 = blockIdx.x * RW_M, e0 = blockIdx.y * RW_N, wm = 32 * (wave & 1), we = 64 * (wave >> 1);
+  const int rn = min(4, (NE - e0 - we + 15) >> 4);          // column tiles this wave has
+  const uint16_t* src[PIECES];
+#pragma unroll
+  for (int j = 0; j < PIECES; ++j) {
+    const int row = (tid >> 3) + 32 * j, ch = tid & 7;
+    src[j] = (row < RW_M ? X + (size_t)min(m0 + row, M - 1) * ldx : R + (size_t)min(e0 + row - RW_M, NE - 1) * D) + ch * 8;
+  }
+  const int chunks = D / 32, steps = (chunks + 1) / 2;
+  u32x4_t v0[PIECES], v1[PIECES];
+  // (D in whole chunks of 32: the last step's second half may lie past the row and is then not read)
+  auto load = [&](u32x4_t (&w)[PIECES], int step) {
+    const int k0 = RW_STEP * min(step, steps - 1) + ((tid & 7) * 8 + RW_STEP * min(step, steps - 1) < D ? 0 : -32);
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) w[j] = *reinterpret_cast<const u32x4_t*>(src[j] + k0);
+  };
+  auto store = [&](int u, const u32x4_t (&w)[PIECES]) {
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j)
+      *reinterpret_cast<u32x4_t*>(&lds[u][((tid >> 3) + 32 * j) * RW_ROW + (tid & 7) * 16]) = w[j];
+  };
+  f32x4_t acc[2][4], sum[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = sum[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  int slice = 0, end = router_chunk(1, chunks);
+  while (end == 0) end = router_chunk(++slice + 1, chunks);
+  // one step from stage u: the next step's operands (in `next`) go to the other stage, those after it into `mine`
+  auto walk = [&](int u, int step, u32x4_t (&mine)[PIECES], const u32x4_t (&next)[PIECES]) __attribute__((always_inline)) {
+    load(mine, step + 2);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int c = 2 * step + h;
+      if (c >= chunks) break;
+      bf16x8_t a[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        a[i] = *reinterpret_cast<const bf16x8_t*>(&lds[u][(wm + 16 * i + r) * RW_ROW + h * 64 + kq * 16]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (j < rn) {
+          const bf16x8_t b = *reinterpret_cast<const bf16x8_t*>(&lds[u][(RW_M + we + 16 * j + r) * RW_ROW + h * 64 + kq * 16]);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b, acc[i][j], 0, 0, 0);
+        }
+      if (c + 1 != end) continue;
+      // the slice that ends here joins the sum (slices without a chunk add nothing)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) sum[i][j][q] = __fadd_rn(sum[i][j][q], acc[i][j][q]);
+          acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        }
+      do end = router_chunk(++slice + 1, chunks);
+      while (slice + 1 < ROUTER_SLICES && end == router_chunk(slice, chunks));
+    }
+    store(1 - u, next);
+    __syncthreads();
+  };
+  load(v0, 0);
+  load(v1, 1);
+  store(0, v0);
+  __syncthreads();
+  for (int step = 0; step < steps; step += 2) {
+    walk(0, step, v0, v1);
+    if (step + 1 < steps) walk(1, step + 1, v1, v0);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int row = m0 + wm + 16 * i + 4 * kq + q, col = e0 + we + 16 * j + r;
+        if (j < rn && row < M && col < NE) out[(size_t)row * NE + col] = sum[i][j][q];
+      }
 }
 
 __global__ void __launch_bounds__(64)
@@ -267,7 +410,23 @@ extern "C" int tf_moe_router(const uint16_t* x, int64_t ldx, const uint16_t* row
   TF_REQUIRE(x && rows && logits && m >= 1 && ne >= 1, "router: null pointer or empty shape");
   TF_REQUIRE(d >= 32 && d % 32 == 0, "router: the hidden size (%d) must be a multiple of 32", d);
   TF_REQUIRE(aligned16(x) && aligned16(rows) && ldx % 8 == 0, "router: x and rows must be 16-byte aligned");
-  router_kernel<<<dim3((m + 15) / 16, (ne + 15) / 16), 64, 0, as_stream(stream)>>>(x, ldx, rows, logits, m, d, ne);
+  hipStream_t s = as_stream(stream);
+  // A compute unit takes 16 to 20 bytes of operands a cycle whatever the tile, so small tiles win while each has a unit
+  // to itself and larger ones (operands read fewer times over) once they do not: 392 tiles x 2688 18.3 us as 16 x 16,
+  // 13.3 as 32 x 32 (128 tiles 7.4 / 13); 1,617 x 2048 14.2 us as 32 x 64, 47 as one wave's 32 x 64; 8,448 x 2048
+  // 30.5 us wide, and from 2,112 tiles on the wide kernel's 28 us against two rounds of the others.
+  const int64_t tiles = (int64_t)((m + 15) / 16) * ((ne + 15) / 16);
+  if (tiles <= 256) {
+    const dim3 grid((m + 15) / 16, (ne + 15) / 16);
+    if (d <= 32 * 8 * ROUTER_SLICES) router_kernel<1, 1, 8><<<grid, 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
+    else router_kernel<1, 1, 12><<<grid, 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
+  } else if (tiles <= 1024) {
+    router_kernel<2, 2, 4><<<dim3((m + 31) / 32, (ne + 31) / 32), 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
+  } else if (tiles <= ROUTER_WIDE_TILES) {
+    router_kernel<2, 4, 4><<<dim3((m + 31) / 32, (ne + 63) / 64), 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
+  } else {
+    router_wide_kernel<<<dim3((m + 63) / 64, (ne + 127) / 128), 256, 0, s>>>(x, ldx, rows, logits, m, d, ne);
+  }
   TF_LAUNCH_OK("tf_moe_router");
   return 0;
 }

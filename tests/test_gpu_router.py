@@ -1,0 +1,25 @@
+"""The router's logits at the edges of its kernels' tiles, against float64 products; a row's bits whatever the call."""
+
+import pytest
+import torch
+
+from tensorfold_amd import moe, synthetic
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("rows,d,ne", [(1, 32, 1), (2, 96, 5), (16, 2688, 128), (17, 512, 129), (70, 2048, 513),
+                                       (257, 2720, 33), (65, 64, 1024), (1030, 480, 513), (4096, 256, 145)])
+def test_router_against_float64_and_row_by_row(rows, d, ne):
+    x = synthetic.activations(rows, d, 3 * rows + d).to(DEV)
+    r = synthetic.activations(ne, d, 5 * ne + d, scale=d ** -0.5).to(DEV)
+    got = moe.router(x, r)
+    want = x.double() @ r.double().t().contiguous()
+    # d products of bf16 values, exact in fp32, added in fp32: each addition rounds by at most 2^-24 of a partial sum
+    bound = d * 2.0 ** -23 * (x.double().abs() @ r.double().abs().t().contiguous())
+    assert bool(((got.double() - want).abs() <= bound).all())
+    for at in {0, rows // 2, rows - 1}:
+        assert torch.equal(moe.router(x[at:at + 1], r)[0], got[at])
+    part = rows - rows // 3
+    assert torch.equal(moe.router(x[:part], r), got[:part])
