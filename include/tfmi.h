@@ -105,8 +105,9 @@ int tf_qmm_group(const uint16_t* x, int64_t ldx, const float* xs, int count, con
 enum { TF_ARITH_F16 = 0, TF_ARITH_BF16 = 1 };
 
 /* Prompt-form matmul on MFMA: each weight rounded once (see TF_ARITH_*), one fp32 chain over K.
- * tile: 0 = chosen from the row count (what kernels/qmm.py:202-205 `prompt_tile` stands for); 1, 4, 8 = the four-wave
- * kernel on 16, 64 or 128 rows a workgroup; 9 = the eight-wave kernel (128 rows x 512 columns; K in whole steps of
+ * tile: 0 = chosen from the rows and columns (what kernels/qmm.py:202-205 `prompt_tile` stands for): 16 x 64, 32 x 64,
+ * 32 x 128 or 64 x 128 tiles while those of 9 would leave compute units idle; 1, 4, 8 = the four-wave kernel on 16, 64 or
+ * 128 rows a workgroup; 9 = the eight-wave kernel (128 rows x 512 columns; K in whole steps of
  * 64 only).  A row's bits are the same whatever the tile.
  * Replaces kernels/qmm.cpp:83-102 `qmm_prefill`. */
 int tf_qmm_prefill(const uint16_t* x, int64_t ldx, const uint32_t* weight, const uint16_t* scales,

@@ -17,6 +17,9 @@
 // scale 2^9 turns two nibble-bytes into the fp16 pair (q0, q1); the operand order this gives, inputs
 // (0, 4, 1, 5, 2, 6, 3, 7) of the eight, is applied to the activations when they are staged.
 
+#include <algorithm>
+#include <type_traits>
+
 #include "tf_common.h"
 
 namespace tf {
@@ -460,6 +463,22 @@ struct DenseSource {
   static __device__ __forceinline__ uint32_t sb_word(const Raw& r, int gi) { return (r.s[gi] & 0xFFFFu) | (r.b[gi] << 16); }
 };
 
+// The transpose of the 4 x 4 matrix whose rows are a wave's four rows of 16 lanes and whose columns are four registers.
+__device__ __forceinline__ void across(uint32_t (&v)[4]) {
+  auto swap32 = [](uint32_t& x, uint32_t& y) {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    x = r[0], y = r[1];
+  };
+  auto swap16 = [](uint32_t& x, uint32_t& y) {
+    const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    x = r[0], y = r[1];
+  };
+  swap32(v[0], v[2]);
+  swap32(v[1], v[3]);
+  swap16(v[0], v[1]);
+  swap16(v[2], v[3]);
+}
+
 // AR: TF_ARITH_F16 (fp16 operands, weights scaled by 2^8) or TF_ARITH_BF16 (the reference's bf16(fma(q, s, b)) weights
 // and untouched bf16 activations on the bf16 matrix instruction): the operand bits of mfma_body's two forms.
 struct NoStaged {
@@ -498,20 +517,6 @@ __device__ __forceinline__ void big_body(const uint16_t* __restrict__ X, int64_t
   // With groups of 64 a step's two chunks share their scale and bias words; the dense kernel keeps them across the two
   // (2 % of its time).  The experts' kernels, a few registers fuller, would spill for it and transpose them again.
   constexpr bool KEEP_SB = WS::KEEPS_GROUP_WORDS && GS == 64;
-  auto across = [](uint32_t (&v)[TJ]) {
-    auto swap32 = [](uint32_t& x, uint32_t& y) {
-      const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
-      x = r[0], y = r[1];
-    };
-    auto swap16 = [](uint32_t& x, uint32_t& y) {
-      const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
-      x = r[0], y = r[1];
-    };
-    swap32(v[0], v[2]);
-    swap32(v[1], v[3]);
-    swap16(v[0], v[1]);
-    swap16(v[2], v[3]);
-  };
   auto take = [&](const Raw& r, int i, uint32_t (&w)[TJ], uint32_t (&sb)[TJ]) {
 #pragma unroll
     for (int j = 0; j < TJ; ++j) w[j] = r.q[i][j];
@@ -1042,6 +1047,204 @@ __global__ void __launch_bounds__(256)
   mfma_body<GS, 1, EPI, RT, AR, true>(X, ldx, KG * GS, ws, rows, cnt, out, N, col0, ok, rows, 0.f, smem);
 }
 
+// The dense prompt matmul where tiles of 128 x 512 would leave compute units idle: WR x WC waves, a wave on 16 RT rows
+// x 16 CT columns, BM x BN = 16 RT WR x 16 CT WC a workgroup, STEP inputs a step.  Such a call is bound by the trip of its
+// operands (100 rows x 4096 x 4096 ran on 8 workgroups), so requests run far ahead of their use: the weights' words and
+// scales four steps in registers, the activations two, through two stages of LDS, one barrier a step.  A wave loads
+// the words its own operands need (lane (column c, quarter kq) word kq of column c: 256 bytes a tile and chunk).
+// The operands, their order along K and the matrix instruction are big_body's, and so are the bits.  
+template <int RT, int CT, int WR, int WC, int STEP>
+struct ShortTile {
+  static constexpr int BM = 16 * RT * WR, BN = 16 * CT * WC, THREADS = 64 * WR * WC;
+  static constexpr int ROW = STEP * 2 + 16;                     // bytes of an LDS row: 16 of padding against conflicts
+  static constexpr int LDS = 2 * BM * ROW;
+  static_assert(LDS <= 64 * 1024, "within what a launch gets without asking");
+  static int64_t workgroups(int64_t m, int64_t n) { return ((m + BM - 1) / BM) * ((n + BN - 1) / BN); }
+};
+typedef ShortTile<1, 1, 1, 4, 256> Short16;          // 16 rows x 64 columns
+typedef ShortTile<2, 1, 1, 4, 256> Short32;          // 32 x 64
+typedef ShortTile<2, 1, 1, 8, 256> Short32Wide;      // 32 x 128, eight waves
+typedef ShortTile<4, 2, 1, 4, 128> Short64;          // 64 x 128
+
+// tiles along the faster grid index, rounded up to whole rounds of the eight XCDs where there are that many
+__host__ __device__ constexpr int short_pad(int tiles) { return tiles < 8 ? tiles : (tiles + 7) & ~7; }
+
+template <int GS, int EPI, int AR, int RT, int CT, int WR, int WC, int STEP>
+__global__ void __launch_bounds__(64 * WR * WC)
+    qmm_prefill_short_kernel(const uint16_t* __restrict__ X, int64_t ldx, const uint32_t* __restrict__ W,
+                             const uint16_t* __restrict__ S, const uint16_t* __restrict__ B, void* __restrict__ out,
+                             int M, int N, int KG, int npad) {
+  typedef ShortTile<RT, CT, WR, WC, STEP> T;
+  constexpr int CPS = STEP / 32, GPS = STEP / GS, PPR = STEP / 8;        // chunks, groups, 16-byte pieces of a row a step
+  constexpr int PPT = T::BM * PPR / T::THREADS;
+  constexpr int WSETS = 4;
+  static_assert(T::BM * PPR % T::THREADS == 0 && T::THREADS % PPR == 0 && 128 % T::BN == 0, "whole pieces a thread");
+  extern __shared__ __align__(16) unsigned char smem[];
+  // neighbours in the grid go to the XCDs in turn: those that read the same part of the larger operand (the weight where
+  // N > 4 M: half a byte against two) are a multiple of eight apart, so it comes into one L2 and not into all eight
+  const int ct = (N + T::BN - 1) / T::BN, mt = (M + T::BM - 1) / T::BM;
+  const bool by_col = N > 4 * M;
+  const int across_n = short_pad(by_col ? ct : mt), slow = blockIdx.x / across_n, fast = blockIdx.x - slow * across_n;
+  const int cbt = by_col ? fast : slow, rt = by_col ? slow : fast;
+  if (cbt >= ct || rt >= mt) return;
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave / WC, wc = wave - wr * WC;
+  const int m0 = rt * T::BM, cnt = min(T::BM, M - m0);
+  const int K = KG * GS, chunks = K / 32, steps = (K + STEP - 1) / STEP;
+  const int col0 = cbt * T::BN + wc * (16 * CT);                 // below npad: columns from N up to it are stored zeros
+
+  // What a lane loads is not what it multiplies: lane (c, kq) loads the four words of column c in chunk 4 j + kq of a
+  // step as one 16-byte load and the scales of group 4 j + kq, and the words change lanes as in big_body.
+  constexpr int QPS = CPS / 4, SPS = (GPS + 3) / 4;
+  struct Words {
+    u32x4_t q[CT][QPS];
+    uint32_t s[CT][SPS], b[CT][SPS];
+  };
+  const uint32_t* wl[CT];
+#pragma unroll
+  for (int t = 0; t < CT; ++t) {
+    const int col = col0 + 16 * t;
+    wl[t] = W + (size_t)(col >> 6) * chunks * 256 + ((col & 63) + c) * 4;
+  }
+  const uint16_t *sl = S + col0 + c, *bl = B + col0 + c;
+  // (past the last step, or the last chunk of a ragged one, the last there is: requested, never used)
+  auto load_w = [&](int step, Words& w) {
+#pragma unroll
+    for (int i = 0; i < QPS; ++i) {
+      const int ch = min(step * CPS + 4 * i + kq, chunks - 1);
+#pragma unroll
+      for (int t = 0; t < CT; ++t) w.q[t][i] = *reinterpret_cast<const u32x4_t*>(wl[t] + (size_t)ch * 256);
+    }
+#pragma unroll
+    for (int i = 0; i < SPS; ++i) {
+      const size_t at = (size_t)min(step * GPS + 4 * i + (GPS < 4 ? kq % GPS : kq), KG - 1) * npad;
+#pragma unroll
+      for (int t = 0; t < CT; ++t) {
+        w.s[t][i] = sl[at + 16 * t];
+        w.b[t][i] = bl[at + 16 * t];
+      }
+    }
+  };
+  // this thread's pieces of the activation tile: piece tid + j THREADS = (row q / PPR, 16 bytes q % PPR)
+  const int ach = (tid % PPR) * 8, arow = tid / PPR;
+  const uint16_t* asrc[PPT];
+#pragma unroll
+  for (int j = 0; j < PPT; ++j) {
+    const int r = arow + j * (T::THREADS / PPR);
+    asrc[j] = X + (size_t)(m0 + (r < cnt ? r : 0)) * ldx;
+  }
+  auto load_a = [&](int step, uint4 (&v)[PPT]) {
+    const int k = min(step * STEP + ach, K - 8);
+#pragma unroll
+    for (int j = 0; j < PPT; ++j) v[j] = *reinterpret_cast<const uint4*>(asrc[j] + k);
+  };
+  auto store_a = [&](int step, int buf, uint4 (&v)[PPT]) {
+    if ((step + 1) * STEP > K) {                                 // inputs past a ragged end count as zeros
+#pragma unroll
+      for (int j = 0; j < PPT; ++j)
+        if (step * STEP + ach >= K) v[j] = make_uint4(0u, 0u, 0u, 0u);
+    }
+#pragma unroll
+    for (int j = 0; j < PPT; ++j)
+      *reinterpret_cast<uint4*>(smem + buf * (T::BM * T::ROW) + (arow + j * (T::THREADS / PPR)) * T::ROW + ach * 2) =
+          AR ? stage8_bf16(v[j]) : stage8(v[j]);
+  };
+
+  f32x4_t acc[RT][CT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int t = 0; t < CT; ++t) acc[r][t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  uint4 a[2][PPT];
+  Words w[WSETS];
+  load_a(0, a[0]);
+  load_w(0, w[0]);
+  load_a(1, a[1]);
+#pragma unroll
+  for (int u = 1; u < WSETS; ++u) load_w(u, w[u]);
+  store_a(0, 0, a[0]);
+  __syncthreads();
+  // one step from landing set U and LDS stage U & 1
+  auto walk = [&](int step, auto U) __attribute__((always_inline)) {
+    constexpr int u = decltype(U)::value;
+    load_a(step + 2, a[u & 1]);
+    const unsigned char* at = smem + (u & 1) * (T::BM * T::ROW) + (wr * 16 * RT + c) * T::ROW + kq * 16;
+    uint32_t q[CT][4], sb[CT][4];
+    u32x4_t av[2][RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) av[0][r] = *reinterpret_cast<const u32x4_t*>(at + 16 * r * T::ROW);
+#pragma unroll
+    for (int i = 0; i < CPS; ++i) {
+      if (i + 1 < CPS) {
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+          av[(i + 1) & 1][r] = *reinterpret_cast<const u32x4_t*>(at + 16 * r * T::ROW + (i + 1) * 64);
+      }
+      u32x4_t bw[CT];
+#pragma unroll
+      for (int t = 0; t < CT; ++t) {
+        if (i % 4 == 0) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) q[t][j] = w[u].q[t][i / 4][j];
+          across(q[t]);
+        }
+        if (32 * i % (4 * GS) == 0) {
+          // four groups' scales; a group past a ragged end has weights of zero
+          const int sg = 32 * i / (4 * GS);
+          const uint32_t word = (w[u].s[t][sg] & 0xFFFFu) | (w[u].b[t][sg] << 16);
+          uint32_t mine = AR ? word : sb_half2(make_uint2(w[u].s[t][sg], w[u].b[t][sg]));
+          if (step * GPS + 4 * sg + (GPS < 4 ? kq % GPS : kq) >= KG) mine = 0u;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) sb[t][j] = mine;
+          across(sb[t]);
+        }
+        const uint32_t qw = q[t][i % 4], sw = sb[t][32 * i / GS % 4];
+        if constexpr (AR) bw[t] = __builtin_bit_cast(u32x4_t, dequant8b(qw, sw));
+        else bw[t] = __builtin_bit_cast(u32x4_t, dequant8h(qw, sw));
+      }
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int t = 0; t < CT; ++t) {
+          if constexpr (AR)
+            acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, bw[t]),
+                                                                __builtin_bit_cast(bf16x8_t, av[i & 1][r]), acc[r][t], 0, 0, 0);
+          else
+            acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, bw[t]),
+                                                               __builtin_bit_cast(f16x8_t, av[i & 1][r]), acc[r][t], 0, 0, 0);
+        }
+    }
+    load_w(step + WSETS, w[u]);
+    store_a(step + 1, 1 - (u & 1), a[1 - (u & 1)]);
+    __syncthreads();
+  };
+  int step = 0;
+  for (; step + WSETS <= steps; step += WSETS) {
+    walk(step, std::integral_constant<int, 0>());
+    walk(step + 1, std::integral_constant<int, 1>());
+    walk(step + 2, std::integral_constant<int, 2>());
+    walk(step + 3, std::integral_constant<int, 3>());
+  }
+  if (step < steps) walk(step, std::integral_constant<int, 0>());
+  if (step + 1 < steps) walk(step + 1, std::integral_constant<int, 1>());
+  if (step + 2 < steps) walk(step + 2, std::integral_constant<int, 2>());
+  // a lane holds row 16 r + c, columns 16 t + 4 kq + (0..3) of each 16 x 16 tile
+  const bool whole = N % 4 == 0;
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    const int row = (wr * RT + r) * 16 + c;
+    if (row >= cnt) continue;
+#pragma unroll
+    for (int t = 0; t < CT; ++t) {
+      const int col = col0 + 16 * t + 4 * kq;
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = acc[r][t][i] * (AR ? 1.f : WUNSCALE);
+      store4<EPI>(out, (size_t)(m0 + row) * N + col, v, v, 0.f, N - col, whole);
+    }
+  }
+}
+
 template <int RT>
 constexpr size_t stage_bytes() {
   return 2 * (size_t)(16 * RT) * AROW;
@@ -1112,7 +1315,7 @@ int launch_experts_prefill(int tile, int arith, const uint16_t* x, int64_t x_str
   return 0;
 }
 
-// tile: 0 = chosen from the row count; 1, 4, 8 = the four-wave kernel on 16, 64 or 128 rows a workgroup; 9 = the
+// tile: 0 = chosen from the rows and columns; 1, 4, 8 = the four-wave kernel on 16, 64 or 128 rows a workgroup; 9 = the
 // eight-wave kernel (128 rows x 512 columns; K in whole steps of 64).  The same bits whatever the tile.
 template <int GS, int EPI>
 int launch_qmm_prefill(int arith, int tile, const uint16_t* x, int64_t ldx, const uint32_t* w, const uint16_t* s,
@@ -1125,7 +1328,39 @@ int launch_qmm_prefill(int arith, int tile, const uint16_t* x, int64_t ldx, cons
   TF_REQUIRE((int64_t)((m + 15) / 16) * ct <= 0x7FFFFFFF, "qmm_prefill: grid too large");
   const bool big_ok = (kg * GS) % KSTEP == 0 && (int64_t)npad * kg * GS / 2 < (1ll << 32);
   TF_REQUIRE(tile != 9 || big_ok, "qmm_prefill: tile 9 (the eight-wave kernel) takes K in whole steps of 64");
-  const int rows = tile == 1 ? 16 : tile == 4 ? 64 : tile == 8 ? 128 : tile == 9 ? 129 : m;     // as if this many rows
+#define TF_SHORT(T_, RT_, CT_, WR_, WC_, STEP_)                                                                      \
+  {                                                                                                                \
+    const int ctn = (n + T_::BN - 1) / T_::BN, mtn = (m + T_::BM - 1) / T_::BM;                                    \
+    const int64_t grid = n > 4 * (int64_t)m ? (int64_t)short_pad(ctn) * mtn : (int64_t)short_pad(mtn) * ctn;       \
+    TF_REQUIRE(grid <= 0x7FFFFFFF, "qmm_prefill: grid too large");                                                 \
+    if (arith)                                                                                                     \
+      qmm_prefill_short_kernel<GS, EPI, 1, RT_, CT_, WR_, WC_, STEP_><<<(unsigned)grid, T_::THREADS, T_::LDS, st>>>( \
+          x, ldx, w, s, b, out, m, n, kg, npad);                                                                   \
+    else                                                                                                           \
+      qmm_prefill_short_kernel<GS, EPI, 0, RT_, CT_, WR_, WC_, STEP_><<<(unsigned)grid, T_::THREADS, T_::LDS, st>>>( \
+          x, ldx, w, s, b, out, m, n, kg, npad);                                                                   \
+    TF_LAUNCH_OK("tf_qmm_prefill");                                                                                \
+    return 0;                                                                                                      \
+  }
+  if (tile == 0) {
+    // A call's time is about a start plus a cost a round of 256 workgroups, in the same unit per input of K (half
+    // microseconds at K = 4096; measured on 17 to 4,096 rows x 512 to 17,408 columns): the least of them is taken.
+    // 17 rows x 4096 x 4096 82.9 -> 12.9 us, 100 rows 86.3 -> 14.4 (32 x 64), 512 rows 89 -> 33 (32 x 128),
+    // 1,000 rows 89 -> 53 (64 x 128); at 2,000 rows the eight-wave kernel's 95.7 is the best again (64 x 128 98.5).
+    auto rounds = [](int64_t workgroups) { return (workgroups + 255) / 256; };
+    const int64_t t16 = 12 + 12 * rounds(Short16::workgroups(m, n)), t32 = 14 + 17 * rounds(Short32::workgroups(m, n)),
+                  t32w = 16 + 26 * rounds(Short32Wide::workgroups(m, n)),
+                  t64 = 32 + 40 * rounds(Short64::workgroups(m, n));
+    const int64_t least = std::min(std::min(t16, t32), std::min(t32w, t64));
+    const int64_t big = 10 + 170 * rounds((int64_t)((m + BIG_ROWS - 1) / BIG_ROWS) * ((n + 511) / 512));
+    if (!big_ok || least < big) {
+      if (least == t16) TF_SHORT(Short16, 1, 1, 1, 4, 256)
+      if (least == t32) TF_SHORT(Short32, 2, 1, 1, 4, 256)
+      if (least == t32w) TF_SHORT(Short32Wide, 2, 1, 1, 8, 256)
+      TF_SHORT(Short64, 4, 2, 1, 4, 128)
+    }
+  }
+  const int rows = tile == 1 ? 16 : tile == 4 ? 64 : tile == 8 ? 128 : 129;     // as if this many rows
   if (rows <= 16) {
     if (arith) TF_SMALL(1, 1);
     else TF_SMALL(1, 0);
@@ -1144,6 +1379,7 @@ int launch_qmm_prefill(int arith, int tile, const uint16_t* x, int64_t ldx, cons
     TF_SMALL(8, 0);
   }
 #undef TF_SMALL
+#undef TF_SHORT
   TF_LAUNCH_OK("tf_qmm_prefill");
   return 0;
 }

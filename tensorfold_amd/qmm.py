@@ -288,9 +288,10 @@ def matmul_group(x: torch.Tensor, qs: list[Q4], xs: torch.Tensor | None = None, 
 
 
 def prompt_tile(m: int, n: int, k: int = 64) -> int:
-    """The prompt matmul's tile for ``m`` rows (cuda/kernels/qmm.py:202-205 names the reference's one tile, tuned for
-    its chip): 1, 4 or 8 = a four-wave workgroup on 16, 64 or 128 rows x 128 columns; 9 = eight waves on 128 rows x
-    512 columns, from 65 rows on, for K in whole steps of 64.  What ``tile=0`` picks."""
+    """A tile code of the prompt matmul by the row count (cuda/kernels/qmm.py:202-205 names the reference's one tile,
+    tuned for its chip): 1, 4 or 8 = a four-wave workgroup on 16, 64 or 128 rows x 128 columns; 9 = eight waves on 128
+    rows x 512 columns, from 65 rows on, for K in whole steps of 64.  ``tile=0`` looks at the columns too and has
+    smaller tiles for what would leave compute units idle (the bits are the same)."""
 
     if m <= 16:
         return 1

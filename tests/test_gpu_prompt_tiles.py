@@ -1,0 +1,42 @@
+"""The prompt matmul's own choice of tile against one kernel asked for by name: the same bits over odd rows, columns
+and ragged K, both arithmetics, both result types, rows with a stride."""
+
+import pytest
+import torch
+
+from tensorfold_amd import qmm, synthetic
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+# (rows, columns, K, group size): each tile the choice has, its row and column edges, one step and less of K, a step
+# that ends inside (K = 32, 96, 736, 1056 are not whole steps of 128 or 256), more columns than rows and the reverse
+SHAPES = [(1, 1, 32, 32), (3, 130, 64, 64), (16, 4096, 96, 32), (17, 640, 256, 64), (33, 1024, 736, 32),
+          (100, 4096, 1056, 32), (129, 515, 320, 64), (257, 4100, 448, 64), (300, 8192, 512, 64),
+          (1000, 2047, 192, 64), (1030, 4096, 544, 32), (2000, 130, 96, 32), (4096, 513, 64, 64)]
+
+
+@pytest.mark.parametrize("m,n,k,gs", SHAPES)
+def test_the_chosen_tile_has_the_bits_of_the_others(m, n, k, gs):
+    q = qmm.pack(*(t.to(DEV) for t in synthetic.affine_general(n, k, gs, 7 * n + k)), gs)
+    wide = synthetic.activations(m, k + 8, m + n).to(DEV)
+    for x in (wide[:, :k].contiguous(), wide[:, :k]):
+        for arith in (0, 1):
+            for f32 in (False, True):
+                got = qmm.prefill_matmul(x, q, f32=f32, arith=arith)
+                assert torch.equal(got, qmm.prefill_matmul(x, q, f32=f32, arith=arith, tile=8)), (arith, f32)
+
+
+def test_a_rows_infinity_stays_in_its_row_at_a_ragged_end():
+    """The inputs past a ragged K count as nothing, also next to an infinity in the last piece of a row."""
+
+    n, k, gs = 200, 96, 32
+    q = qmm.pack(*(t.to(DEV) for t in synthetic.affine_general(n, k, gs, 5)), gs)
+    x = synthetic.activations(40, k, 6).to(DEV)
+    want = qmm.prefill_matmul(x, q, f32=True, arith=1)
+    x[7, k - 1] = float("inf")
+    got = qmm.prefill_matmul(x, q, f32=True, arith=1)
+    others = [r for r in range(40) if r != 7]
+    assert torch.equal(got[others], want[others])
+    assert torch.equal(got[7].isnan(), qmm.prefill_matmul(x, q, f32=True, arith=1, tile=8)[7].isnan())
