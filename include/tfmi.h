@@ -56,8 +56,8 @@ int tf_qmm_unpack(const uint32_t* weight, const uint16_t* scales_t, const uint16
 int tf_group_sums(const uint16_t* x, int64_t ldx, int m, int k, int gs, float* xs, tf_stream_t stream);
 /* Decode-form matmul: per group in order acc = fma(xs, b, fma(P, s, acc)), P = sum x*q with exact q; K in `sk`
  * slices summed in slice order; one rounding to bf16 (or fp32 with f32).  `part` fp32 [sk, m, n] is required when
- * sk > 1 (with reduce == 0 the slices are left there unadded; with few rows and reduce != 0 the slices are added
- * inside the one launch, in the same order, and `part` goes unused).  sb_stride = elements between scale rows
+ * sk > 1 (with reduce == 0 the slices are left there unadded).  `bm` (16, 32 or 64) is a row tile: a workgroup takes 16
+ * rows of a call of up to 16 and 32 of a longer one, whatever it says.  sb_stride = elements between scale rows
  * (>= npad).  `counters` (may be NULL): n_counters arrival counters of the weight, TF_QMM_COUNTER_STRIDE ints apart,
  * zero on entry and left zero; with one for every column tile of 64, the slices of up to eight rows are added up in the
  * matmul's own launch by the last workgroup of a tile to finish (same order, same bits);

@@ -1,22 +1,22 @@
 // Decode-form 4-bit matmuls for 1..16 rows an item: the routed-expert GEMV (tf_experts_run) and the dense lane
 // matmul (tf_qmm), plus tf_group_sums.  HBM-bound: one pass over the packed weights.
 //
-// Mapping.  A lane owns one output column and walks K; the 64 lanes of a wave read 1 KB of codes with one
+// Mapping of the experts' GEMV (the dense matmul's is with it below).  A lane owns one output column and walks K; the 64 lanes of a wave read 1 KB of codes with one
 // 16-byte load each (a chunk: 32 inputs x 64 columns).  The activations of the item's rows are the same for every
 // lane: each lane loads dword (lane % 16) of the chunk (one coalesced 64-byte read, fetched with the weights,
 // DEPTH groups ahead) and v_dot2c_f32_bf16's DPP form broadcasts dword j across each row of 16 lanes inside the
 // multiply itself (row_newbcast:j), so there is no cross-lane reduction, no scalar-cache traffic and no LDS
 // traffic in the inner loop.
 //
-// K is cut into SLICES fixed slices (a function of the shape alone).  A workgroup's waves each walk a run of
+// The experts' K is cut into SLICES fixed slices (a function of the shape alone).  A workgroup's waves each walk a run of
 // consecutive slices, park each slice's fp32 sum in LDS, and the sums are added in slice order; how many waves
 // share the slices (16, 8 or 4, picked from the launch size) therefore never changes a bit, and neither do the
 // other rows of the call.
 //
 // Arithmetic per group, as the reference's decode form (experts.cu:94-106, qmm.cu:66-76):
 //   acc = fma(xs, b, fma(P, s, acc)),   P = sum x * q,   xs = sum x
-// with q exact: a nibble OR-ed into the bf16 pattern of 128 is 128 + q, so the dot product gives P + 128 xs and
-// P = fma(-128, xs, that).
+// with q exact.  For the experts a nibble OR-ed into the bf16 pattern of 128 is 128 + q, so the dot product gives
+// P + 128 xs and P = fma(-128, xs, that).
 
 #include <cstdlib>
 #include <mutex>
@@ -72,44 +72,167 @@ __global__ void __launch_bounds__(WAVES * 64)
 
 // ---- dense lane matmul ---------------------------------------------------------------------------------------------
 
-constexpr int QRB = 8;          // rows a pass of the dense split kernels (the one-launch form keeps pairs)
+//
+// A wave takes 64 columns and a run of groups; up to 16 RT rows of the call are the rows of v_mfma_f32_16x16x32_bf16, so
+// a weight is unpacked once for all of them (rows are independent there: a row's bits do not depend on the others, on
+// RT or on the row tile).  Lane L loads column L's four words of a chunk with one 16-byte load and its scale and bias,
+// which change lanes by the lane swaps (`across`) to where the matrix instruction wants them.  A nibble in a byte is
+// the e4m3 number q * 2^-9, so v_cvt_scalef32_pk_bf16_fp8 with scale 2^9 makes the operand's bf16 pair, exactly q.  The
+// first form made vector dot products of 8 rows a pass and was bound by them: 21 rows x 17408 x 5120 72 -> 28 us
+// with its reduce, 64 rows 178 -> 50, 8 rows 31 -> 20, one row 16 as before, and eight times closer to 64 bits (8e-7 ->
+// 1e-7 relative: the codes no longer ride on 128, whose part was taken off again).
 
-struct NoFlush {
-  template <class A>
-  __device__ __forceinline__ void operator()(int, A&) const {}
+// one packed word -> eight bf16 codes, inputs in the order (0, 4, 1, 5, 2, 6, 3, 7)
+__device__ __forceinline__ bf16x8_t codes8(uint32_t w) {
+  const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
+  const u32x4_t r = {__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.f, false)),
+                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.f, true)),
+                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.f, false)),
+                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.f, true))};
+  return __builtin_bit_cast(bf16x8_t, r);
+}
+
+// lane I of the reader's row of 16 lanes
+template <int I>
+__device__ __forceinline__ float row16_lane(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + I, 0xF, 0xF, true));
+}
+
+constexpr int QPART = 68;          // floats of a row of a wave's 64 parked sums: padded against bank conflicts
+
+// LDS floats of a workgroup
+constexpr size_t qmm_lds_floats(int waves, int rt) { return (size_t)waves * 16 * rt * QPART; }
+
+// A group in registers: the lane's column's codes, scale and bias; of row tile r the lane's eight inputs of each chunk
+// (row 16 r + row_of(c), inputs 8 kq ..) and the group sum of row 16 r + kq + 4 (c % NI).
+template <int GS, int RT>
+struct DenseStage {
+  uint4 w[GS / 32], x[RT][GS / 32];
+  uint32_t s, b;
+  float xs[RT];
 };
 
-// One pass of a row tile: RB rows r0 .. r0 + RB - 1 against the workgroup's 64 columns and K slice.
-template <int GS, int WAVES, int RB, bool COH, class WQ, class SB>
-__device__ __forceinline__ void qmm_pass(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
-                                         const WQ& wq, const SB& sb, int r0, int tile, int slice, int gs0, int per,
-                                         int g0, int g1, void* __restrict__ out, float* __restrict__ part_out, int M,
-                                         int N, int KG, int SK, int f32, float* xs, float* part,
-                                         Stage<GS, 1, QRB> (&st)[DEPTH], bool loaded, int valid) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint32_t* xl[RB];
-  const_u32_ptr xsr[RB];
+// grid (column tiles of 64 x row tiles of 16 RT, 1, SK).  Slice z takes groups [z * per, (z + 1) * per), its waves
+// split them again (added in wave order); SK > 1 leaves the slice's fp32 sums in part[z].
+// A lane ends with four of the matrix instruction's rows: 4 kq + (0..3).  The call's row p is put into row
+// 4 (p % 4) + p / 4, so that up to four rows fill the lanes' first results and up to eight the first two: a call of at
+// most 4 NI rows adds NI results up a lane, not four (17408 x 5120, one row: 17.9 -> 16.3 us).
+template <int GS, int WAVES, int RT, int NI, bool COH = false>
+__device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
+                                          const uint32_t* __restrict__ W, const uint16_t* __restrict__ S,
+                                          const uint16_t* __restrict__ B, int64_t sb_stride, void* __restrict__ out,
+                                          float* __restrict__ part_out, int M, int N, int KG, int SK, int f32, int block,
+                                          int slice, float* part) {
+  constexpr int CH = GS / 32, ROWS = 16 * RT;
+  const int tiles = (N + 63) >> 6, tile = block % tiles, r0 = block / tiles * ROWS, valid = min(ROWS, M - r0);
+  const int per = KG / SK, gs0 = slice * per;
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  static_assert(RT == 1 || NI == 4, "more than 16 rows need every result");
+  const uint32_t* wt = W + ((size_t)tile * KG) * (size_t)(CH * 256);
+  const uint32_t wo = lane * 4, co = tile * 64 + lane;
+  const uint16_t* xl[RT];
+  const float* xsl[RT];
 #pragma unroll
-  for (int r = 0; r < RB; ++r) {
-    const int row = r0 + (r < valid ? r : valid - 1);          // a pass past the last row walks that row again, unstored
-    xl[r] = reinterpret_cast<const uint32_t*>(X + (size_t)row * ldx) + (lane & 15);
-    xsr[r] = as_const(XS + (size_t)row * KG);
+  for (int r = 0; r < RT; ++r) {          // rows past the last are the last one again, unstored
+    xl[r] = X + (size_t)(r0 + min(16 * r + (c >> 2) + 4 * (c & 3), valid - 1)) * ldx + 8 * kq;
+    xsl[r] = XS + (size_t)(r0 + min(16 * r + kq + 4 * (c & (NI - 1)), valid - 1)) * KG;
   }
-  __syncthreads();                                  // the previous pass is done with part
-  float acc[1][RB];
+  float acc[RT][4][NI];
 #pragma unroll
-  for (int r = 0; r < RB; ++r) acc[0][r] = 0.f;
-  NoFlush none;
-  auto xsum = [&](int r, int g) { return __uint_as_float(xsr[r][g]); };
-  gemv_stream<GS, 1, RB, 0>(acc, st, loaded, wq, sb, xl, xsum, g0, g1, none);
+  for (int r = 0; r < RT; ++r)
 #pragma unroll
-  for (int r = 0; r < RB; ++r) part[(wave * RB + r) * 64 + lane] = acc[0][r];
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < NI; ++i) acc[r][t][i] = 0.f;
+  typedef DenseStage<GS, RT> Stg;
+  auto load = [&](Stg& st, int g) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < CH; ++i) st.w[i] = ldg16(wt + ((size_t)g * CH + i) * 256 + wo);
+    st.s = (S + (size_t)g * sb_stride)[co];
+    st.b = (B + (size_t)g * sb_stride)[co];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+#pragma unroll
+      for (int i = 0; i < CH; ++i) st.x[r][i] = *reinterpret_cast<const uint4*>(xl[r] + (size_t)g * GS + 32 * i);
+      st.xs[r] = xsl[r][g];
+    }
+    // With one row tile a stage's requests stay apart from the next's: left alone, the compiler merges the stages' group
+    // sums into one load, which arrives with the last stage.  (Two row tiles: 30.2 us so where 28.4 without.)
+    if constexpr (RT == 1) asm volatile("" ::: "memory");
+  };
+  auto add = [&](const Stg& st) __attribute__((always_inline)) {
+    f32x4_t p[RT][4];
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      uint32_t w[4] = {st.w[i].x, st.w[i].y, st.w[i].z, st.w[i].w};
+      across(w);
+      bf16x8_t xa[RT];
+#pragma unroll
+      for (int r = 0; r < RT; ++r) xa[r] = __builtin_bit_cast(bf16x8_t, stage8_bf16(st.x[r][i]));
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const bf16x8_t q = codes8(w[t]);
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+          p[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[r], q, i ? p[r][t] : (f32x4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      }
+    }
+    uint32_t sb[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) sb[t] = (st.s & 0xFFFFu) | (st.b << 16);
+    across(sb);
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      float sc[NI];
+      if constexpr (NI == 1) sc[0] = st.xs[r];
+      if constexpr (NI > 1) sc[0] = row16_lane<0>(st.xs[r]), sc[1] = row16_lane<1>(st.xs[r]);
+      if constexpr (NI > 2) sc[2] = row16_lane<2>(st.xs[r]), sc[3] = row16_lane<3>(st.xs[r]);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+          acc[r][t][i] = fmaf(sc[i], bf16_hi(sb[t]), fmaf(p[r][t][i], bf16_lo(sb[t]), acc[r][t][i]));
+    }
+  };
+  Stg st[DEPTH];
+  int g = gs0 + (int)((long long)wave * per / WAVES);
+  const int g1 = gs0 + (int)((long long)(wave + 1) * per / WAVES);
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d)
+    if (g + d < g1) load(st[d], g + d);
+  const int n = g1 - g;
+  for (; g + 2 * DEPTH <= g1; g += DEPTH) {
+    prio_by_progress(g1 - g, n);
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      add(st[d]);
+      load(st[d], g + DEPTH + d);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d)
+    if (g + d < g1) {
+      add(st[d]);
+      if (g + DEPTH + d < g1) load(st[d], g + DEPTH + d);
+    }
+#pragma unroll
+  for (int d = 0; d < DEPTH - 1; ++d)
+    if (g + DEPTH + d < g1) add(st[d]);
+  // result i of tile (r, t): row 16 r + kq + 4 i, column 16 t + c
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < NI; ++i) part[(wave * ROWS + 16 * r + kq + 4 * i) * QPART + 16 * t + c] = acc[r][t][i];
   __syncthreads();
   for (int o = tid; o < valid * 64; o += WAVES * 64) {
     const int r = o >> 6, l = o & 63, cc = tile * 64 + l;
     if (cc >= N) continue;
-    float s = part[r * 64 + l];
-    for (int w = 1; w < WAVES; ++w) s += part[(w * RB + r) * 64 + l];
+    float s = part[r * QPART + l];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) s += part[(w * ROWS + r) * QPART + l];
     const size_t at = (size_t)(r0 + r) * N + cc;
     if (SK > 1) {
       // COH: another workgroup adds the slices up in this launch: the store goes through to where it can read it
@@ -120,87 +243,37 @@ __device__ __forceinline__ void qmm_pass(const uint16_t* __restrict__ X, int64_t
   }
 }
 
-// grid (column tiles of 64 x row tiles of BM, 1, SK).  Slice z takes groups [z * per, (z + 1) * per), its waves
-// split them again (added in wave order); SK > 1 leaves the slice's fp32 sums in part[z].  Rows go in passes of 8, 4,
-// 2 or 1 (a row's arithmetic is the same in each: what a pass shares is the unpacked weights); 5 to 7 rows take the
-// pass of 8 and 3 rows the pass of 4, rather than two passes over the weights.
-template <int GS, int WAVES, bool COH = false>
-__device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
-                                          const uint32_t* __restrict__ W, const uint16_t* __restrict__ S,
-                                          const uint16_t* __restrict__ B, int64_t sb_stride, void* __restrict__ out,
-                                          float* __restrict__ part_out, int M, int N, int KG, int SK, int BM, int f32,
-                                          int block, int slice, float* lds) {
-  const int tiles = (N + 63) >> 6;
-  const int tile = block % tiles, rt = block / tiles;
-  const int per = KG / SK, gs0 = slice * per;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  constexpr int CH = GS / 32;
-  const uint32_t* wbase = W + ((size_t)tile * KG) * (size_t)(CH * 256) + lane * 4;
-  const int col = tile * 64 + lane;
-  auto wq = [&](int g, int m, int i) { return ldg16(wbase + ((size_t)g * CH + i) * 256); };
-  auto sb = [&](int g, int m, uint32_t& s, uint32_t& b) {
-    s = S[(size_t)g * sb_stride + col];
-    b = B[(size_t)g * sb_stride + col];
-  };
-  const int g0 = gs0 + (int)((long long)wave * per / WAVES), g1 = gs0 + (int)((long long)(wave + 1) * per / WAVES);
-  float* xs = nullptr;
-  float* part = lds;
-  const int m_end = min(M, (rt + 1) * BM);
-  int r0 = rt * BM;
-  Stage<GS, 1, QRB> st[DEPTH];
-#pragma unroll
-  for (int d = 0; d < DEPTH; ++d)
-    if (g0 + d < g1) load_weights<GS, 1>(st[d], wq, sb, g0 + d);
-  bool loaded = true;
-#define TF_QMM_PASS(RB_)                                                                                             \
-  {                                                                                                                  \
-    const int valid = min(RB_, m_end - r0);                                                                          \
-    qmm_pass<GS, WAVES, RB_, COH>(X, ldx, XS, wq, sb, r0, tile, slice, gs0, per, g0, g1, out, part_out, M, N, KG, SK, \
-                                  f32, xs, part, st, loaded, valid);                                                 \
-    loaded = g1 - g0 <= DEPTH;                                                                                       \
-    r0 += valid;                                                                                                     \
-  }
-  while (m_end - r0 >= 5) TF_QMM_PASS(8)
-  if (m_end - r0 >= 3) TF_QMM_PASS(4)
-  if (m_end - r0 == 2) TF_QMM_PASS(2)
-  if (m_end - r0 == 1) TF_QMM_PASS(1)
-#undef TF_QMM_PASS
-}
-
-template <int GS, int WAVES>
+template <int GS, int WAVES, int RT, int NI>
 __global__ void __launch_bounds__(WAVES * 64)
     qmm_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
                const uint32_t* __restrict__ W, const uint16_t* __restrict__ S, const uint16_t* __restrict__ B,
                int64_t sb_stride, void* __restrict__ out, float* __restrict__ part_out, int M, int N, int KG, int SK,
-               int BM, int f32) {
-  extern __shared__ float lds[];            // partials [WAVES][QRB][64]
-  qmm_block<GS, WAVES>(X, ldx, XS, W, S, B, sb_stride, out, part_out, M, N, KG, SK, BM, f32, blockIdx.x, blockIdx.z, lds);
+               int f32) {
+  extern __shared__ float lds[];
+  qmm_block<GS, WAVES, RT, NI>(X, ldx, XS, W, S, B, sb_stride, out, part_out, M, N, KG, SK, f32, blockIdx.x, blockIdx.z,
+                               lds);
 }
 
-// The split matmul with its reduce in the same launch: a slice's workgroup leaves its sums in part[z] with stores
-// that go through to memory, waits for them to be acknowledged and counts itself in at the (column tile, row tile)'s
-// counter; the workgroup that finds the others there adds the slices in slice order (qmm_reduce_kernel's arithmetic)
-// and puts the counter back to zero.  A thousand short workgroups fill the chip where the one-launch form above has
-// one workgroup a column tile.
+// The split matmul of up to eight rows with its reduce in the same launch: a slice's workgroup leaves its sums in
+// part[z] with stores that go through to memory, waits for them to be acknowledged and counts itself in at the column
+// tile's counter; the workgroup that finds the others there adds the slices in slice order (qmm_reduce_kernel's
+// arithmetic) and puts the counter back to zero.
 // What a slice's workgroup does once its sums are in part[z] (stored through to memory): wait for the stores'
 // acknowledgement, count itself in at the tile's counter, and if every other slice is there already add them up.
 template <int WAVES>
 __device__ __forceinline__ void qmm_arrive_tail(int* __restrict__ counter, const float* __restrict__ part_out,
-                                                void* __restrict__ out, int M, int N, int SK, int BM, int f32, int block,
-                                                int* last) {
+                                                void* __restrict__ out, int M, int N, int SK, int f32, int tile, int* last) {
   __builtin_amdgcn_s_waitcnt(0);        // this wave's stores are acknowledged ...
   __syncthreads();                      // ... every wave's are ...
   if (threadIdx.x == 0)                 // ... then the workgroup counts itself in
     *last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == SK - 1;
   __syncthreads();
   if (!*last) return;
-  const int tiles = (N + 63) >> 6, tile = block % tiles, rt = block / tiles;
-  const int r_first = rt * BM, rows = min(M, r_first + BM) - r_first;
   const long long total = (long long)M * N;
-  for (int o = threadIdx.x; o < rows * 64; o += WAVES * 64) {
+  for (int o = threadIdx.x; o < M * 64; o += WAVES * 64) {
     const int cc = tile * 64 + (o & 63);
     if (cc >= N) continue;
-    const size_t at = (size_t)(r_first + (o >> 6)) * N + cc;
+    const size_t at = (size_t)(o >> 6) * N + cc;
     // eight slices' loads go out together, then the sums in slice order
     float acc = 0.f;
     for (int z0 = 0; z0 < SK; z0 += 8) {
@@ -219,123 +292,18 @@ __device__ __forceinline__ void qmm_arrive_tail(int* __restrict__ counter, const
   if (threadIdx.x == 0) *counter = 0;   // every slice of the tile has arrived: ready for the next call
 }
 
-template <int GS, int WAVES>
+template <int GS, int WAVES, int NI>
 __global__ void __launch_bounds__(WAVES * 64)
     qmm_arrive_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
                       const uint32_t* __restrict__ W, const uint16_t* __restrict__ S, const uint16_t* __restrict__ B,
                       int64_t sb_stride, void* __restrict__ out, float* __restrict__ part_out, int* __restrict__ counters,
-                      int M, int N, int KG, int SK, int BM, int f32) {
+                      int M, int N, int KG, int SK, int f32) {
   extern __shared__ float lds[];
   __shared__ int last;
-  qmm_block<GS, WAVES, true>(X, ldx, XS, W, S, B, sb_stride, out, part_out, M, N, KG, SK, BM, f32, blockIdx.x, blockIdx.z, lds);
-  qmm_arrive_tail<WAVES>(counters + (size_t)blockIdx.x * TF_QMM_COUNTER_STRIDE, part_out, out, M, N, SK, BM, f32,
-                         blockIdx.x, &last);
-}
-
-// The split matmul and its reduce in ONE launch, with no traffic between workgroups: a workgroup of FW waves takes a
-// (column tile, row tile) with ALL of K.  The 4 * SK sub-slices (SK slices x the 4 waves qmm_kernel runs a slice on)
-// keep their boundaries; wave w streams 4 * SK / FW consecutive ones, parking each sum in LDS, and the end adds a
-// slice's four in wave order, then the slices in slice order: the arithmetic, and so the bits, of qmm_kernel followed
-// by qmm_reduce_kernel.  The same waves are in flight as in the split launch; only the grouping differs.
-template <int GS, int FW, int RB, class WQ, class SB>
-__device__ __forceinline__ void qmm_fat_pass(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
-                                             const WQ& wq, const SB& sb, int r0, int tile, int per, int SK, int gA,
-                                             int gB, void* __restrict__ out, int N, int KG, int f32, float* part,
-                                             Stage<GS, 1> (&st)[DEPTH], bool loaded) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int U = 4 * SK, SPW = U / FW;
-  auto sub_begin = [&](int u) { return (u >> 2) * per + (int)((long long)(u & 3) * per / 4); };
-  const uint32_t* xl[RB];
-  const_u32_ptr xsr[RB];
-#pragma unroll
-  for (int r = 0; r < RB; ++r) {
-    xl[r] = reinterpret_cast<const uint32_t*>(X + (size_t)(r0 + r) * ldx) + (lane & 15);
-    xsr[r] = as_const(XS + (size_t)(r0 + r) * KG);
-  }
-  __syncthreads();                                  // the previous pass is done with part
-  if (per < 4) {                                    // sub-slices with no group still take part in the sums: as zeros
-    for (int q = 0; q < SPW; ++q)
-#pragma unroll
-      for (int r = 0; r < RB; ++r) part[((wave * SPW + q) * RB + r) * 64 + lane] = 0.f;
-  }
-  float acc[1][RB];
-#pragma unroll
-  for (int r = 0; r < RB; ++r) acc[0][r] = 0.f;
-  int sub = wave * SPW;
-  const int sub_last = (wave + 1) * SPW;
-  while (sub < sub_last && sub_begin(sub + 1) == sub_begin(sub)) ++sub;
-  int sub_end = sub < sub_last ? sub_begin(sub + 1) : -1;
-  auto flush = [&](int g, float (&a)[1][RB]) {
-    if (g + 1 != sub_end) return;
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-      part[(sub * RB + r) * 64 + lane] = a[0][r];
-      a[0][r] = 0.f;
-    }
-    ++sub;
-    while (sub < sub_last && sub_begin(sub + 1) == sub_begin(sub)) ++sub;
-    sub_end = sub < sub_last ? sub_begin(sub + 1) : -1;
-  };
-  auto xsum = [&](int r, int g) { return __uint_as_float(xsr[r][g]); };
-  gemv_stream<GS, 1, RB, 0>(acc, st, loaded, wq, sb, xl, xsum, gA, gB, flush);
-  __syncthreads();
-  for (int o = tid; o < RB * 64; o += FW * 64) {
-    const int r = o >> 6, l = o & 63, cc = tile * 64 + l;
-    if (cc >= N) continue;
-    float total = 0.f;
-    for (int z = 0; z < SK; ++z) {
-      float t = part[((4 * z) * RB + r) * 64 + l];
-      for (int j = 1; j < 4; ++j) t += part[((4 * z + j) * RB + r) * 64 + l];
-      total = z ? total + t : t;
-    }
-    const size_t at = (size_t)(r0 + r) * N + cc;
-    if (f32) reinterpret_cast<float*>(out)[at] = total;
-    else reinterpret_cast<uint16_t*>(out)[at] = (uint16_t)f32_bf16_bits(total);
-  }
-}
-
-template <int GS, int FW>
-__device__ __forceinline__ void qmm_fat_block(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
-                                              const uint32_t* __restrict__ W, const uint16_t* __restrict__ S,
-                                              const uint16_t* __restrict__ B, int64_t sb_stride,
-                                              void* __restrict__ out, int M, int N, int KG, int SK, int BM, int f32,
-                                              int block, float* lds) {
-  const int tiles = (N + 63) >> 6;
-  const int tile = block % tiles, rt = block / tiles;
-  const int per = KG / SK;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  constexpr int CH = GS / 32;
-  const uint32_t* wbase = W + ((size_t)tile * KG) * (size_t)(CH * 256) + lane * 4;
-  const int col = tile * 64 + lane;
-  auto wq = [&](int g, int m, int i) { return ldg16(wbase + ((size_t)g * CH + i) * 256); };
-  auto sb = [&](int g, int m, uint32_t& s, uint32_t& b) {
-    s = S[(size_t)g * sb_stride + col];
-    b = B[(size_t)g * sb_stride + col];
-  };
-  auto sub_begin = [&](int u) { return (u >> 2) * per + (int)((long long)(u & 3) * per / 4); };
-  const int SPW = 4 * SK / FW;
-  const int gA = sub_begin(wave * SPW), gB = sub_begin((wave + 1) * SPW);
-  const int m_end = min(M, (rt + 1) * BM);
-  int r0 = rt * BM;
-  Stage<GS, 1> st[DEPTH];
-#pragma unroll
-  for (int d = 0; d < DEPTH; ++d)
-    if (gA + d < gB) load_weights<GS, 1>(st[d], wq, sb, gA + d);
-  bool loaded = true;
-  for (; r0 + 2 <= m_end; r0 += 2) {
-    qmm_fat_pass<GS, FW, 2>(X, ldx, XS, wq, sb, r0, tile, per, SK, gA, gB, out, N, KG, f32, lds, st, loaded);
-    loaded = gB - gA <= DEPTH;
-  }
-  if (r0 < m_end) qmm_fat_pass<GS, FW, 1>(X, ldx, XS, wq, sb, r0, tile, per, SK, gA, gB, out, N, KG, f32, lds, st, loaded);
-}
-
-template <int GS, int FW>
-__global__ void __launch_bounds__(FW * 64)
-    qmm_fat_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
-                   const uint32_t* __restrict__ W, const uint16_t* __restrict__ S, const uint16_t* __restrict__ B,
-                   int64_t sb_stride, void* __restrict__ out, int M, int N, int KG, int SK, int BM, int f32) {
-  extern __shared__ float lds[];            // sub-slice sums [4 * SK][RBMAX][64]
-  qmm_fat_block<GS, FW>(X, ldx, XS, W, S, B, sb_stride, out, M, N, KG, SK, BM, f32, blockIdx.x, lds);
+  qmm_block<GS, WAVES, 1, NI, true>(X, ldx, XS, W, S, B, sb_stride, out, part_out, M, N, KG, SK, f32, blockIdx.x,
+                                    blockIdx.z, lds);
+  qmm_arrive_tail<WAVES>(counters + (size_t)blockIdx.x * TF_QMM_COUNTER_STRIDE, part_out, out, M, N, SK, f32, blockIdx.x,
+                         &last);
 }
 
 // Up to four weights against one x in one launch (and one reduce launch): workgroups [first[w], first[w + 1]) take
@@ -354,27 +322,26 @@ struct GroupArgs {
   int count;
 };
 
-template <int GS, int WAVES>
+template <int GS, int WAVES, int RT, int NI>
 __global__ void __launch_bounds__(WAVES * 64)
     qmm_group_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS, GroupArgs a, int M,
-                     int KG, int BM, int f32) {
+                     int KG, int f32) {
   extern __shared__ float lds[];
   int w = 0;
 #pragma unroll
   for (int i = 1; i < GROUP_MAX; ++i)
     if (i < a.count && (int)blockIdx.x >= a.first[i]) w = i;
   if ((int)blockIdx.z >= a.sk[w]) return;
-  qmm_block<GS, WAVES>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], a.part[w], M, a.n[w], KG, a.sk[w],
-                       BM, f32, blockIdx.x - a.first[w], blockIdx.z, lds);
+  qmm_block<GS, WAVES, RT, NI>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], a.part[w], M, a.n[w], KG,
+                               a.sk[w], f32, blockIdx.x - a.first[w], blockIdx.z, lds);
 }
 
-// The grouped launch in the one-launch form (see qmm_fat_block): every weight's K split is 4, 8 or 16.
 // the grouped launch whose slices are added up by the last workgroup of a tile to finish (qmm_arrive_kernel's way);
 // a weight whose K is not split stores its rows itself
-template <int GS, int WAVES>
+template <int GS, int WAVES, int NI>
 __global__ void __launch_bounds__(WAVES * 64)
     qmm_group_arrive_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS, GroupArgs a, int M,
-                            int KG, int BM, int f32) {
+                            int KG, int f32) {
   extern __shared__ float lds[];
   __shared__ int last;
   int w = 0;
@@ -383,24 +350,11 @@ __global__ void __launch_bounds__(WAVES * 64)
     if (i < a.count && (int)blockIdx.x >= a.first[i]) w = i;
   if ((int)blockIdx.z >= a.sk[w]) return;
   const int block = blockIdx.x - a.first[w];
-  qmm_block<GS, WAVES, true>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], a.part[w], M, a.n[w], KG,
-                             a.sk[w], BM, f32, block, blockIdx.z, lds);
+  qmm_block<GS, WAVES, 1, NI, true>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], a.part[w], M, a.n[w], KG,
+                                    a.sk[w], f32, block, blockIdx.z, lds);
   if (a.sk[w] > 1)
     qmm_arrive_tail<WAVES>(a.counters[w] + (size_t)block * TF_QMM_COUNTER_STRIDE, a.part[w], a.out[w], M, a.n[w],
-                           a.sk[w], BM, f32, block, &last);
-}
-
-template <int GS>
-__global__ void __launch_bounds__(1024)
-    qmm_group_fat_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS, GroupArgs a, int M,
-                         int KG, int BM, int f32) {
-  extern __shared__ float lds[];
-  int w = 0;
-#pragma unroll
-  for (int i = 1; i < GROUP_MAX; ++i)
-    if (i < a.count && (int)blockIdx.x >= a.first[i]) w = i;
-  qmm_fat_block<GS, 16>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], M, a.n[w], KG, a.sk[w], BM, f32,
-                        blockIdx.x - a.first[w], lds);
+                           a.sk[w], f32, block, &last);
 }
 
 // p[0] + p[stride] + ... (n terms, in that order); eight loads go out together before they are added
@@ -451,8 +405,7 @@ __global__ void __launch_bounds__(256)
 }
 
 constexpr int QMM_WAVES = 4;
-constexpr int FAT_ROWS = 8;          // rows up to which tf_qmm runs the one-launch form
-constexpr int ARRIVE_ROWS = QRB;      // rows up to which, given arrival counters, the split launch adds its own slices
+constexpr int ARRIVE_ROWS = 8;        // rows up to which, given arrival counters, the split launch adds its own slices
 
 // Waves a workgroup of the expert GEMV: few workgroups (a small batch) spread each one's K over 16 waves, many
 // workgroups keep 4 longer-running waves each so that more of them are resident.  Scheduling only: bits do not move.
@@ -579,52 +532,43 @@ static int qmm_launch(const uint16_t* x, int64_t ldx, const float* xs, const uin
   TF_REQUIRE(aligned16(weight), "packed weight must be 16-byte aligned");
   TF_REQUIRE(sk == 1 || part, "part: at least (SK, M, n) fp32 is needed when K is split");
   hipStream_t s = as_stream(stream);
-  const int tiles = (n + 63) / 64, rts = (m + bm - 1) / bm, per = kg / sk;
-  const size_t smem = sizeof(float) * ((size_t)QMM_WAVES * QRB * 64);
+  // up to 16 rows are one row tile of the matrix instruction; past that a workgroup takes two (`bm` is the caller's row
+  // tile: accepted, and no longer what decides)
+  const int rt = m <= 16 ? 1 : 2, tiles = (n + 63) / 64, rts = (m + 16 * rt - 1) / (16 * rt);
+  const size_t smem = sizeof(float) * qmm_lds_floats(QMM_WAVES, rt);
   TF_REQUIRE((int64_t)tiles * rts <= 0x7FFFFFFF && sk <= 65535, "qmm: grid too large");
-  const int64_t fat_blocks = (int64_t)((n + 63) / 64) * ((m + RBMAX - 1) / RBMAX);
   const dim3 grid((unsigned)(tiles * rts), 1, (unsigned)sk);
-  if (reduce && sk > 1 && counters && m <= ARRIVE_ROWS && (int64_t)tiles * rts <= n_counters) {
-    // one pass of rows, and arrival counters: the slices are added up by the last workgroup of a tile to finish.
-    // Hundreds of four-wave workgroups beat the one-launch form's workgroup a column tile and row pair: 4096 x 4096
-    // 6.0 us at 1 row against 7.5, 7.1 at 4 against 8.5 (9.1 against 8.3 at 8, the one shape where that form wins);
-    // 5120 x 17408 at 8 rows 24 against 40
-    if (gs == 64)
-      qmm_arrive_kernel<64, QMM_WAVES><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, weight, scales, biases, sb_stride,
-                                                                           out, part, counters, m, n, kg, sk, bm, f32);
-    else
-      qmm_arrive_kernel<32, QMM_WAVES><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, weight, scales, biases, sb_stride,
-                                                                           out, part, counters, m, n, kg, sk, bm, f32);
-    TF_LAUNCH_OK("tf_qmm");
-    return 0;
-  }
-  if (reduce && (m <= RBMAX || (m <= FAT_ROWS && fat_blocks <= 512)) && (sk == 2 || sk == 4 || sk == 8 || sk == 16)) {
-    // few rows: split and reduce in one launch, a workgroup of 8 or 16 waves taking every slice of a tile for RBMAX
-    // rows in one pass (same bits), while those workgroups fit the chip at once (512 of 16 waves).  Past that, and
-    // with many rows, the split launch is better: its waves keep their one or two groups in registers from pass to
-    // pass.
-    bm = RBMAX;
-    const dim3 fat((unsigned)(tiles * ((m + RBMAX - 1) / RBMAX)));
-    const size_t fat_smem = sizeof(float) * ((size_t)4 * sk * RBMAX * 64);
-#define TF_FAT(GS_, FW_) \
-  qmm_fat_kernel<GS_, FW_><<<fat, FW_ * 64, fat_smem, s>>>(x, ldx, xs, weight, scales, biases, sb_stride, out, m, n, kg, sk, bm, f32)
+  if (reduce && sk > 1 && counters && m <= ARRIVE_ROWS && tiles <= n_counters) {
+    // few rows and arrival counters: the slices are added up by the last workgroup of a tile to finish
+#define TF_GO(GS_, NI_)                                                                                             \
+  qmm_arrive_kernel<GS_, QMM_WAVES, NI_><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, weight, scales, biases, sb_stride, \
+                                                                            out, part, counters, m, n, kg, sk, f32)
     if (gs == 64) {
-      if (sk == 2) TF_FAT(64, 8);
-      else TF_FAT(64, 16);
+      if (m <= 4) TF_GO(64, 1);
+      else TF_GO(64, 2);
     } else {
-      if (sk == 2) TF_FAT(32, 8);
-      else TF_FAT(32, 16);
+      if (m <= 4) TF_GO(32, 1);
+      else TF_GO(32, 2);
     }
-#undef TF_FAT
+#undef TF_GO
     TF_LAUNCH_OK("tf_qmm");
     return 0;
   }
-  if (gs == 64)
-    qmm_kernel<64, QMM_WAVES><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, weight, scales, biases, sb_stride, out,
-                                                                part, m, n, kg, sk, bm, f32);
-  else
-    qmm_kernel<32, QMM_WAVES><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, weight, scales, biases, sb_stride, out,
-                                                                part, m, n, kg, sk, bm, f32);
+#define TF_GO(GS_, RT_, NI_)                                                                                             \
+  qmm_kernel<GS_, QMM_WAVES, RT_, NI_><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, weight, scales, biases, sb_stride, \
+                                                                          out, part, m, n, kg, sk, f32)
+  if (gs == 64) {
+    if (m <= 4) TF_GO(64, 1, 1);
+    else if (m <= 8) TF_GO(64, 1, 2);
+    else if (m <= 16) TF_GO(64, 1, 4);
+    else TF_GO(64, 2, 4);
+  } else {
+    if (m <= 4) TF_GO(32, 1, 1);
+    else if (m <= 8) TF_GO(32, 1, 2);
+    else if (m <= 16) TF_GO(32, 1, 4);
+    else TF_GO(32, 2, 4);
+  }
+#undef TF_GO
   TF_LAUNCH_OK("tf_qmm");
   if (sk > 1 && reduce) {
     const long long total = (long long)m * n;
@@ -712,17 +656,8 @@ extern "C" int tf_qmm_group(const uint16_t* x, int64_t ldx, const float* xs, int
   // one pass of rows and every split weight's arrival counters: the arriving form, as tf_qmm
   bool arrive = counters && m <= ARRIVE_ROWS;
   for (int i = 0; i < count && arrive; ++i)
-    arrive = ns && sks && (sks[i] == 1 || (counters[i] && (ns[i] + 63) / 64 * ((m + bm - 1) / bm) <= n_counters[i]));
-  // few rows and every K split 4, 8 or 16: the one-launch form (two rows a workgroup), as tf_qmm
-  bool fat = !arrive && m <= FAT_ROWS;
-  int64_t fat_blocks = 0;
-  for (int i = 0; i < count && fat; ++i) {
-    fat = ns && sks && ns[i] >= 1 && (sks[i] == 4 || sks[i] == 8 || sks[i] == 16);
-    if (fat) fat_blocks += (int64_t)((ns[i] + 63) / 64) * ((m + RBMAX - 1) / RBMAX);
-  }
-  fat = fat && (m <= RBMAX || fat_blocks <= 512);
-  if (fat) bm = RBMAX;
-  const int rts = (m + bm - 1) / bm;
+    arrive = sks[i] == 1 || (counters[i] && (ns[i] + 63) / 64 <= n_counters[i]);
+  const int rt = m <= 16 ? 1 : 2, rts = (m + 16 * rt - 1) / (16 * rt);
   GroupArgs a{}, r{};
   int max_sk = 1;
   int64_t blocks = 0, chunks = 0;
@@ -754,23 +689,36 @@ extern "C" int tf_qmm_group(const uint16_t* x, int64_t ldx, const float* xs, int
   a.count = count;
   a.first[count] = (int)blocks;
   hipStream_t s = as_stream(stream);
-  if (fat) {
-    const size_t fat_smem = sizeof(float) * ((size_t)4 * max_sk * RBMAX * 64);
-    if (gs == 64) qmm_group_fat_kernel<64><<<(unsigned)blocks, 1024, fat_smem, s>>>(x, ldx, xs, a, m, kg, bm, f32);
-    else qmm_group_fat_kernel<32><<<(unsigned)blocks, 1024, fat_smem, s>>>(x, ldx, xs, a, m, kg, bm, f32);
-    TF_LAUNCH_OK("tf_qmm_group");
-    return 0;
-  }
-  const size_t smem = sizeof(float) * ((size_t)QMM_WAVES * QRB * 64);
+  const size_t smem = sizeof(float) * qmm_lds_floats(QMM_WAVES, rt);
   const dim3 grid((unsigned)blocks, 1, (unsigned)max_sk);
   if (arrive) {
-    if (gs == 64) qmm_group_arrive_kernel<64, QMM_WAVES><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, a, m, kg, bm, f32);
-    else qmm_group_arrive_kernel<32, QMM_WAVES><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, a, m, kg, bm, f32);
+#define TF_GO(GS_, NI_) \
+  qmm_group_arrive_kernel<GS_, QMM_WAVES, NI_><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, a, m, kg, f32)
+    if (gs == 64) {
+      if (m <= 4) TF_GO(64, 1);
+      else TF_GO(64, 2);
+    } else {
+      if (m <= 4) TF_GO(32, 1);
+      else TF_GO(32, 2);
+    }
+#undef TF_GO
     TF_LAUNCH_OK("tf_qmm_group");
     return 0;
   }
-  if (gs == 64) qmm_group_kernel<64, QMM_WAVES><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, a, m, kg, bm, f32);
-  else qmm_group_kernel<32, QMM_WAVES><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, a, m, kg, bm, f32);
+#define TF_GO(GS_, RT_, NI_) \
+  qmm_group_kernel<GS_, QMM_WAVES, RT_, NI_><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, a, m, kg, f32)
+  if (gs == 64) {
+    if (m <= 4) TF_GO(64, 1, 1);
+    else if (m <= 8) TF_GO(64, 1, 2);
+    else if (m <= 16) TF_GO(64, 1, 4);
+    else TF_GO(64, 2, 4);
+  } else {
+    if (m <= 4) TF_GO(32, 1, 1);
+    else if (m <= 8) TF_GO(32, 1, 2);
+    else if (m <= 16) TF_GO(32, 1, 4);
+    else TF_GO(32, 2, 4);
+  }
+#undef TF_GO
   TF_LAUNCH_OK("tf_qmm_group");
   if (any_split) {
     int first[GROUP_MAX + 1];

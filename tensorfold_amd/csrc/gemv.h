@@ -1,4 +1,4 @@
-// The decode-form GEMV core shared by the stand-alone expert and lane kernels (decode.hip) and the fused MoE layer
+// The decode-form GEMV core shared by the stand-alone expert kernels (decode.hip) and the fused MoE layer
 // (fused.hip): one wave's streaming loop, the per-item pass with its ordered K-slice sums and epilogues.
 #pragma once
 
@@ -6,12 +6,6 @@
 
 namespace tf {
 namespace {
-
-typedef const __attribute__((address_space(4))) uint32_t* const_u32_ptr;   // constant address space: scalar loads
-
-__device__ __forceinline__ const_u32_ptr as_const(const void* p) {
-  return (const_u32_ptr)(reinterpret_cast<uintptr_t>(p));
-}
 
 __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
@@ -80,18 +74,17 @@ __device__ __forceinline__ float dot2_bcast(float acc, uint32_t x, uint32_t q) {
 
 // A group in registers: the weights of NM matrices (GS/32 16-byte chunks, scale and bias) and, of each of RB rows,
 // the lane's dword of each chunk of the group's inputs.  Scale and bias stay as they were loaded (bf16 bits: the
-// scale in the low half of `s`, the bias in the low half of `b`, or with BHI in its high half) until the group is
-// added: turning them into floats where they are loaded would make the wave wait for every load it has just issued.
-// RBM: the most rows a pass of the kernel holding the stage takes.
-template <int GS, int NM, int RBM = RBMAX>
+// scale in the low half of `s`, the bias in the high half of `b`) until the group is added: turning them into floats
+// where they are loaded would make the wave wait for every load it has just issued.
+template <int GS, int NM>
 struct Stage {
   uint4 w[NM][GS / 32];
   uint32_t s[NM], b[NM];
-  uint32_t x[RBM][GS / 32];
+  uint32_t x[RBMAX][GS / 32];
 };
 
-template <int GS, int NM, int RBM, class WQ, class SB>
-__device__ __forceinline__ void load_weights(Stage<GS, NM, RBM>& st, const WQ& wq, const SB& sb, int g) {
+template <int GS, int NM, class WQ, class SB>
+__device__ __forceinline__ void load_weights(Stage<GS, NM>& st, const WQ& wq, const SB& sb, int g) {
 #pragma unroll
   for (int m = 0; m < NM; ++m) {
 #pragma unroll
@@ -115,8 +108,8 @@ __device__ __forceinline__ float row16_sum(float s) {
 
 // Row r's sum over the staged group, from the dwords the dot products read anyway: a lane adds its two inputs of
 // each chunk in chunk order (a dot product against ones), then the sixteen lanes that share the row add up.
-template <int GS, int NM, int RBM>
-__device__ __forceinline__ float stage_row_sum(const Stage<GS, NM, RBM>& st, int r) {
+template <int GS, int NM>
+__device__ __forceinline__ float stage_row_sum(const Stage<GS, NM>& st, int r) {
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < GS / 32; ++i) s = dot2(st.x[r][i], BF16_ONES, s);
@@ -124,8 +117,8 @@ __device__ __forceinline__ float stage_row_sum(const Stage<GS, NM, RBM>& st, int
 }
 
 // xl[r]: row r's inputs as dwords, already offset by (lane % 16)
-template <int GS, int NM, int RB, int COH, int RBM>
-__device__ __forceinline__ void load_inputs(Stage<GS, NM, RBM>& st, const uint32_t* const (&xl)[RB], int g) {
+template <int GS, int NM, int RB, int COH>
+__device__ __forceinline__ void load_inputs(Stage<GS, NM>& st, const uint32_t* const (&xl)[RB], int g) {
 #pragma unroll
   for (int r = 0; r < RB; ++r)
 #pragma unroll
@@ -150,8 +143,8 @@ __device__ __forceinline__ void word_dot(float (&p)[NM][RB], const uint32_t (&wo
 }
 
 // p += sum over chunk i of x * (128 + q)
-template <int GS, int NM, int RB, int RBM>
-__device__ __forceinline__ void chunk_dot(float (&p)[NM][RB], const Stage<GS, NM, RBM>& st, int i) {
+template <int GS, int NM, int RB>
+__device__ __forceinline__ void chunk_dot(float (&p)[NM][RB], const Stage<GS, NM>& st, int i) {
   const uint32_t magic = BF16_128;
   uint32_t x[RB];
 #pragma unroll
@@ -178,18 +171,16 @@ __device__ __forceinline__ float group_term(float pq, float scale, float sc, flo
 //   wq(g, m, i)     -> the lane's 16 bytes of chunk i of group g of matrix m
 //   sb(g, m, s, b)  -> the lane's column's scale and bias of that group, as loaded (see Stage)
 //   xl[r]           -> row r's inputs as dwords, offset by lane % 16
-//   xsum(r, g)      -> row r's sum over group g (wave-uniform); with XIN the sums are taken from the staged inputs
 //   flush(g, acc)   -> called after group g has been added (wave-uniform); may park and clear acc
-// `st` holds the weights of groups gA .. gA + DEPTH - 1 on entry when `loaded`.
+// The rows' group sums are taken from the staged inputs.  `st` holds the weights of groups gA .. gA + DEPTH - 1 on entry when `loaded`.
 // SEPG: a group's term is rounded by itself, t = fma(xs, b, P s), and added to the running sum (acc + t) instead of
 // being chained through it.  The down projection of the routed experts sums this way, so that a kernel that holds one
 // group of an expert's inputs (the decode layer cut along the intermediate width) can leave t for another workgroup
 // to add and arrive at the same bits.
-template <int GS, int NM, int RB, int COH, bool XIN = false, bool BHI = false, bool SEPG = false, int RBM, class WQ,
-          class SB, class XS, class FLUSH>
-__device__ __forceinline__ void gemv_stream(float (&acc)[NM][RB], Stage<GS, NM, RBM> (&st)[DEPTH], bool loaded,
-                                            const WQ& wq, const SB& sb, const uint32_t* const (&xl)[RB],
-                                            const XS& xsum, int gA, int gB, FLUSH& flush) {
+template <int GS, int NM, int RB, int COH, bool SEPG, class WQ, class SB, class FLUSH>
+__device__ __forceinline__ void gemv_stream(float (&acc)[NM][RB], Stage<GS, NM> (&st)[DEPTH], bool loaded,
+                                            const WQ& wq, const SB& sb, const uint32_t* const (&xl)[RB], int gA, int gB,
+                                            FLUSH& flush) {
   constexpr int CH = GS / 32;
   if (gA >= gB) return;
 #pragma unroll
@@ -220,14 +211,12 @@ __device__ __forceinline__ void gemv_stream(float (&acc)[NM][RB], Stage<GS, NM, 
           for (int r = 0; r < RB; ++r) asm volatile("s_nop 2" : "+v"(p[m][r]));
 #pragma unroll
         for (int r = 0; r < RB; ++r) {
-          float sc;
-          if constexpr (XIN) sc = stage_row_sum<GS, NM>(st[d], r);
-          else sc = xsum(r, g);
+          const float sc = stage_row_sum<GS, NM>(st[d], r);
 #pragma unroll
           for (int m = 0; m < NM; ++m) {
             const float pq = fmaf(-128.f, sc, p[m][r]);
             const float scale = __uint_as_float(st[d].s[m] << 16);
-            const float bias = __uint_as_float(BHI ? st[d].b[m] & 0xFFFF0000u : st[d].b[m] << 16);
+            const float bias = __uint_as_float(st[d].b[m] & 0xFFFF0000u);
             if constexpr (SEPG) acc[m][r] = __fadd_rn(acc[m][r], group_term(pq, scale, sc, bias));
             else acc[m][r] = fmaf(sc, bias, fmaf(pq, scale, acc[m][r]));
           }
@@ -306,10 +295,9 @@ __device__ __forceinline__ void expert_pass(const uint16_t* __restrict__ X, int6
     slice_end = slice < SLICES ? slice_begin(slice + 1, KG) : -1;
   };
   const int gA = slice_begin(wave * SPW, KG), gB = slice_begin((wave + 1) * SPW, KG);
-  auto no_sums = [](int, int) { return 0.f; };
   if (first_pass) TF_MARK(2);
   // the down projection (EPI 0) adds each group's term by itself: see gemv_stream
-  gemv_stream<GS, NM, RB, COH, true, true, EPI == 0>(acc, st, loaded, wq, sb, xl, no_sums, gA, gB, flush);
+  gemv_stream<GS, NM, RB, COH, EPI == 0>(acc, st, loaded, wq, sb, xl, gA, gB, flush);
   TF_MARK(3);
   sink.streamed();
   __syncthreads();

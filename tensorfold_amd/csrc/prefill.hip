@@ -87,12 +87,6 @@ __device__ __forceinline__ f16x8_t dequant8h(uint32_t w, uint32_t sb) {
 // dequantization work and eight times the rounding error of the fp16 form above; it is what callers get when a
 // table's scales or biases do not fit fp16 after the 2^8 scaling, or when they ask for it.
 
-// eight consecutive bf16 inputs in the operand order (0, 4, 1, 5, 2, 6, 3, 7), unchanged
-__device__ __forceinline__ uint4 stage8_bf16(uint4 v) {
-  return make_uint4(__builtin_amdgcn_perm(v.z, v.x, 0x05040100u), __builtin_amdgcn_perm(v.z, v.x, 0x07060302u),
-                    __builtin_amdgcn_perm(v.w, v.y, 0x05040100u), __builtin_amdgcn_perm(v.w, v.y, 0x07060302u));
-}
-
 __device__ __forceinline__ uint32_t pack_bf16_rn(float lo, float hi) {
   typedef __attribute__((ext_vector_type(2))) __bf16 bf2;
   bf2 r;
@@ -462,22 +456,6 @@ struct DenseSource {
   }
   static __device__ __forceinline__ uint32_t sb_word(const Raw& r, int gi) { return (r.s[gi] & 0xFFFFu) | (r.b[gi] << 16); }
 };
-
-// The transpose of the 4 x 4 matrix whose rows are a wave's four rows of 16 lanes and whose columns are four registers.
-__device__ __forceinline__ void across(uint32_t (&v)[4]) {
-  auto swap32 = [](uint32_t& x, uint32_t& y) {
-    const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
-    x = r[0], y = r[1];
-  };
-  auto swap16 = [](uint32_t& x, uint32_t& y) {
-    const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
-    x = r[0], y = r[1];
-  };
-  swap32(v[0], v[2]);
-  swap32(v[1], v[3]);
-  swap16(v[0], v[1]);
-  swap16(v[2], v[3]);
-}
 
 // AR: TF_ARITH_F16 (fp16 operands, weights scaled by 2^8) or TF_ARITH_BF16 (the reference's bf16(fma(q, s, b)) weights
 // and untouched bf16 activations on the bf16 matrix instruction): the operand bits of mfma_body's two forms.

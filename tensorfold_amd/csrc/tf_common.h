@@ -171,4 +171,26 @@ constexpr uint32_t BF16_128 = 0x43004300u;   // the bf16 pair (128, 128): OR-ing
 // int32 words of an experts block: 32 columns x gs inputs of codes, then 32 (scale | bias << 16) words
 __host__ __device__ constexpr int block_words(int gs) { return 32 * gs / 8 + 32; }
 
+// The transpose of the 4 x 4 matrix whose rows are a wave's four rows of 16 lanes and whose columns are four registers.
+__device__ __forceinline__ void across(uint32_t (&v)[4]) {
+  auto swap32 = [](uint32_t& x, uint32_t& y) {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    x = r[0], y = r[1];
+  };
+  auto swap16 = [](uint32_t& x, uint32_t& y) {
+    const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    x = r[0], y = r[1];
+  };
+  swap32(v[0], v[2]);
+  swap32(v[1], v[3]);
+  swap16(v[0], v[1]);
+  swap16(v[2], v[3]);
+}
+
+// eight consecutive bf16 inputs in the operand order (0, 4, 1, 5, 2, 6, 3, 7), unchanged
+__device__ __forceinline__ uint4 stage8_bf16(uint4 v) {
+  return make_uint4(__builtin_amdgcn_perm(v.z, v.x, 0x05040100u), __builtin_amdgcn_perm(v.z, v.x, 0x07060302u),
+                    __builtin_amdgcn_perm(v.w, v.y, 0x05040100u), __builtin_amdgcn_perm(v.w, v.y, 0x07060302u));
+}
+
 }  // namespace tf

@@ -142,7 +142,7 @@ def split_k(n: int, k: int, gs: int = 64, target: int = 768) -> int:
 
 
 def bucket(m: int) -> int:
-    """Rows a workgroup walks: 16, 32 or 64.  Purely a scheduling choice; bits do not change with it."""
+    """The row tile ``tf_qmm`` is told: 16, 32 or 64.  The launch sizes its own; bits do not change with it."""
 
     if m < 1:
         raise ValueError("the lane matmul takes at least one row")
