@@ -108,7 +108,7 @@ __global__ void __launch_bounds__(WK * 64, K2 <= 12 ? 4 : 1)
     for (int j = 0; j < 8; ++j) acc[j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     // the A operand's row: lane (row c, quarter kq); rows past the pass read a valid row and are dropped later
     const uint16_t* xr = xh + (size_t)(m0 + (c < R ? c : R - 1)) * K + 2 * kq;
-    uint32_t* stage = reinterpret_cast<uint32_t*>(red) + wave * (16 * 128);       // 16 tiles of TW + 2 words
+    uint32_t* stage = reinterpret_cast<uint32_t*>(red) + wave * (16 * 128);       // 16 tiles of TW words
     if (pass) __syncthreads();                 // the previous pass is done with red
     TF_MARK(1);
     wave_block<K2, CB>(xr, tiles, stride_k, pr0, pr1, stage, lane, L, h, acc);

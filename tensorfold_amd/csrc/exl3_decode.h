@@ -44,21 +44,24 @@ __host__ __device__ constexpr int delta(int j) {
 }
 
 // The stored words lane (L, h) needs of a tile for its four values p0 .. p0 + 3 (p0 = 8 L + 4 h): two, or three when
-// a window can reach past the second.
+// the four windows span more than 32 bits.  The first window starts 1 to 32 bits into the first word (not 0 to 31): the
+// shift that lines it up is then 31 to 0 and one v_alignbit_b32 does it.  With 0 to 31 the case of no shift needed a
+// select, and the compiler made it a branch around the second word's LDS read, one in every column tile: the walk
+// waited on two LDS round trips in a row sixteen times a pair (that and the runs' wider loads: 8 rows through 288 experts at 4
+// bits 250 -> 234 us, an MLP at 3 bits and one row 63.3 -> 59.4; a pair of k tiles is 241 vector instructions at 4 bits).
 template <int K2>
 struct Windows {
   static constexpr int TW = tile_words<K2>(), R = 32 * TW;
-  static constexpr bool NEED_LO = delta<K2>(3) + 16 > 32;      // a window reaches past the first aligned word
-  static constexpr bool NEED_W2 = 31 + delta<K2>(3) + 16 > 64; // ... and past the second stored word
-  static constexpr int NW = NEED_LO && NEED_W2 ? 3 : 2;
-  int wi, wi1, wi2, o;                                         // the words and the bit offset: the same for every tile
+  static constexpr int NW = delta<K2>(3) > 16 ? 3 : 2;
+  int wi, wi1, wi2, sh;                                        // the words and the shift: the same for every tile
   __device__ __forceinline__ Windows(int L, int h) {
     const int p0 = 8 * L + 4 * h;
-    const int first = (stream_end<K2>(0) + p0 * K2 / 2 - 16 + R) % R;   // E(p0) - 16; p0 is even, p0 * K2 / 2 whole
-    wi = first >> 5;
+    // one bit before the first window, E(p0) - 16 - 1; p0 is even, p0 * K2 / 2 whole
+    const int before = (stream_end<K2>(0) + p0 * K2 / 2 - 17 + R) % R;
+    wi = before >> 5;
     wi1 = (wi + 1) % TW;
     wi2 = (wi + 2) % TW;
-    o = first & 31;
+    sh = 31 - (before & 31);
   }
   __device__ __forceinline__ void load(const uint32_t* tile, uint32_t (&w)[NW]) const {
     w[0] = tile[wi];
@@ -67,35 +70,18 @@ struct Windows {
   }
   // the 16-bit states of the four values
   __device__ __forceinline__ void states(const uint32_t (&w)[NW], uint32_t (&s)[4]) const {
-    const uint32_t hi = __funnelshift_l(w[1], w[0], o);        // the stream from the first window on, 32 bits
+    const uint32_t hi = __builtin_amdgcn_alignbit(w[0], w[1], sh);        // the stream from the first window on, 32 bits
     uint32_t lo = 0;
-    if constexpr (NEED_LO) lo = __funnelshift_l(NW == 3 ? w[NW - 1] : 0u, w[1], o);
+    if constexpr (NW == 3) lo = __builtin_amdgcn_alignbit(w[1], w[2], sh);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int d = delta<K2>(j);
       if (d + 16 <= 32) s[j] = (hi >> (16 - d)) & 0xFFFFu;
-      else if (d < 32) s[j] = __funnelshift_l(lo, hi, d) >> 16;
+      else if (d < 32) s[j] = __builtin_amdgcn_alignbit(hi, lo, 48 - d) & 0xFFFFu;
       else s[j] = (lo >> (48 - d)) & 0xFFFFu;
     }
   }
 };
-
-// fp16 bits of the codebook value of state s
-template <int CB>
-__device__ __forceinline__ uint16_t code_value(uint32_t s) {
-  if constexpr (CB == 2) {
-    const uint32_t x = s * 0x83DCD12Du;
-    const uint32_t hs = 1024u + (x & 255u) + ((x >> 8) & 255u) + ((x >> 16) & 255u) + (x >> 24);
-    const __half hv = __ushort_as_half((unsigned short)(0x6400u + (hs - 1024u)));   // fp16 of 1024 + byte sum (< 2048)
-    const __half r = __hfma(hv, __ushort_as_half((unsigned short)0x1EEE), __ushort_as_half((unsigned short)0xC931));
-    return __half_as_ushort(r);
-  } else {
-    uint32_t x = CB == 1 ? s * 0xCBAC1FEDu : s * 89226354u + 64248484u;
-    x = (x & 0x8FFF8FFFu) ^ 0x3B603B60u;
-    const __half r = __hadd(__ushort_as_half((unsigned short)(x & 0xFFFFu)), __ushort_as_half((unsigned short)(x >> 16)));
-    return __half_as_ushort(r);
-  }
-}
 
 // The hashed word of a state of the 3inst and mcg codebooks: the value is the fp16 sum of its two halves.
 template <int CB>
@@ -116,6 +102,19 @@ __device__ __forceinline__ uint32_t half_sums(uint32_t xa, uint32_t xb) {
   return r;
 }
 
+// The mul1 values of two states, packed.  v_sad_u8 against zero adds a word's four bytes to an accumulator, its _hi
+// form to the upper half; the accumulator starts as fp16 1024 in both halves (0x6400 + a sum of at most 1,020 is the fp16
+// of 1024 + the sum), and one packed fp16 fma
+// scales and shifts both.
+__device__ __forceinline__ uint32_t mul1_pair(uint32_t sa, uint32_t sb) {
+  uint32_t t = __builtin_amdgcn_sad_u8(sa * 0x83DCD12Du, 0u, 0x64006400u);
+  t = __builtin_amdgcn_sad_hi_u8(sb * 0x83DCD12Du, 0u, t);
+  typedef __attribute__((ext_vector_type(2))) _Float16 f16x2_t;
+  const f16x2_t r = __builtin_elementwise_fma(__builtin_bit_cast(f16x2_t, t), __builtin_bit_cast(f16x2_t, 0x1EEE1EEEu),
+                                              __builtin_bit_cast(f16x2_t, 0xC931C931u));
+  return __builtin_bit_cast(uint32_t, r);
+}
+
 // the fp16 bits of the lane's four values of one tile, as two packed words
 template <int K2, int CB>
 __device__ __forceinline__ void decode4(const Windows<K2>& win, const uint32_t (&w)[Windows<K2>::NW], uint32_t& lo,
@@ -123,8 +122,8 @@ __device__ __forceinline__ void decode4(const Windows<K2>& win, const uint32_t (
   uint32_t s[4];
   win.states(w, s);
   if constexpr (CB == 2) {
-    lo = (uint32_t)code_value<CB>(s[0]) | ((uint32_t)code_value<CB>(s[1]) << 16);
-    hi = (uint32_t)code_value<CB>(s[2]) | ((uint32_t)code_value<CB>(s[3]) << 16);
+    lo = mul1_pair(s[0], s[1]);
+    hi = mul1_pair(s[2], s[3]);
   } else {
     lo = half_sums(code_word<CB>(s[0]), code_word<CB>(s[1]));
     hi = half_sums(code_word<CB>(s[2]), code_word<CB>(s[3]));
@@ -245,42 +244,55 @@ template <int K2, int CB>
 __device__ __forceinline__ void wave_block(const uint16_t* xr, const uint32_t* tiles, int64_t stride_k, int pr0, int pr1,
                                            uint32_t* stage, int lane, int L, int h, f32x4_t (&acc)[8]) {
   constexpr int TW = tile_words<K2>();
-  // The stored words of a k-tile pair (two runs of 8 tiles) come in with coalesced loads, a dword a lane, one pair
-  // ahead, and go through the wave's own part of LDS: each lane then reads the two or three words its windows
-  // start in.  (A lane loading its words itself costs sixteen times the load instructions, and the kernel was
-  // bound by their issue.)  A staged tile repeats its first two words at its end, so a window never wraps.
+  // The stored words of a k-tile pair (two runs of 8 tiles) come in with coalesced loads of up to 16 bytes a lane, one
+  // pair ahead, and go through the wave's own part of LDS as they lie: each lane then reads the two or three words its
+  // windows start in.  (A lane loading its words itself costs sixteen times the load instructions, and the kernel was
+  // bound by their issue.)  Each lane keeps its wrapped word numbers, the same in every tile, so no tile needs a copy of
+  // its first words at its end; a tile's words are at most 64, one a bank.  The pair's number is a scalar (the same
+  // in the whole wave), so a run's address costs no vector instructions.
   constexpr int NW = Windows<K2>::NW;
-  constexpr int TWP = TW + 2, RUN = 8 * TW, GL = (RUN + 63) / 64;
+  constexpr int RUN = 8 * TW, PER = RUN / 64, N4 = PER / 4, REM = PER % 4;      // words a run; whole words a lane
+  constexpr bool HALF = RUN % 64 != 0;                                          // an odd K2: 32 words more
+  typedef uint32_t __attribute__((ext_vector_type(4), aligned(4))) words4_t;    // a trellis may start on any word
   const Windows<K2> win(L, h);
-  uint32_t g[2][GL];
+  pr0 = __builtin_amdgcn_readfirstlane(pr0);
+  pr1 = __builtin_amdgcn_readfirstlane(pr1);
+  const uint32_t* own0 = stage + win.wi;
+  const uint32_t* own1 = stage + win.wi1;
+  const uint32_t* own2 = stage + win.wi2;
+  const int rem_at = 256 * N4 + REM * lane, half_at = 64 * PER + (lane & 31);
+  u32x4_t g4[2][N4 + 1];
+  uint32_t gr[2][REM + 1], gh[2];
   u32x4_t av, an;
-  auto fetch = [&](int pr, uint32_t (&w)[2][GL], u32x4_t& a) {
+  auto fetch = [&](int pr, u32x4_t& a) {
     const uint32_t* xk = reinterpret_cast<const uint32_t*>(xr + 32 * pr);
     a = (u32x4_t){xk[0], xk[4], xk[8], xk[12]};
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
-      const uint32_t* run = tiles + (size_t)(2 * pr + r) * stride_k;
+      const uint32_t* run = tiles + (2 * (int64_t)pr + r) * stride_k;
 #pragma unroll
-      for (int i = 0; i < GL; ++i) w[r][i] = lane + 64 * i < RUN ? run[lane + 64 * i] : 0u;
+      for (int i = 0; i < N4; ++i) g4[r][i] = *reinterpret_cast<const words4_t*>(run + 256 * i + 4 * lane);
+#pragma unroll
+      for (int i = 0; i < REM; ++i) gr[r][i] = run[rem_at + i];
+      if constexpr (HALF) gh[r] = run[half_at];
     }
   };
-  auto put = [&](const uint32_t (&w)[2][GL]) {
+  auto put = [&]() {
 #pragma unroll
-    for (int r = 0; r < 2; ++r)
+    for (int r = 0; r < 2; ++r) {
+      uint32_t* dst = stage + r * RUN;
 #pragma unroll
-      for (int i = 0; i < GL; ++i) {
-        const int idx = lane + 64 * i, j = idx / TW, q = idx - j * TW;
-        if (idx < RUN) {
-          stage[(8 * r + j) * TWP + q] = w[r][i];
-          if (q < 2) stage[(8 * r + j) * TWP + TW + q] = w[r][i];
-        }
-      }
+      for (int i = 0; i < N4; ++i) *reinterpret_cast<u32x4_t*>(dst + 256 * i + 4 * lane) = g4[r][i];
+#pragma unroll
+      for (int i = 0; i < REM; ++i) dst[rem_at + i] = gr[r][i];
+      if constexpr (HALF) dst[half_at] = gh[r];            // both halves of the wave, the same words
+    }
   };
-  if (pr0 < pr1) fetch(pr0, g, av);
+  if (pr0 < pr1) fetch(pr0, av);
   for (int pr = pr0; pr < pr1; ++pr) {
-    put(g);
+    put();
     __builtin_amdgcn_wave_barrier();         // the wave's LDS accesses run in program order: no wait beyond the data's
-    fetch(pr + 1 < pr1 ? pr + 1 : pr, g, an);
+    fetch(pr + 1 < pr1 ? pr + 1 : pr, an);
     const f16x8_t a = __builtin_bit_cast(f16x8_t, av);
     // 3inst and mcg: a value is the sum of the two fp16 halves of its hashed word.  The matrix unit adds them: the
     // four hashed words of a tile are the B operand as they stand (eight fp16 numbers) against every input twice
@@ -297,12 +309,12 @@ __device__ __forceinline__ void wave_block(const uint16_t* xr, const uint32_t* t
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
+      // the widths with three words a window: half of the tiles' reads at a time, or they spill
+      if (NW == 3 && j == 4) __builtin_amdgcn_sched_barrier(0);
       uint32_t w0[NW], w1[NW];
-#pragma unroll
-      for (int q = 0; q < NW; ++q) {
-        w0[q] = stage[j * TWP + win.wi + q];
-        w1[q] = stage[(8 + j) * TWP + win.wi + q];
-      }
+      w0[0] = own0[j * TW], w1[0] = own0[(8 + j) * TW];
+      w0[1] = own1[j * TW], w1[1] = own1[(8 + j) * TW];
+      if constexpr (NW == 3) w0[2] = own2[j * TW], w1[2] = own2[(8 + j) * TW];
       if constexpr (CB != 2) {
         uint32_t s0[4], s1[4];
         win.states(w0, s0);

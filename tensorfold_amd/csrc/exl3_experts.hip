@@ -182,9 +182,10 @@ __device__ __forceinline__ void grouped_body(const GroupedArgs& g, const uint32_
   }
 }
 
-// grid (N / 128, SK, max items * mats); the width is the expert's own
+// grid (N / 128, SK, max items * mats); the width is the expert's own.  Four waves a SIMD (128 registers): without the
+// bound the widest width's needs would leave every width three; with it 8 bits alone spills, five words a pair.
 template <int CB>
-__global__ void __launch_bounds__(XWK * 64) grouped_kernel(const GroupedArgs g) {
+__global__ void __launch_bounds__(XWK * 64, 4) grouped_kernel(const GroupedArgs g) {
   extern __shared__ __align__(16) float red[];              // [XWK][16][128]
   const int it = blockIdx.z / g.mats, mat = blockIdx.z - it * g.mats;
   if (it >= g.counts[0]) return;
