@@ -113,7 +113,8 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the handle of torch.cuda.current_stream() without the Stream object around it: every launch asks for it
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def call(name: str, *args) -> None:

@@ -8,7 +8,9 @@ do not depend on its neighbours.
 
 from __future__ import annotations
 
+import ctypes
 import dataclasses
+from functools import lru_cache
 
 import torch
 
@@ -126,6 +128,7 @@ def matmul_rows(x: torch.Tensor, parts: list[Q4]) -> torch.Tensor:
     return torch.cat([matmul(x, p, xs, sk=sk) for p in parts], dim=1)
 
 
+@lru_cache(maxsize=4096)
 def split_k(n: int, k: int, gs: int = 64, target: int = 768) -> int:
     """Number of K slices of an (n, k) weight - from the shape alone, never the row count.
 
@@ -183,7 +186,8 @@ def matmul(x: torch.Tensor, q: Q4, xs: torch.Tensor | None = None, *, sk: int | 
 
     x = _check_x(x, q, "matmul")
     m = int(x.shape[0])
-    xs = group_sums(x, q.gs) if xs is None else xs
+    own_xs = xs is None
+    xs = group_sums(x, q.gs) if own_xs else xs
     sk = split_k(q.n, q.k, q.gs) if not sk else sk
     if out is None:
         out = x.new_empty((m, q.n), dtype=torch.float32 if f32 else torch.bfloat16)
@@ -195,8 +199,8 @@ def matmul(x: torch.Tensor, q: Q4, xs: torch.Tensor | None = None, *, sk: int | 
     elif sk > 1 and (part.dtype != torch.float32 or part.numel() < sk * m * q.n or not part.is_contiguous()
                      or part.device != x.device):
         raise ValueError(f"matmul: part must hold {sk} x {m} x {q.n} fp32 values (split_k gives the slice count)")
-    if xs.dtype != torch.float32 or tuple(xs.shape) != (m, q.k // q.gs) or not xs.is_contiguous() \
-            or xs.device != x.device:
+    if not own_xs and (xs.dtype != torch.float32 or tuple(xs.shape) != (m, q.k // q.gs) or not xs.is_contiguous()
+                       or xs.device != x.device):
         raise ValueError(f"matmul: xs must be contiguous fp32 ({m}, {q.k // q.gs}), the group sums of x")
     counters = q.counters if reduce and sk > 1 and m <= 8 else None
     _lib.call("tf_qmm", _lib.ptr(x), x.stride(0), _lib.ptr(xs), _lib.ptr(q.weight), _lib.ptr(q.scales),
@@ -245,45 +249,70 @@ def matmul_group(x: torch.Tensor, qs: list[Q4], xs: torch.Tensor | None = None, 
     """``[matmul(x, q) for q in qs]`` for one to four weights of the same K and group size in one launch (plus one
     reduce launch), same bits.  ``outs`` and ``parts`` may bring preallocated buffers (a part where sks[i] > 1)."""
 
-    import ctypes
-
-    if not 1 <= len(qs) <= 4:
+    n = len(qs)
+    if not 1 <= n <= 4:
         raise ValueError("matmul_group: one to four weights")
-    if x.dtype != torch.bfloat16 or x.dim() != 2 or any(x.shape[1] != q.k for q in qs):
+    gs, k = qs[0].gs, qs[0].k
+    if x.dtype != torch.bfloat16 or x.dim() != 2:
         raise ValueError("matmul_group: x must be (M, K) bf16 with every weight's K")
-    if any(q.gs != qs[0].gs for q in qs):
-        raise ValueError("matmul_group: the weights must share a group size")
-    if len({id(q.counters) for q in qs}) != len(qs):
+    m, width = x.shape
+    for q in qs:
+        if q.k != width:
+            raise ValueError("matmul_group: x must be (M, K) bf16 with every weight's K")
+        if q.gs != gs:
+            raise ValueError("matmul_group: the weights must share a group size")
+    counters = [q.counters for q in qs]
+    if len(set(map(id, counters))) != n:
         raise ValueError("matmul_group: a weight given twice would share its arrival counters with itself; "
                          "give the second one as dataclasses.replace(q)")
-    x = _check_x(x, qs[0], "matmul_group")
-    m, gs, k = int(x.shape[0]), qs[0].gs, qs[0].k
+    _lib.on_gpu(x)
+    x = _aligned_rows(x)
     xs = group_sums(x, gs) if xs is None else xs
-    if xs.dtype != torch.float32 or tuple(xs.shape) != (m, k // gs) or not xs.is_contiguous() or xs.device != x.device:
+    if xs.dtype != torch.float32 or xs.shape != (m, k // gs) or not xs.is_contiguous() or xs.device != x.device:
         raise ValueError(f"matmul_group: xs must be contiguous fp32 ({m}, {k // gs}), the group sums of x")
-    sks = list(sks) if sks else [split_k(q.n, q.k, q.gs) for q in qs]
+    sks = list(sks) if sks else [split_k(q.n, q.k, gs) for q in qs]
     dtype = torch.float32 if f32 else torch.bfloat16
-    if outs is None:
+    given = outs is not None
+    if not given:
         outs = [x.new_empty((m, q.n), dtype=dtype) for q in qs]
-    parts = list(parts) if parts else [None] * len(qs)
-    if len(sks) != len(qs) or len(outs) != len(qs) or len(parts) != len(qs):
+    parts = list(parts) if parts else [None] * n
+    if len(sks) != n or len(outs) != n or len(parts) != n:
         raise ValueError("matmul_group: one slice count, output and part a weight")
-    for i, (q, sk, out) in enumerate(zip(qs, sks, outs)):
-        if tuple(out.shape) != (m, q.n) or out.dtype != dtype or not out.is_contiguous() or out.device != x.device:
+    part_at, own = [None] * n, 0        # a part's address, or its place (256-byte steps) in one buffer for all of the call's
+    for i, q in enumerate(qs):
+        out, part, sk = outs[i], parts[i], sks[i]
+        if given and (tuple(out.shape) != (m, q.n) or out.dtype != dtype or not out.is_contiguous()
+                      or out.device != x.device):
             raise ValueError(f"matmul_group: outs[{i}] must be contiguous ({m}, {q.n}) {'fp32' if f32 else 'bf16'}")
-        if sk > 1 and parts[i] is None:
-            parts[i] = x.new_empty((sk, m, q.n), dtype=torch.float32)
-        elif sk > 1 and (parts[i].dtype != torch.float32 or parts[i].numel() < sk * m * q.n
-                         or not parts[i].is_contiguous() or parts[i].device != x.device):
+        if part is None:
+            if sk > 1:
+                part_at[i] = own
+                own += -(-sk * m * q.n // 64) * 256
+        elif sk > 1 and (part.dtype != torch.float32 or part.numel() < sk * m * q.n
+                         or not part.is_contiguous() or part.device != x.device):
             raise ValueError(f"matmul_group: parts[{i}] must hold {sk} x {m} x {q.n} fp32 values")
-    n = len(qs)
-    ptrs = lambda ts: (ctypes.c_void_p * n)(*[None if t is None else t.data_ptr() for t in ts])
-    counters = [q.counters if sk > 1 and m <= 8 else None for q, sk in zip(qs, sks)]
-    _lib.call("tf_qmm_group", _lib.ptr(x), x.stride(0), _lib.ptr(xs), n, ptrs([q.weight for q in qs]),
-              ptrs([q.scales for q in qs]), ptrs([q.biases for q in qs]),
-              (ctypes.c_int64 * n)(*[q.scales.stride(0) for q in qs]), ptrs(outs), ptrs(parts), ptrs(counters),
-              (ctypes.c_int * n)(*[0 if c is None else c.numel() // COUNTER_STRIDE for c in counters]),
-              (ctypes.c_int * n)(*[q.n for q in qs]), (ctypes.c_int * n)(*sks), m, k, gs, bucket(m), int(f32))
+        else:
+            part_at[i] = part.data_ptr()
+    if own:
+        buffer = x.new_empty((own // 4,), dtype=torch.float32)
+        base = buffer.data_ptr()
+        part_at = [at + base if part is None and at is not None else at for at, part in zip(part_at, parts)]
+    if m > 8:
+        counters = [None] * n
+    else:
+        counters = [c if sk > 1 else None for c, sk in zip(counters, sks)]
+    # The entry point's tables side by side in two arrays (addresses and strides, then counts) and one buffer for the
+    # parts: at a row the GPU needs 11 us for the norm and q, k and v (4096 + 1024 + 1024 columns) and the host bounds
+    # the pair of calls: 37 us, with nine arrays, a part a weight and a Stream object a launch; 26 so.
+    wide = (ctypes.c_int64 * (7 * n))(
+        *[q.weight.data_ptr() for q in qs], *[q.scales.data_ptr() for q in qs], *[q.biases.data_ptr() for q in qs],
+        *[q.scales.stride(0) for q in qs], *[out.data_ptr() for out in outs], *[at or 0 for at in part_at],
+        *[0 if c is None else c.data_ptr() for c in counters])
+    narrow = (ctypes.c_int * (3 * n))(*[0 if c is None else c.numel() // COUNTER_STRIDE for c in counters],
+                                      *[q.n for q in qs], *sks)
+    w, c = ctypes.addressof(wide), ctypes.addressof(narrow)
+    _lib.call("tf_qmm_group", x.data_ptr(), x.stride(0), xs.data_ptr(), n, w, w + 8 * n, w + 16 * n, w + 24 * n,
+              w + 32 * n, w + 40 * n, w + 48 * n, c, c + 4 * n, c + 8 * n, m, k, gs, bucket(m), int(f32))
     return outs
 
 
