@@ -3,6 +3,8 @@
 //
 // The decode primitives are in exl3_decode.h.
 
+#include <algorithm>
+
 #include "exl3_decode.h"
 
 namespace tf {
@@ -237,9 +239,10 @@ __global__ void __launch_bounds__(256)
 
 // ---- prompt matmul: y = ((xh @ W_q) H / sqrt(128)) * svh + bias on decoded weights (exl3/prefill.py:15-95) -----------
 //
-// xh fp16 [M, K] (rot_in's output), W8 fp16 [K / 8][N][8] (unpack_k8's).  A workgroup of WAVES waves takes 128 rows x
-// 64 WAVES columns; a wave owns 64 columns = four B operands and all eight 16-row tiles, so one B operand feeds eight MFMAs
-// and one LDS read of xh four: per 32 inputs a wave issues 32 MFMAs against 8 LDS reads and 4 global loads.  B
+// xh fp16 [M, K] (rot_in's output), W8 fp16 [K / 8][N][8] (unpack_k8's).  A workgroup of four waves takes 16 RT rows (128,
+// fewer where that fills the chip better: gemm_row_tiles) x 256 columns, two workgroups a compute unit: one's first loads
+// and its epilogue run under the other's MFMAs.  A wave owns 64 columns = four B operands and all RT 16-row tiles, so one
+// B operand feeds RT MFMAs and one LDS read of xh four: at RT = 8, per 32 inputs, 32 MFMAs against 8 LDS reads and 4 global loads.  B
 // operands come straight from W8 into registers (16 bytes a lane, 16 neighbouring lanes one 256-byte run: the cache
 // sees 8 full lines a load, not 64 lanes' separate pieces), requested two steps of 64 inputs ahead; xh goes a step
 // ahead through registers into LDS (two stages, 144-byte rows), one barrier a step.
@@ -249,16 +252,17 @@ __global__ void __launch_bounds__(256)
 // Workgroups reach the XCDs round-robin (blockIdx % 8) and each XCD has its own L2: the workgroups an XCD runs
 // together (2^g_log2 consecutive ones) take an RG x CG block of tiles, so what they stream in step from beyond L2 is
 // RG tiles of xh and CG of W8, not one of each a workgroup.
-constexpr int GEMM_KSTEP = 64, GEMM_AROW = 2 * GEMM_KSTEP + 16, GEMM_STAGE = 128 * GEMM_AROW;     // bytes
-constexpr int GEMM_LDS = 2 * GEMM_STAGE;         // two stages of xh; the epilogue's 16 x 516 floats fit too
-static_assert(16 * 516 * 4 <= GEMM_LDS, "the epilogue's tile must fit the staging buffers");
+constexpr int GEMM_KSTEP = 64, GEMM_AROW = 2 * GEMM_KSTEP + 16, GEMM_WAVES = 4, GEMM_COLS = 64 * GEMM_WAVES;
+// two stages of xh, or the epilogue's 16 rows of a workgroup's columns if those are more
+constexpr int gemm_lds(int rt) { return max(2 * 16 * rt * GEMM_AROW, 16 * (GEMM_COLS + 4) * 4); }     // bytes
 
-template <int WAVES>
-__global__ void __launch_bounds__(64 * WAVES, 8 / WAVES)
+template <int RT>
+__global__ void __launch_bounds__(64 * GEMM_WAVES, 2)
     gemm_kernel(const uint16_t* __restrict__ xh, const uint16_t* __restrict__ W8, const uint16_t* __restrict__ svh,
                 const uint16_t* __restrict__ bias, void* __restrict__ y, int y_dtype, int64_t y_stride, int M, int K,
                 int N, int rts, int cts, int rg_log2, int g_log2) {
-  constexpr int THREADS = 64 * WAVES, COLS = 64 * WAVES, RED = COLS + 4;     // RED: floats a row of the epilogue's tile
+  constexpr int WAVES = GEMM_WAVES, THREADS = 64 * WAVES, COLS = GEMM_COLS, RED = COLS + 4;     // RED: floats a row of the epilogue's tile
+  constexpr int ROWS = 16 * RT, GEMM_STAGE = ROWS * GEMM_AROW;
   extern __shared__ __align__(16) unsigned char smem[];
   const int RG = 1 << rg_log2, CG = 1 << (g_log2 - rg_log2);
   const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
@@ -267,7 +271,7 @@ __global__ void __launch_bounds__(64 * WAVES, 8 / WAVES)
   const int sc = super / rgs, sr = super - sc * rgs;
   const int rt = sr * RG + (place & (RG - 1)), ct = sc * CG + (place >> rg_log2);
   if (rt >= rts || ct >= cts) return;
-  const int m0 = rt * 128, col0 = ct * COLS;
+  const int m0 = rt * ROWS, col0 = ct * COLS;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, kq = lane >> 4;
   const bool wok = col0 + 64 * wave < N;                   // N is a multiple of 128: a pair of waves falls out together
   const int steps = K / GEMM_KSTEP, last = steps - 1;
@@ -290,8 +294,9 @@ __global__ void __launch_bounds__(64 * WAVES, 8 / WAVES)
   };
   // A: the workgroup's rows of xh as one buffer; this thread's 16-byte pieces of a step: piece q = (row q / 8,
   // 8 inputs q % 8); rows past M read the last row and are dropped at the end
-  constexpr int PPT = 1024 / THREADS;
-  const int nrows = min(128, M - m0);
+  constexpr int PPT = 8 * ROWS / THREADS;
+  static_assert(8 * ROWS % THREADS == 0, "whole pieces a thread");
+  const int nrows = min(ROWS, M - m0);
   const __amdgpu_buffer_rsrc_t asrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(xh + (size_t)m0 * K), 0, (uint32_t)nrows * (uint32_t)K * 2u, 0x00020000);
   uint32_t aoff[PPT];
@@ -313,11 +318,11 @@ __global__ void __launch_bounds__(64 * WAVES, 8 / WAVES)
     }
   };
 
-  f32x4_t acc[4][8];
+  f32x4_t acc[4][RT];
 #pragma unroll
   for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int r = 0; r < 8; ++r) acc[j][r] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < RT; ++r) acc[j][r] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 
   load_b(0, 0, b[0]);
   load_b(0, 1, b[0]);
@@ -334,18 +339,18 @@ __global__ void __launch_bounds__(64 * WAVES, 8 / WAVES)
       load_a(min(step + 1, last));
       __builtin_amdgcn_sched_barrier(0);                // the request leaves now, not when its registers are needed
       const unsigned char* abuf = smem + u * GEMM_STAGE + c * GEMM_AROW + kq * 16;
-      // operand t of the step is (chunk t / 8, row tile t % 8), requested two row tiles before its MFMAs
+      // operand t of the step is (chunk t / RT, row tile t % RT), requested two row tiles before its MFMAs
       auto read_a = [&](int t) {
-        return *reinterpret_cast<const f16x8_t*>(abuf + 16 * (t & 7) * GEMM_AROW + (t >> 3) * 64);
+        return *reinterpret_cast<const f16x8_t*>(abuf + 16 * (t % RT) * GEMM_AROW + (t / RT) * 64);
       };
       f16x8_t a = read_a(0), a1 = read_a(1);
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-          const int t = 8 * i + r;
+        for (int r = 0; r < RT; ++r) {
+          const int t = RT * i + r;
           f16x8_t a2 = a1;
-          if (t + 2 < 16) a2 = read_a(t + 2);
+          if (t + 2 < 2 * RT) a2 = read_a(t + 2);
 #pragma unroll
           for (int j = 0; j < 4; ++j)
             acc[j][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(f16x8_t, b[u][j][i]), acc[j][r], 0, 0, 0);
@@ -353,7 +358,7 @@ __global__ void __launch_bounds__(64 * WAVES, 8 / WAVES)
           a1 = a2;
           // keep the order written here: one LDS read two row tiles ahead of the four MFMAs it feeds
           if (t == 0) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-          if (t + 2 < 16) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          if (t + 2 < 2 * RT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
           __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -367,7 +372,7 @@ __global__ void __launch_bounds__(64 * WAVES, 8 / WAVES)
   // D[row 4 kq + e][column c] of tile (j, r) -> LDS [16 rows][RED] a row tile at a time, then a wave a (row, block)
   float* red = reinterpret_cast<float*>(smem);
 #pragma unroll
-  for (int r = 0; r < 8; ++r) {
+  for (int r = 0; r < RT; ++r) {
     if (r) __syncthreads();
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -530,6 +535,54 @@ extern "C" int tf_exl3_unpack_k8(const uint32_t* T, uint16_t* W8, int k, int n, 
   return 1;
 }
 
+// The tiles along the grid's XCD order: an XCD's 2^g_log2 consecutive workgroups take 2^rg_log2 row tiles x the rest
+// column tiles; smaller groups when the whole grid would not give every XCD two of them.
+struct GemmGrid {
+  int64_t rts, cts, supers;
+  int g_log2, rg_log2;
+  GemmGrid(int m, int n, int rt) {
+    rts = ((int64_t)m + 16 * rt - 1) / (16 * rt), cts = (n + GEMM_COLS - 1) / GEMM_COLS;
+    for (g_log2 = 6;; --g_log2) {
+      rg_log2 = 0;
+      while (rg_log2 < 3 && rg_log2 < g_log2 && (1 << rg_log2) < rts) ++rg_log2;
+      const int64_t cg = 1 << (g_log2 - rg_log2);
+      supers = ((rts + (1 << rg_log2) - 1) >> rg_log2) * ((cts + cg - 1) / cg);
+      if (supers >= 16 || g_log2 == 3) break;
+    }
+  }
+  // the tiles of the XCD that has the most
+  int64_t fullest() const {
+    int64_t tiles[8] = {}, most = 0;
+    const int64_t rg = 1 << rg_log2, cg = 1 << (g_log2 - rg_log2), rgs = (rts + rg - 1) / rg;
+    for (int64_t s = 0; s < supers; ++s) {
+      const int64_t sc = s / rgs, sr = s - sc * rgs;
+      const int64_t t = tiles[s & 7] += std::min(rg, rts - sr * rg) * std::min(cg, cts - sc * cg);
+      most = std::max(most, t);
+    }
+    return most;
+  }
+};
+
+// Row tiles (of 16) a workgroup: 8 where the chip is full, fewer where 128-row tiles would leave compute units idle or
+// a last round nearly empty.  Estimated time: the fullest XCD's tiles a compute unit, times what a tile takes there,
+// measured in us at K = 5120 alone (38, 48, 63, 80 for 32, 64, 96, 128 rows: a chain over K) and among others (32, 40,
+// 55, 70: a smaller tile reads as much of W8 for fewer rows).  Against 128 rows always: 200 x 1024 80 -> 38 us, 777 x 3072
+// 82 -> 52, 1,400 x 5120 122 -> 89, 1,000 x 17408 216 -> 206 by itself (the whole
+// call 269 either way); over 70 shapes 0.69 at the (geometric) mean, none
+// slower.  An odd count of row tiles leaves half the threads a piece more to load and is 1.3 to 2 times slower.
+static int gemm_row_tiles(int m, int n) {
+  if (((int64_t)m + 127) / 128 * ((n + GEMM_COLS - 1) / GEMM_COLS) > 4096) return 8;         // eight rounds and more
+  constexpr int ALONE[4] = {38, 48, 63, 80}, AMONG[4] = {32, 40, 55, 70};
+  int best = 8;
+  int64_t least = INT64_MAX;
+  for (int i = 3; i >= 0; --i) {
+    const int64_t per = (GemmGrid(m, n, 2 * (i + 1)).fullest() + 31) / 32;                   // 32 compute units an XCD
+    const int64_t time = per <= 1 ? ALONE[i] : per * AMONG[i];
+    if (time < least) least = time, best = 2 * (i + 1);
+  }
+  return best;
+}
+
 extern "C" int tf_exl3_gemm(const uint16_t* xh, const uint16_t* w8, const uint16_t* svh, const uint16_t* bias, void* y,
                             int y_dtype, int64_t y_stride, int m, int k, int n, tf_stream_t stream) {
   clear_error();
@@ -539,26 +592,18 @@ extern "C" int tf_exl3_gemm(const uint16_t* xh, const uint16_t* w8, const uint16
   TF_REQUIRE(y_dtype == TF_F16 || y_dtype == TF_BF16 || y_dtype == TF_F32, "y: expected fp16, bf16 or fp32");
   TF_REQUIRE(y_stride >= n && y_stride % 2 == 0, "y rows hold at least N values, an even stride apart");
   TF_REQUIRE(aligned16(xh) && aligned16(w8) && ((uintptr_t)y & 7) == 0, "xh, W8 16-byte and y 8-byte aligned");
-  // 128 x 256 tiles, four waves, two workgroups a CU: one workgroup's first loads and its epilogue run under the
-  // other's MFMAs, and the last, part-filled round of tiles is spread thinner
-  constexpr int WAVES = 4, COLS = 64 * WAVES;
-  const int64_t rts = ((int64_t)m + 127) / 128, cts = (n + COLS - 1) / COLS;
-  TF_REQUIRE(rts <= 0x3FFFFF, "gemm: too many rows for one launch");
-  // an XCD's 2^g_log2 consecutive workgroups: 2^rg_log2 row tiles x the rest column tiles; smaller groups when the
-  // whole grid would not give every XCD two of them
-  int g_log2 = WAVES == 4 ? 6 : 5, rg_log2 = 0;
-  int64_t supers = 0;
-  for (;; --g_log2) {
-    rg_log2 = 0;
-    while (rg_log2 < 3 && rg_log2 < g_log2 && (1 << rg_log2) < rts) ++rg_log2;
-    const int64_t cg = 1 << (g_log2 - rg_log2);
-    supers = ((rts + (1 << rg_log2) - 1) >> rg_log2) * ((cts + cg - 1) / cg);
-    if (supers >= 16 || g_log2 == 3) break;
-  }
-  const int64_t grid = (supers + 7) / 8 * (8 << g_log2);
+  const int tile = gemm_row_tiles(m, n);
+  const GemmGrid gg(m, n, tile);
+  TF_REQUIRE(gg.rts <= 0x3FFFFF, "gemm: too many rows for one launch");
+  const int64_t grid = (gg.supers + 7) / 8 * (8 << gg.g_log2);
   TF_REQUIRE(grid <= 0x7FFFFFFF, "gemm: %lld workgroups exceed the grid limit", (long long)grid);
-  gemm_kernel<WAVES><<<dim3((unsigned)grid), 64 * WAVES, GEMM_LDS, as_stream(stream)>>>(
-      xh, w8, svh, bias, y, y_dtype, y_stride, m, k, n, (int)rts, (int)cts, rg_log2, g_log2);
+#define TF_GEMM(RT_)                                                                                                 \
+  case RT_:                                                                                                          \
+    gemm_kernel<RT_><<<dim3((unsigned)grid), 64 * GEMM_WAVES, gemm_lds(RT_), as_stream(stream)>>>(                   \
+        xh, w8, svh, bias, y, y_dtype, y_stride, m, k, n, (int)gg.rts, (int)gg.cts, gg.rg_log2, gg.g_log2);          \
+    break;
+  switch (tile) { TF_GEMM(2) TF_GEMM(4) TF_GEMM(6) TF_GEMM(8) }
+#undef TF_GEMM
   TF_LAUNCH_OK("tf_exl3_gemm");
   return 0;
 }
