@@ -23,3 +23,10 @@ def test_router_against_float64_and_row_by_row(rows, d, ne):
         assert torch.equal(moe.router(x[at:at + 1], r)[0], got[at])
     part = rows - rows // 3
     assert torch.equal(moe.router(x[:part], r), got[:part])
+
+
+# slices of 2 to 28 chunks: fewer than a workgroup requests together, as many, and one to a few more (each tile's kernel)
+@pytest.mark.parametrize("rows,d,ne", [(32, 512, 128), (8, 896, 16), (40, 2080, 64), (8, 4096, 128), (3, 7168, 17),
+                                       (300, 736, 513), (290, 1504, 257), (777, 1056, 513), (530, 3104, 500)])
+def test_slices_of_any_length(rows, d, ne):
+    test_router_against_float64_and_row_by_row(rows, d, ne)
