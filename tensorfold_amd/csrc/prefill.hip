@@ -1044,8 +1044,15 @@ typedef ShortTile<2, 1, 1, 4, 256> Short32;          // 32 x 64
 typedef ShortTile<2, 1, 1, 8, 256> Short32Wide;      // 32 x 128, eight waves
 typedef ShortTile<4, 2, 1, 4, 128> Short64;          // 64 x 128
 
-// tiles along the faster grid index, rounded up to whole rounds of the eight XCDs where there are that many
+// tiles of `size` that `count` rows or columns take, and those tiles along the faster grid index rounded up to whole
+// rounds of the eight XCDs where there are that many
+__host__ __device__ constexpr int short_tiles(int count, int size) { return (count - 1) / size + 1; }
 __host__ __device__ constexpr int short_pad(int tiles) { return tiles < 8 ? tiles : (tiles + 7) & ~7; }
+// Which index is the faster one: the launch sizes its grid by this and the kernel reads its place off it, so both ask
+// here.  Neighbours in the grid go to the XCDs in turn: those that read the same part of the larger operand (the weight
+// where n > 4 m: half a byte against two) are a multiple of eight apart, so it comes into one L2 and not into all eight.
+__host__ __device__ constexpr bool short_by_col(int m, int n) { return n > 4ll * m; }
+static_assert(!short_by_col(1 << 29, 64) && short_by_col(1, 5), "4 m does not fit 32 bits from 2^29 rows on");
 
 template <int GS, int EPI, int AR, int RT, int CT, int WR, int WC, int STEP>
 __global__ void __launch_bounds__(64 * WR * WC)
@@ -1058,10 +1065,8 @@ __global__ void __launch_bounds__(64 * WR * WC)
   constexpr int WSETS = 4;
   static_assert(T::BM * PPR % T::THREADS == 0 && T::THREADS % PPR == 0 && 128 % T::BN == 0, "whole pieces a thread");
   extern __shared__ __align__(16) unsigned char smem[];
-  // neighbours in the grid go to the XCDs in turn: those that read the same part of the larger operand (the weight where
-  // N > 4 M: half a byte against two) are a multiple of eight apart, so it comes into one L2 and not into all eight
-  const int ct = (N + T::BN - 1) / T::BN, mt = (M + T::BM - 1) / T::BM;
-  const bool by_col = N > 4 * M;
+  const int ct = short_tiles(N, T::BN), mt = short_tiles(M, T::BM);
+  const bool by_col = short_by_col(M, N);
   const int across_n = short_pad(by_col ? ct : mt), slow = blockIdx.x / across_n, fast = blockIdx.x - slow * across_n;
   const int cbt = by_col ? fast : slow, rt = by_col ? slow : fast;
   if (cbt >= ct || rt >= mt) return;
@@ -1308,8 +1313,8 @@ int launch_qmm_prefill(int arith, int tile, const uint16_t* x, int64_t ldx, cons
   TF_REQUIRE(tile != 9 || big_ok, "qmm_prefill: tile 9 (the eight-wave kernel) takes K in whole steps of 64");
 #define TF_SHORT(T_, RT_, CT_, WR_, WC_, STEP_)                                                                      \
   {                                                                                                                \
-    const int ctn = (n + T_::BN - 1) / T_::BN, mtn = (m + T_::BM - 1) / T_::BM;                                    \
-    const int64_t grid = n > 4 * (int64_t)m ? (int64_t)short_pad(ctn) * mtn : (int64_t)short_pad(mtn) * ctn;       \
+    const int ctn = short_tiles(n, T_::BN), mtn = short_tiles(m, T_::BM);                                          \
+    const int64_t grid = short_by_col(m, n) ? (int64_t)short_pad(ctn) * mtn : (int64_t)short_pad(mtn) * ctn;       \
     TF_REQUIRE(grid <= 0x7FFFFFFF, "qmm_prefill: grid too large");                                                 \
     if (arith)                                                                                                     \
       qmm_prefill_short_kernel<GS, EPI, 1, RT_, CT_, WR_, WC_, STEP_><<<(unsigned)grid, T_::THREADS, T_::LDS, st>>>( \
