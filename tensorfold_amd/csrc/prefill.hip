@@ -1030,7 +1030,7 @@ __global__ void __launch_bounds__(256)
 // operands (100 rows x 4096 x 4096 ran on 8 workgroups), so requests run far ahead of their use: the weights' words and
 // scales four steps in registers, the activations two, through two stages of LDS, one barrier a step.  A wave loads
 // the words its own operands need (lane (column c, quarter kq) word kq of column c: 256 bytes a tile and chunk).
-// The operands, their order along K and the matrix instruction are big_body's, and so are the bits.  
+// The operands, their order along K and the matrix instruction are big_body's, and so are the bits.
 template <int RT, int CT, int WR, int WC, int STEP>
 struct ShortTile {
   static constexpr int BM = 16 * RT * WR, BN = 16 * CT * WC, THREADS = 64 * WR * WC;
@@ -1298,19 +1298,47 @@ int launch_experts_prefill(int tile, int arith, const uint16_t* x, int64_t x_str
   return 0;
 }
 
-// tile: 0 = chosen from the rows and columns; 1, 4, 8 = the four-wave kernel on 16, 64 or 128 rows a workgroup; 9 = the
-// eight-wave kernel (128 rows x 512 columns; K in whole steps of 64).  The same bits whatever the tile.
+// The eight-wave kernel takes K in whole steps and a weight whose codes a 32-bit byte offset reaches.
+static bool big_takes(int64_t n, int64_t k) {
+  return k % KSTEP == 0 && (n + 127) / 128 * 128 * k / 2 < (1ll << 32);
+}
+
+// The tile codes of tf_qmm_prefill: 1, 4, 8 = the four-wave kernel on 16, 64 or 128 rows a workgroup; 2, 3, 5, 6 = the
+// short tiles; 9 = the eight-wave kernel.  The same bits whatever the tile.
+//
+// What code 0 stands for.  A call's time is about a start plus a cost a round of 256 workgroups, in the same unit per
+// input of K (half microseconds at K = 4096; measured on 17 to 4,096 rows x 512 to 17,408 columns): the least of them is
+// taken.  17 rows x 4096 x 4096 82.9 -> 12.9 us, 100 rows 86.3 -> 14.4 (32 x 64), 512 rows 89 -> 33 (32 x 128),
+// 1,000 rows 89 -> 53 (64 x 128); at 2,000 rows the eight-wave kernel's 95.7 is the best again (64 x 128 98.5).
+static int prompt_tile(int64_t m, int64_t n, int64_t k) {
+  auto rounds = [](int64_t workgroups) { return (workgroups + 255) / 256; };
+  const int64_t t16 = 12 + 12 * rounds(Short16::workgroups(m, n)), t32 = 14 + 17 * rounds(Short32::workgroups(m, n)),
+                t32w = 16 + 26 * rounds(Short32Wide::workgroups(m, n)),
+                t64 = 32 + 40 * rounds(Short64::workgroups(m, n));
+  const int64_t least = std::min(std::min(t16, t32), std::min(t32w, t64));
+  const int64_t big = 10 + 170 * rounds((m + BIG_ROWS - 1) / BIG_ROWS * ((n + 511) / 512));
+  if (big_takes(n, k) && big <= least) return 9;
+  return least == t16 ? 2 : least == t32 ? 3 : least == t32w ? 5 : 6;
+}
+
 template <int GS, int EPI>
 int launch_qmm_prefill(int arith, int tile, const uint16_t* x, int64_t ldx, const uint32_t* w, const uint16_t* s,
                        const uint16_t* b, void* out, int m, int n, int kg, hipStream_t st) {
   const int npad = (n + 127) / 128 * 128;
   const int ct = (n + 127) / 128;
-#define TF_SMALL(RT_, AR_)                                                                                       \
-  qmm_prefill_kernel<GS, EPI, RT_, AR_><<<(unsigned)(((m + 16 * RT_ - 1) / (16 * RT_)) * ct), 256, stage_bytes<RT_>(), \
-                                          st>>>(x, ldx, w, s, b, out, m, n, kg, npad)
   TF_REQUIRE((int64_t)((m + 15) / 16) * ct <= 0x7FFFFFFF, "qmm_prefill: grid too large");
-  const bool big_ok = (kg * GS) % KSTEP == 0 && (int64_t)npad * kg * GS / 2 < (1ll << 32);
-  TF_REQUIRE(tile != 9 || big_ok, "qmm_prefill: tile 9 (the eight-wave kernel) takes K in whole steps of 64");
+  if (tile == 0) tile = prompt_tile(m, n, (int64_t)kg * GS);
+  TF_REQUIRE(tile != 9 || big_takes(n, (int64_t)kg * GS),
+             "qmm_prefill: tile 9 (the eight-wave kernel) takes K in whole steps of 64");
+#define TF_SMALL(RT_)                                                                                             \
+  {                                                                                                               \
+    const unsigned grid = (unsigned)(((m + 16 * RT_ - 1) / (16 * RT_)) * ct);                                     \
+    if (arith)                                                                                                    \
+      qmm_prefill_kernel<GS, EPI, RT_, 1><<<grid, 256, stage_bytes<RT_>(), st>>>(x, ldx, w, s, b, out, m, n, kg, npad); \
+    else                                                                                                          \
+      qmm_prefill_kernel<GS, EPI, RT_, 0><<<grid, 256, stage_bytes<RT_>(), st>>>(x, ldx, w, s, b, out, m, n, kg, npad); \
+    break;                                                                                                        \
+  }
 #define TF_SHORT(T_, RT_, CT_, WR_, WC_, STEP_)                                                                      \
   {                                                                                                                \
     const int ctn = short_tiles(n, T_::BN), mtn = short_tiles(m, T_::BM);                                          \
@@ -1322,44 +1350,23 @@ int launch_qmm_prefill(int arith, int tile, const uint16_t* x, int64_t ldx, cons
     else                                                                                                           \
       qmm_prefill_short_kernel<GS, EPI, 0, RT_, CT_, WR_, WC_, STEP_><<<(unsigned)grid, T_::THREADS, T_::LDS, st>>>( \
           x, ldx, w, s, b, out, m, n, kg, npad);                                                                   \
-    TF_LAUNCH_OK("tf_qmm_prefill");                                                                                \
-    return 0;                                                                                                      \
+    break;                                                                                                         \
   }
-  if (tile == 0) {
-    // A call's time is about a start plus a cost a round of 256 workgroups, in the same unit per input of K (half
-    // microseconds at K = 4096; measured on 17 to 4,096 rows x 512 to 17,408 columns): the least of them is taken.
-    // 17 rows x 4096 x 4096 82.9 -> 12.9 us, 100 rows 86.3 -> 14.4 (32 x 64), 512 rows 89 -> 33 (32 x 128),
-    // 1,000 rows 89 -> 53 (64 x 128); at 2,000 rows the eight-wave kernel's 95.7 is the best again (64 x 128 98.5).
-    auto rounds = [](int64_t workgroups) { return (workgroups + 255) / 256; };
-    const int64_t t16 = 12 + 12 * rounds(Short16::workgroups(m, n)), t32 = 14 + 17 * rounds(Short32::workgroups(m, n)),
-                  t32w = 16 + 26 * rounds(Short32Wide::workgroups(m, n)),
-                  t64 = 32 + 40 * rounds(Short64::workgroups(m, n));
-    const int64_t least = std::min(std::min(t16, t32), std::min(t32w, t64));
-    const int64_t big = 10 + 170 * rounds((int64_t)((m + BIG_ROWS - 1) / BIG_ROWS) * ((n + 511) / 512));
-    if (!big_ok || least < big) {
-      if (least == t16) TF_SHORT(Short16, 1, 1, 1, 4, 256)
-      if (least == t32) TF_SHORT(Short32, 2, 1, 1, 4, 256)
-      if (least == t32w) TF_SHORT(Short32Wide, 2, 1, 1, 8, 256)
-      TF_SHORT(Short64, 4, 2, 1, 4, 128)
+  switch (tile) {
+    case 1: TF_SMALL(1)
+    case 4: TF_SMALL(4)
+    case 8: TF_SMALL(8)
+    case 2: TF_SHORT(Short16, 1, 1, 1, 4, 256)
+    case 3: TF_SHORT(Short32, 2, 1, 1, 4, 256)
+    case 5: TF_SHORT(Short32Wide, 2, 1, 1, 8, 256)
+    case 6: TF_SHORT(Short64, 4, 2, 1, 4, 128)
+    default: {
+      const unsigned grid = (unsigned)((int64_t)((m + BIG_ROWS - 1) / BIG_ROWS) * ((n + 511) / 512));
+      if (arith)
+        qmm_prefill_big_kernel<GS, EPI, 1><<<grid, BIG_THREADS, BIG_LDS, st>>>(x, ldx, w, s, b, out, m, n, kg, npad);
+      else
+        qmm_prefill_big_kernel<GS, EPI, 0><<<grid, BIG_THREADS, BIG_LDS, st>>>(x, ldx, w, s, b, out, m, n, kg, npad);
     }
-  }
-  const int rows = tile == 1 ? 16 : tile == 4 ? 64 : tile == 8 ? 128 : 129;     // as if this many rows
-  if (rows <= 16) {
-    if (arith) TF_SMALL(1, 1);
-    else TF_SMALL(1, 0);
-  } else if (rows <= 64) {
-    if (arith) TF_SMALL(4, 1);
-    else TF_SMALL(4, 0);
-  } else if (big_ok && tile != 8) {
-    const unsigned grid = (unsigned)((int64_t)((m + BIG_ROWS - 1) / BIG_ROWS) * ((n + 511) / 512));
-    if (arith)
-      qmm_prefill_big_kernel<GS, EPI, 1><<<grid, BIG_THREADS, BIG_LDS, st>>>(x, ldx, w, s, b, out, m, n, kg, npad);
-    else
-      qmm_prefill_big_kernel<GS, EPI, 0><<<grid, BIG_THREADS, BIG_LDS, st>>>(x, ldx, w, s, b, out, m, n, kg, npad);
-  } else if (arith) {
-    TF_SMALL(8, 1);
-  } else {
-    TF_SMALL(8, 0);
   }
 #undef TF_SMALL
 #undef TF_SHORT
@@ -1397,13 +1404,15 @@ extern "C" int tf_experts_prefill(int gs, int epi, const uint16_t* x, int64_t x_
   return 1;
 }
 
+extern "C" int tf_qmm_prompt_tile(int m, int n, int k) { return prompt_tile(m < 1 ? 1 : m, n < 1 ? 1 : n, k); }
+
 extern "C" int tf_qmm_prefill(const uint16_t* x, int64_t ldx, const uint32_t* weight, const uint16_t* scales,
                               const uint16_t* biases, void* out, int m, int n, int k, int gs, int f32, int tile,
                               int arith, tf_stream_t stream) {
   clear_error();
   TF_REQUIRE(arith == TF_ARITH_F16 || arith == TF_ARITH_BF16, "prefill arithmetic %d: TF_ARITH_F16 or TF_ARITH_BF16", arith);
   TF_REQUIRE(gs == 32 || gs == 64, "groups of 32 or 64");
-  TF_REQUIRE(tile == 0 || tile == 1 || tile == 4 || tile == 8 || tile == 9, "qmm_prefill: tile 0 (chosen from the row count), 1, 4, 8 or 9, not %d", tile);
+  TF_REQUIRE((tile >= 0 && tile <= 6) || tile == 8 || tile == 9, "qmm_prefill: tile 0 (chosen from the sizes), 1 to 6, 8 or 9, not %d", tile);
   TF_REQUIRE(x && weight && scales && biases && out && m >= 1 && n >= 1, "qmm_prefill: null pointer or empty shape");
   TF_REQUIRE(aligned16(x) && (m == 1 || ldx % 8 == 0), "x rows must start on 16-byte boundaries");
   TF_REQUIRE(k >= gs && k % gs == 0, "K splits into whole groups");

@@ -317,16 +317,13 @@ def matmul_group(x: torch.Tensor, qs: list[Q4], xs: torch.Tensor | None = None, 
 
 
 def prompt_tile(m: int, n: int, k: int = 64) -> int:
-    """A tile code of the prompt matmul by the row count (cuda/kernels/qmm.py:202-205 names the reference's one tile,
-    tuned for its chip): 1, 4 or 8 = a four-wave workgroup on 16, 64 or 128 rows x 128 columns; 9 = eight waves on 128
-    rows x 512 columns, from 65 rows on, for K in whole steps of 64.  ``tile=0`` looks at the columns too and has
-    smaller tiles for what would leave compute units idle (the bits are the same)."""
+    """The tile code that ``prefill_matmul(..., tile=0)`` takes for ``m`` rows of an (n, k) weight
+    (cuda/kernels/qmm.py:202-205 names the reference's one tile, tuned for its chip): 1, 4 or 8 = a four-wave workgroup
+    on 16, 64 or 128 rows x 128 columns; 2, 3, 5 or 6 = 16 x 64, 32 x 64, 32 x 128 or 64 x 128 of a pipeline for what
+    would leave compute units idle at larger tiles; 9 = eight waves on 128 rows x 512 columns, for K in whole steps of
+    64.  The launch asks the same rule; it needs no GPU."""
 
-    if m <= 16:
-        return 1
-    if m <= 64:
-        return 4
-    return 9 if k % 64 == 0 else 8
+    return _lib.lib().tf_qmm_prompt_tile(m, n, k)
 
 
 def prefill_matmul(x: torch.Tensor, q: Q4, *, f32: bool = False, tile: int = 0,
@@ -337,8 +334,8 @@ def prefill_matmul(x: torch.Tensor, q: Q4, *, f32: bool = False, tile: int = 0,
     bf16's range; None: what ``pack`` found the weight's scales and biases to need.  ``tile``: 0 or a ``prompt_tile``
     code; the bits are the same whatever the tile."""
 
-    if tile not in (0, 1, 4, 8, 9):
-        raise ValueError("prefill_matmul: tile 0, 1, 4, 8 or 9 (see prompt_tile)")
+    if tile not in (0, 1, 2, 3, 4, 5, 6, 8, 9):
+        raise ValueError("prefill_matmul: tile 0 to 6, 8 or 9 (see prompt_tile)")
     x = _check_x(x, q, "prefill_matmul")
     m = int(x.shape[0])
     if out is None:

@@ -1,0 +1,34 @@
+"""The rule behind the prompt matmul's tile, without a GPU: what ``prompt_tile`` names is what the launch takes."""
+
+import pytest
+
+from tensorfold_amd import qmm
+
+CODES = {1, 2, 3, 4, 5, 6, 8, 9}
+
+
+def test_the_rule_looks_at_rows_and_columns():
+    assert qmm.prompt_tile(100, 4096, 4096) == 3           # 128 x 512 tiles would be 8 workgroups
+    assert qmm.prompt_tile(512, 4096, 4096) == 5
+    assert qmm.prompt_tile(1000, 4096, 4096) == 6
+    assert qmm.prompt_tile(2000, 4096, 4096) == 9
+    assert qmm.prompt_tile(4096, 17408, 5120) == 9
+
+
+@pytest.mark.parametrize("k", [32, 64, 96, 4096, 4128, 5120])
+def test_every_size_has_a_tile(k):
+    for m in (0, 1, 16, 17, 64, 65, 300, 1000, 4096, 1 << 20, (1 << 31) - 1):
+        for n in (1, 64, 130, 4096, 17408, 248320):
+            tile = qmm.prompt_tile(m, n, k)
+            assert tile in CODES and (tile != 9 or k % 64 == 0), (m, n)
+
+
+def test_a_weight_past_a_32_bit_offset_keeps_off_the_eight_wave_tile():
+    assert qmm.prompt_tile(4096, 1 << 20, 8128) == 9       # 0xFE000000 bytes of codes
+    assert qmm.prompt_tile(4096, 1 << 20, 8192) != 9       # 2^32
+
+
+def test_a_code_that_names_nothing_is_refused():
+    for tile in (-1, 7, 10):
+        with pytest.raises(ValueError, match="tile"):
+            qmm.prefill_matmul(None, None, tile=tile)
