@@ -1310,6 +1310,8 @@ static bool big_takes(int64_t n, int64_t k) {
 // input of K (half microseconds at K = 4096; measured on 17 to 4,096 rows x 512 to 17,408 columns): the least of them is
 // taken.  17 rows x 4096 x 4096 82.9 -> 12.9 us, 100 rows 86.3 -> 14.4 (32 x 64), 512 rows 89 -> 33 (32 x 128),
 // 1,000 rows 89 -> 53 (64 x 128); at 2,000 rows the eight-wave kernel's 95.7 is the best again (64 x 128 98.5).
+constexpr int SHORT_K = 192;
+
 static int prompt_tile(int64_t m, int64_t n, int64_t k) {
   auto rounds = [](int64_t workgroups) { return (workgroups + 255) / 256; };
   const int64_t t16 = 12 + 12 * rounds(Short16::workgroups(m, n)), t32 = 14 + 17 * rounds(Short32::workgroups(m, n)),
@@ -1318,7 +1320,17 @@ static int prompt_tile(int64_t m, int64_t n, int64_t k) {
   const int64_t least = std::min(std::min(t16, t32), std::min(t32w, t64));
   const int64_t big = 10 + 170 * rounds((m + BIG_ROWS - 1) / BIG_ROWS * ((n + 511) / 512));
   if (big_takes(n, k) && big <= least) return 9;
-  return least == t16 ? 2 : least == t32 ? 3 : least == t32w ? 5 : 6;
+  const int best = least == t16 ? 2 : least == t32 ? 3 : least == t32w ? 5 : 6;
+  if (k >= SHORT_K) return best;
+  // With so short a K a workgroup is its start and its stores: four steps of requests have nothing to run ahead of, and a
+  // round of the small tiles costs more than the unit above says.  Where there are many workgroups (w, of 64 x 128) the
+  // four- and eight-wave kernels are faster: 4,096 rows x 17408 x 96 62 us (64 x 128: 76), 17 x 151936 x 64 8.4 (32 x 128:
+  // 14.0), 65 x 65536 x 64 11.7 (16.3); with a few hundred 64 x 128 is: 1,500 x 2048 x 96 6.8 (32 x 128: 9.8).  From 192
+  // inputs on none of them is.
+  const int64_t w = Short64::workgroups(m, n);
+  if (m <= 64) return w > (k <= 64 ? 64 : 512) || (k < 64 && m <= 16) ? (m <= 16 ? 1 : 4) : best;
+  if (w >= (k < 64 ? 512 : 1024)) return big_takes(n, k) ? 9 : 8;
+  return w >= 192 ? 6 : best;
 }
 
 template <int GS, int EPI>

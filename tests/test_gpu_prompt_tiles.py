@@ -12,11 +12,11 @@ DEV = "cuda"
 
 # (rows, columns, K, group size) and the tile that the call takes: its row and column edges, one step and less of K, a
 # step that ends inside (K = 32, 96, 736, 1056 are not whole steps of 128 or 256), more columns than rows and the reverse
-SHAPES = [(1, 1, 32, 32, 2), (3, 130, 64, 64, 2), (16, 4096, 96, 32, 2), (17, 640, 256, 64, 2),
+SHAPES = [(1, 1, 32, 32, 1), (3, 130, 64, 64, 2), (16, 4096, 96, 32, 2), (17, 640, 256, 64, 2),
           (33, 1024, 736, 32, 2), (100, 4096, 1056, 32, 3), (129, 515, 320, 64, 2), (257, 4100, 448, 64, 3),
           (300, 8192, 512, 64, 5), (1000, 4096, 192, 64, 6), (999, 4099, 320, 64, 5), (1000, 2047, 192, 64, 5),
           (1030, 4096, 544, 32, 5), (2000, 130, 96, 32, 3), (2000, 4100, 192, 64, 9), (1999, 4096, 320, 32, 9),
-          (4096, 513, 64, 64, 5)]
+          (4096, 513, 64, 64, 6)]
 
 
 def operands(m, n, k, gs):

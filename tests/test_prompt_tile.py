@@ -15,6 +15,18 @@ def test_the_rule_looks_at_rows_and_columns():
     assert qmm.prompt_tile(4096, 17408, 5120) == 9
 
 
+def test_a_short_k_keeps_the_tiles_that_start_quickly():
+    assert qmm.prompt_tile(4096, 17408, 96) == 8           # 62 us; 64 x 128 76
+    assert qmm.prompt_tile(4096, 8192, 160) == 8           # 39 us; 47
+    assert qmm.prompt_tile(200, 17408, 32) == 8            # 7.6 us; 32 x 128 11.3
+    assert qmm.prompt_tile(1500, 2048, 96) == 6            # 6.8 us; 32 x 128 9.8
+    assert qmm.prompt_tile(65, 65536, 64) == 9             # 11.7 us; 32 x 128 16.3
+    assert qmm.prompt_tile(64, 17408, 64) == 4             # 4.9 us; 32 x 64 5.9
+    assert qmm.prompt_tile(8, 17408, 64) == 1              # 3.6 us; 16 x 64 4.1
+    assert qmm.prompt_tile(33, 8192, 64) == 3              # 4.2 us; four-wave 4.5
+    assert qmm.prompt_tile(4096, 8192, 224) == 6           # from 192 inputs on the other rule
+
+
 @pytest.mark.parametrize("k", [32, 64, 96, 4096, 4128, 5120])
 def test_every_size_has_a_tile(k):
     for m in (0, 1, 16, 17, 64, 65, 300, 1000, 4096, 1 << 20, (1 << 31) - 1):
