@@ -14,7 +14,7 @@ namespace {
 // form spent its time on (11 us at 1 to 8 rows x 128 experts x 2688, 131 us at 4,096 x 513 x 2048).
 
 constexpr int ROUTER_SLICES = 8;
-constexpr int64_t ROUTER_WIDE_TILES = 2048;      // more 16 x 16 tiles than this: the wide kernel
+constexpr int64_t ROUTER_ROUND = 512;      // workgroups of 32 x 64 that the chip holds at once: beyond, the wide kernel
 
 __device__ __forceinline__ int router_chunk(int s, int chunks) { return s * chunks / ROUTER_SLICES; }
 
@@ -418,15 +418,20 @@ extern "C" int tf_moe_router(const uint16_t* x, int64_t ldx, const uint16_t* row
   // A compute unit takes 16 to 20 bytes of operands a cycle whatever the tile, so small tiles win while each has a unit
   // to itself and larger ones (operands read fewer times over) once they do not: 392 tiles x 2688 18.3 us as 16 x 16,
   // 13.3 as 32 x 32 (128 tiles 7.4 / 13); 1,617 x 2048 14.2 us as 32 x 64, 47 as one wave's 32 x 64; 8,448 x 2048
-  // 30.5 us wide, and from 2,112 tiles on the wide kernel's 28 us against two rounds of the others.
+  // 30.5 us wide.  The wide kernel takes what would be more than one round of 32 x 64, two workgroups a unit: below that its
+  // own 64 x 128 leave units idle (4,096 rows x 129 x 512 11.8 us on 128 workgroups, 8.6 as 32 x 64; x 2048 28.3, 21.3).
+  // With up to 32 experts a column tile of 64 or 128 would be mostly padding: 32,768 rows x 8 x 2048 36 us as 32 x 64,
+  // 24.7 as 64 x 16 (one wave a tile, the single chain: 27); 16,384 x 32 x 1024 13.1 as 32 x 64, 10.7 as 32 x 32.
   const int64_t tiles = (int64_t)((m + 15) / 16) * ((ne + 15) / 16);
   if (tiles <= 256) {
     const dim3 grid((m + 15) / 16, (ne + 15) / 16);
     if (d <= 32 * 8 * ROUTER_SLICES) router_kernel<1, 1, 8><<<grid, 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
     else router_kernel<1, 1, 12><<<grid, 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
-  } else if (tiles <= 1024) {
+  } else if (tiles > 1024 && ne <= 16) {
+    router_kernel<4, 1, 4><<<dim3((m + 63) / 64), 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
+  } else if (tiles <= 1024 || ne <= 32) {
     router_kernel<2, 2, 4><<<dim3((m + 31) / 32, (ne + 31) / 32), 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
-  } else if (tiles <= ROUTER_WIDE_TILES) {
+  } else if ((int64_t)((m + 31) / 32) * ((ne + 63) / 64) <= ROUTER_ROUND) {
     router_kernel<2, 4, 4><<<dim3((m + 31) / 32, (ne + 63) / 64), 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
   } else {
     router_wide_kernel<<<dim3((m + 63) / 64, (ne + 127) / 128), 256, 0, s>>>(x, ldx, rows, logits, m, d, ne);

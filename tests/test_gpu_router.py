@@ -30,3 +30,12 @@ def test_router_against_float64_and_row_by_row(rows, d, ne):
                                        (300, 736, 513), (290, 1504, 257), (777, 1056, 513), (530, 3104, 500)])
 def test_slices_of_any_length(rows, d, ne):
     test_router_against_float64_and_row_by_row(rows, d, ne)
+
+
+# the edges between the kernels that the rows and experts choose: many rows of few experts, and either side of where the
+# wide kernel starts (512 workgroups of 32 x 64)
+@pytest.mark.parametrize("rows,d,ne", [(16390, 96, 8), (16400, 352, 16), (33000, 64, 1), (16385, 160, 17), (16400, 512, 32),
+                                       (4100, 256, 128), (4096, 512, 129), (1055, 288, 513), (5460, 96, 145),
+                                       (5471, 352, 180), (8192, 128, 128), (8193, 288, 128)])
+def test_many_rows_of_few_experts(rows, d, ne):
+    test_router_against_float64_and_row_by_row(rows, d, ne)
