@@ -114,8 +114,12 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream() -> int:
-    # the handle of torch.cuda.current_stream() without the Stream object around it: every launch asks for it
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    # the handle of torch.cuda.current_stream() without the Stream object around it: every launch asks for it.  The two
+    # names are torch's own and not public: a build that lacks them is asked the public way
+    try:
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    except AttributeError:
+        return torch.cuda.current_stream().cuda_stream
 
 
 def call(name: str, *args) -> None:
