@@ -18,6 +18,7 @@
 // with q exact.  For the experts a nibble OR-ed into the bf16 pattern of 128 is 128 + q, so the dot product gives
 // P + 128 xs and P = fma(-128, xs, that).
 
+#include <algorithm>
 #include <cstdlib>
 #include <mutex>
 
@@ -71,7 +72,6 @@ __global__ void __launch_bounds__(WAVES * 64)
 }
 
 // ---- dense lane matmul ---------------------------------------------------------------------------------------------
-
 //
 // A wave takes 64 columns and a run of groups; up to 16 RT rows of the call are the rows of v_mfma_f32_16x16x32_bf16, so
 // a weight is unpacked once for all of them (rows are independent there: a row's bits do not depend on the others, on
@@ -112,22 +112,19 @@ struct DenseStage {
   float xs[RT];
 };
 
-// grid (column tiles of 64 x row tiles of 16 RT, 1, SK).  Slice z takes groups [z * per, (z + 1) * per), its waves
-// split them again (added in wave order); SK > 1 leaves the slice's fp32 sums in part[z].
+// A wave's walk over groups [g, g1) of a column tile for rows r0 .. r0 + valid - 1.  `flush(g, acc)` is called after
+// group g has been added (wave-uniform); it may park and clear acc.  Result i of acc[r][t]: row 16 r + kq + 4 i, column
+// 16 t + c.
 // A lane ends with four of the matrix instruction's rows: 4 kq + (0..3).  The call's row p is put into row
 // 4 (p % 4) + p / 4, so that up to four rows fill the lanes' first results and up to eight the first two: a call of at
-// most 4 NI rows adds NI results up a lane, not four (17408 x 5120, one row: 17.9 -> 16.3 us).
-template <int GS, int WAVES, int RT, int NI, bool COH = false>
-__device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
-                                          const uint32_t* __restrict__ W, const uint16_t* __restrict__ S,
-                                          const uint16_t* __restrict__ B, int64_t sb_stride, void* __restrict__ out,
-                                          float* __restrict__ part_out, int M, int N, int KG, int SK, int f32, int block,
-                                          int slice, float* part) {
-  constexpr int CH = GS / 32, ROWS = 16 * RT;
-  const int tiles = (N + 63) >> 6, tile = block % tiles, r0 = block / tiles * ROWS, valid = min(ROWS, M - r0);
-  const int per = KG / SK, gs0 = slice * per;
-  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, kq = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+// most 4 NI rows adds NI results up a lane, not four (17408 x 5120, one row: 17.9 us with NI = 4 for every call, 16.3 so).
+template <int GS, int RT, int NI, class FLUSH>
+__device__ __forceinline__ void qmm_walk(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
+                                         const uint32_t* __restrict__ W, const uint16_t* __restrict__ S,
+                                         const uint16_t* __restrict__ B, int64_t sb_stride, int KG, int tile, int r0,
+                                         int valid, int g, int g1, float (&acc)[RT][4][NI], const FLUSH& flush) {
+  constexpr int CH = GS / 32;
+  const int lane = threadIdx.x & 63, c = lane & 15, kq = lane >> 4;
   static_assert(RT == 1 || NI == 4, "more than 16 rows need every result");
   const uint32_t* wt = W + ((size_t)tile * KG) * (size_t)(CH * 256);
   const uint32_t wo = lane * 4, co = tile * 64 + lane;
@@ -138,7 +135,6 @@ __device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_
     xl[r] = X + (size_t)(r0 + min(16 * r + (c >> 2) + 4 * (c & 3), valid - 1)) * ldx + 8 * kq;
     xsl[r] = XS + (size_t)(r0 + min(16 * r + kq + 4 * (c & (NI - 1)), valid - 1)) * KG;
   }
-  float acc[RT][4][NI];
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
@@ -161,7 +157,7 @@ __device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_
     // sums into one load, which arrives with the last stage.  (Two row tiles: 30.2 us so where 28.4 without.)
     if constexpr (RT == 1) asm volatile("" ::: "memory");
   };
-  auto add = [&](const Stg& st) __attribute__((always_inline)) {
+  auto add = [&](const Stg& st, int at) __attribute__((always_inline)) {
     f32x4_t p[RT][4];
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
@@ -194,10 +190,9 @@ __device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_
         for (int i = 0; i < NI; ++i)
           acc[r][t][i] = fmaf(sc[i], bf16_hi(sb[t]), fmaf(p[r][t][i], bf16_lo(sb[t]), acc[r][t][i]));
     }
+    flush(at, acc);
   };
   Stg st[DEPTH];
-  int g = gs0 + (int)((long long)wave * per / WAVES);
-  const int g1 = gs0 + (int)((long long)(wave + 1) * per / WAVES);
 #pragma unroll
   for (int d = 0; d < DEPTH; ++d)
     if (g + d < g1) load(st[d], g + d);
@@ -206,20 +201,37 @@ __device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_
     prio_by_progress(g1 - g, n);
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
-      add(st[d]);
+      add(st[d], g + d);
       load(st[d], g + DEPTH + d);
     }
   }
 #pragma unroll
   for (int d = 0; d < DEPTH; ++d)
     if (g + d < g1) {
-      add(st[d]);
+      add(st[d], g + d);
       if (g + DEPTH + d < g1) load(st[d], g + DEPTH + d);
     }
 #pragma unroll
   for (int d = 0; d < DEPTH - 1; ++d)
-    if (g + DEPTH + d < g1) add(st[d]);
-  // result i of tile (r, t): row 16 r + kq + 4 i, column 16 t + c
+    if (g + DEPTH + d < g1) add(st[d], g + DEPTH + d);
+}
+
+// grid (column tiles of 64 x row tiles of 16 RT, 1, SK).  Slice z takes groups [z * per, (z + 1) * per), its waves
+// split them again (added in wave order); SK > 1 leaves the slice's fp32 sums in part[z].
+template <int GS, int WAVES, int RT, int NI, bool COH = false>
+__device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
+                                          const uint32_t* __restrict__ W, const uint16_t* __restrict__ S,
+                                          const uint16_t* __restrict__ B, int64_t sb_stride, void* __restrict__ out,
+                                          float* __restrict__ part_out, int M, int N, int KG, int SK, int f32, int block,
+                                          int slice, float* part) {
+  constexpr int ROWS = 16 * RT;
+  const int tiles = (N + 63) >> 6, tile = block % tiles, r0 = block / tiles * ROWS, valid = min(ROWS, M - r0);
+  const int per = KG / SK, gs0 = slice * per;
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  float acc[RT][4][NI];
+  qmm_walk<GS, RT, NI>(X, ldx, XS, W, S, B, sb_stride, KG, tile, r0, valid, gs0 + (int)((long long)wave * per / WAVES),
+                       gs0 + (int)((long long)(wave + 1) * per / WAVES), acc, [](int, float (&)[RT][4][NI]) {});
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
@@ -254,10 +266,78 @@ __global__ void __launch_bounds__(WAVES * 64)
                                lds);
 }
 
-// The split matmul of up to eight rows with its reduce in the same launch: a slice's workgroup leaves its sums in
-// part[z] with stores that go through to memory, waits for them to be acknowledged and counts itself in at the column
-// tile's counter; the workgroup that finds the others there adds the slices in slice order (qmm_reduce_kernel's
-// arithmetic) and puts the counter back to zero.
+// The split matmul of a few rows and its reduce in one launch with no traffic between workgroups, for callers without
+// arrival counters (whole_takes): a workgroup takes a column tile with all of K.  A second launch costs 1.5 to 2 us:
+// one row x 2048 x 512 4.3 us in two launches, 2.7 so; 8192 x 1024 4.8, 3.6; 17408 x 1024 5.8, 4.6.  The 4 SK runs of groups that qmm_kernel's waves
+// take (slice z, wave w: run 4 z + w) keep their ends; a wave walks 4 SK / WAVES of them one after the other, parks each
+// one's sums in LDS, and the end adds a slice's four and then the slices in order: the bits of qmm_kernel and
+// qmm_reduce_kernel.
+template <int GS, int WAVES, int NI>
+__device__ __forceinline__ void qmm_whole_block(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
+                                                const uint32_t* __restrict__ W, const uint16_t* __restrict__ S,
+                                                const uint16_t* __restrict__ B, int64_t sb_stride,
+                                                void* __restrict__ out, int M, int N, int KG, int SK, int f32, int tile,
+                                                float* part) {
+  constexpr int ROWS = 4 * NI;
+  const int per = KG / SK, runs = 4 * SK / WAVES;
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  auto begin = [&](int u) { return (u >> 2) * per + (int)((long long)(u & 3) * per / 4); };
+  auto park = [&](int u, float (&a)[1][4][NI]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < NI; ++i) part[(u * ROWS + kq + 4 * i) * QPART + 16 * t + c] = a[0][t][i], a[0][t][i] = 0.f;
+  };
+  float acc[1][4][NI];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < NI; ++i) acc[0][t][i] = 0.f;
+  const int u0 = wave * runs, u1 = u0 + runs;
+  if (per < 4)                              // runs without a group take part in the sums as zeros
+    for (int u = u0; u < u1; ++u) park(u, acc);
+  int u = u0;
+  while (u < u1 && begin(u + 1) == begin(u)) ++u;
+  int end = u < u1 ? begin(u + 1) : -1;
+  auto flush = [&](int g, float (&a)[1][4][NI]) __attribute__((always_inline)) {
+    if (g + 1 != end) return;
+    park(u, a);
+    ++u;
+    while (u < u1 && begin(u + 1) == begin(u)) ++u;
+    end = u < u1 ? begin(u + 1) : -1;
+  };
+  qmm_walk<GS, 1, NI>(X, ldx, XS, W, S, B, sb_stride, KG, tile, 0, M, begin(u0), begin(u1), acc, flush);
+  __syncthreads();
+  for (int o = tid; o < M * 64; o += WAVES * 64) {
+    const int r = o >> 6, l = o & 63, cc = tile * 64 + l;
+    if (cc >= N) continue;
+    float total = 0.f;
+    for (int z = 0; z < SK; ++z) {
+      const float* p = part + (4 * z * ROWS + r) * QPART + l;
+      float s = p[0];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) s += p[w * ROWS * QPART];
+      total = z ? total + s : s;
+    }
+    const size_t at = (size_t)r * N + cc;
+    if (f32) reinterpret_cast<float*>(out)[at] = total;
+    else reinterpret_cast<uint16_t*>(out)[at] = (uint16_t)f32_bf16_bits(total);
+  }
+}
+
+// LDS bytes of a workgroup (at most 34 KB: eight slices come with NI = 1 only)
+constexpr size_t qmm_whole_lds(int sk, int ni) { return sizeof(float) * 4 * sk * 4 * ni * QPART; }
+
+template <int GS, int WAVES, int NI>
+__global__ void __launch_bounds__(WAVES * 64)
+    qmm_whole_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
+                     const uint32_t* __restrict__ W, const uint16_t* __restrict__ S, const uint16_t* __restrict__ B,
+                     int64_t sb_stride, void* __restrict__ out, int M, int N, int KG, int SK, int f32) {
+  extern __shared__ float lds[];
+  qmm_whole_block<GS, WAVES, NI>(X, ldx, XS, W, S, B, sb_stride, out, M, N, KG, SK, f32, blockIdx.x, lds);
+}
+
 // What a slice's workgroup does once its sums are in part[z] (stored through to memory): wait for the stores'
 // acknowledgement, count itself in at the tile's counter, and if every other slice is there already add them up.
 template <int WAVES>
@@ -292,6 +372,10 @@ __device__ __forceinline__ void qmm_arrive_tail(int* __restrict__ counter, const
   if (threadIdx.x == 0) *counter = 0;   // every slice of the tile has arrived: ready for the next call
 }
 
+// The split matmul of up to eight rows with its reduce in the same launch: a slice's workgroup leaves its sums in
+// part[z] with stores that go through to memory, waits for them to be acknowledged and counts itself in at the column
+// tile's counter; the workgroup that finds the others there adds the slices in slice order (qmm_reduce_kernel's
+// arithmetic) and puts the counter back to zero.
 template <int GS, int WAVES, int NI>
 __global__ void __launch_bounds__(WAVES * 64)
     qmm_arrive_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
@@ -334,6 +418,20 @@ __global__ void __launch_bounds__(WAVES * 64)
   if ((int)blockIdx.z >= a.sk[w]) return;
   qmm_block<GS, WAVES, RT, NI>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], a.part[w], M, a.n[w], KG,
                                a.sk[w], f32, blockIdx.x - a.first[w], blockIdx.z, lds);
+}
+
+// the grouped launch on whole column tiles (qmm_whole_kernel's way) of weights that are all cut into 4 or 8 slices
+template <int GS, int NI>
+__global__ void __launch_bounds__(1024)
+    qmm_group_whole_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS, GroupArgs a, int M,
+                           int KG, int f32) {
+  extern __shared__ float lds[];
+  int w = 0;
+#pragma unroll
+  for (int i = 1; i < GROUP_MAX; ++i)
+    if (i < a.count && (int)blockIdx.x >= a.first[i]) w = i;
+  qmm_whole_block<GS, 16, NI>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], M, a.n[w], KG, a.sk[w], f32,
+                              blockIdx.x - a.first[w], lds);
 }
 
 // the grouped launch whose slices are added up by the last workgroup of a tile to finish (qmm_arrive_kernel's way);
@@ -406,6 +504,17 @@ __global__ void __launch_bounds__(256)
 
 constexpr int QMM_WAVES = 4;
 constexpr int ARRIVE_ROWS = 8;        // rows up to which, given arrival counters, the split launch adds its own slices
+
+// Without arrival counters: whether whole column tiles (one launch) are faster than the split launch and its reduce.
+// `tiles` column tiles of 64, two a compute unit for SK = 2 (eight waves), else one.  They are while K is short: 0.61 to
+// 0.97 of the time up to 1,536 inputs, and up to 3,072 (0.84 to 1.02) where the tiles fill half the chip; beyond, a tile's
+// 8 or 16 waves walk too long (8192 x 5120 1.00 to 1.16).  Eight slices are two runs a wave: only up to 1,024
+// inputs (0.84 to 0.98; at 1,536 1.02 to 1.11), and a call of more than four rows would not fit LDS.
+bool whole_takes(int64_t tiles, int sk, int m, int k) {
+  if (m > ARRIVE_ROWS || (sk != 2 && sk != 4 && sk != 8) || (sk > 2 && tiles > 256)) return false;
+  if (sk == 8) return m <= 4 && k <= 1024 && tiles >= 16;
+  return k <= 1536 || (k <= 3072 && tiles >= 128);
+}
 
 // Waves a workgroup of the expert GEMV: few workgroups (a small batch) spread each one's K over 16 waves, many
 // workgroups keep 4 longer-running waves each so that more of them are resident.  Scheduling only: bits do not move.
@@ -554,6 +663,26 @@ static int qmm_launch(const uint16_t* x, int64_t ldx, const float* xs, const uin
     TF_LAUNCH_OK("tf_qmm");
     return 0;
   }
+  if (reduce && whole_takes(tiles, sk, m, k)) {
+    const size_t whole = qmm_whole_lds(sk, m <= 4 ? 1 : 2);
+#define TF_GO(GS_, W_, NI_)                                                                                              \
+  qmm_whole_kernel<GS_, W_, NI_><<<(unsigned)tiles, W_ * 64, whole, s>>>(x, ldx, xs, weight, scales, biases, sb_stride, out, \
+                                                                         m, n, kg, sk, f32)
+    if (gs == 64) {
+      if (sk == 2 && m <= 4) TF_GO(64, 8, 1);
+      else if (sk == 2) TF_GO(64, 8, 2);
+      else if (m <= 4) TF_GO(64, 16, 1);
+      else TF_GO(64, 16, 2);
+    } else {
+      if (sk == 2 && m <= 4) TF_GO(32, 8, 1);
+      else if (sk == 2) TF_GO(32, 8, 2);
+      else if (m <= 4) TF_GO(32, 16, 1);
+      else TF_GO(32, 16, 2);
+    }
+#undef TF_GO
+    TF_LAUNCH_OK("tf_qmm");
+    return 0;
+  }
 #define TF_GO(GS_, RT_, NI_)                                                                                             \
   qmm_kernel<GS_, QMM_WAVES, RT_, NI_><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, weight, scales, biases, sb_stride, \
                                                                           out, part, m, n, kg, sk, f32)
@@ -657,6 +786,16 @@ extern "C" int tf_qmm_group(const uint16_t* x, int64_t ldx, const float* xs, int
   bool arrive = counters && m <= ARRIVE_ROWS;
   for (int i = 0; i < count && arrive; ++i)
     arrive = sks[i] == 1 || (counters[i] && (ns[i] + 63) / 64 <= n_counters[i]);
+  // no counters, and every K split four or eight ways: whole column tiles, as tf_qmm
+  bool whole = !arrive;
+  int64_t all_tiles = 0;
+  int most = 1;
+  for (int i = 0; i < count && whole; ++i) {
+    whole = sks[i] == 4 || sks[i] == 8;
+    all_tiles += ((int64_t)ns[i] + 63) / 64;
+    most = std::max(most, sks[i]);
+  }
+  whole = whole && whole_takes(all_tiles, most, m, k);
   const int rt = m <= 16 ? 1 : 2, rts = (m + 16 * rt - 1) / (16 * rt);
   GroupArgs a{}, r{};
   int max_sk = 1;
@@ -694,6 +833,20 @@ extern "C" int tf_qmm_group(const uint16_t* x, int64_t ldx, const float* xs, int
   if (arrive) {
 #define TF_GO(GS_, NI_) \
   qmm_group_arrive_kernel<GS_, QMM_WAVES, NI_><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, a, m, kg, f32)
+    if (gs == 64) {
+      if (m <= 4) TF_GO(64, 1);
+      else TF_GO(64, 2);
+    } else {
+      if (m <= 4) TF_GO(32, 1);
+      else TF_GO(32, 2);
+    }
+#undef TF_GO
+    TF_LAUNCH_OK("tf_qmm_group");
+    return 0;
+  }
+  if (whole) {
+    const size_t lds = qmm_whole_lds(max_sk, m <= 4 ? 1 : 2);
+#define TF_GO(GS_, NI_) qmm_group_whole_kernel<GS_, NI_><<<(unsigned)blocks, 1024, lds, s>>>(x, ldx, xs, a, m, kg, f32)
     if (gs == 64) {
       if (m <= 4) TF_GO(64, 1);
       else TF_GO(64, 2);
