@@ -60,7 +60,8 @@ int tf_group_sums(const uint16_t* x, int64_t ldx, int m, int k, int gs, float* x
  * rows of a call of up to 16 and 32 of a longer one, whatever it says.  sb_stride = elements between scale rows
  * (>= npad).  `counters` (may be NULL): n_counters arrival counters of the weight, TF_QMM_COUNTER_STRIDE ints apart,
  * zero on entry and left zero; with one for every column tile of 64, the slices of up to eight rows are added up in the
- * matmul's own launch by the last workgroup of a tile to finish (same order, same bits);
+ * matmul's own launch by the last workgroup of a tile to finish (same order, same bits); without, up to eight rows of a
+ * short K take one launch too (`part` then goes unused), and a longer K a reduce launch after the matmul's;
  * calls on one weight's counters must not overlap.  Replaces kernels/qmm.cpp:18-48 `qmm`. */
 #define TF_QMM_COUNTER_STRIDE 16
 int tf_qmm(const uint16_t* x, int64_t ldx, const float* xs, const uint32_t* weight, const uint16_t* scales,
@@ -82,8 +83,8 @@ int tf_qmm(const uint16_t* x, int64_t ldx, const float* xs, const uint32_t* weig
 int tf_qmm_static(const uint16_t* x, int64_t ldx, const float* xs, const uint32_t* weight, const uint16_t* scales,
                   const uint16_t* biases, int64_t sb_stride, void* out, int m, int n, int k, int sk, int gs, int bm,
                   int f32, tf_stream_t stream);
-/* `count` (1 to 4) weights against one x in one launch (plus one reduce launch when any K is split and the rows are
- * many): the bits of tf_qmm on each.  The arrays are host arrays of `count` entries, read during the call: packed weights, transposed
+/* `count` (1 to 4) weights against one x in one launch (plus one reduce launch when any K is split, unless up to eight
+ * rows have counters or a short K): the bits of tf_qmm on each.  The arrays are host arrays of `count` entries, read during the call: packed weights, transposed
  * scales and biases with their row strides, outputs, parts (fp32 [sks[i], m, ns[i]], may be NULL where sks[i] == 1),
  * column counts and slice counts; `counters` (may be NULL) the weights' arrival counters with their counts, as in
  * tf_qmm: with them up to eight rows take one launch in which every weight's slices are added up by the last

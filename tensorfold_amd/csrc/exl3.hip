@@ -566,10 +566,11 @@ struct GemmGrid {
 // Row tiles (of 16) a workgroup: 8 where the chip is full, fewer where 128-row tiles would leave compute units idle or
 // a last round nearly empty.  Estimated time: the fullest XCD's tiles a compute unit, times what a tile takes there,
 // measured in us at K = 5120 alone (38, 48, 63, 80 for 32, 64, 96, 128 rows: a chain over K) and among others (32, 40,
-// 55, 70: a smaller tile reads as much of W8 for fewer rows).  Against 128 rows always: 200 x 1024 80 -> 38 us, 777 x 3072
-// 82 -> 52, 1,400 x 5120 122 -> 89, 1,000 x 17408 216 -> 206 by itself (the whole
-// call 269 either way); over 70 shapes 0.69 at the (geometric) mean, none
-// slower.  An odd count of row tiles leaves half the threads a piece more to load and is 1.3 to 2 times slower.
+// 55, 70: a smaller tile reads as much of W8 for fewer rows).  Against 128 rows always: 200 x 1024 80 -> 38 us, 777 x
+// 3072 82 -> 52, 1,400 x 5120 122 -> 89, 1,000 x 17408 216 -> 206 by itself (the whole call 269 either way); over 70
+// shapes 0.69 at the (geometric) mean, none slower, and none of 240 with K = 128 to 2048 (0.55).  The rule does not look
+// at K, whose shorter chains favour smaller tiles still more: 1,000 x 5120 x 1536 46 us with the 128 rows it picks, 37
+// with 32.  An odd count of row tiles leaves half the threads a piece more to load and is 1.3 to 2 times slower.
 static int gemm_row_tiles(int m, int n) {
   if (((int64_t)m + 127) / 128 * ((n + GEMM_COLS - 1) / GEMM_COLS) > 4096) return 8;         // eight rounds and more
   constexpr int ALONE[4] = {38, 48, 63, 80}, AMONG[4] = {32, 40, 55, 70};

@@ -48,7 +48,8 @@ __host__ __device__ constexpr int delta(int j) {
 // shift that lines it up is then 31 to 0 and one v_alignbit_b32 does it.  With 0 to 31 the case of no shift needed a
 // select, and the compiler made it a branch around the second word's LDS read, one in every column tile: the walk
 // waited on two LDS round trips in a row sixteen times a pair (that and the runs' wider loads: 8 rows through 288 experts at 4
-// bits 250 -> 234 us, an MLP at 3 bits and one row 63.3 -> 59.4; a pair of k tiles is 241 vector instructions at 4 bits).
+// bits 250 -> 234 us, an MLP at 3 bits and one row 63.3 -> 59.4; a pair of k tiles is 225 vector instructions beside 16
+// matrix ones at 4 bits of mcg, 291 at 3 bits of 3inst).
 template <int K2>
 struct Windows {
   static constexpr int TW = tile_words<K2>(), R = 32 * TW;

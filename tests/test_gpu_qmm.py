@@ -101,8 +101,8 @@ def test_rows_do_not_depend_on_row_count(n, k, gs):
 @pytest.mark.parametrize("n,k,gs", [(4096, 4096, 64), (200, 1024, 32), (1536, 2048, 32)])
 def test_the_slices_added_in_the_matmuls_own_launch(n, k, gs):
     """Up to eight rows with a weight's arrival counters: the last workgroup of a tile adds the K slices up; without
-    them the one-launch form runs (or, past eight rows, a second launch).  The same bits, the counters zero again
-    afterwards, also on replays of a graph; more rows take the other forms whatever is passed."""
+    them (at these K) and past eight rows a second launch does.  The same bits, the counters zero again afterwards,
+    also on replays of a graph."""
 
     from tensorfold_amd import _lib
 

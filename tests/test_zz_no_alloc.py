@@ -39,8 +39,8 @@ def test_static_scratch_matches_the_part_buffer_twice(f32):
         x = synthetic.activations(rows, k, seed).to(DEV)
         want, got = both(x, q, sk, f32)
         assert torch.equal(want, got), (rows, f32)
-    # up to eight rows finish in one launch: the library's own arrival counters there, tf_qmm (given none) in its
-    # one-launch form; the counters are back at zero after each call, so calls in a row agree
+    # up to eight rows finish in one launch on the library's own arrival counters, tf_qmm (given none, and a long K) in
+    # two; the counters are back at zero after each call, so calls in a row agree
     for rows, seed in ((3, 3), (8, 4), (1, 5), (1, 6), (5, 7)):
         x = synthetic.activations(rows, k, seed).to(DEV)
         want, got = both(x, q, sk, f32)
