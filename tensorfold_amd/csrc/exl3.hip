@@ -95,10 +95,10 @@ __global__ void __launch_bounds__(WK * 64, K2 <= 12 ? 4 : 1)
     if (counters && !mlp) counters += z * 8 * NB * TF_EXL3_COUNTER_STRIDE;
   }
   const int arrivals = mlp ? 2 * SK : SK;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane & 15, kq = lane >> 4;
   const int L = 4 * (c & 7) + kq, h = c >> 3;
   const int pairs = K >> 5, slot = split * WK + wave, nslots = SK * WK;
-  const int pr0 = (int)((long long)slot * pairs / nslots), pr1 = (int)((long long)(slot + 1) * pairs / nslots);
+  const int pr0 = first_pair(slot, pairs, nslots), pr1 = first_pair(slot + 1, pairs, nslots);
   const uint32_t* tiles = T + (size_t)nb * stride_nb;
   const int col0 = nb * 128;
   TF_MARK(0);
@@ -115,13 +115,9 @@ __global__ void __launch_bounds__(WK * 64, K2 <= 12 ? 4 : 1)
     TF_MARK(1);
     wave_block<K2, CB>(xr, tiles, stride_k, pr0, pr1, stage, lane, L, h, acc);
     TF_MARK(2);
-    // D[row 4 kq + i][column c] of column tile j -> red[wave][row][16 j + c]
     __syncthreads();
     TF_MARK(3);
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) red[(wave * 16 + 4 * kq + i) * 128 + 16 * j + c] = acc[j][i];
+    store_rows(red + wave * (16 * 128), acc, R, c, kq);
     __syncthreads();
     // a wave a row: the waves' sums in wave order, two columns a lane
     for (int r = wave; r < R; r += WK) {

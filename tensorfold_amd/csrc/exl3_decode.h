@@ -49,7 +49,7 @@ __host__ __device__ constexpr int delta(int j) {
 // select, and the compiler made it a branch around the second word's LDS read, one in every column tile: the walk
 // waited on two LDS round trips in a row sixteen times a pair (that and the runs' wider loads: 8 rows through 288 experts at 4
 // bits 250 -> 234 us, an MLP at 3 bits and one row 63.3 -> 59.4; a pair of k tiles is 225 vector instructions beside 16
-// matrix ones at 4 bits of mcg, 291 at 3 bits of 3inst).
+// matrix ones at 4 bits of mcg).
 template <int K2>
 struct Windows {
   static constexpr int TW = tile_words<K2>(), R = 32 * TW;
@@ -84,10 +84,20 @@ struct Windows {
   }
 };
 
-// The hashed word of a state of the 3inst and mcg codebooks: the value is the fp16 sum of its two halves.
+// The hashed word of a state of the 3inst and mcg codebooks: the value is the fp16 sum of its two halves.  3inst's multiply
+// and add are one v_mad_u64_u32 (2.08 ns a wave and SIMD against 1.75 each for a multiply and an add; the upper half of its
+// result is not used, which the compiler must not learn): 227 vector instructions a pair of k tiles instead of 291, an MLP
+// 5120 -> 17408 -> 5120 at 3 bits and one row 59.7 -> 55.9 us.
 template <int CB>
 __device__ __forceinline__ uint32_t code_word(uint32_t s) {
-  const uint32_t x = CB == 1 ? s * 0xCBAC1FEDu : s * 89226354u + 64248484u;
+  uint32_t x;
+  if constexpr (CB == 1) {
+    x = s * 0xCBAC1FEDu;
+  } else {
+    uint64_t wide = (uint64_t)s * 89226354u + 64248484u;
+    asm("" : "+v"(wide));
+    x = (uint32_t)wide;
+  }
   return (x & 0x8FFF8FFFu) ^ 0x3B603B60u;
 }
 
@@ -239,6 +249,13 @@ __device__ __forceinline__ void swiglu_rot(float g0, float g1, float u0, float u
   store2(xh, TF_F16, at, a * HAD_SCALE, b * HAD_SCALE);
 }
 
+// The first of `pairs` k-tile pairs of slot `slot` out of `nslots` (at most 65,535): floor(slot * pairs / nslots) without
+// a 64-bit division.
+__device__ __forceinline__ int first_pair(uint32_t slot, uint32_t pairs, uint32_t nslots) {
+  const uint32_t q = pairs / nslots, r = pairs - q * nslots;
+  return (int)(slot * q + slot * r / nslots);
+}
+
 // One wave's sums of up to 16 rows over the k-tile pairs [pr0, pr1) of a 128-column block: acc[j] is the 16 x 16
 // tile of column tile j.  xr: the lane's A row (row c of the pass) + 2 kq; stage: this wave's own 16 * 128 words of LDS.
 template <int K2, int CB>
@@ -335,6 +352,20 @@ __device__ __forceinline__ void wave_block(const uint16_t* xr, const uint32_t* t
     }
     __builtin_amdgcn_wave_barrier();
     av = an;
+  }
+}
+
+// A pass's sums, D[row 4 kq + i][column c] of column tile j, to red[row][16 j + c]: the rows the pass has, no others.  A wave walks
+// four to six pairs, so what it does once weighs: with one row a quarter of the stores are left (that MLP 55.9 -> 51.6 us, 8 rows
+// through 288 experts 230 -> 223).
+__device__ __forceinline__ void store_rows(float* red, const f32x4_t (&acc)[8], int rows, int c, int kq) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (i >= rows) break;
+    if (4 * kq + i < rows) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) red[(4 * kq + i) * 128 + 16 * j + c] = acc[j][i];
+    }
   }
 }
 

@@ -148,10 +148,10 @@ __device__ __forceinline__ void grouped_body(const GroupedArgs& g, const uint32_
                                              int cnt, int mat, float* red) {
   constexpr int TW = tile_words<K2>();
   const int nb = blockIdx.x, split = blockIdx.y;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane & 15, kq = lane >> 4;
   const int L = 4 * (c & 7) + kq, h = c >> 3;
   const int pairs = g.K >> 5, slot = split * XWK + wave, nslots = g.SK * XWK;
-  const int pr0 = (int)((long long)slot * pairs / nslots), pr1 = (int)((long long)(slot + 1) * pairs / nslots);
+  const int pr0 = first_pair(slot, pairs, nslots), pr1 = first_pair(slot + 1, pairs, nslots);
   const int64_t stride_k = (int64_t)(g.N >> 4) * TW;          // the checkpoint's order: [K / 16][N / 16][TW] words
   const uint32_t* tiles = T + (size_t)nb * 8 * TW;
   f32x4_t acc[8];
@@ -162,12 +162,8 @@ __device__ __forceinline__ void grouped_body(const GroupedArgs& g, const uint32_
   const uint16_t* xr = xh + (size_t)pc * g.K + 2 * kq;
   uint32_t* stage = reinterpret_cast<uint32_t*>(red) + wave * (16 * 128);
   wave_block<K2, CB>(xr, tiles, stride_k, pr0, pr1, stage, lane, L, h, acc);
-  // D[row 4 kq + i][column c] of column tile j -> red[wave][row][16 j + c]
   __syncthreads();
-#pragma unroll
-  for (int j = 0; j < 8; ++j)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) red[(wave * 16 + 4 * kq + i) * 128 + 16 * j + c] = acc[j][i];
+  store_rows(red + wave * (16 * 128), acc, cnt, c, kq);
   __syncthreads();
   // a wave a row: the waves' sums in wave order, two columns a lane
   float* zs = g.Z + (size_t)(mat * g.SK + split) * g.P * g.N + nb * 128 + 2 * lane;
