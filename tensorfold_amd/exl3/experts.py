@@ -156,11 +156,13 @@ def prepare_stacked(gt: torch.Tensor, ut: torch.Tensor, dt: torch.Tensor, suh_g,
 
 def default_config(k: int, n: int, gateup: bool = True) -> int:
     """K splits of a K -> N projection: the shape's alone, so a row's sums run in one order at every row count.
-    As many as keep four tile pairs a wave and at most 128 (column block, split) workgroups an item."""
+    As many as keep three tile pairs a wave and at most 64 (column block, split) workgroups an item: a wave's head and tail cost
+    it about a pair (4096 -> 2048 -> 4096 at 4 bits with (4, 2) splits, (8, 4) before: 50.7 us at one row, was 50.3; 220.5 at 8
+    rows, was 232.0; 379.6 at 16, was 396.3; 2048 -> 768 -> 2048 with (4, 2), (4, 1) before: 27.3, was 29.3)."""
 
     pairs, nb = k // 32, n // 128
     for sk in (8, 4, 2):
-        if pairs // (WAVES * sk) >= 4 and nb * sk <= 128:
+        if pairs // (WAVES * sk) >= 3 and nb * sk <= 64:
             return sk
     if pairs < WAVES:
         raise ValueError(f"K={k} is too short for {WAVES} waves")

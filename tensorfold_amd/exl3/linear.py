@@ -28,10 +28,19 @@ def k2_of(bits: float) -> int:
 
 def plan(k: int, n: int, waves: int = 4096, min_pairs: int = 4) -> tuple[int, int]:
     """(K splits, waves a workgroup) of a K x N layer, from the shape alone so that a layer keeps one reduction
-    order at every row count.  The decode is bound by vector arithmetic, every wave of a launch is resident at once,
-    and the launch ends with the busiest SIMD: a column block of 128 gets as many waves (splits x waves a workgroup)
-    as put just under four on each of an MI355X's 1,024 SIMDs, none of them with fewer than ``min_pairs`` pairs of k
-    tiles.  Many waves a block go eight a workgroup, so that the splits' partial sums stay few."""
+    order at every row count.
+
+    A launch ends with its busiest compute unit, so a pair (sk, wk) is priced by what that unit does: the four-wave
+    workgroups it gets (2.5 at the least: SIMDs of one or two waves issue less often), each as long as its longest wave's
+    pairs of k tiles plus two for a wave's head and tail, and 0.4 for every split whose partial sums the last
+    workgroup of a column block reads back (fitted to 14 shapes).  A layer wider than it is deep is priced by itself and, half, as
+    one of a stack of two (an MLP's gate and up).  The cheapest wins, the fewest splits among equals, where
+    it is a twelfth cheaper than a fixed number of waves a SIMD (closer than that the price is not to be trusted).  Against
+    that number (us, 3 bits, 1 / 12 rows): 12288 x 4096 (8, 8) 14.3 / 17.3, was (12, 8) 16.7 / 21.9;
+    2048 x 2048 (8, 8) 8.4 / 11.0, was (4, 4) 9.7 / 13.3; an MLP 4096 -> 12288 35.1 / 42.3 at 1 / 8 rows, was 37.0 / 45.8;
+    1024 -> 2048 16.8 / 20.8, was 19.8 / 26.0.
+    Layers of more than 512 column blocks, and callers that give ``waves`` or ``min_pairs``, keep the fixed number: so many
+    waves in a launch, none with fewer pairs."""
 
     pairs, nb = k // 32, n // 128
     slots = max(2, min(waves // max(nb, 1), pairs // min_pairs, 512))
@@ -39,7 +48,20 @@ def plan(k: int, n: int, waves: int = 4096, min_pairs: int = 4) -> tuple[int, in
     sk = max(1, min(64, slots // wk))
     while wk > 2 and sk * wk > pairs:
         wk //= 2
-    return min(sk, max(1, pairs // wk)), wk
+    even = min(sk, max(1, pairs // wk)), wk
+    if nb > 512 or pairs < 8 or (waves, min_pairs) != (4096, 4):
+        return even
+
+    def price(sk: int, wk: int, layers: int) -> float:
+        units = max(2.5, -(-nb * sk * layers // 256) * wk / 4)
+        return units * (-(-pairs // (sk * wk)) + 2) + (0.4 * sk if sk > 1 else 0)
+
+    def cost(split: tuple[int, int]) -> tuple[float, int, int]:
+        sk, wk = split
+        return price(sk, wk, 1) + (price(sk, wk, 2) / 2 if n > k else 0), sk, -wk
+
+    best = min(((sk, wk) for wk in (8, 4) for sk in range(1, 65) if sk * wk <= pairs), key=cost)
+    return best if 12 * cost(best)[0] < 11 * cost(even)[0] else even
 
 
 def strips(words: torch.Tensor) -> torch.Tensor:
