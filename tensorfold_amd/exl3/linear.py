@@ -9,6 +9,7 @@ order and applies the output Hadamard, svh and the bias.
 from __future__ import annotations
 
 import dataclasses
+import functools
 
 import torch
 
@@ -26,6 +27,7 @@ def k2_of(bits: float) -> int:
     return int(2 * fmt.check_bits(bits))
 
 
+@functools.lru_cache(maxsize=1024)
 def plan(k: int, n: int, waves: int = 4096, min_pairs: int = 4) -> tuple[int, int]:
     """(K splits, waves a workgroup) of a K x N layer, from the shape alone so that a layer keeps one reduction
     order at every row count.
