@@ -10,36 +10,37 @@
 namespace tf {
 namespace {
 
-// xh = fp16(((x * suh) H) / sqrt(128)), a wave a (row, block of 128); a workgroup walks rows blockIdx.y, + gridDim.y, ...
-// blockIdx.z is the layer of a stack: its own suh [K] and xh [M, K] over the one x.
+// xh = fp16(((x * suh) H) / sqrt(128)), sixteen lanes a (row, block of 128), eight values a lane; groups of lanes walk the
+// blocks of x as they lie in memory, two at a time.  blockIdx.y is the layer of a stack: its own suh [K] and xh [M, K] over the one
+// x.  Bound by memory once the butterflies stay in registers (1,000 rows x 5120: 11.2 us with a wave a block and
+// ds_bpermute, 6.5 now).
 __global__ void __launch_bounds__(256)
     rot_in_kernel(const void* __restrict__ x, int x_dtype, const uint16_t* __restrict__ suh, uint16_t* __restrict__ xh,
-                  int M, int K) {
-  const int blk = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (blk * 128 >= K) return;
-  suh += (size_t)blockIdx.z * K;
-  xh += (size_t)blockIdx.z * M * K;
-  const int k = blk * 128 + 2 * lane;
-  float sa, sb;
-  load2(suh, TF_F16, k, sa, sb);
-  // four rows' loads are in flight together
-  for (int row0 = blockIdx.y; row0 < M; row0 += 4 * gridDim.y) {
-    float a[4], b[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int row = row0 + u * gridDim.y;
-      if (row < M) load2(x, x_dtype, (size_t)row * K + k, a[u], b[u]);
+                  uint32_t blocks, int K) {
+  const int lane = threadIdx.x & 63, sub = lane & 15;
+  suh += (size_t)blockIdx.y * K;
+  xh += (size_t)blockIdx.y * blocks * 128;
+  const uint32_t groups = gridDim.x * 16, kb = (uint32_t)K >> 7;
+  for (uint32_t u = blockIdx.x * 16 + (threadIdx.x >> 4); u < blocks; u += 2 * groups) {
+    const uint32_t u1 = u + groups;                                           // the second block of the two
+    const bool two = u1 < blocks;
+    float s[8], s1[8], v[8], v1[8];
+    load8(x, x_dtype, (size_t)u * 128 + 8 * sub, v);
+    load8(suh, TF_F16, (u % kb) * 128 + 8 * sub, s);
+    if (two) {
+      load8(x, x_dtype, (size_t)u1 * 128 + 8 * sub, v1);
+      load8(suh, TF_F16, (u1 % kb) * 128 + 8 * sub, s1);
     }
+    auto finish = [&](uint32_t at, float (&w)[8], const float (&f)[8]) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int row = row0 + u * gridDim.y;
-      if (row < M) {
-        a[u] *= sa;
-        b[u] *= sb;
-        fwht128(a[u], b[u], lane);
-        store2(xh, TF_F16, (size_t)row * K + k, a[u] * HAD_SCALE, b[u] * HAD_SCALE);
-      }
-    }
+      for (int i = 0; i < 8; ++i) w[i] *= f[i];
+      fwht128x8(w, lane);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) w[i] *= HAD_SCALE;
+      store8(xh, TF_F16, (size_t)at * 128 + 8 * sub, w);
+    };
+    finish(u, v, s);
+    if (two) finish(u1, v1, s1);
   }
 }
 
@@ -242,15 +243,15 @@ __global__ void __launch_bounds__(256)
 // operands come straight from W8 into registers (16 bytes a lane, 16 neighbouring lanes one 256-byte run: the cache
 // sees 8 full lines a load, not 64 lanes' separate pieces), requested two steps of 64 inputs ahead; xh goes a step
 // ahead through registers into LDS (two stages, 144-byte rows), one barrier a step.
-// The epilogue is linear_kernel's: a row tile's sums through LDS, a wave a (row, 128-column block): FWHT, scale, bias.
+// The epilogue is linear_kernel's: a row tile's sums through LDS, sixteen lanes a (row, 128-column block): FWHT, scale, bias.
 // A row's arithmetic does not depend on the other rows, on M or on the tile it falls in.
 //
 // Workgroups reach the XCDs round-robin (blockIdx % 8) and each XCD has its own L2: the workgroups an XCD runs
 // together (2^g_log2 consecutive ones) take an RG x CG block of tiles, so what they stream in step from beyond L2 is
 // RG tiles of xh and CG of W8, not one of each a workgroup.
 constexpr int GEMM_KSTEP = 64, GEMM_AROW = 2 * GEMM_KSTEP + 16, GEMM_WAVES = 4, GEMM_COLS = 64 * GEMM_WAVES;
-// two stages of xh, or the epilogue's 16 rows of a workgroup's columns if those are more
-constexpr int gemm_lds(int rt) { return max(2 * 16 * rt * GEMM_AROW, 16 * (GEMM_COLS + 4) * 4); }     // bytes
+// two stages of xh, or the epilogue's two row tiles of a workgroup's columns if those are more
+constexpr int gemm_lds(int rt) { return max(2 * 16 * rt * GEMM_AROW, 2 * 16 * (GEMM_COLS + 4) * 4); }     // bytes
 
 template <int RT>
 __global__ void __launch_bounds__(64 * GEMM_WAVES, 2)
@@ -349,7 +350,7 @@ __global__ void __launch_bounds__(64 * GEMM_WAVES, 2)
           if (t + 2 < 2 * RT) a2 = read_a(t + 2);
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            acc[j][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(f16x8_t, b[u][j][i]), acc[j][r], 0, 0, 0);
+            acc[j][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, b[u][j][i]), a, acc[j][r], 0, 0, 0);
           a = a1;
           a1 = a2;
           // keep the order written here: one LDS read two row tiles ahead of the four MFMAs it feeds
@@ -365,23 +366,37 @@ __global__ void __launch_bounds__(64 * GEMM_WAVES, 2)
       __syncthreads();
     }
   }
-  // D[row 4 kq + e][column c] of tile (j, r) -> LDS [16 rows][RED] a row tile at a time, then a wave a (row, block)
+  // With the weights first a tile comes out columns down: the lane holds columns 4 kq .. 4 kq + 3 of row c, one 16-byte LDS
+  // write.  A row tile goes to LDS [16 rows][RED], two of them in turn (one barrier a row tile), and sixteen lanes finish
+  // a (row, 128-column block): a thread's block and columns are the same in every row, so its scales are loaded once.
   float* red = reinterpret_cast<float*>(smem);
+  const int blk = (tid >> 4) & (WAVES / 2 - 1), col = col0 + 128 * blk + 8 * (tid & 15);
+  const bool cok = col0 + 128 * blk < N;
+  float sv[8], bv[8];
+  if (cok) load8(svh, TF_F16, col, sv);
+  if (cok && bias) load8(bias, TF_F16, col, bv);
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
-    if (r) __syncthreads();
+    float* buf = red + (r & 1) * 16 * RED;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) red[(4 * kq + e) * RED + 64 * wave + 16 * j + c] = acc[j][r][e];
+    for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4_t*>(buf + c * RED + 64 * wave + 16 * j + 4 * kq) = acc[j][r];
     __syncthreads();
-    for (int unit = wave; unit < 8 * WAVES; unit += WAVES) {
-      const int row = unit / (WAVES / 2), blk = unit % (WAVES / 2);
-      const int grow = m0 + 16 * r + row, col = col0 + 128 * blk + 2 * lane;
-      if (grow < M && col0 + 128 * blk < N) {
-        const float2 v = *reinterpret_cast<const float2*>(red + row * RED + 128 * blk + 2 * lane);
-        finish_row(v.x, v.y, lane, svh, bias, col, y, y_dtype, (size_t)grow * y_stride + col);
+    if (!cok) continue;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int row = 8 * u + (tid >> 4) / (WAVES / 2), grow = m0 + 16 * r + row;
+      if (grow >= M) continue;                             // the sixteen lanes of a block leave together
+      const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(buf + row * RED + 128 * blk + 8 * (tid & 15));
+      const f32x4_t hi = *reinterpret_cast<const f32x4_t*>(buf + row * RED + 128 * blk + 8 * (tid & 15) + 4);
+      float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      fwht128x8(v, lane);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = v[i] * HAD_SCALE * sv[i];
+      if (bias) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] += bv[i];
       }
+      store8(y, y_dtype, (size_t)grow * y_stride + col, v);
     }
   }
 }
@@ -400,7 +415,10 @@ static int rot_in_launch(const char* who, const void* x, int x_dtype, const uint
   TF_REQUIRE(m >= 1 && k >= 128 && k % 128 == 0, "x and xh must be [M, K], K a multiple of 128, suh [K]");
   TF_REQUIRE(layers >= 1 && layers <= 64, "%s: 1 to 64 layers a stack", who);
   TF_REQUIRE(aligned16(x) && aligned16(xh), "x: must be 16-byte aligned");
-  rot_in_kernel<<<dim3((k / 128 + 3) / 4, m < 1024 ? m : 1024, layers), 256, 0, as_stream(stream)>>>(x, x_dtype, suh, xh, m, k);
+  // sixteen blocks a workgroup, thirty-two once that fills the chip; past 4,096 workgroups they walk
+  const int64_t blocks = (int64_t)m * (k / 128), groups = blocks < 16384 ? (blocks + 15) / 16 : (blocks + 31) / 32;
+  TF_REQUIRE(blocks < (1LL << 31), "%s: %lld blocks of 128 are more than a launch counts", who, (long long)blocks);
+  rot_in_kernel<<<dim3((unsigned)(groups < 4096 ? groups : 4096), layers), 256, 0, as_stream(stream)>>>(x, x_dtype, suh, xh, (uint32_t)blocks, k);
   TF_LAUNCH_OK(who);
   return 0;
 }

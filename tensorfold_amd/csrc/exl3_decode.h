@@ -153,17 +153,108 @@ __device__ __forceinline__ void values4(const uint32_t* tile, int L, int h, uint
   v[3] = (uint16_t)(hi >> 16);
 }
 
+// The lane's value of another lane of its row of 16: lane ^ M.  gfx9 has quad permutes, a row's halves mirrored (lane ^ 7) and a
+// rotation of the row, so 4 is two moves.
+template <int M>
+__device__ __forceinline__ float row_xor(float v) {
+  static_assert(M == 1 || M == 2 || M == 4 || M == 8, "inside a row of 16 lanes");
+  int u = __builtin_bit_cast(int, v);
+  if constexpr (M == 1) u = __builtin_amdgcn_mov_dpp(u, 0xB1, 0xF, 0xF, true);
+  if constexpr (M == 2) u = __builtin_amdgcn_mov_dpp(u, 0x4E, 0xF, 0xF, true);
+  if constexpr (M == 4) u = __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(u, 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF, true);
+  if constexpr (M == 8) u = __builtin_amdgcn_mov_dpp(u, 0x128, 0xF, 0xF, true);
+  return __builtin_bit_cast(float, u);
+}
+
+// One butterfly step between lane and lane ^ M: the lower lane's sum, the upper lane's (lower - upper) difference, each one
+// rounding.  Steps of 16 and 32 lanes are the lane-swap instructions: of two copies of a value one ends with the lower
+// lane's in both places, the other with the upper's.  All six steps stay in registers; through LDS (ds_bpermute) a step
+// was a round trip of a hundred cycles, and the steps bound the prompt's rotation and the tail of every decode launch.
+template <int M>
+__device__ __forceinline__ float butterfly(float v, int lane) {
+  const float sign = (lane & M) ? -1.f : 1.f;
+  if constexpr (M < 16) {
+    return fmaf(v, sign, row_xor<M>(v));
+  } else {
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto t = M == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false) : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return fmaf(__builtin_bit_cast(float, (uint32_t)t[1]), sign, __builtin_bit_cast(float, (uint32_t)t[0]));
+  }
+}
+
 // Unscaled Walsh-Hadamard transform of 128 values, two a lane (elements 2 lane, 2 lane + 1), fixed butterfly order.
 __device__ __forceinline__ void fwht128(float& a, float& b, int lane) {
   const float s = a + b, d = a - b;
-  a = s;
-  b = d;
+  a = butterfly<1>(s, lane), b = butterfly<1>(d, lane);
+  a = butterfly<2>(a, lane), b = butterfly<2>(b, lane);
+  a = butterfly<4>(a, lane), b = butterfly<4>(b, lane);
+  a = butterfly<8>(a, lane), b = butterfly<8>(b, lane);
+  a = butterfly<16>(a, lane), b = butterfly<16>(b, lane);
+  a = butterfly<32>(a, lane), b = butterfly<32>(b, lane);
+}
+
+// The same transform of four blocks a wave, eight values a lane (elements 8 (lane % 16) on): the same sums in the same
+// order, so the same bits; three steps between a lane's own values, four between lanes, for eight values at once.
+__device__ __forceinline__ void fwht128x8(float (&v)[8], int lane) {
 #pragma unroll
-  for (int m = 1; m < 64; m <<= 1) {
-    const float oa = __shfl_xor(a, m), ob = __shfl_xor(b, m);
-    a = (lane & m) ? oa - a : a + oa;
-    b = (lane & m) ? ob - b : b + ob;
+  for (int m = 1; m < 8; m <<= 1)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (!(i & m)) {
+        const float s = v[i] + v[i + m], d = v[i] - v[i + m];
+        v[i] = s;
+        v[i + m] = d;
+      }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = butterfly<1>(v[i], lane);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = butterfly<2>(v[i], lane);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = butterfly<4>(v[i], lane);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = butterfly<8>(v[i], lane);
+}
+
+// eight values at element i, a multiple of 8, of a tensor that starts on any 4 bytes
+typedef uint32_t __attribute__((ext_vector_type(4), aligned(4))) words4_t;
+
+__device__ __forceinline__ void load8(const void* p, int dtype, size_t i, float (&v)[8]) {
+  if (dtype == TF_F32) {
+    const words4_t u = *reinterpret_cast<const words4_t*>(static_cast<const float*>(p) + i);
+    const words4_t w = *reinterpret_cast<const words4_t*>(static_cast<const float*>(p) + i + 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = __builtin_bit_cast(float, (uint32_t)u[j]), v[4 + j] = __builtin_bit_cast(float, (uint32_t)w[j]);
+    return;
   }
+  const words4_t u = *reinterpret_cast<const words4_t*>(static_cast<const uint16_t*>(p) + i);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (dtype == TF_BF16) {
+      v[2 * j] = bf16_lo(u[j]);
+      v[2 * j + 1] = bf16_hi(u[j]);
+    } else {
+      const uint32_t w = u[j];
+      const __half2 h = __builtin_bit_cast(__half2, w);
+      v[2 * j] = __low2float(h);
+      v[2 * j + 1] = __high2float(h);
+    }
+  }
+}
+
+__device__ __forceinline__ void store8(void* p, int dtype, size_t i, const float (&v)[8]) {
+  if (dtype == TF_F32) {
+    words4_t u, w;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) u[j] = __builtin_bit_cast(uint32_t, v[j]), w[j] = __builtin_bit_cast(uint32_t, v[4 + j]);
+    *reinterpret_cast<words4_t*>(static_cast<float*>(p) + i) = u;
+    *reinterpret_cast<words4_t*>(static_cast<float*>(p) + i + 4) = w;
+    return;
+  }
+  words4_t u;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    u[j] = dtype == TF_BF16 ? pack_bf16(v[2 * j], v[2 * j + 1]) : __builtin_bit_cast(uint32_t, __floats2half2_rn(v[2 * j], v[2 * j + 1]));
+  *reinterpret_cast<words4_t*>(static_cast<uint16_t*>(p) + i) = u;
 }
 
 __device__ __forceinline__ void load2(const void* p, int dtype, size_t i, float& a, float& b) {
@@ -271,7 +362,6 @@ __device__ __forceinline__ void wave_block(const uint16_t* xr, const uint32_t* t
   constexpr int NW = Windows<K2>::NW;
   constexpr int RUN = 8 * TW, PER = RUN / 64, N4 = PER / 4, REM = PER % 4;      // words a run; whole words a lane
   constexpr bool HALF = RUN % 64 != 0;                                          // an odd K2: 32 words more
-  typedef uint32_t __attribute__((ext_vector_type(4), aligned(4))) words4_t;    // a trellis may start on any word
   const Windows<K2> win(L, h);
   pr0 = __builtin_amdgcn_readfirstlane(pr0);
   pr1 = __builtin_amdgcn_readfirstlane(pr1);
