@@ -246,10 +246,11 @@ __global__ void __launch_bounds__(256)
 // The epilogue is linear_kernel's: a row tile's sums through LDS, sixteen lanes a (row, 128-column block): FWHT, scale, bias.
 // A row's arithmetic does not depend on the other rows, on M or on the tile it falls in.
 //
-// Workgroups reach the XCDs round-robin (blockIdx % 8) and each XCD has its own L2: the workgroups an XCD runs
-// together (2^g_log2 consecutive ones) take an RG x CG block of tiles, so what they stream in step from beyond L2 is
-// RG tiles of xh and CG of W8, not one of each a workgroup.
-constexpr int GEMM_KSTEP = 64, GEMM_AROW = 2 * GEMM_KSTEP + 16, GEMM_WAVES = 4, GEMM_COLS = 64 * GEMM_WAVES;
+// Workgroups reach the XCDs round-robin (blockIdx % 8) and each XCD has its own L2: an XCD takes one run of the tiles,
+// walked down groups of GEMM_GROUP row tiles, so its 64 co-resident workgroups are about 8 x 8 tiles and what they stream in
+// step from beyond L2 is 8 tiles of xh and 8 of W8, not one of each a workgroup.  The runs differ by one tile at most
+// (whole 8 x 8 or 8 x 4 blocks dealt out to the XCDs gave the fullest of them 96 of 1,000 x 17408's 544 tiles, where 68 are its share).
+constexpr int GEMM_GROUP = 8, GEMM_KSTEP = 64, GEMM_AROW = 2 * GEMM_KSTEP + 16, GEMM_WAVES = 4, GEMM_COLS = 64 * GEMM_WAVES;
 // two stages of xh, or the epilogue's two row tiles of a workgroup's columns if those are more
 constexpr int gemm_lds(int rt) { return max(2 * 16 * rt * GEMM_AROW, 2 * 16 * (GEMM_COLS + 4) * 4); }     // bytes
 
@@ -257,17 +258,15 @@ template <int RT>
 __global__ void __launch_bounds__(64 * GEMM_WAVES, 2)
     gemm_kernel(const uint16_t* __restrict__ xh, const uint16_t* __restrict__ W8, const uint16_t* __restrict__ svh,
                 const uint16_t* __restrict__ bias, void* __restrict__ y, int y_dtype, int64_t y_stride, int M, int K,
-                int N, int rts, int cts, int rg_log2, int g_log2) {
+                int N, int rts, int cts, int per_xcd) {
   constexpr int WAVES = GEMM_WAVES, THREADS = 64 * WAVES, COLS = GEMM_COLS, RED = COLS + 4;     // RED: floats a row of the epilogue's tile
   constexpr int ROWS = 16 * RT, GEMM_STAGE = ROWS * GEMM_AROW;
   extern __shared__ __align__(16) unsigned char smem[];
-  const int RG = 1 << rg_log2, CG = 1 << (g_log2 - rg_log2);
-  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
-  const int super = (local >> g_log2) * 8 + xcd, place = local & ((1 << g_log2) - 1);
-  const int rgs = (rts + RG - 1) >> rg_log2;
-  const int sc = super / rgs, sr = super - sc * rgs;
-  const int rt = sr * RG + (place & (RG - 1)), ct = sc * CG + (place >> rg_log2);
-  if (rt >= rts || ct >= cts) return;
+  // an XCD's share of the tiles, GEMM_GROUP row tiles of a column, then the next column's
+  const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (tile >= rts * cts) return;
+  const int group = tile / (GEMM_GROUP * cts), at = tile - group * (GEMM_GROUP * cts), high = min(GEMM_GROUP, rts - group * GEMM_GROUP);
+  const int ct = at / high, rt = group * GEMM_GROUP + at - ct * high;
   const int m0 = rt * ROWS, col0 = ct * COLS;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, kq = lane >> 4;
   const bool wok = col0 + 64 * wave < N;                   // N is a multiple of 128: a pair of waves falls out together
@@ -290,9 +289,11 @@ __global__ void __launch_bounds__(64 * GEMM_WAVES, 2)
       dst[j][i] = __builtin_amdgcn_raw_buffer_load_b128(wsrc, boff[j], (step * 8 + 4 * i) * octet, 0);
   };
   // A: the workgroup's rows of xh as one buffer; this thread's 16-byte pieces of a step: piece q = (row q / 8,
-  // 8 inputs q % 8); rows past M read the last row and are dropped at the end
-  constexpr int PPT = 8 * ROWS / THREADS;
-  static_assert(8 * ROWS % THREADS == 0, "whole pieces a thread");
+  // 8 inputs q % 8); rows past M read the last row and are dropped at the end.  An odd row tile is 8 bytes a thread (a
+  // 16-byte piece for half of the threads cost every step a wait of its own: 1.3 to 2 times the time).
+  constexpr int PPT = RT / 2;
+  constexpr bool ODD = RT % 2;
+  typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
   const int nrows = min(ROWS, M - m0);
   const __amdgpu_buffer_rsrc_t asrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(xh + (size_t)m0 * K), 0, (uint32_t)nrows * (uint32_t)K * 2u, 0x00020000);
@@ -302,10 +303,14 @@ __global__ void __launch_bounds__(64 * GEMM_WAVES, 2)
     const int q = tid + THREADS * j;
     aoff[j] = ((uint32_t)min(q >> 3, nrows - 1) * (uint32_t)K + (q & 7) * 8) * 2u;
   }
+  const int odd_row = 16 * (RT - 1) + (tid >> 4);
+  const uint32_t odd_off = ((uint32_t)min(odd_row, nrows - 1) * (uint32_t)K + (tid & 15) * 4) * 2u;
   u32x4_t ar[PPT];
+  u32x2_t ao;
   auto load_a = [&](int step) {
 #pragma unroll
     for (int j = 0; j < PPT; ++j) ar[j] = __builtin_amdgcn_raw_buffer_load_b128(asrc, aoff[j], step * (GEMM_KSTEP * 2), 0);
+    if constexpr (ODD) ao = __builtin_amdgcn_raw_buffer_load_b64(asrc, odd_off, step * (GEMM_KSTEP * 2), 0);
   };
   auto store_a = [&](int buf) {
 #pragma unroll
@@ -313,6 +318,7 @@ __global__ void __launch_bounds__(64 * GEMM_WAVES, 2)
       const int q = tid + THREADS * j;
       *reinterpret_cast<u32x4_t*>(smem + buf * GEMM_STAGE + (q >> 3) * GEMM_AROW + (q & 7) * 16) = ar[j];
     }
+    if constexpr (ODD) *reinterpret_cast<u32x2_t*>(smem + buf * GEMM_STAGE + odd_row * GEMM_AROW + (tid & 15) * 8) = ao;
   };
 
   f32x4_t acc[4][RT];
@@ -549,51 +555,23 @@ extern "C" int tf_exl3_unpack_k8(const uint32_t* T, uint16_t* W8, int k, int n, 
   return 1;
 }
 
-// The tiles along the grid's XCD order: an XCD's 2^g_log2 consecutive workgroups take 2^rg_log2 row tiles x the rest
-// column tiles; smaller groups when the whole grid would not give every XCD two of them.
-struct GemmGrid {
-  int64_t rts, cts, supers;
-  int g_log2, rg_log2;
-  GemmGrid(int m, int n, int rt) {
-    rts = ((int64_t)m + 16 * rt - 1) / (16 * rt), cts = (n + GEMM_COLS - 1) / GEMM_COLS;
-    for (g_log2 = 6;; --g_log2) {
-      rg_log2 = 0;
-      while (rg_log2 < 3 && rg_log2 < g_log2 && (1 << rg_log2) < rts) ++rg_log2;
-      const int64_t cg = 1 << (g_log2 - rg_log2);
-      supers = ((rts + (1 << rg_log2) - 1) >> rg_log2) * ((cts + cg - 1) / cg);
-      if (supers >= 16 || g_log2 == 3) break;
-    }
-  }
-  // the tiles of the XCD that has the most
-  int64_t fullest() const {
-    int64_t tiles[8] = {}, most = 0;
-    const int64_t rg = 1 << rg_log2, cg = 1 << (g_log2 - rg_log2), rgs = (rts + rg - 1) / rg;
-    for (int64_t s = 0; s < supers; ++s) {
-      const int64_t sc = s / rgs, sr = s - sc * rgs;
-      const int64_t t = tiles[s & 7] += std::min(rg, rts - sr * rg) * std::min(cg, cts - sc * cg);
-      most = std::max(most, t);
-    }
-    return most;
-  }
-};
-
-// Row tiles (of 16) a workgroup: 8 where the chip is full, fewer where 128-row tiles would leave compute units idle or
-// a last round nearly empty.  Estimated time: the fullest XCD's tiles a compute unit, times what a tile takes there,
-// measured in us at K = 5120 alone (38, 48, 63, 80 for 32, 64, 96, 128 rows: a chain over K) and among others (32, 40,
-// 55, 70: a smaller tile reads as much of W8 for fewer rows).  Against 128 rows always: 200 x 1024 80 -> 38 us, 777 x
-// 3072 82 -> 52, 1,400 x 5120 122 -> 89, 1,000 x 17408 216 -> 206 by itself (the whole call 269 either way); over 70
-// shapes 0.69 at the (geometric) mean, none slower, and none of 240 with K = 128 to 2048 (0.55).  The rule does not look
-// at K, whose shorter chains favour smaller tiles still more: 1,000 x 5120 x 1536 46 us with the 128 rows it picks, 37
-// with 32.  An odd count of row tiles leaves half the threads a piece more to load and is 1.3 to 2 times slower.
+// Row tiles (of 16) a workgroup, 2 to 9.  Estimated time: the tiles a compute unit gets, times what a tile takes there,
+// measured in us at K = 5120 alone (a chain over K) and among others (a smaller tile reads as much of W8 for fewer rows).
+// Nine row tiles are what 256 registers hold; they earn their place where seven of 144 rows end a round that eight of 128 would
+// start another for.  1,000 x 5120 x 17408: 185 us with the 64-row tiles taken when 32, 64, 96 and 128 rows were the choice, 146
+// with 144; 512 rows 112 -> 90 (80-row tiles); 1,000 x 5120 x 5120 68 -> 56; 3,000 x 4096 x 12288 265 -> 239; 4,096 x 5120 x
+// 17408 602 -> 577 (128 rows as before: the XCDs' even shares).  The rule does not look at K, whose shorter chains favour smaller
+// tiles still more.
 static int gemm_row_tiles(int m, int n) {
   if (((int64_t)m + 127) / 128 * ((n + GEMM_COLS - 1) / GEMM_COLS) > 4096) return 8;         // eight rounds and more
-  constexpr int ALONE[4] = {38, 48, 63, 80}, AMONG[4] = {32, 40, 55, 70};
+  constexpr int ALONE[10] = {0, 0, 36, 39, 41, 47, 53, 60, 66, 74}, AMONG[10] = {0, 0, 30, 36, 39, 44, 51, 57, 63, 72};
   int best = 8;
   int64_t least = INT64_MAX;
-  for (int i = 3; i >= 0; --i) {
-    const int64_t per = (GemmGrid(m, n, 2 * (i + 1)).fullest() + 31) / 32;                   // 32 compute units an XCD
-    const int64_t time = per <= 1 ? ALONE[i] : per * AMONG[i];
-    if (time < least) least = time, best = 2 * (i + 1);
+  for (int rt = 9; rt >= 2; --rt) {
+    const int64_t tiles = ((int64_t)m + 16 * rt - 1) / (16 * rt) * ((n + GEMM_COLS - 1) / GEMM_COLS);
+    const int64_t per = (tiles + 255) / 256;
+    const int64_t time = per <= 1 ? ALONE[rt] : per * AMONG[rt];
+    if (time < least) least = time, best = rt;
   }
   return best;
 }
@@ -608,16 +586,16 @@ extern "C" int tf_exl3_gemm(const uint16_t* xh, const uint16_t* w8, const uint16
   TF_REQUIRE(y_stride >= n && y_stride % 2 == 0, "y rows hold at least N values, an even stride apart");
   TF_REQUIRE(aligned16(xh) && aligned16(w8) && ((uintptr_t)y & 7) == 0, "xh, W8 16-byte and y 8-byte aligned");
   const int tile = gemm_row_tiles(m, n);
-  const GemmGrid gg(m, n, tile);
-  TF_REQUIRE(gg.rts <= 0x3FFFFF, "gemm: too many rows for one launch");
-  const int64_t grid = (gg.supers + 7) / 8 * (8 << gg.g_log2);
+  const int64_t rts = ((int64_t)m + 16 * tile - 1) / (16 * tile), cts = (n + GEMM_COLS - 1) / GEMM_COLS;
+  const int64_t per_xcd = (rts * cts + 7) / 8, grid = 8 * per_xcd;
+  TF_REQUIRE(rts <= 0x3FFFFF, "gemm: too many rows for one launch");
   TF_REQUIRE(grid <= 0x7FFFFFFF, "gemm: %lld workgroups exceed the grid limit", (long long)grid);
 #define TF_GEMM(RT_)                                                                                                 \
   case RT_:                                                                                                          \
     gemm_kernel<RT_><<<dim3((unsigned)grid), 64 * GEMM_WAVES, gemm_lds(RT_), as_stream(stream)>>>(                   \
-        xh, w8, svh, bias, y, y_dtype, y_stride, m, k, n, (int)gg.rts, (int)gg.cts, gg.rg_log2, gg.g_log2);          \
+        xh, w8, svh, bias, y, y_dtype, y_stride, m, k, n, (int)rts, (int)cts, (int)per_xcd);          \
     break;
-  switch (tile) { TF_GEMM(2) TF_GEMM(4) TF_GEMM(6) TF_GEMM(8) }
+  switch (tile) { TF_GEMM(2) TF_GEMM(3) TF_GEMM(4) TF_GEMM(5) TF_GEMM(6) TF_GEMM(7) TF_GEMM(8) TF_GEMM(9) }
 #undef TF_GEMM
   TF_LAUNCH_OK("tf_exl3_gemm");
   return 0;
