@@ -214,23 +214,49 @@ __global__ void __launch_bounds__(64)
 }
 
 // W_q as [K / 8][N][8] fp16, the order an MFMA B operand is read in: the 8 consecutive inputs a lane holds are 16
-// bytes, and the 16 columns of a tile lie side by side, so a wave's operand load is four runs of 256 bytes.  A lane's
-// four values are two pairs of consecutive inputs of one column: two 4-byte stores, a wave's a run of 256 bytes each.
-// A workgroup takes four k-tiles of a 128-column block, a wave the eight tiles of one of them.
+// bytes, and the 16 columns of a tile lie side by side, so a wave's operand load is four runs of 256 bytes.
+// A workgroup takes four k-tiles of a 128-column block, a wave the eight tiles of one of them: their stored words come in by
+// 16-byte loads and go through the wave's part of LDS to the lanes whose windows start there; the decoded pairs of inputs go
+// back through it and leave as four stores of 16 bytes a lane, runs of 2 KB.  (With a lane loading its own words and
+// storing its own pairs, 32 memory instructions of 4 bytes a wave, the address unit's 16 cycles an instruction were the whole
+// time: 5120 x 17408 at 3 bits 43 us, now 34.)
 template <int K2, int CB>
 __global__ void __launch_bounds__(256)
     unpack_k8_kernel(const uint32_t* __restrict__ T, uint16_t* __restrict__ W8, int N, int64_t stride_k,
                      int64_t stride_nb) {
-  const int kt = 4 * blockIdx.y + (threadIdx.x >> 6), nb = blockIdx.x, lane = threadIdx.x & 63, L = lane & 31, h = lane >> 5;
-  const uint32_t* tiles = T + (size_t)kt * stride_k + (size_t)nb * stride_nb;
-  const int col = (L >> 2) + 8 * h;                      // values j = 0, 1: inputs 2 (L & 3), + 1; j = 2, 3: those + 8
-  uint32_t* dst = reinterpret_cast<uint32_t*>(W8) + ((size_t)(2 * kt) * N + nb * 128 + col) * 4 + (L & 3);
+  constexpr int TW = tile_words<K2>(), PIECES = 2 * TW;                    // a run of eight tiles in 16-byte pieces
+  static_assert(8 * TW <= 1024, "the run fits where the values go");
+  __shared__ __align__(16) uint32_t stage[4][1024];                        // [octet of two][column][4 pairs of inputs]
+  const int wave = threadIdx.x >> 6, kt = 4 * blockIdx.y + wave, nb = blockIdx.x, lane = threadIdx.x & 63, L = lane & 31, h = lane >> 5;
+  const uint32_t* run = T + (size_t)kt * stride_k + (size_t)nb * stride_nb;
+  uint32_t* own = stage[wave];
+#pragma unroll
+  for (int i = 0; i < (PIECES + 63) / 64; ++i) {
+    const int piece = 64 * i + lane;
+    if (PIECES % 64 == 0 || piece < PIECES)
+      *reinterpret_cast<u32x4_t*>(own + 4 * piece) = *reinterpret_cast<const words4_t*>(run + 4 * piece);
+  }
+  __builtin_amdgcn_wave_barrier();                       // the wave's LDS accesses run in program order
+  const Windows<K2> win(L, h);
+  uint32_t lo[8], hi[8];                                 // inputs 2 (L & 3), + 1 of column (L >> 2) + 8 h; those + 8
 #pragma unroll
   for (int t = 0; t < 8; ++t) {
-    uint16_t v[4];
-    values4<K2, CB>(tiles + t * tile_words<K2>(), L, h, v);
-    dst[t * 64] = (uint32_t)v[0] | ((uint32_t)v[1] << 16);
-    dst[(size_t)N * 4 + t * 64] = (uint32_t)v[2] | ((uint32_t)v[3] << 16);
+    uint32_t w[Windows<K2>::NW];
+    win.load(own + t * TW, w);
+    decode4<K2, CB>(win, w, lo[t], hi[t]);
+  }
+  __builtin_amdgcn_wave_barrier();
+  const int at = 4 * ((L >> 2) + 8 * h) + (L & 3);
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    own[64 * t + at] = lo[t];
+    own[512 + 64 * t + at] = hi[t];
+  }
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {                          // octet i / 2, columns 64 (i % 2) + lane
+    uint16_t* dst = W8 + ((size_t)(2 * kt + i / 2) * N + nb * 128 + 64 * (i % 2) + lane) * 8;
+    *reinterpret_cast<u32x4_t*>(dst) = *reinterpret_cast<const u32x4_t*>(own + 4 * (64 * i + lane));
   }
 }
 
