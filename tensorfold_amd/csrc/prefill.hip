@@ -96,19 +96,17 @@ __device__ __forceinline__ uint32_t pack_bf16_rn(float lo, float hi) {
 }
 
 // one packed word -> the B operand in the same input order, each bf16(fma(q, s, b)) with s and b the stored bf16
-// values: round to nearest even, as the reference's __float2bfloat16_rn
+// values: round to nearest even, as the reference's __float2bfloat16_rn.  The codes convert two an instruction (a nibble in a byte
+// is the e4m3 number q * 2^-9): 19 vector instructions a word, 23 with a conversion a code, which the experts' bf16 form
+// is bound by (777 rows x 128 experts of 2688 x 1856, routing and all: 326 -> 314 us; dense 4096 cubed 127.4 -> 126.0).
 __device__ __forceinline__ bf16x8_t dequant8b(uint32_t w, uint32_t sb) {
   const float s = bf16_lo(sb), b = bf16_hi(sb);
-  uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
-  // the compiler is not to know that these are w's nibbles: knowing it, it extracts each of the eight from w and
-  // converts that (16 instructions), where a byte of lo or hi converts as it lies (v_cvt_f32_ubyte0..3: 8)
-  asm("" : "+v"(lo));
-  asm("" : "+v"(hi));
-  auto q = [](uint32_t v, int byte) { return (float)((v >> (8 * byte)) & 0xFFu); };
-  const u32x4_t r = {pack_bf16_rn(fmaf(q(lo, 0), s, b), fmaf(q(lo, 1), s, b)),
-                     pack_bf16_rn(fmaf(q(lo, 2), s, b), fmaf(q(lo, 3), s, b)),
-                     pack_bf16_rn(fmaf(q(hi, 0), s, b), fmaf(q(hi, 1), s, b)),
-                     pack_bf16_rn(fmaf(q(hi, 2), s, b), fmaf(q(hi, 3), s, b))};
+  const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
+  auto two = [&](uint32_t v, auto HI) {
+    const auto q = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(v, 512.f, decltype(HI)::value);
+    return pack_bf16_rn(fmaf(q[0], s, b), fmaf(q[1], s, b));
+  };
+  const u32x4_t r = {two(lo, std::false_type()), two(lo, std::true_type()), two(hi, std::false_type()), two(hi, std::true_type())};
   return __builtin_bit_cast(bf16x8_t, r);
 }
 
@@ -381,7 +379,7 @@ __global__ void __launch_bounds__(256)
 // ---- routed experts, big items ---------------------------------------------------------------------------------------
 //
 // An item of up to 128 pairs against 512 weight columns (NM = 1: 512 output columns; NM = 2: 256 output columns of
-// gate and of up).  Each of the eight waves owns 64 weight columns = four B operands and all eight 16-row tiles, so
+// gate and of up), or half as many (expert_waves).  Each of the eight or four waves owns 64 weight columns = four B operands and all eight 16-row tiles, so
 // one dequantized operand feeds eight MFMAs and one LDS read of the activations feeds four: per 32 inputs a wave
 // issues 32 MFMAs against 8 LDS reads and 4 dequantizations.  Weights are requested a step and a half (96 inputs)
 // ahead into registers and change lanes there, activations one step ahead through registers into the workgroup's
@@ -467,12 +465,12 @@ struct NoStaged {
 // then, and with them (a wave's vector memory operations complete in issue order) whatever the caller requested
 // before calling, which it can put away there without a wait of its own.
 template <int GS, int NM, int EPI, int RT, int AR, bool SWAP, class WS, int TJ = 4, int NTHREADS = BIG_THREADS,
-          bool STAGE_OUT = false, class STAGED = NoStaged>
+          bool STAGE_OUT = false, class STAGED = NoStaged, bool SKIP_IDLE = false>
 __device__ __forceinline__ void big_body(const uint16_t* __restrict__ X, int64_t x_stride, const WS& ws,
                                          const int (&ocol)[TJ], const bool (&jok)[TJ],
                                          int K, const int* src_rows, const int* dst_rows, int cnt,
                                          void* __restrict__ out, int N, float limit, unsigned char* smem,
-                                         STAGED&& staged = STAGED(), int thread = -1) {
+                                         STAGED&& staged = STAGED(), int thread = -1, bool busy = true) {
   constexpr int CPS = KSTEP / 32, GPS = KSTEP / GS;
   constexpr int ROWS = 16 * RT;
   constexpr int PIECES = ROWS * 8;                // 16-byte pieces of a staged tile
@@ -541,6 +539,22 @@ __device__ __forceinline__ void big_body(const uint16_t* __restrict__ X, int64_t
       return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, first), __builtin_bit_cast(f16x8_t, second), c, 0, 0, 0);
   };
   constexpr float UNSCALE = AR ? 1.f : WUNSCALE;
+
+  if (SKIP_IDLE && !busy) {
+    // a wave past the last column: its share of the activations only, not a dequantization that takes the others' issue
+    // slots (1856 columns are 29 tiles of 64 in units of four; 777 rows 314 -> 310 us)
+    uint4 v[PPT];
+    load_a(0, v);
+    store_a(0, v);
+    __syncthreads();
+    staged();
+    for (int step = 0; step < K / KSTEP; ++step) {
+      load_a(min(step + 1, K / KSTEP - 1), v);
+      store_a(~step & 1, v);
+      __syncthreads();
+    }
+    return;
+  }
 
   f32x4_t acc[TJ][RT];
 #pragma unroll
@@ -648,7 +662,7 @@ __device__ __forceinline__ void big_body(const uint16_t* __restrict__ X, int64_t
       constexpr int OJ = NM == 2 ? TJ / 2 : TJ;                  // 16-column tiles of output a wave
       constexpr int OROW = 16 * OJ * ES + 16;                    // bytes of a staged row (padded against bank conflicts)
       constexpr int CPR = 16 * OJ * ES / 16;                     // 16-byte pieces a row
-      static_assert(BIG_WAVES * 16 * OROW <= 2 * STAGE, "the output tiles of a workgroup's waves fit the activation stages");
+      static_assert(NTHREADS / 64 * 16 * OROW <= 2 * STAGE, "the output tiles of a workgroup's waves fit the activation stages");
       unsigned char* mine = smem + (tid >> 6) * (16 * OROW);
       const int col0 = ocol[0] - c;                              // the wave's first output column (its tiles are neighbours)
       unsigned okmask = 0;
@@ -736,17 +750,25 @@ __device__ __forceinline__ void big_body(const uint16_t* __restrict__ X, int64_t
   }
 }
 
+// Waves a workgroup of the experts' kernels, each 64 weight columns.  The bf16 form is bound by the vector instructions of its
+// dequantization (54 % of a launch's issue cycles, 25 % matrix, the two seldom side by side; requests three steps ahead gained
+// nothing): four waves, two workgroups a compute unit, whose barriers, heads and stores fall apart and whose units even out better
+// at the launch's end (777 rows x 128 experts of 2688 x 1856, routing and all: 360 -> 326 us).  The fp16 form spends half as much
+// on a weight, and staging the activations twice as often costs it more than that gains (4,096 rows x 512 experts 551 ->
+// 556 us, 500 rows 184 -> 193): eight waves.
+constexpr int expert_waves(int ar) { return ar == TF_ARITH_BF16 ? 4 : 8; }
+constexpr int expert_threads(int ar) { return 64 * expert_waves(ar); }
 // 32-column blocks a workgroup of the big kernel covers
-constexpr int big_blocks(int nm) { return nm == 2 ? BIG_WAVES : 2 * BIG_WAVES; }
+constexpr int big_blocks(int nm, int ar) { return nm == 2 ? expert_waves(ar) : 2 * expert_waves(ar); }
 
 template <int GS, int NM, int EPI, int AR>
-__global__ void __launch_bounds__(BIG_THREADS, 1)
+__global__ void __launch_bounds__(expert_threads(AR), expert_threads(AR) == 256 ? 2 : 1)
     experts_prefill_big_kernel(const uint16_t* __restrict__ X, int64_t x_stride, int slots,
                                const uint32_t* __restrict__ W, int KG, int NB, const int* __restrict__ items,
                                const int* __restrict__ counts, const int* __restrict__ members,
                                void* __restrict__ out, int N, float limit) {
   constexpr int BW = block_words(GS);
-  constexpr int NBW = big_blocks(NM);
+  constexpr int NBW = big_blocks(NM, AR);
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int src_rows[BIG_ROWS], dst_rows[BIG_ROWS];
   const int nbt = (NB + NBW - 1) / NBW;
@@ -786,9 +808,11 @@ __global__ void __launch_bounds__(BIG_THREADS, 1)
   // lines out through LDS (4 % of the launch); gate and up with the SwiGLU between them: neither (3 % the other way)
   constexpr bool OUT_LINES = NM == 1;
   const int K = KG * GS;
-  if (cnt <= 32) big_body<GS, NM, EPI, 2, AR, OUT_LINES, ExpertSource<GS, NM>, 4, BIG_THREADS, OUT_LINES>(X, x_stride, ws, ocol, jok, K, src_rows, dst_rows, cnt, out, N, limit, smem);
-  else if (cnt <= 64) big_body<GS, NM, EPI, 4, AR, OUT_LINES, ExpertSource<GS, NM>, 4, BIG_THREADS, OUT_LINES>(X, x_stride, ws, ocol, jok, K, src_rows, dst_rows, cnt, out, N, limit, smem);
-  else big_body<GS, NM, EPI, 8, AR, OUT_LINES, ExpertSource<GS, NM>, 4, BIG_THREADS, OUT_LINES>(X, x_stride, ws, ocol, jok, K, src_rows, dst_rows, cnt, out, N, limit, smem);
+  const bool busy = cbt * NBW + (NM == 2 ? wave : 2 * wave) < NB;          // the wave has a column
+  constexpr bool SKIP = AR == TF_ARITH_BF16;          // (the fp16 form's loop came out 1 % slower for it)
+  if (cnt <= 32) big_body<GS, NM, EPI, 2, AR, OUT_LINES, ExpertSource<GS, NM>, 4, expert_threads(AR), OUT_LINES, NoStaged, SKIP>(X, x_stride, ws, ocol, jok, K, src_rows, dst_rows, cnt, out, N, limit, smem, NoStaged(), tid, busy);
+  else if (cnt <= 64) big_body<GS, NM, EPI, 4, AR, OUT_LINES, ExpertSource<GS, NM>, 4, expert_threads(AR), OUT_LINES, NoStaged, SKIP>(X, x_stride, ws, ocol, jok, K, src_rows, dst_rows, cnt, out, N, limit, smem, NoStaged(), tid, busy);
+  else big_body<GS, NM, EPI, 8, AR, OUT_LINES, ExpertSource<GS, NM>, 4, expert_threads(AR), OUT_LINES, NoStaged, SKIP>(X, x_stride, ws, ocol, jok, K, src_rows, dst_rows, cnt, out, N, limit, smem, NoStaged(), tid, busy);
   TF_MARK(4);
 #ifdef TF_TIMELINE
   __builtin_amdgcn_s_waitcnt(0);         // mark 5 is the results written, not only issued
@@ -796,8 +820,8 @@ __global__ void __launch_bounds__(BIG_THREADS, 1)
   TF_MARK(5);
 }
 
-// The same units taken by workgroups that stay, one a compute unit (a unit = an item's 512 weight columns, as a
-// workgroup of experts_prefill_big_kernel takes).  A workgroup has a compute unit to itself (the body's registers), so
+// The same units taken by workgroups that stay, eight waves a compute unit (a unit = an item's 512 weight columns, 256 in the
+// bf16 form, as a workgroup of experts_prefill_big_kernel takes).  A workgroup has a compute unit to itself (the body's registers), so
 // in the kernel above nothing runs under a unit's head (the item's rows looked up through two dependent reads, then
 // the first operands' trip), its results' drain, and the dispatch of the next workgroup; and with five or six
 // workgroups of 47 to 67 us to a compute unit, those that got five sit idle for the last tenth of the launch.  Here
@@ -832,7 +856,7 @@ __device__ __forceinline__ void resident_unit(const uint16_t* __restrict__ X, in
                                               void* __restrict__ out, int N, float limit, int parity, int tid,
                                               STAGED& staged) {
   constexpr int BW = block_words(GS);
-  constexpr int NBW = big_blocks(NM);
+  constexpr int NBW = big_blocks(NM, AR);
   extern __shared__ __align__(16) unsigned char smem[];
   const int lane = tid & 63, wave = tid >> 6, c = lane & 15, kq = lane >> 4;
   ExpertSource<GS, NM> ws;
@@ -854,19 +878,21 @@ __device__ __forceinline__ void resident_unit(const uint16_t* __restrict__ X, in
     ws.sp = (blk + 32 * GS / 8 + (lane & 31)) * 4u;
   }
   constexpr bool OUT_LINES = NM == 1;
-  big_body<GS, NM, EPI, RT, AR, OUT_LINES, ExpertSource<GS, NM>, 4, BIG_THREADS, OUT_LINES>(
+  const bool busy = cbt * NBW + (NM == 2 ? wave : 2 * wave) < NB;          // the wave has a column
+  constexpr bool SKIP = AR == TF_ARITH_BF16;          // (the fp16 form's loop came out 1 % slower for it)
+  big_body<GS, NM, EPI, RT, AR, OUT_LINES, ExpertSource<GS, NM>, 4, expert_threads(AR), OUT_LINES, STAGED&, SKIP>(
       X, x_stride, ws, ocol, jok, KG * GS, resident_rows(parity, 0), resident_rows(parity, 1), cnt, out, N, limit, smem,
-      staged, tid);
+      staged, tid, busy);
 }
 
 template <int GS, int NM, int EPI, int AR>
-__global__ void __launch_bounds__(BIG_THREADS, 1)
+__global__ void __launch_bounds__(expert_threads(AR), expert_threads(AR) == 256 ? 2 : 1)
     experts_prefill_resident_kernel(const uint16_t* __restrict__ X, int64_t x_stride, int slots,
                                     const uint32_t* __restrict__ W, int KG, int NB, const int* __restrict__ items,
                                     const int* __restrict__ counts, int* __restrict__ ticket,
                                     const int* __restrict__ members, void* __restrict__ out, int N, float limit) {
   constexpr int BW = block_words(GS);
-  constexpr int NBW = big_blocks(NM);
+  constexpr int NBW = big_blocks(NM, AR);
   const int nbt = (NB + NBW - 1) / NBW;
   const int total = counts[0] * nbt, G = gridDim.x;
   // place q of the walk -> unit: two from the front of the plan (full items: matrix work), then one from its back
@@ -1269,29 +1295,24 @@ int launch_experts_prefill(int tile, int arith, const uint16_t* x, int64_t x_str
       else TF_SMALL(8, 0);
     }
   } else {
-    constexpr int NBW = big_blocks(NM);
-    const int64_t big = max_items * ((nb + NBW - 1) / NBW);
+    const int64_t big = max_items * ((nb + big_blocks(NM, arith) - 1) / big_blocks(NM, arith));
     TF_REQUIRE(big <= 0x7FFFFFFF, "experts: %lld workgroups exceed the grid limit", (long long)big);
-    // workgroups that stay and walk the units by stride, one a compute unit, once there are units to walk
-    const int cus = compute_units();
-    if (big > 2 * cus) {
-      const dim3 rg((unsigned)cus);
-      if (arith)
-        experts_prefill_resident_kernel<GS, NM, EPI, 1><<<rg, BIG_THREADS, RESIDENT_LDS, s>>>(
-            x, x_stride, slots, w, kg, nb, items, counts, counts + 2, members, out, n, limit);
-      else
-        experts_prefill_resident_kernel<GS, NM, EPI, 0><<<rg, BIG_THREADS, RESIDENT_LDS, s>>>(
-            x, x_stride, slots, w, kg, nb, items, counts, counts + 2, members, out, n, limit);
-      TF_LAUNCH_OK("tf_experts_prefill");
-      return 0;
-    }
-    const dim3 bg((unsigned)big);
-    if (arith)
-      experts_prefill_big_kernel<GS, NM, EPI, 1><<<bg, BIG_THREADS, BIG_LDS, s>>>(
-          x, x_stride, slots, w, kg, nb, items, counts, members, out, n, limit);
-    else
-      experts_prefill_big_kernel<GS, NM, EPI, 0><<<bg, BIG_THREADS, BIG_LDS, s>>>(
-          x, x_stride, slots, w, kg, nb, items, counts, members, out, n, limit);
+    // workgroups that stay and walk the units by stride, as many as the compute units hold, once there are units to walk
+    const int stay = compute_units() * 8 / expert_waves(arith);
+    const bool walk = big > 2 * stay;
+    const dim3 rg((unsigned)(walk ? stay : big));
+#define TF_BIG(AR_)                                                                                                      \
+  {                                                                                                                     \
+    if (walk)                                                                                                           \
+      experts_prefill_resident_kernel<GS, NM, EPI, AR_><<<rg, expert_threads(AR_), RESIDENT_LDS, s>>>(                   \
+          x, x_stride, slots, w, kg, nb, items, counts, counts + 2, members, out, n, limit);                            \
+    else                                                                                                                \
+      experts_prefill_big_kernel<GS, NM, EPI, AR_><<<rg, expert_threads(AR_), BIG_LDS, s>>>(                             \
+          x, x_stride, slots, w, kg, nb, items, counts, members, out, n, limit);                                        \
+  }
+    if (arith) TF_BIG(TF_ARITH_BF16)
+    else TF_BIG(TF_ARITH_F16)
+#undef TF_BIG
   }
 #undef TF_SMALL
   TF_LAUNCH_OK("tf_experts_prefill");
