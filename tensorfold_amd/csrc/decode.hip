@@ -216,9 +216,132 @@ __device__ __forceinline__ void qmm_walk(const uint16_t* __restrict__ X, int64_t
     if (g + DEPTH + d < g1) add(st[d], g + DEPTH + d);
 }
 
+// The walk of a call of 9 rows and more.  There qmm_walk's stages (one or two row tiles' inputs beside the weights) take 112 to 168
+// registers, and the compiler requested two of them together after adding both: every pair of groups waited for a whole
+// trip.  Here a stage is the wave's own corner of LDS, filled by loads that go straight there: a group's operands are read out, its
+// place takes the request for the group RING_STAGES on, and the arithmetic runs under both requests.  A wave waits for its
+// own loads by count; nothing crosses waves.  The same operands and the same order of sums as qmm_walk: the same bits.  17408 x
+// 5120: 9 rows 20.9 -> 19.4 us, 16 24.2 -> 20.4, 21 27.7 -> 22.9, 32 33.6 -> 26.4, 64 51.5 -> 37.4 (reduce and group
+// sums included); up to 8 rows qmm_walk is not so held up and keeps more workgroups a compute unit.  Two stages: three would take
+// the third workgroup's LDS.
+constexpr int RING_STAGES = 2;
+
+template <int GS, int RT>
+struct QmmRing {
+  static constexpr int CH = GS / 32;
+  static constexpr int AT_SB = CH * 1024, AT_X = AT_SB + 256, AT_XS = AT_X + RT * 16 * GS * 2, STAGE = AT_XS + RT * 64;      // bytes
+  static constexpr int LOADS = CH + 1 + RT * CH + 1;             // load instructions a group
+  static constexpr int WAVE = RING_STAGES * STAGE;
+};
+
+// Loads into LDS: a lane's 16 or 4 bytes go to `lds` + its share of the wave's run.  Written as instructions because the compiler
+// would wait for every load in flight ahead of any LDS read.
+__device__ __forceinline__ void to_lds16(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}
+__device__ __forceinline__ void to_lds4(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}
+__device__ __forceinline__ void lane_to_lds4(const void* p, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(p) : "memory");
+}
+
+template <int GS, int RT>
+__device__ __forceinline__ void qmm_ring_walk(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
+                                              const uint32_t* __restrict__ W, const uint16_t* __restrict__ S,
+                                              const uint16_t* __restrict__ B, int64_t sb_stride, int KG, int tile, int r0,
+                                              int valid, int g0, int g1, float (&acc)[RT][4][4], unsigned char* ring) {
+  typedef QmmRing<GS, RT> R;
+  constexpr int CH = R::CH, P = R::LOADS, ROW = GS * 2, PIECES = ROW / 16;       // bytes of a row's group of inputs; 16-byte pieces
+  const int lane = threadIdx.x & 63, c = lane & 15, kq = lane >> 4;
+  // operand row o of the matrix instruction's 16 RT holds this row of the call (qmm_walk has the reason)
+  auto call_row = [&](int o) { return min((o & ~15) + ((o & 15) >> 2) + 4 * (o & 3), valid - 1); };
+  // a row's pieces lie turned by its number, so that 16 lanes reading a piece of 16 rows meet different banks
+  auto turn = [&](int o) { return PIECES == 8 ? o & 7 : (o >> 1) & 3; };
+  uint32_t xoff[RT * CH];
+#pragma unroll
+  for (int j = 0; j < RT * CH; ++j) {
+    const int o = (64 / PIECES) * j + lane / PIECES;
+    xoff[j] = (uint32_t)call_row(o) * (uint32_t)ldx * 2u + (((lane % PIECES) ^ turn(o)) * 16);
+  }
+  const uint32_t xsoff = (uint32_t)call_row(lane & (16 * RT - 1)) * (uint32_t)KG * 4u;
+  const uint16_t* sb = (lane < 32 ? S : B) + tile * 64 + 2 * (lane & 31);
+  const uint16_t* x0 = X + (size_t)r0 * ldx;
+  const float* xs0 = XS + (size_t)r0 * KG;
+  const uint32_t* w0 = W + (size_t)tile * KG * (CH * 256);
+  const uint32_t at = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)ring);
+  auto request = [&](int g) {
+    const uint32_t lds = at + (g & (RING_STAGES - 1)) * R::STAGE;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) to_lds16(w0 + ((size_t)g * CH + i) * 256, lane * 16, lds + i * 1024);
+    lane_to_lds4(sb + (size_t)g * sb_stride, lds + R::AT_SB);
+#pragma unroll
+    for (int j = 0; j < RT * CH; ++j) to_lds16(x0 + (size_t)g * GS, xoff[j], lds + R::AT_X + j * 1024);
+    if (lane < 16 * RT) to_lds4(xs0 + g, xsoff, lds + R::AT_XS);
+  };
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[r][t][i] = 0.f;
+  for (int d = 0; d < RING_STAGES; ++d)
+    if (g0 + d < g1) request(g0 + d);
+  for (int g = g0; g < g1; ++g) {
+    static_assert(RING_STAGES == 2, "one group's loads may be on their way past the one waited for");
+    if (g + 1 < g1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(P) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const unsigned char* stage = ring + (g & (RING_STAGES - 1)) * R::STAGE;
+    uint32_t w[CH][4], s[4], b[4];
+    uint4 x[RT][CH];
+    float4 sums[RT];
+#pragma unroll
+    for (int i = 0; i < CH; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) w[i][t] = *reinterpret_cast<const uint32_t*>(stage + i * 1024 + (16 * t + c) * 16 + kq * 4);
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+#pragma unroll
+      for (int i = 0; i < CH; ++i)
+        x[r][i] = *reinterpret_cast<const uint4*>(stage + R::AT_X + (16 * r + c) * ROW + (((4 * i + kq) ^ turn(c)) * 16));
+      sums[r] = *reinterpret_cast<const float4*>(stage + R::AT_XS + (16 * r + 4 * kq) * 4);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      s[t] = *reinterpret_cast<const uint16_t*>(stage + R::AT_SB + (16 * t + c) * 2);
+      b[t] = *reinterpret_cast<const uint16_t*>(stage + R::AT_SB + 128 + (16 * t + c) * 2);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");          // the stage is read: its place is free
+    if (g + RING_STAGES < g1) request(g + RING_STAGES);
+    f32x4_t p[RT][4];
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      bf16x8_t xa[RT];
+#pragma unroll
+      for (int r = 0; r < RT; ++r) xa[r] = __builtin_bit_cast(bf16x8_t, stage8_bf16(x[r][i]));
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const bf16x8_t q = codes8(w[i][t]);
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+          p[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[r], q, i ? p[r][t] : (f32x4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      const float sc[4] = {sums[r].x, sums[r].y, sums[r].z, sums[r].w};
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc[r][t][i] = fmaf(sc[i], __uint_as_float(b[t] << 16), fmaf(p[r][t][i], __uint_as_float(s[t] << 16), acc[r][t][i]));
+    }
+  }
+}
+
 // grid (column tiles of 64 x row tiles of 16 RT, 1, SK).  Slice z takes groups [z * per, (z + 1) * per), its waves
 // split them again (added in wave order); SK > 1 leaves the slice's fp32 sums in part[z].
-template <int GS, int WAVES, int RT, int NI, bool COH = false>
+template <int GS, int WAVES, int RT, int NI, bool COH = false, bool RING = false>
 __device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
                                           const uint32_t* __restrict__ W, const uint16_t* __restrict__ S,
                                           const uint16_t* __restrict__ B, int64_t sb_stride, void* __restrict__ out,
@@ -230,8 +353,14 @@ __device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, kq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   float acc[RT][4][NI];
-  qmm_walk<GS, RT, NI>(X, ldx, XS, W, S, B, sb_stride, KG, tile, r0, valid, gs0 + (int)((long long)wave * per / WAVES),
-                       gs0 + (int)((long long)(wave + 1) * per / WAVES), acc, [](int, float (&)[RT][4][NI]) {});
+  const int g0 = gs0 + (int)((long long)wave * per / WAVES), g1 = gs0 + (int)((long long)(wave + 1) * per / WAVES);
+  if constexpr (RING) {
+    qmm_ring_walk<GS, RT>(X, ldx, XS, W, S, B, sb_stride, KG, tile, r0, valid, g0, g1, acc,
+                          reinterpret_cast<unsigned char*>(part) + wave * QmmRing<GS, RT>::WAVE);
+    __syncthreads();                                     // the rings are read: the sums take their place
+  } else {
+    qmm_walk<GS, RT, NI>(X, ldx, XS, W, S, B, sb_stride, KG, tile, r0, valid, g0, g1, acc, [](int, float (&)[RT][4][NI]) {});
+  }
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
@@ -255,14 +384,14 @@ __device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_
   }
 }
 
-template <int GS, int WAVES, int RT, int NI>
+template <int GS, int WAVES, int RT, int NI, bool RING = false>
 __global__ void __launch_bounds__(WAVES * 64)
     qmm_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
                const uint32_t* __restrict__ W, const uint16_t* __restrict__ S, const uint16_t* __restrict__ B,
                int64_t sb_stride, void* __restrict__ out, float* __restrict__ part_out, int M, int N, int KG, int SK,
                int f32) {
   extern __shared__ float lds[];
-  qmm_block<GS, WAVES, RT, NI>(X, ldx, XS, W, S, B, sb_stride, out, part_out, M, N, KG, SK, f32, blockIdx.x, blockIdx.z,
+  qmm_block<GS, WAVES, RT, NI, false, RING>(X, ldx, XS, W, S, B, sb_stride, out, part_out, M, N, KG, SK, f32, blockIdx.x, blockIdx.z,
                                lds);
 }
 
@@ -406,7 +535,7 @@ struct GroupArgs {
   int count;
 };
 
-template <int GS, int WAVES, int RT, int NI>
+template <int GS, int WAVES, int RT, int NI, bool RING = false>
 __global__ void __launch_bounds__(WAVES * 64)
     qmm_group_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS, GroupArgs a, int M,
                      int KG, int f32) {
@@ -416,7 +545,7 @@ __global__ void __launch_bounds__(WAVES * 64)
   for (int i = 1; i < GROUP_MAX; ++i)
     if (i < a.count && (int)blockIdx.x >= a.first[i]) w = i;
   if ((int)blockIdx.z >= a.sk[w]) return;
-  qmm_block<GS, WAVES, RT, NI>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], a.part[w], M, a.n[w], KG,
+  qmm_block<GS, WAVES, RT, NI, false, RING>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], a.part[w], M, a.n[w], KG,
                                a.sk[w], f32, blockIdx.x - a.first[w], blockIdx.z, lds);
 }
 
@@ -503,6 +632,16 @@ __global__ void __launch_bounds__(256)
 }
 
 constexpr int QMM_WAVES = 4;
+// What the ring walk takes besides 9 rows or more: its loads into LDS are of whole dwords (two columns' scales: an even row length on a 4-byte boundary) and
+// of 32-bit offsets from 32 rows' first.
+static bool ring_takes(int64_t ldx, int64_t sb_stride, const void* scales, const void* biases) {
+  return sb_stride % 2 == 0 && (((uintptr_t)scales | (uintptr_t)biases) & 3) == 0 && ldx < (1ll << 25);
+}
+// LDS of its workgroup: the waves' rings, and later their sums in the same place
+static size_t ring_lds(int gs, int rt) {
+  const int wave = gs == 64 ? (rt == 1 ? QmmRing<64, 1>::WAVE : QmmRing<64, 2>::WAVE) : rt == 1 ? QmmRing<32, 1>::WAVE : QmmRing<32, 2>::WAVE;
+  return std::max((size_t)QMM_WAVES * wave, sizeof(float) * qmm_lds_floats(QMM_WAVES, rt));
+}
 constexpr int ARRIVE_ROWS = 8;        // rows up to which, given arrival counters, the split launch adds its own slices
 
 // Without arrival counters: whether whole column tiles (one launch) are faster than the split launch and its reduce.
@@ -644,7 +783,8 @@ static int qmm_launch(const uint16_t* x, int64_t ldx, const float* xs, const uin
   // up to 16 rows are one row tile of the matrix instruction; past that a workgroup takes two (`bm` is the caller's row
   // tile: accepted, and no longer what decides)
   const int rt = m <= 16 ? 1 : 2, tiles = (n + 63) / 64, rts = (m + 16 * rt - 1) / (16 * rt);
-  const size_t smem = sizeof(float) * qmm_lds_floats(QMM_WAVES, rt);
+  const bool ring = m > 8 && ring_takes(ldx, sb_stride, scales, biases);
+  const size_t smem = ring ? ring_lds(gs, rt) : sizeof(float) * qmm_lds_floats(QMM_WAVES, rt);
   TF_REQUIRE((int64_t)tiles * rts <= 0x7FFFFFFF && sk <= 65535, "qmm: grid too large");
   const dim3 grid((unsigned)(tiles * rts), 1, (unsigned)sk);
   if (reduce && sk > 1 && counters && m <= ARRIVE_ROWS && tiles <= n_counters) {
@@ -683,19 +823,23 @@ static int qmm_launch(const uint16_t* x, int64_t ldx, const float* xs, const uin
     TF_LAUNCH_OK("tf_qmm");
     return 0;
   }
-#define TF_GO(GS_, RT_, NI_)                                                                                             \
-  qmm_kernel<GS_, QMM_WAVES, RT_, NI_><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, weight, scales, biases, sb_stride, \
-                                                                          out, part, m, n, kg, sk, f32)
+#define TF_GO(GS_, RT_, NI_, RING_)                                                                                      \
+  qmm_kernel<GS_, QMM_WAVES, RT_, NI_, RING_><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, weight, scales, biases,     \
+                                                                                 sb_stride, out, part, m, n, kg, sk, f32)
   if (gs == 64) {
-    if (m <= 4) TF_GO(64, 1, 1);
-    else if (m <= 8) TF_GO(64, 1, 2);
-    else if (m <= 16) TF_GO(64, 1, 4);
-    else TF_GO(64, 2, 4);
+    if (m <= 4) TF_GO(64, 1, 1, false);
+    else if (m <= 8) TF_GO(64, 1, 2, false);
+    else if (ring && m <= 16) TF_GO(64, 1, 4, true);
+    else if (ring) TF_GO(64, 2, 4, true);
+    else if (m <= 16) TF_GO(64, 1, 4, false);
+    else TF_GO(64, 2, 4, false);
   } else {
-    if (m <= 4) TF_GO(32, 1, 1);
-    else if (m <= 8) TF_GO(32, 1, 2);
-    else if (m <= 16) TF_GO(32, 1, 4);
-    else TF_GO(32, 2, 4);
+    if (m <= 4) TF_GO(32, 1, 1, false);
+    else if (m <= 8) TF_GO(32, 1, 2, false);
+    else if (ring && m <= 16) TF_GO(32, 1, 4, true);
+    else if (ring) TF_GO(32, 2, 4, true);
+    else if (m <= 16) TF_GO(32, 1, 4, false);
+    else TF_GO(32, 2, 4, false);
   }
 #undef TF_GO
   TF_LAUNCH_OK("tf_qmm");
@@ -828,7 +972,9 @@ extern "C" int tf_qmm_group(const uint16_t* x, int64_t ldx, const float* xs, int
   a.count = count;
   a.first[count] = (int)blocks;
   hipStream_t s = as_stream(stream);
-  const size_t smem = sizeof(float) * qmm_lds_floats(QMM_WAVES, rt);
+  bool ring = m > 8;
+  for (int i = 0; i < count && ring; ++i) ring = ring_takes(ldx, sb_strides[i], scales[i], biases[i]);
+  const size_t smem = ring ? ring_lds(gs, rt) : sizeof(float) * qmm_lds_floats(QMM_WAVES, rt);
   const dim3 grid((unsigned)blocks, 1, (unsigned)max_sk);
   if (arrive) {
 #define TF_GO(GS_, NI_) \
@@ -858,18 +1004,22 @@ extern "C" int tf_qmm_group(const uint16_t* x, int64_t ldx, const float* xs, int
     TF_LAUNCH_OK("tf_qmm_group");
     return 0;
   }
-#define TF_GO(GS_, RT_, NI_) \
-  qmm_group_kernel<GS_, QMM_WAVES, RT_, NI_><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, a, m, kg, f32)
+#define TF_GO(GS_, RT_, NI_, RING_) \
+  qmm_group_kernel<GS_, QMM_WAVES, RT_, NI_, RING_><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, a, m, kg, f32)
   if (gs == 64) {
-    if (m <= 4) TF_GO(64, 1, 1);
-    else if (m <= 8) TF_GO(64, 1, 2);
-    else if (m <= 16) TF_GO(64, 1, 4);
-    else TF_GO(64, 2, 4);
+    if (m <= 4) TF_GO(64, 1, 1, false);
+    else if (m <= 8) TF_GO(64, 1, 2, false);
+    else if (ring && m <= 16) TF_GO(64, 1, 4, true);
+    else if (ring) TF_GO(64, 2, 4, true);
+    else if (m <= 16) TF_GO(64, 1, 4, false);
+    else TF_GO(64, 2, 4, false);
   } else {
-    if (m <= 4) TF_GO(32, 1, 1);
-    else if (m <= 8) TF_GO(32, 1, 2);
-    else if (m <= 16) TF_GO(32, 1, 4);
-    else TF_GO(32, 2, 4);
+    if (m <= 4) TF_GO(32, 1, 1, false);
+    else if (m <= 8) TF_GO(32, 1, 2, false);
+    else if (ring && m <= 16) TF_GO(32, 1, 4, true);
+    else if (ring) TF_GO(32, 2, 4, true);
+    else if (m <= 16) TF_GO(32, 1, 4, false);
+    else TF_GO(32, 2, 4, false);
   }
 #undef TF_GO
   TF_LAUNCH_OK("tf_qmm_group");
