@@ -88,11 +88,15 @@ struct Windows {
 // and add are one v_mad_u64_u32 (2.08 ns a wave and SIMD against 1.75 each for a multiply and an add; the upper half of its
 // result is not used, which the compiler must not learn): 227 vector instructions a pair of k tiles instead of 291, an MLP
 // 5120 -> 17408 -> 5120 at 3 bits and one row 59.7 -> 55.9 us.
-template <int CB>
+// At 5 bits and more the 64-bit results do not fit beside the windows (8 rows through experts at 6 bits spilled and took 1.4
+// times as long): a multiply and an add there.
+template <int CB, int K2>
 __device__ __forceinline__ uint32_t code_word(uint32_t s) {
   uint32_t x;
   if constexpr (CB == 1) {
     x = s * 0xCBAC1FEDu;
+  } else if constexpr (K2 >= 10) {
+    x = s * 89226354u + 64248484u;
   } else {
     uint64_t wide = (uint64_t)s * 89226354u + 64248484u;
     asm("" : "+v"(wide));
@@ -136,8 +140,8 @@ __device__ __forceinline__ void decode4(const Windows<K2>& win, const uint32_t (
     lo = mul1_pair(s[0], s[1]);
     hi = mul1_pair(s[2], s[3]);
   } else {
-    lo = half_sums(code_word<CB>(s[0]), code_word<CB>(s[1]));
-    hi = half_sums(code_word<CB>(s[2]), code_word<CB>(s[3]));
+    lo = half_sums(code_word<CB, K2>(s[0]), code_word<CB, K2>(s[1]));
+    hi = half_sums(code_word<CB, K2>(s[2]), code_word<CB, K2>(s[3]));
   }
 }
 
@@ -427,8 +431,8 @@ __device__ __forceinline__ void wave_block(const uint16_t* xr, const uint32_t* t
         uint32_t s0[4], s1[4];
         win.states(w0, s0);
         win.states(w1, s1);
-        const u32x4_t x0 = {code_word<CB>(s0[0]), code_word<CB>(s0[1]), code_word<CB>(s0[2]), code_word<CB>(s0[3])};
-        const u32x4_t x1 = {code_word<CB>(s1[0]), code_word<CB>(s1[1]), code_word<CB>(s1[2]), code_word<CB>(s1[3])};
+        const u32x4_t x0 = {code_word<CB, K2>(s0[0]), code_word<CB, K2>(s0[1]), code_word<CB, K2>(s0[2]), code_word<CB, K2>(s0[3])};
+        const u32x4_t x1 = {code_word<CB, K2>(s1[0]), code_word<CB, K2>(s1[1]), code_word<CB, K2>(s1[2]), code_word<CB, K2>(s1[3])};
         acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, __builtin_bit_cast(f16x8_t, x0), acc[j], 0, 0, 0);
         acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, __builtin_bit_cast(f16x8_t, x1), acc[j], 0, 0, 0);
       } else {

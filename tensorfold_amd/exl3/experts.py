@@ -156,13 +156,15 @@ def prepare_stacked(gt: torch.Tensor, ut: torch.Tensor, dt: torch.Tensor, suh_g,
 
 def default_config(k: int, n: int, gateup: bool = True) -> int:
     """K splits of a K -> N projection: the shape's alone, so a row's sums run in one order at every row count.
-    As many as keep three tile pairs a wave and at most 64 (column block, split) workgroups an item: a wave's head and tail cost
-    it about a pair (4096 -> 2048 -> 4096 at 4 bits with (4, 2) splits, (8, 4) before: 50.7 us at one row, was 50.3; 220.5 at 8
-    rows, was 232.0; 379.6 at 16, was 396.3; 2048 -> 768 -> 2048 with (4, 2), (4, 1) before: 27.3, was 29.3)."""
+    As many as keep three tile pairs a wave (three and a half with four or eight splits) and at most 64 (column block, split)
+    workgroups an item: a wave's head and tail cost it about a pair (4096 -> 2048 -> 4096 at 4 bits with (4, 2) splits, (8, 4)
+    before: 50.7 us at one row, was 50.3; 220.5 at 8 rows, was 232.0; 379.6 at 16, was 396.3; 2048 -> 768 -> 2048 with (4, 2),
+    (4, 1) before: 27.3, was 29.3; 3968 -> 640 with (8, 1), (4, 1) before: 111 at 12 rows, was 119; but 3328 -> 768 with (8, 2),
+    3.25 pairs: 109 at 11 rows against 103 with (4, 1))."""
 
     pairs, nb = k // 32, n // 128
     for sk in (8, 4, 2):
-        if pairs // (WAVES * sk) >= 3 and nb * sk <= 64:
+        if 2 * pairs >= (6 if sk == 2 else 7) * WAVES * sk and nb * sk <= 64:
             return sk
     if pairs < WAVES:
         raise ValueError(f"K={k} is too short for {WAVES} waves")
