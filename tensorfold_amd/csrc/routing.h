@@ -337,19 +337,22 @@ struct PlanLds {
 // Whole workgroup (PLAN_THREADS threads, barriers inside); thread e brings expert e's pair count c (0 past E).
 // Fills L and writes the plan's items and counts: experts ascending, an expert's pairs cut into runs of T.  The
 // items are written a thread an item (an expert that holds thousands of a prompt chunk's pairs has dozens): item i
-// belongs to the last expert whose first item is not past i, found by bisection of the non-decreasing istart.
-__device__ void place_items(PlanLds& L, int c, int E, int T, int* __restrict__ items, int* __restrict__ counts) {
+// belongs to the last expert whose first item is not past i, found by bisection of the non-decreasing istart.  Of
+// several workgroups that need L one writes the plan.
+__device__ void place_items(PlanLds& L, int c, int E, int T, int* __restrict__ items, int* __restrict__ counts,
+                            bool write = true) {
   const int tid = threadIdx.x;
   int val[3] = {c, (c + T - 1) / T, c > 0 ? 1 : 0}, excl[3], tot[3];
   scan3(val, excl, tot);
   L.cnt[tid] = c;
   L.first[tid] = excl[0];
   L.istart[tid] = excl[1];
-  if (tid == 0) {
+  if (write && tid == 0) {
     counts[0] = tot[1];
     counts[1] = tot[2];
   }
   __syncthreads();
+  if (!write) return;
   for (int i = tid; i < tot[1]; i += PLAN_THREADS) {
     int lo = 0, hi = E - 1;
     while (lo < hi) {

@@ -89,6 +89,28 @@ def test_plan_groups_pairs_by_expert(rows, prefill, tile):
     assert np.array_equal(plan.members.cpu().numpy(), members)
 
 
+# 1,024 pairs a workgroup: the second's first pair, a whole second one, the most whose workgroups place their own pairs, one past
+# that, and one more; few experts and the most, some picks of none
+@pytest.mark.parametrize("e", [1, 50, 1024])
+@pytest.mark.parametrize("pairs", [1025, 2048, 20000, 256 * 1024 - 1, 256 * 1024, 256 * 1024 + 1])
+def test_plan_of_several_workgroups(pairs, e):
+    g = torch.Generator().manual_seed(pairs + e)
+    picks = (torch.rand((pairs, 1), generator=g).square() * e).to(torch.int32).clamp(max=e - 1)
+    picks[::97] = e
+    picks[5::101] = -1
+    plan = experts.Plan(pairs, 1, e, DEV, prefill=True)
+    experts.route(picks.to(DEV), plan, 128)
+    flat = picks.numpy()[:, 0]
+    held = np.flatnonzero((flat >= 0) & (flat < e))
+    members = held[np.argsort(flat[held], kind="stable")]
+    assert np.array_equal(plan.members.cpu().numpy()[:len(members)], members)
+    count = np.bincount(flat[held], minlength=e)
+    first = np.cumsum(count) - count
+    want = [(x, first[x] + j, min(128, count[x] - j)) for x in range(e) for j in range(0, count[x], 128)]
+    assert plan.counts[:2].tolist() == [len(want), int((count > 0).sum())]
+    assert plan.items[:len(want)].tolist() == [list(map(int, w)) for w in want]
+
+
 @pytest.mark.parametrize("gs", [32, 64])
 def test_the_sums_a_wave_takes_from_its_inputs(gs):
     """The affine form needs the sum of every group of inputs; each wave takes it from the inputs it streams.  A table
