@@ -455,7 +455,9 @@ extern "C" int tf_moe_router(const uint16_t* x, int64_t ldx, const uint16_t* row
   hipStream_t s = as_stream(stream);
   // A compute unit takes 16 to 20 bytes of operands a cycle whatever the tile, so small tiles win while each has a unit
   // to itself and larger ones (operands read fewer times over) once they do not: 392 tiles x 2688 18.3 us as 16 x 16,
-  // 13.3 as 32 x 32 (128 tiles 7.4 / 13); 1,617 x 2048 14.2 us as 32 x 64, 47 as one wave's 32 x 64; 8,448 x 2048
+  // 13.3 as 32 x 32 (128 tiles 7.4 / 13).  Between the two, 32 x 16 while each has a unit to itself, all of a slice in
+  // flight up to 3,072 inputs: 777 rows x 128 x 2688 11.3 us as 32 x 32 (100 units of the 256 at work), 9.6 so; 250 x 512 x 4096
+  // 16.8, 13.2; 8,000 x 16 x 512 3.6, 3.5; 1,617 x 2048 14.2 us as 32 x 64, 47 as one wave's 32 x 64; 8,448 x 2048
   // 30.5 us wide.  The wide kernel takes what would be more than one round of 32 x 64, two workgroups a unit: below that its
   // own 64 x 128 leave units idle (4,096 rows x 129 x 512 11.8 us on 128 workgroups, 8.6 as 32 x 64; x 2048 28.3, 21.3).
   // With up to 32 experts a column tile of 64 or 128 would be mostly padding: 32,768 rows x 8 x 2048 36 us as 32 x 64,
@@ -465,6 +467,10 @@ extern "C" int tf_moe_router(const uint16_t* x, int64_t ldx, const uint16_t* row
     const dim3 grid((m + 15) / 16, (ne + 15) / 16);
     if (d <= 32 * 8 * ROUTER_SLICES) router_kernel<1, 1, 8><<<grid, 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
     else router_kernel<1, 1, 12><<<grid, 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
+  } else if ((int64_t)((m + 31) / 32) * ((ne + 15) / 16) <= 256) {
+    const dim3 grid((m + 31) / 32, (ne + 15) / 16);
+    if (d <= 32 * 8 * ROUTER_SLICES) router_kernel<2, 1, 8><<<grid, 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
+    else router_kernel<2, 1, 12><<<grid, 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
   } else if (tiles > 1024 && ne <= 16) {
     router_kernel<4, 1, 4><<<dim3((m + 63) / 64), 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
   } else if (tiles <= 1024 || ne <= 32) {

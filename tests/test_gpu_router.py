@@ -39,3 +39,11 @@ def test_slices_of_any_length(rows, d, ne):
                                        (5471, 352, 180), (8192, 128, 128), (8193, 288, 128)])
 def test_many_rows_of_few_experts(rows, d, ne):
     test_router_against_float64_and_row_by_row(rows, d, ne)
+
+
+# 32 x 16 tiles, a compute unit each: from the first call past 256 tiles of 16 x 16 to 256 such tiles and one more; slices that
+# are requested in one go, and in two
+@pytest.mark.parametrize("rows,d,ne", [(257, 2688, 241), (513, 2048, 113), (1024, 2080, 128), (1025, 352, 128), (8192, 64, 9),
+                                       (8193, 64, 9), (17, 4096, 2044), (250, 3104, 500), (4000, 32, 17)])
+def test_tiles_of_32_rows_and_16_experts(rows, d, ne):
+    test_router_against_float64_and_row_by_row(rows, d, ne)
