@@ -99,6 +99,20 @@ def test_planners_are_functions_of_the_shape():
     assert linear.plan(17408, 5120)[0] > linear.plan(5120, 17408)[0]      # the narrow layer splits K further
 
 
+def test_the_exl3_splits_are_ones_the_launches_take():
+    """Over layers of every depth and of widths from one column block to past the priced range: the splits and waves that
+    tf_exl3_linear and tf_exl3x_grouped accept."""
+
+    from tensorfold_amd.exl3 import experts as routed
+
+    for k in range(128, 20481, 128):
+        for nb in (1, 2, 5, 16, 33, 136, 511, 512, 513, 1200):
+            sk, wk = linear.plan(k, 128 * nb)
+            assert wk in (2, 4, 8) and 1 <= sk <= 64 and sk * wk <= k // 32, (k, nb)
+            splits = routed.default_config(k, 128 * nb)
+            assert splits in (1, 2, 4, 8) and splits * routed.WAVES <= k // 32, (k, nb)
+
+
 def test_format_facts():
     assert fmt.tile_words(3) == 48 and fmt.bits_of((320, 1088, 48)) == 3 and fmt.bits_of((4, 4, 40)) == 2.5
     assert linear.k2_of(3) == 6 and linear.k2_of(2.5) == 5
