@@ -67,10 +67,13 @@ __global__ void __launch_bounds__(256)
 // grid (N / 128, SK, layers); WK waves a block; each wave walks its range of k-tile pairs over the block's eight column
 // tiles.  The layers of a stack share K, N, width and codebook; layer z has its own xh [M, K], trellis (stride_layer
 // words on), svh and bias [N], y [M, N], Z [SK, M, N] and counters.
-// (The second launch bound, waves a SIMD, keeps the kernel within 128 registers at the widths where that costs no
-// spill; the widest decodes need a few more and run three waves a SIMD.)
+// The second launch bound, waves a SIMD, keeps every width within 128 registers: two workgroups of eight waves a compute unit,
+// which `plan` counts on.  What the tail makes of the lane number (the butterflies' six signs, addresses) the compiler works out
+// ahead of the walk and keeps in ten to twenty registers all through it.  From 6 bits on those are not there: the kernels spilled, or
+// without the bound ran a workgroup of eight waves alone on its compute unit, so there the tail has a lane number of its own.  17408 ->
+// 5120, one row: 6 bits 3inst 29.1 -> 25.8 us, 7 bits 30.9 -> 26.8, 8 bits 31.0 -> 27.7; at 4 bits it would cost (mcg 20.6 -> 21.9).
 template <int K2, int CB, int WK>
-__global__ void __launch_bounds__(WK * 64, K2 <= 12 ? 4 : 1)
+__global__ void __launch_bounds__(WK * 64, 4)
     linear_kernel(const uint16_t* __restrict__ xh, const uint32_t* __restrict__ T, int64_t stride_k, int64_t stride_nb,
                   int64_t stride_layer, const uint16_t* __restrict__ svh, const uint16_t* __restrict__ bias,
                   void* __restrict__ y, int y_dtype, float* __restrict__ Z, int* __restrict__ counters, int M, int K,
@@ -96,7 +99,7 @@ __global__ void __launch_bounds__(WK * 64, K2 <= 12 ? 4 : 1)
     if (counters && !mlp) counters += z * 8 * NB * TF_EXL3_COUNTER_STRIDE;
   }
   const int arrivals = mlp ? 2 * SK : SK;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave_lane = threadIdx.x & 63, c = wave_lane & 15, kq = wave_lane >> 4;
   const int L = 4 * (c & 7) + kq, h = c >> 3;
   const int pairs = K >> 5, slot = split * WK + wave, nslots = SK * WK;
   const int pr0 = first_pair(slot, pairs, nslots), pr1 = first_pair(slot + 1, pairs, nslots);
@@ -114,8 +117,10 @@ __global__ void __launch_bounds__(WK * 64, K2 <= 12 ? 4 : 1)
     uint32_t* stage = reinterpret_cast<uint32_t*>(red) + wave * (16 * 128);       // 16 tiles of TW words
     if (pass) __syncthreads();                 // the previous pass is done with red
     TF_MARK(1);
-    wave_block<K2, CB>(xr, tiles, stride_k, pr0, pr1, stage, lane, L, h, acc);
+    wave_block<K2, CB>(xr, tiles, stride_k, pr0, pr1, stage, wave_lane, L, h, acc);
     TF_MARK(2);
+    int lane = wave_lane;
+    if constexpr (K2 >= 12) asm volatile("" : "+v"(lane));       // the compiler is not to know that it is the same
     __syncthreads();
     TF_MARK(3);
     store_rows(red + wave * (16 * 128), acc, R, c, kq);
