@@ -235,16 +235,27 @@ struct QmmRing {
 };
 
 // Loads into LDS: a lane's 16 or 4 bytes go to `lds` + its share of the wave's run.  Written as instructions because the compiler
-// would wait for every load in flight ahead of any LDS read.
+// would wait for every load in flight ahead of any LDS read.  m0 is the compiler's as well, so each says that it writes it.
+// A vector memory instruction may read a scalar register five wait states after a vector instruction wrote it, which the
+// compiler does not see to in here: bases that come out of `settled` have four of them behind them, the move to m0 is the fifth.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"          // "m0 is reserved": no value is kept there, but the compiler writes it too
+#define TF_TO_LDS(LOAD, ...) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" LOAD ::"s"(lds), __VA_ARGS__ : "memory", "m0")
 __device__ __forceinline__ void to_lds16(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+  TF_TO_LDS("global_load_lds_dwordx4 %1, %2", "v"(off), "s"(base));
 }
 __device__ __forceinline__ void to_lds4(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+  TF_TO_LDS("global_load_lds_dword %1, %2", "v"(off), "s"(base));
 }
 __device__ __forceinline__ void lane_to_lds4(const void* p, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(p) : "memory");
+  TF_TO_LDS("global_load_lds_dword %1, off", "v"(p));
 }
+template <class A, class B, class C>
+__device__ __forceinline__ void settled(A*& a, B*& b, C*& c) {
+  asm volatile("s_nop 3" : "+s"(a), "+s"(b), "+s"(c));
+}
+#undef TF_TO_LDS
+#pragma clang diagnostic pop
 
 template <int GS, int RT>
 __device__ __forceinline__ void qmm_ring_walk(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
@@ -272,12 +283,16 @@ __device__ __forceinline__ void qmm_ring_walk(const uint16_t* __restrict__ X, in
   const uint32_t at = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)ring);
   auto request = [&](int g) {
     const uint32_t lds = at + (g & (RING_STAGES - 1)) * R::STAGE;
+    const uint32_t* w = w0 + (size_t)g * (CH * 256);
+    const uint16_t* x = x0 + (size_t)g * GS;
+    const float* xs = xs0 + g;
+    settled(w, x, xs);
 #pragma unroll
-    for (int i = 0; i < CH; ++i) to_lds16(w0 + ((size_t)g * CH + i) * 256, lane * 16, lds + i * 1024);
+    for (int i = 0; i < CH; ++i) to_lds16(w + i * 256, lane * 16, lds + i * 1024);
     lane_to_lds4(sb + (size_t)g * sb_stride, lds + R::AT_SB);
 #pragma unroll
-    for (int j = 0; j < RT * CH; ++j) to_lds16(x0 + (size_t)g * GS, xoff[j], lds + R::AT_X + j * 1024);
-    if (lane < 16 * RT) to_lds4(xs0 + g, xsoff, lds + R::AT_XS);
+    for (int j = 0; j < RT * CH; ++j) to_lds16(x, xoff[j], lds + R::AT_X + j * 1024);
+    if (lane < 16 * RT) to_lds4(xs, xsoff, lds + R::AT_XS);
   };
 #pragma unroll
   for (int r = 0; r < RT; ++r)
