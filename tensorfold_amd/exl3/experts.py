@@ -154,21 +154,25 @@ def prepare_stacked(gt: torch.Tensor, ut: torch.Tensor, dt: torch.Tensor, suh_g,
                   cb, stacks, gt.device)
 
 
-def default_config(k: int, n: int, gateup: bool = True) -> int:
-    """K splits of a K -> N projection: the shape's alone, so a row's sums run in one order at every row count.
-    As many as keep three tile pairs a wave (three and a half with four or eight splits) and at most 64 (column block, split)
-    workgroups an item: a wave's head and tail cost it about a pair (4096 -> 2048 -> 4096 at 4 bits with (4, 2) splits, (8, 4)
-    before: 50.7 us at one row, was 50.3; 220.5 at 8 rows, was 232.0; 379.6 at 16, was 396.3; 2048 -> 768 -> 2048 with (4, 2),
-    (4, 1) before: 27.3, was 29.3; 3968 -> 640 with (8, 1), (4, 1) before: 111 at 12 rows, was 119; but 3328 -> 768 with (8, 2),
-    3.25 pairs: 109 at 11 rows against 103 with (4, 1))."""
+def default_config(k: int, n: int, gateup: bool = True, slots: int = 8) -> int:
+    """K splits of a K -> N projection: the shape's and the layer's picks a row alone, so a row's sums run in one order at
+    every row count.
 
-    pairs, nb = k // 32, n // 128
-    for sk in (8, 4, 2):
-        if 2 * pairs >= (6 if sk == 2 else 7) * WAVES * sk and nb * sk <= 64:
-            return sk
+    As many as give a row's launch 1,024 workgroups (column blocks x splits x picks, both matrices for gate and up): four to a
+    compute unit, what it holds.  Fewer leave the chip to waves that walk longer where a layer has few picks; more only add heads
+    and tails, a pair's worth of time each (4096 -> 2048 -> 4096 at 4 bits, one row: one pick 22-24 us with (8, 4) splits,
+    30 with (4, 2); 8 picks 47.5 with (4, 4), 48.5 with (4, 2), and at 8 rows 161 and 160, with (8, 4) 166; 4096 -> 6144: one
+    pick 31 with (8, 8), 70 with (1, 2); 8 picks 97 with (2, 4), 104 with (1, 2)).  A wave keeps three tile pairs, three and a
+    half with four or eight splits (2048 -> 768 -> 2048 with (4, 2), (4, 1) before: 27.3 us at one row of 8 picks, was 29.3;
+    3328 -> 768 with (8, 2), 3.25 pairs: 109 at 11 rows against 103 with (4, 1))."""
+
+    pairs, row = k // 32, n // 128 * slots * (2 if gateup else 1)
     if pairs < WAVES:
         raise ValueError(f"K={k} is too short for {WAVES} waves")
-    return 1
+    sk = 1
+    while sk < 8 and row * sk < 1024 and pairs >= (3 if sk == 1 else 3.5) * WAVES * 2 * sk:
+        sk *= 2
+    return sk
 
 
 class Scratch:
@@ -180,8 +184,8 @@ class Scratch:
     def __init__(self, ex: Exl3RoutedExperts, rows: int, slots: int, sk_gu: int | None = None, sk_d: int | None = None,
                  device: str | torch.device = "cuda") -> None:
         self.rows, self.slots, self.count_experts = rows, slots, ex.count
-        self.sk_gu = sk_gu or default_config(ex.dims, ex.width, True)
-        self.sk_d = sk_d or default_config(ex.width, ex.dims, False)
+        self.sk_gu = sk_gu or default_config(ex.dims, ex.width, True, slots)
+        self.sk_d = sk_d or default_config(ex.width, ex.dims, False, slots)
         pairs = rows * slots
 
         def buffer(columns: int, dtype: torch.dtype) -> torch.Tensor:
