@@ -220,10 +220,12 @@ __device__ __forceinline__ void qmm_walk(const uint16_t* __restrict__ X, int64_t
 // registers, and the compiler requested two of them together after adding both: every pair of groups waited for a whole
 // trip.  Here a stage is the wave's own corner of LDS, filled by loads that go straight there: a group's operands are read out, its
 // place takes the request for the group RING_STAGES on, and the arithmetic runs under both requests.  A wave waits for its
-// own loads by count; nothing crosses waves.  The same operands and the same order of sums as qmm_walk: the same bits.  17408 x
-// 5120: 9 rows 20.9 -> 19.4 us, 16 24.2 -> 20.4, 21 27.7 -> 22.9, 32 33.6 -> 26.4, 64 51.5 -> 37.4 (reduce and group
-// sums included); up to 8 rows qmm_walk is not so held up and keeps more workgroups a compute unit.  Two stages: three would take
-// the third workgroup's LDS.
+// own loads by count; nothing crosses waves.  The same operands and the same order of sums as qmm_walk: the same bits.  Up to 8 rows
+// qmm_walk is not so held up and keeps more workgroups a compute unit.  What the ring gains depends on where the weights come from.
+// 17408 x 5120, reduce included, weights in the last-level cache (four of them, 200 MB): 9 rows 17.6 -> 16.1 us, 12 18.9 -> 16.6, 16
+// 20.6 -> 17.2, 21 24.6 -> 20.5, 32 30.4 -> 22.6, 64 46.9 -> 33.2; from HBM (25 of them): 17.7 -> 18.2, 18.8 -> 18.9, 20.5 ->
+// 20.0, 24.6 -> 24.4, 30.3 -> 28.0, 46.7 -> 38.0 (4096 x 4096 from HBM: 9 rows 7.5 -> 8.0, 21 10.0 -> 9.7, 64 17.0 -> 15.8).
+// Two stages: three (four in groups of 32) take the fourth workgroup's LDS and were slower from either (16 rows 17.8 and 20.4 us).
 constexpr int RING_STAGES = 2;
 
 template <int GS, int RT>
@@ -647,10 +649,22 @@ __global__ void __launch_bounds__(256)
 }
 
 constexpr int QMM_WAVES = 4;
-// What the ring walk takes besides 9 rows or more: its loads into LDS are of whole dwords (two columns' scales: an even row length on a 4-byte boundary) and
-// of 32-bit offsets from 32 rows' first.
+// What the ring walk's loads into LDS take: whole dwords (two columns' scales: an even row length on a 4-byte boundary) and 32-bit offsets from 32
+// rows' first.
 static bool ring_takes(int64_t ldx, int64_t sb_stride, const void* scales, const void* biases) {
   return sb_stride % 2 == 0 && (((uintptr_t)scales | (uintptr_t)biases) & 3) == 0 && ldx < (1ll << 25);
+}
+// Whether it is the better walk of a weight in sk slices.  Besides up to 8 rows it is not, wherever the weights come from,
+// - up to 16 rows where waves have fewer than two groups and nothing to request ahead, in a grouped launch (`least` = 5 halves) two
+//   and a half, its narrow weights' waves having fewer still (1536 x 3072 in groups of 32, 12 rows: 8.4 us, 8.7 as a ring; q, k and
+//   v of 4096 + 1024 + 1024 columns x 4096 12.0, 12.4; 2048 + 256 + 256 x 2048 in groups of 32 8.8, 9.2; but 4096 + 512 + 512 x
+//   7168, three and a half groups, 14.1, 13.0);
+// - at 9 and 10 rows of a long walk along a deep K in groups of 64 (9 rows x 8192 x 8192 from the cache 12.7 us, 12.8 as a
+//   ring, from HBM 12.7, 13.3; 4096 x 12288 10.6, 10.5, and 10.4, 11.2; 5120 x 17408 16.1, 15.7, and 15.9, 17.3; but 5120 x 8192, four groups a
+//   wave, 12.9, 11.9, and 11.5, 11.9; in groups of 32 5120 x 17408 19.1, 17.1, and 19.3, 20.1).
+static bool ring_pays(int m, int gs, int kg, int sk, int least) {
+  if (m <= 8 || (m <= 16 && 2 * kg < least * QMM_WAVES * sk)) return false;
+  return m > 10 || gs != 64 || kg < 128 || kg < 6 * QMM_WAVES * sk;
 }
 // LDS of its workgroup: the waves' rings, and later their sums in the same place
 static size_t ring_lds(int gs, int rt) {
@@ -798,7 +812,7 @@ static int qmm_launch(const uint16_t* x, int64_t ldx, const float* xs, const uin
   // up to 16 rows are one row tile of the matrix instruction; past that a workgroup takes two (`bm` is the caller's row
   // tile: accepted, and no longer what decides)
   const int rt = m <= 16 ? 1 : 2, tiles = (n + 63) / 64, rts = (m + 16 * rt - 1) / (16 * rt);
-  const bool ring = m > 8 && ring_takes(ldx, sb_stride, scales, biases);
+  const bool ring = ring_pays(m, gs, kg, sk, 4) && ring_takes(ldx, sb_stride, scales, biases);
   const size_t smem = ring ? ring_lds(gs, rt) : sizeof(float) * qmm_lds_floats(QMM_WAVES, rt);
   TF_REQUIRE((int64_t)tiles * rts <= 0x7FFFFFFF && sk <= 65535, "qmm: grid too large");
   const dim3 grid((unsigned)(tiles * rts), 1, (unsigned)sk);
@@ -987,7 +1001,8 @@ extern "C" int tf_qmm_group(const uint16_t* x, int64_t ldx, const float* xs, int
   a.count = count;
   a.first[count] = (int)blocks;
   hipStream_t s = as_stream(stream);
-  bool ring = m > 8;
+  bool ring = false;                          // the weight that gains most decides
+  for (int i = 0; i < count; ++i) ring = ring || ring_pays(m, gs, kg, sks[i], 5);
   for (int i = 0; i < count && ring; ++i) ring = ring_takes(ldx, sb_strides[i], scales[i], biases[i]);
   const size_t smem = ring ? ring_lds(gs, rt) : sizeof(float) * qmm_lds_floats(QMM_WAVES, rt);
   const dim3 grid((unsigned)blocks, 1, (unsigned)max_sk);
