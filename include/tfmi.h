@@ -324,7 +324,9 @@ int tf_exl3_unpack_k8(const uint32_t* T, uint16_t* W8, int k, int n, int64_t str
 /* y[m, block] = ((xh[m] @ W_q[:, block]) H / sqrt(128)) * svh + bias for any m: xh fp16 [m, k] from tf_exl3_rot_in,
  * w8 from tf_exl3_unpack_k8 (k * n < 2^31), K added in order in fp32 (a row's bits do not depend on m or on the
  * rows beside it), the rotation exact in fp32.  y rows are y_stride elements apart.  Replaces exl3/prefill.py:16-44
- * `_gemm`. */
+ * `_gemm`.  A workgroup takes 16 times as many rows as tf_exl3_gemm_tile gives for the call's rows and columns (2 to 9;
+ * host arithmetic alone, no GPU, returns the count). */
+int tf_exl3_gemm_tile(int m, int n);
 int tf_exl3_gemm(const uint16_t* xh, const uint16_t* w8, const uint16_t* svh, const uint16_t* bias, void* y, int y_dtype,
                  int64_t y_stride, int m, int k, int n, tf_stream_t stream);
 

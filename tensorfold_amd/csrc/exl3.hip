@@ -279,8 +279,9 @@ __global__ void __launch_bounds__(256)
 //
 // Workgroups reach the XCDs round-robin (blockIdx % 8) and each XCD has its own L2: an XCD takes one run of the tiles,
 // walked down groups of GEMM_GROUP row tiles, so its 64 co-resident workgroups are about 8 x 8 tiles and what they stream in
-// step from beyond L2 is 8 tiles of xh and 8 of W8, not one of each a workgroup.  The runs differ by one tile at most
-// (whole 8 x 8 or 8 x 4 blocks dealt out to the XCDs gave the fullest of them 96 of 1,000 x 17408's 544 tiles, where 68 are its share).
+// step from beyond L2 is 8 tiles of xh and 8 of W8, not one of each a workgroup.  No run is longer than an eighth of the tiles
+// rounded up, the last ones may be shorter (whole 8 x 8 or 8 x 4 blocks dealt out to the XCDs gave the fullest of them 96 of 1,000 x
+// 17408's 544 tiles, where 68 are its share).
 constexpr int GEMM_GROUP = 8, GEMM_KSTEP = 64, GEMM_AROW = 2 * GEMM_KSTEP + 16, GEMM_WAVES = 4, GEMM_COLS = 64 * GEMM_WAVES;
 // two stages of xh, or the epilogue's two row tiles of a workgroup's columns if those are more
 constexpr int gemm_lds(int rt) { return max(2 * 16 * rt * GEMM_AROW, 2 * 16 * (GEMM_COLS + 4) * 4); }     // bytes
@@ -592,7 +593,8 @@ extern "C" int tf_exl3_unpack_k8(const uint32_t* T, uint16_t* W8, int k, int n, 
 // start another for.  1,000 x 5120 x 17408: 185 us with the 64-row tiles taken when 32, 64, 96 and 128 rows were the choice, 146
 // with 144; 512 rows 112 -> 90 (80-row tiles); 1,000 x 5120 x 5120 68 -> 56; 3,000 x 4096 x 12288 265 -> 239; 4,096 x 5120 x
 // 17408 602 -> 577 (128 rows as before: the XCDs' even shares).  The rule does not look at K, whose shorter chains favour smaller
-// tiles still more.
+// tiles still more; all the same no call of 110 (130 to 4,096 rows; K 128 to 5120; 1024 to 17408 columns) is slower than with that
+// choice of four (0.33 to 0.93 of the time; 1,000 x 1536 x 5120 45.7 -> 24.2 us, 1,000 x 5120 x 1536 39.8 -> 35.6).
 static int gemm_row_tiles(int m, int n) {
   if (((int64_t)m + 127) / 128 * ((n + GEMM_COLS - 1) / GEMM_COLS) > 4096) return 8;         // eight rounds and more
   constexpr int ALONE[10] = {0, 0, 36, 39, 41, 47, 53, 60, 66, 74}, AMONG[10] = {0, 0, 30, 36, 39, 44, 51, 57, 63, 72};
@@ -606,6 +608,8 @@ static int gemm_row_tiles(int m, int n) {
   }
   return best;
 }
+
+extern "C" int tf_exl3_gemm_tile(int m, int n) { return gemm_row_tiles(m < 1 ? 1 : m, n < 1 ? 1 : n); }
 
 extern "C" int tf_exl3_gemm(const uint16_t* xh, const uint16_t* w8, const uint16_t* svh, const uint16_t* bias, void* y,
                             int y_dtype, int64_t y_stride, int m, int k, int n, tf_stream_t stream) {

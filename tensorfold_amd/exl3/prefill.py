@@ -51,6 +51,13 @@ def decode(layer: Exl3Linear, ws: Workspace) -> torch.Tensor:
     return w8
 
 
+def row_tiles(m: int, n: int) -> int:
+    """16-row tiles a workgroup of ``matmul`` takes for ``m`` rows and ``n`` columns, 2 to 9: what the launch asks (no GPU
+    needed)."""
+
+    return _lib.lib().tf_exl3_gemm_tile(m, n)
+
+
 def matmul(layer: Exl3Linear, x: torch.Tensor, out: torch.Tensor, ws: Workspace,
            wt: torch.Tensor | None = None) -> torch.Tensor:
     """out [M, N] (row stride free) = x [M, K] @ W + bias for any M, the prompt path's arithmetic

@@ -13,8 +13,10 @@ DEV = "cuda"
 
 
 # rows x columns whose calls take 3, 4, 5, 6, 7, 8 and 9 row tiles a workgroup
-@pytest.mark.parametrize("rows,n", [(700, 4224), (777, 4224), (1000, 4224), (1400, 4224), (1000, 6272), (1400, 5120), (2050, 4224)])
-def test_rows_do_not_depend_on_the_tile(rows, n):
+@pytest.mark.parametrize("tiles,rows,n", [(3, 700, 4224), (4, 777, 4224), (5, 1000, 4224), (6, 1400, 4224), (7, 1000, 6272),
+                                          (8, 1400, 5120), (9, 2050, 4224)])
+def test_rows_do_not_depend_on_the_tile(tiles, rows, n):
+    assert prefill.row_tiles(rows, n) == tiles and prefill.row_tiles(31, n) == 2
     trellis, suh, svh = synthetic.exl3_layer(256, n, 3, n)
     layer = linear.Exl3Linear.from_tensors(trellis, suh, svh, "3inst", device=DEV)
     layer.bias = torch.linspace(-1, 1, n, device=DEV).half()
