@@ -158,19 +158,22 @@ def default_config(k: int, n: int, gateup: bool = True, slots: int = 8) -> int:
     """K splits of a K -> N projection: the shape's and the layer's picks a row alone, so a row's sums run in one order at
     every row count.
 
-    As many as give a row's launch 1,024 workgroups (column blocks x splits x picks, both matrices for gate and up): four to a
-    compute unit, what it holds.  Fewer leave the chip to waves that walk longer where a layer has few picks; more only add heads
-    and tails, a pair's worth of time each (4096 -> 2048 -> 4096 at 4 bits, one row: one pick 22-24 us with (8, 4) splits,
-    30 with (4, 2); 8 picks 47.5 with (4, 4), 48.5 with (4, 2), and at 8 rows 161 and 160, with (8, 4) 166; 4096 -> 6144: one
-    pick 31 with (8, 8), 70 with (1, 2); 8 picks 97 with (2, 4), 104 with (1, 2)).  A wave keeps three tile pairs, three and a
-    half with four or eight splits (2048 -> 768 -> 2048 with (4, 2), (4, 1) before: 27.3 us at one row of 8 picks, was 29.3;
-    3328 -> 768 with (8, 2), 3.25 pairs: 109 at 11 rows against 103 with (4, 1))."""
+    As many as give a row's launch 512 workgroups (column blocks x splits x picks, both matrices for gate and up), two to a
+    compute unit, and 1,024 while a wave keeps five tile pairs.  Fewer leave the chip to waves that walk longer where a layer
+    has few picks; more only add heads and tails, a pair's worth of time each (4096 -> 2048 -> 4096 at 4 bits, one row: one pick
+    22-24 us with (8, 4) splits, 30 with (4, 2); 8 picks 47.8 and 48.5, and at 8 rows 166 and 160; 4096 -> 6144: one pick 31
+    with (8, 8), 70 with (1, 2); 8 picks 97 with (2, 4), 104 with (1, 2)).  At the least a wave keeps three tile pairs, three
+    and a half with four or eight splits (2048 -> 768 -> 2048 with (4, 2), (4, 1) before: 27.3 us at one row of 8 picks, was
+    29.3; 3328 -> 768 with (8, 2), 3.25 pairs: 109 at 11 rows against 103 with (4, 1))."""
 
     pairs, row = k // 32, n // 128 * slots * (2 if gateup else 1)
     if pairs < WAVES:
         raise ValueError(f"K={k} is too short for {WAVES} waves")
     sk = 1
-    while sk < 8 and row * sk < 1024 and pairs >= (3 if sk == 1 else 3.5) * WAVES * 2 * sk:
+    while sk < 8:
+        keeps = pairs / (2 * sk * WAVES)             # pairs a wave with twice the splits
+        if keeps < (3 if sk == 1 else 3.5) or row * sk >= (1024 if keeps >= 5 else 512):
+            break
         sk *= 2
     return sk
 
