@@ -753,7 +753,9 @@ __device__ __forceinline__ void big_body(const uint16_t* __restrict__ X, int64_t
 // Waves a workgroup of the experts' kernels, each 64 weight columns.  The bf16 form is bound by the vector instructions of its
 // dequantization (54 % of a launch's issue cycles, 25 % matrix, the two seldom side by side; requests three steps ahead gained
 // nothing): four waves, two workgroups a compute unit, whose barriers, heads and stores fall apart and whose units even out better
-// at the launch's end (777 rows x 128 experts of 2688 x 1856, routing and all: 360 -> 326 us).  The fp16 form spends half as much
+// at the launch's end (777 rows x 128 experts of 2688 x 1856, routing and all: 360 -> 326 us; over 168 launches of 500 to 4,096
+// rows x 32 to 128 experts 0.60 to 1.08 of the time, 0.92 at the geometric mean, the slower ones where full units of eight waves end a round evenly: up, 4,096 rows
+// x 64 experts of 2048 x 768 204 -> 214 us, 3,000 rows 195 -> 168).  The fp16 form spends half as much
 // on a weight, and staging the activations twice as often costs it more than that gains (4,096 rows x 512 experts 551 ->
 // 556 us, 500 rows 184 -> 193): eight waves.
 constexpr int expert_waves(int ar) { return ar == TF_ARITH_BF16 ? 4 : 8; }
@@ -821,10 +823,11 @@ __global__ void __launch_bounds__(expert_threads(AR), expert_threads(AR) == 256 
 }
 
 // The same units taken by workgroups that stay, eight waves a compute unit (a unit = an item's 512 weight columns, 256 in the
-// bf16 form, as a workgroup of experts_prefill_big_kernel takes).  A workgroup has a compute unit to itself (the body's registers), so
-// in the kernel above nothing runs under a unit's head (the item's rows looked up through two dependent reads, then
-// the first operands' trip), its results' drain, and the dispatch of the next workgroup; and with five or six
-// workgroups of 47 to 67 us to a compute unit, those that got five sit idle for the last tenth of the launch.  Here
+// bf16 form, as a workgroup of experts_prefill_big_kernel takes).  The body's registers leave room for eight waves a compute unit: in
+// the fp16 form one workgroup, so in the kernel above nothing runs under a unit's head (the item's rows looked up through two
+// dependent reads, then the first operands' trip), its results' drain, and the dispatch of the next workgroup (in the bf16
+// form one other workgroup does); and with five or six workgroups of 47 to 67 us to a compute unit, those that got five
+// sit idle for the last tenth of the launch.  Here
 //   * the units are walked in one order, place q = 0, 1, 2, ...: workgroup w of G takes places w and w + G, then
 //     whichever place is next on a ticket counter in memory (an atomic add that returns: ticket t is place 2 G + t),
 //     so a compute unit that finishes early takes more and the launch ends within a unit's time of the moment the

@@ -294,9 +294,9 @@ __global__ void __launch_bounds__(PLAN_THREADS)
 // own pairs of an expert begin, and puts them there; the first writes items and counts.  What bounds it is the launch and
 // three trips to memory in a row (counts, then a place in LDS, then the store); with the offsets a launch of one workgroup and
 // the placing a third, both passes of it over the counts were on that chain: the whole sort 12.2 -> 10.5 us at 4,662 pairs x
-// 128 experts, 16.9 -> 13.6 at 45,056 x 513, 38.8 -> 26.1 at 262,144 x 513 (graph replays).  Every workgroup reads
-// all counts, so the reads grow with the square of the pairs: past 256 blocks (the chip holds them at once; 138 MB at 513
-// experts) one workgroup adds the counts up for all of them, as below.
+// 128 experts, 16.9 -> 13.6 at 45,056 x 513, 39.1 -> 25.7 at 262,144 x 513, 46.4 -> 27.5 x 1,024 (graph replays).  Every
+// workgroup reads all counts, so the reads grow with the square of the pairs: past 256 blocks (the chip holds them at once; 134 MB
+// at 513 experts, 268 MB at 1,024) one workgroup adds the counts up for all of them, as below.
 constexpr int PLACE_BLOCKS = 256;
 __global__ void __launch_bounds__(PLAN_THREADS)
     plan_place_kernel(const int* __restrict__ picks, int P, int E, int T, const int* __restrict__ rank,

@@ -40,7 +40,9 @@ def plan(k: int, n: int, waves: int = 4096, min_pairs: int = 4) -> tuple[int, in
     it is a twelfth cheaper than a fixed number of waves a SIMD (closer than that the price is not to be trusted).  Against
     that number (us, 3 bits, 1 / 12 rows): 12288 x 4096 (8, 8) 14.3 / 17.3, was (12, 8) 16.7 / 21.9;
     2048 x 2048 (8, 8) 8.4 / 11.0, was (4, 4) 9.7 / 13.3; an MLP 4096 -> 12288 35.1 / 42.3 at 1 / 8 rows, was 37.0 / 45.8;
-    1024 -> 2048 16.8 / 20.8, was 19.8 / 26.0.
+    1024 -> 2048 16.8 / 20.8, was 19.8 / 26.0.  The price knows no width; at 2 to 8 bits of every codebook no layer of nine
+    shapes timed is slower with it (8 bits of mcg, 1 / 8 rows: 12288 x 4096 17.6 / 18.9, was 21.8 / 23.6; 5120 x 5120 13.7 / 15.3,
+    was 14.7 / 18.1).
     Layers of more than 512 column blocks, and callers that give ``waves`` or ``min_pairs``, keep the fixed number: so many
     waves in a launch, none with fewer pairs."""
 
