@@ -391,8 +391,10 @@ constexpr int BIG_THREADS = BIG_WAVES * 64;
 // LDS of a workgroup: two stages of activations
 constexpr int BIG_LDS = 2 * BIG_ROWS * AROW;
 static_assert(BIG_LDS + 2 * 2 * BIG_ROWS * 4 + 16 <= 64 * 1024, "within what a launch gets without asking");
+// LDS of one stage where a workgroup takes RT row tiles (the dense kernel's 9 are more rows than an item has)
+constexpr int big_stage(int rt) { return std::max(16 * rt, BIG_ROWS) * AROW; }
 
-// The pipeline for an item of at most 16 * RT rows (RT = 2, 4 or 8).  K is a multiple of KSTEP and nothing inside a
+// The pipeline for an item of at most 16 * RT rows (RT = 2, 4 or 8; the dense prompt matmul's tiles: 2 to 9).  K is a multiple of KSTEP and nothing inside a
 // step is conditional (prefetches past the end re-read the last step, rows past the item read its first row), so the
 // compiler is free to keep the LDS reads of the next row tile in flight under the MFMAs of this one.
 // Where a wave's weights come from.  A wave takes 64 weight columns (four operands of 16), and for loading them lane L
@@ -475,7 +477,7 @@ __device__ __forceinline__ void big_body(const uint16_t* __restrict__ X, int64_t
   constexpr int ROWS = 16 * RT;
   constexpr int PIECES = ROWS * 8;                // 16-byte pieces of a staged tile
   constexpr int PPT = (PIECES + NTHREADS - 1) / NTHREADS;
-  constexpr int STAGE = BIG_ROWS * AROW;
+  constexpr int STAGE = big_stage(RT);
   const int tid = thread < 0 ? (int)threadIdx.x : thread, lane = tid & 63, c = lane & 15, kq = lane >> 4;
   const int steps = K / KSTEP;
   typedef typename WS::Raw Raw;
@@ -504,24 +506,30 @@ __device__ __forceinline__ void big_body(const uint16_t* __restrict__ X, int64_t
     for (int j = 0; j < TJ; ++j) sb[j] = mine;
     across(sb);
   };
-  // this thread's pieces of the activation tile: piece q = (row q / 8, 16 bytes q % 8)
+  // this thread's pieces of the activation tile: piece q = (row q / 8, 16 bytes q % 8).  A thread past the last piece takes its
+  // first one again: requests under a condition would make the wait for the weights ahead of them one for everything (7
+  // row tiles of 8 waves: 129 -> 101 us a tile of K = 5120)
+  constexpr bool PAST = PIECES > NTHREADS && PIECES % NTHREADS != 0;
   const uint16_t* asrc[PPT];
 #pragma unroll
   for (int j = 0; j < PPT; ++j) {
-    const int q = tid + j * NTHREADS, r = q >> 3, ch = q & 7;
+    int q = tid + j * NTHREADS;
+    if (PAST && q >= PIECES) q = tid;
+    const int r = q >> 3, ch = q & 7;
     asrc[j] = X + (size_t)src_rows[r < cnt ? r : 0] * x_stride + ch * 8;
   }
   auto load_a = [&](int step, uint4 (&v)[PPT]) {
 #pragma unroll
     for (int j = 0; j < PPT; ++j)
-      if (PIECES % NTHREADS == 0 || tid + j * NTHREADS < PIECES)
+      if (PIECES >= NTHREADS || tid < PIECES)
         v[j] = *reinterpret_cast<const uint4*>(asrc[j] + (size_t)step * KSTEP);
   };
   auto store_a = [&](int buf, const uint4 (&v)[PPT]) {
 #pragma unroll
     for (int j = 0; j < PPT; ++j) {
-      const int q = tid + j * NTHREADS;
-      if (PIECES % NTHREADS == 0 || q < PIECES)
+      int q = tid + j * NTHREADS;
+      if (PAST && q >= PIECES) q = tid;
+      if (PIECES >= NTHREADS || q < PIECES)
         *reinterpret_cast<uint4*>(smem + buf * STAGE + (q >> 3) * AROW + (q & 7) * 16) =
             AR ? stage8_bf16(v[j]) : stage8(v[j]);
     }
@@ -589,7 +597,7 @@ __device__ __forceinline__ void big_body(const uint16_t* __restrict__ X, int64_t
       bb[1][j] = (u32x4_t){0u, 0u, 0u, 0u};
     }
   }
-  constexpr bool DEFER = RT == 8;          // with fewer row tiles a step the tile put off is too large a part of it
+  constexpr bool DEFER = RT >= 5;          // with fewer row tiles a step the tile put off is too large a part of it
   auto last_tile = [&]() {
     if constexpr (!DEFER) return;
 #pragma unroll
@@ -968,20 +976,23 @@ __global__ void __launch_bounds__(expert_threads(AR), expert_threads(AR) == 256 
   }
 }
 
-// The dense prompt matmul on the same pipeline: 128 rows x 512 columns a workgroup, a wave a 64-column tile.
-template <int GS, int EPI, int AR>
+// The dense prompt matmul on the same pipeline: a workgroup takes 16 RT rows (the first `tall` row tiles) or 16 (RT - 1) x 512
+// columns, a wave a 64-column tile.
+template <int GS, int EPI, int AR, int RT>
 __global__ void __launch_bounds__(BIG_THREADS, 1)
     qmm_prefill_big_kernel(const uint16_t* __restrict__ X, int64_t ldx, const uint32_t* __restrict__ W,
                            const uint16_t* __restrict__ S, const uint16_t* __restrict__ B, void* __restrict__ out,
-                           int M, int N, int KG, int npad) {
+                           int M, int N, int KG, int npad, int tall) {
+  constexpr int ROWS = 16 * RT, LOW = RT > 2 ? RT - 1 : RT;
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ int rows[BIG_ROWS];
+  __shared__ int rows[ROWS];
   const int ct = (N + 511) >> 9;
   const int rt = blockIdx.x / ct, cbt = blockIdx.x - rt * ct;
-  const int m0 = rt * BIG_ROWS, cnt = min(BIG_ROWS, M - m0);
+  const bool high = rt < tall;
+  const int m0 = high ? rt * ROWS : tall * ROWS + (rt - tall) * (16 * LOW), cnt = min(high ? ROWS : 16 * LOW, M - m0);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, kq = lane >> 4;
   TF_MARK(0);
-  if (tid < BIG_ROWS) rows[tid] = m0 + (tid < cnt ? tid : 0);
+  if (tid < ROWS) rows[tid] = m0 + (tid < cnt ? tid : 0);
   __syncthreads();
   TF_MARK(1);
   const int tiles = npad >> 6, tile = cbt * 8 + wave;
@@ -1002,9 +1013,8 @@ __global__ void __launch_bounds__(BIG_THREADS, 1)
   ws.qp = ((uint32_t)(ok ? tile : 0) * KG * (GS / 32) * 256u + lane * 4) * 4u;      // the column this lane loads: lane
   ws.cp = ((ok ? tile : 0) * 64 + lane) * 2;
   const int K = KG * GS;
-  if (cnt <= 32) big_body<GS, 1, EPI, 2, AR, true>(X, ldx, ws, ocol, jok, K, rows, rows, cnt, out, N, 0.f, smem);
-  else if (cnt <= 64) big_body<GS, 1, EPI, 4, AR, true>(X, ldx, ws, ocol, jok, K, rows, rows, cnt, out, N, 0.f, smem);
-  else big_body<GS, 1, EPI, 8, AR, true>(X, ldx, ws, ocol, jok, K, rows, rows, cnt, out, N, 0.f, smem);
+  if (LOW == RT || high) big_body<GS, 1, EPI, RT, AR, true>(X, ldx, ws, ocol, jok, K, rows, rows, cnt, out, N, 0.f, smem);
+  else big_body<GS, 1, EPI, LOW, AR, true>(X, ldx, ws, ocol, jok, K, rows, rows, cnt, out, N, 0.f, smem);
   TF_MARK(4);
 #ifdef TF_TIMELINE
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1336,13 +1346,48 @@ static bool big_takes(int64_t n, int64_t k) {
 // 1,000 rows 89 -> 53 (64 x 128); at 2,000 rows the eight-wave kernel's 95.7 is the best again (64 x 128 98.5).
 constexpr int SHORT_K = 192;
 
+// The eight-wave kernel's row tiles.  Where all are 128 rows the last round of 256 workgroups is seldom full and costs what a
+// full one does: 1,000 rows x 17408 columns are 272 tiles, two rounds.  So a call of r rounds takes as many row tiles as
+// those have room for, its 16-row units dealt out over them evenly: `tall` tiles of `rt` units, then tiles of one unit less.
+// `cost`: half microseconds at K = 4096 by the most units a tile has, for a round whose workgroups leave half the chip idle
+// and for a full one, where the clock is lower (17408 x 5120: 34 tiles of 128 rows 110 us, 238 tiles 139).  The rounds
+// whose cost is least are taken.  17408 x 5120, 1,000 rows: 239 -> 156 us (63 units on 7 row tiles), 512 rows 112 -> 101, 2,000 rows 380 ->
+// 305, 4,096 rows 656 -> 625; 12288 x 4096, 1,500 rows 200 -> 155; 4096 x 4096, 1,300 rows 78 -> 62.
+struct BigTiles {
+  int64_t tiles, tall;
+  int rt;
+  int64_t cost;
+};
+
+static BigTiles big_tiles(int64_t m, int64_t n) {
+  constexpr int64_t CU = 256;
+  static const int idle[10] = {0, 0, 100, 114, 132, 142, 152, 163, 176, 202}, full[10] = {0, 0, 104, 125, 146, 166, 182, 203, 221, 250};
+  const int64_t ct = (n + 511) / 512, units = (m + 15) / 16;
+  auto price = [](int64_t h, int64_t load) { return idle[h] * 100 + (full[h] - idle[h]) * load; };
+  // 0 where the workgroups of r rounds leave half the chip idle, 100 where they fill it
+  auto load = [&](int64_t tiles, int64_t r) { return std::max<int64_t>(0, 200 * tiles * ct / (CU * r) - 100); };
+  // all of 128 rows: the fastest a row where they come out even (4096 x 4096, 3,500 rows 106 us, on 32 tiles 110)
+  const int64_t even = (units + 7) / 8, rounds = (even * ct + CU - 1) / CU;
+  BigTiles best{even, even, 8, rounds * price(8, load(even, rounds)) / 100};
+  // fewest rounds that tiles of 144 rows fill, and up to three more
+  const int64_t least = ((units + 8) / 9 * ct + CU - 1) / CU;
+  for (int64_t r = least; r < least + 4; ++r) {
+    const int64_t tiles = std::min(std::max(CU * r / ct, (units + 8) / 9), (units + 1) / 2);
+    const int64_t rt = std::max<int64_t>(2, (units + tiles - 1) / tiles), tall = rt == 2 ? tiles : units - tiles * (rt - 1);
+    const int64_t at = load(tiles, r), low = std::max<int64_t>(2, rt - 1);
+    const int64_t cost = r * (price(rt, at) * tall + price(low, at) * (tiles - tall)) / tiles * 103 / 10000;
+    if (cost < best.cost) best = {tiles, tall, (int)rt, cost};
+  }
+  return best;
+}
+
 static int prompt_tile(int64_t m, int64_t n, int64_t k) {
   auto rounds = [](int64_t workgroups) { return (workgroups + 255) / 256; };
   const int64_t t16 = 12 + 12 * rounds(Short16::workgroups(m, n)), t32 = 14 + 17 * rounds(Short32::workgroups(m, n)),
                 t32w = 16 + 26 * rounds(Short32Wide::workgroups(m, n)),
                 t64 = 32 + 40 * rounds(Short64::workgroups(m, n));
   const int64_t least = std::min(std::min(t16, t32), std::min(t32w, t64));
-  const int64_t big = 10 + 170 * rounds((m + BIG_ROWS - 1) / BIG_ROWS * ((n + 511) / 512));
+  const int64_t big = 10 + 10240 / std::max<int64_t>(k, 64) + big_tiles(m, n).cost;
   if (big_takes(n, k) && big <= least) return 9;
   const int best = least == t16 ? 2 : least == t32 ? 3 : least == t32w ? 5 : 6;
   if (k >= SHORT_K) return best;
@@ -1397,11 +1442,19 @@ int launch_qmm_prefill(int arith, int tile, const uint16_t* x, int64_t ldx, cons
     case 5: TF_SHORT(Short32Wide, 2, 1, 1, 8, 256)
     case 6: TF_SHORT(Short64, 4, 2, 1, 4, 128)
     default: {
-      const unsigned grid = (unsigned)((int64_t)((m + BIG_ROWS - 1) / BIG_ROWS) * ((n + 511) / 512));
-      if (arith)
-        qmm_prefill_big_kernel<GS, EPI, 1><<<grid, BIG_THREADS, BIG_LDS, st>>>(x, ldx, w, s, b, out, m, n, kg, npad);
-      else
-        qmm_prefill_big_kernel<GS, EPI, 0><<<grid, BIG_THREADS, BIG_LDS, st>>>(x, ldx, w, s, b, out, m, n, kg, npad);
+      const BigTiles t = big_tiles(m, n);
+      const unsigned grid = (unsigned)(t.tiles * ((n + 511) / 512));
+#define TF_BIG(RT_)                                                                                                       \
+  case RT_:                                                                                                              \
+    if (arith)                                                                                                           \
+      qmm_prefill_big_kernel<GS, EPI, 1, RT_><<<grid, BIG_THREADS, 2 * big_stage(RT_), st>>>(x, ldx, w, s, b, out, m, n, kg, \
+                                                                                             npad, (int)t.tall);         \
+    else                                                                                                                 \
+      qmm_prefill_big_kernel<GS, EPI, 0, RT_><<<grid, BIG_THREADS, 2 * big_stage(RT_), st>>>(x, ldx, w, s, b, out, m, n, kg, \
+                                                                                             npad, (int)t.tall);         \
+    break;
+      switch (t.rt) { TF_BIG(2) TF_BIG(3) TF_BIG(4) TF_BIG(5) TF_BIG(6) TF_BIG(7) TF_BIG(8) TF_BIG(9) }
+#undef TF_BIG
     }
   }
 #undef TF_SMALL
@@ -1439,6 +1492,8 @@ extern "C" int tf_experts_prefill(int gs, int epi, const uint16_t* x, int64_t x_
   set_error("experts: no prefill kernel for group %d and epilogue %d", gs, epi);
   return 1;
 }
+
+extern "C" int tf_qmm_prompt_rows(int m, int n) { return 16 * big_tiles(m < 1 ? 1 : m, n < 1 ? 1 : n).rt; }
 
 extern "C" int tf_qmm_prompt_tile(int m, int n, int k) { return prompt_tile(m < 1 ? 1 : m, n < 1 ? 1 : n, k); }
 

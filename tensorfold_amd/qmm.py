@@ -320,8 +320,8 @@ def prompt_tile(m: int, n: int, k: int = 64) -> int:
     """The tile code that ``prefill_matmul(..., tile=0)`` takes for ``m`` rows of an (n, k) weight
     (cuda/kernels/qmm.py:202-205 names the reference's one tile, tuned for its chip): 1, 4 or 8 = a four-wave workgroup
     on 16, 64 or 128 rows x 128 columns; 2, 3, 5 or 6 = 16 x 64, 32 x 64, 32 x 128 or 64 x 128 of a pipeline for what
-    would leave compute units idle at larger tiles; 9 = eight waves on 128 rows x 512 columns, for K in whole steps of
-    64.  The launch asks the same rule; it needs no GPU."""
+    would leave compute units idle at larger tiles; 9 = eight waves on 32 to 144 rows x 512 columns, for K in whole steps
+    of 64.  The launch asks the same rule; it needs no GPU."""
 
     return _lib.lib().tf_qmm_prompt_tile(m, n, k)
 
