@@ -67,6 +67,10 @@ int tf_group_sums(const uint16_t* x, int64_t ldx, int m, int k, int gs, float* x
 int tf_qmm(const uint16_t* x, int64_t ldx, const float* xs, const uint32_t* weight, const uint16_t* scales,
            const uint16_t* biases, int64_t sb_stride, void* out, float* part, int32_t* counters, int n_counters, int m,
            int n, int k, int sk, int gs, int bm, int f32, int reduce, tf_stream_t stream);
+/* tf_qmm without xs: the launch takes the group sums itself, with tf_group_sums' bits. */
+int tf_qmm_own_sums(const uint16_t* x, int64_t ldx, const uint32_t* weight, const uint16_t* scales,
+                    const uint16_t* biases, int64_t sb_stride, void* out, float* part, int32_t* counters, int n_counters,
+                    int m, int n, int k, int sk, int gs, int bm, int f32, int reduce, tf_stream_t stream);
 /* tf_qmm (reduce != 0) for callers that cannot allocate or pass a workspace: code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc.  The K slices that tf_qmm keeps in `part` live in a fixed array
  * inside the library's device image (TF_QMM_STATIC_FLOATS fp32 = 16 MiB, held by every GPU the library runs on

@@ -20,6 +20,7 @@ PROTOTYPES = {
     "tf_qmm_unpack": [P, P, P, I, I, I, P, P, P, P],
     "tf_group_sums": [P, L, I, I, I, P, P],
     "tf_qmm": [P, L, P, P, P, P, L, P, P, P, I, I, I, I, I, I, I, I, I, P],
+    "tf_qmm_own_sums": [P, L, P, P, P, L, P, P, P, I, I, I, I, I, I, I, I, I, P],
     "tf_qmm_static": [P, L, P, P, P, P, L, P, I, I, I, I, I, I, I, P],
     "tf_qmm_group": [P, L, P, I, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, P],
     "tf_qmm_prompt_tile": [I, I, I],

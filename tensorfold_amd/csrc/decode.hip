@@ -105,12 +105,21 @@ constexpr size_t qmm_lds_floats(int waves, int rt) { return (size_t)waves * 16 *
 
 // A group in registers: the lane's column's codes, scale and bias; of row tile r the lane's eight inputs of each chunk
 // (row 16 r + row_of(c), inputs 8 kq ..) and the group sum of row 16 r + kq + 4 (c % NI).
-template <int GS, int RT>
+template <int GS, int RT, bool OWN>
 struct DenseStage {
   uint4 w[GS / 32], x[RT][GS / 32];
   uint32_t s, b;
   float xs[RT];
 };
+
+// The group sums of OWN calls, which no launch has taken ahead: the row tile's inputs (as the matrix instruction multiplies them)
+// times a column of ones, the chunks' sums added in fp32.  Result i is the row of result i of every product, so it is where the
+// group's fma wants it.  group_sums_kernel takes them the same way, so both forms of a call have the same bits.  Against 64 bits
+// (64 normal inputs, rms of the sum of magnitudes) 4.50e-10, 4.49e-10 with the lanes' own adds before.
+__device__ __forceinline__ f32x4_t ones_sum(bf16x8_t x) {
+  const u32x4_t one = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, __builtin_bit_cast(bf16x8_t, one), (f32x4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+}
 
 // A wave's walk over groups [g, g1) of a column tile for rows r0 .. r0 + valid - 1.  `flush(g, acc)` is called after
 // group g has been added (wave-uniform); it may park and clear acc.  Result i of acc[r][t]: row 16 r + kq + 4 i, column
@@ -118,7 +127,7 @@ struct DenseStage {
 // A lane ends with four of the matrix instruction's rows: 4 kq + (0..3).  The call's row p is put into row
 // 4 (p % 4) + p / 4, so that up to four rows fill the lanes' first results and up to eight the first two: a call of at
 // most 4 NI rows adds NI results up a lane, not four (17408 x 5120, one row: 17.9 us with NI = 4 for every call, 16.3 so).
-template <int GS, int RT, int NI, class FLUSH>
+template <int GS, int RT, int NI, bool OWN, class FLUSH>
 __device__ __forceinline__ void qmm_walk(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
                                          const uint32_t* __restrict__ W, const uint16_t* __restrict__ S,
                                          const uint16_t* __restrict__ B, int64_t sb_stride, int KG, int tile, int r0,
@@ -133,7 +142,7 @@ __device__ __forceinline__ void qmm_walk(const uint16_t* __restrict__ X, int64_t
 #pragma unroll
   for (int r = 0; r < RT; ++r) {          // rows past the last are the last one again, unstored
     xl[r] = X + (size_t)(r0 + min(16 * r + (c >> 2) + 4 * (c & 3), valid - 1)) * ldx + 8 * kq;
-    xsl[r] = XS + (size_t)(r0 + min(16 * r + kq + 4 * (c & (NI - 1)), valid - 1)) * KG;
+    xsl[r] = OWN ? nullptr : XS + (size_t)(r0 + min(16 * r + kq + 4 * (c & (NI - 1)), valid - 1)) * KG;
   }
 #pragma unroll
   for (int r = 0; r < RT; ++r)
@@ -141,7 +150,7 @@ __device__ __forceinline__ void qmm_walk(const uint16_t* __restrict__ X, int64_t
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int i = 0; i < NI; ++i) acc[r][t][i] = 0.f;
-  typedef DenseStage<GS, RT> Stg;
+  typedef DenseStage<GS, RT, OWN> Stg;
   auto load = [&](Stg& st, int g) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < CH; ++i) st.w[i] = ldg16(wt + ((size_t)g * CH + i) * 256 + wo);
@@ -151,21 +160,24 @@ __device__ __forceinline__ void qmm_walk(const uint16_t* __restrict__ X, int64_t
     for (int r = 0; r < RT; ++r) {
 #pragma unroll
       for (int i = 0; i < CH; ++i) st.x[r][i] = *reinterpret_cast<const uint4*>(xl[r] + (size_t)g * GS + 32 * i);
-      st.xs[r] = xsl[r][g];
+      if constexpr (!OWN) st.xs[r] = xsl[r][g];
     }
     // With one row tile a stage's requests stay apart from the next's: left alone, the compiler merges the stages' group
     // sums into one load, which arrives with the last stage.  (Two row tiles: 30.2 us so where 28.4 without.)
     if constexpr (RT == 1) asm volatile("" ::: "memory");
   };
   auto add = [&](const Stg& st, int at) __attribute__((always_inline)) {
-    f32x4_t p[RT][4];
+    f32x4_t p[RT][4], own[RT];
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
       uint32_t w[4] = {st.w[i].x, st.w[i].y, st.w[i].z, st.w[i].w};
       across(w);
       bf16x8_t xa[RT];
 #pragma unroll
-      for (int r = 0; r < RT; ++r) xa[r] = __builtin_bit_cast(bf16x8_t, stage8_bf16(st.x[r][i]));
+      for (int r = 0; r < RT; ++r) {
+        xa[r] = __builtin_bit_cast(bf16x8_t, stage8_bf16(st.x[r][i]));
+        if constexpr (OWN) own[r] = i ? own[r] + ones_sum(xa[r]) : ones_sum(xa[r]);
+      }
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const bf16x8_t q = codes8(w[t]);
@@ -181,9 +193,14 @@ __device__ __forceinline__ void qmm_walk(const uint16_t* __restrict__ X, int64_t
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
       float sc[NI];
-      if constexpr (NI == 1) sc[0] = st.xs[r];
-      if constexpr (NI > 1) sc[0] = row16_lane<0>(st.xs[r]), sc[1] = row16_lane<1>(st.xs[r]);
-      if constexpr (NI > 2) sc[2] = row16_lane<2>(st.xs[r]), sc[3] = row16_lane<3>(st.xs[r]);
+      if constexpr (OWN) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) sc[i] = own[r][i];
+      } else if constexpr (NI == 1) {
+        sc[0] = st.xs[r];
+      }
+      if constexpr (!OWN && NI > 1) sc[0] = row16_lane<0>(st.xs[r]), sc[1] = row16_lane<1>(st.xs[r]);
+      if constexpr (!OWN && NI > 2) sc[2] = row16_lane<2>(st.xs[r]), sc[3] = row16_lane<3>(st.xs[r]);
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -228,11 +245,11 @@ __device__ __forceinline__ void qmm_walk(const uint16_t* __restrict__ X, int64_t
 // Two stages: three (four in groups of 32) take the fourth workgroup's LDS and were slower from either (16 rows 17.8 and 20.4 us).
 constexpr int RING_STAGES = 2;
 
-template <int GS, int RT>
+template <int GS, int RT, bool OWN = false>
 struct QmmRing {
   static constexpr int CH = GS / 32;
-  static constexpr int AT_SB = CH * 1024, AT_X = AT_SB + 256, AT_XS = AT_X + RT * 16 * GS * 2, STAGE = AT_XS + RT * 64;      // bytes
-  static constexpr int LOADS = CH + 1 + RT * CH + 1;             // load instructions a group
+  static constexpr int AT_SB = CH * 1024, AT_X = AT_SB + 256, AT_XS = AT_X + RT * 16 * GS * 2, STAGE = AT_XS + (OWN ? 0 : RT * 64);      // bytes
+  static constexpr int LOADS = CH + 1 + RT * CH + (OWN ? 0 : 1);             // load instructions a group
   static constexpr int WAVE = RING_STAGES * STAGE;
 };
 
@@ -243,8 +260,17 @@ struct QmmRing {
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"          // "m0 is reserved": no value is kept there, but the compiler writes it too
 #define TF_TO_LDS(LOAD, ...) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" LOAD ::"s"(lds), __VA_ARGS__ : "memory", "m0")
-__device__ __forceinline__ void to_lds16(const void* base, uint32_t off, uint32_t lds) {
-  TF_TO_LDS("global_load_lds_dwordx4 %1, %2", "v"(off), "s"(base));
+// N loads in one statement, the j-th with 1,024 j added to both its address and its place
+__device__ __forceinline__ void to_lds16(const void* base, const uint32_t (&off)[1], uint32_t lds) {
+  TF_TO_LDS("global_load_lds_dwordx4 %1, %2", "v"(off[0]), "s"(base));
+}
+__device__ __forceinline__ void to_lds16(const void* base, const uint32_t (&off)[2], uint32_t lds) {
+  TF_TO_LDS("global_load_lds_dwordx4 %1, %3\n\tglobal_load_lds_dwordx4 %2, %3 offset:1024", "v"(off[0]), "v"(off[1]), "s"(base));
+}
+__device__ __forceinline__ void to_lds16(const void* base, const uint32_t (&off)[4], uint32_t lds) {
+  TF_TO_LDS("global_load_lds_dwordx4 %1, %5\n\tglobal_load_lds_dwordx4 %2, %5 offset:1024\n\t"
+            "global_load_lds_dwordx4 %3, %5 offset:2048\n\tglobal_load_lds_dwordx4 %4, %5 offset:3072",
+            "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(base));
 }
 __device__ __forceinline__ void to_lds4(const void* base, uint32_t off, uint32_t lds) {
   TF_TO_LDS("global_load_lds_dword %1, %2", "v"(off), "s"(base));
@@ -259,42 +285,50 @@ __device__ __forceinline__ void settled(A*& a, B*& b, C*& c) {
 #undef TF_TO_LDS
 #pragma clang diagnostic pop
 
-template <int GS, int RT>
+template <int GS, int RT, bool OWN>
 __device__ __forceinline__ void qmm_ring_walk(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
                                               const uint32_t* __restrict__ W, const uint16_t* __restrict__ S,
                                               const uint16_t* __restrict__ B, int64_t sb_stride, int KG, int tile, int r0,
                                               int valid, int g0, int g1, float (&acc)[RT][4][4], unsigned char* ring) {
-  typedef QmmRing<GS, RT> R;
+  typedef QmmRing<GS, RT, OWN> R;
   constexpr int CH = R::CH, P = R::LOADS, ROW = GS * 2, PIECES = ROW / 16;       // bytes of a row's group of inputs; 16-byte pieces
   const int lane = threadIdx.x & 63, c = lane & 15, kq = lane >> 4;
   // operand row o of the matrix instruction's 16 RT holds this row of the call (qmm_walk has the reason)
   auto call_row = [&](int o) { return min((o & ~15) + ((o & 15) >> 2) + 4 * (o & 3), valid - 1); };
   // a row's pieces lie turned by its number, so that 16 lanes reading a piece of 16 rows meet different banks
   auto turn = [&](int o) { return PIECES == 8 ? o & 7 : (o >> 1) & 3; };
-  uint32_t xoff[RT * CH];
+  // (the j-th load adds 1,024 j to its address, which its offset does without: all of them 4,096 ahead of the row's)
+  uint32_t xoff[RT * CH], woff[CH];
 #pragma unroll
   for (int j = 0; j < RT * CH; ++j) {
     const int o = (64 / PIECES) * j + lane / PIECES;
-    xoff[j] = (uint32_t)call_row(o) * (uint32_t)ldx * 2u + (((lane % PIECES) ^ turn(o)) * 16);
+    xoff[j] = (uint32_t)call_row(o) * (uint32_t)ldx * 2u + (((lane % PIECES) ^ turn(o)) * 16) + (4096 - 1024 * j);
   }
+#pragma unroll
+  for (int i = 0; i < CH; ++i) woff[i] = lane * 16;
   const uint32_t xsoff = (uint32_t)call_row(lane & (16 * RT - 1)) * (uint32_t)KG * 4u;
-  const uint16_t* sb = (lane < 32 ? S : B) + tile * 64 + 2 * (lane & 31);
-  const uint16_t* x0 = X + (size_t)r0 * ldx;
-  const float* xs0 = XS + (size_t)r0 * KG;
-  const uint32_t* w0 = W + (size_t)tile * KG * (CH * 256);
+  const uint16_t* sb = (lane < 32 ? S : B) + tile * 64 + 2 * (lane & 31) + (size_t)g0 * sb_stride;
+  const uint16_t* xg = X + (size_t)r0 * ldx + (size_t)g0 * GS - 2048;
+  const float* xsg = OWN ? nullptr : XS + (size_t)r0 * KG + g0;
+  const uint32_t* wg = W + ((size_t)tile * KG + g0) * (CH * 256);
   const uint32_t at = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)ring);
+  // group g's operands; the groups are asked for in turn
   auto request = [&](int g) {
     const uint32_t lds = at + (g & (RING_STAGES - 1)) * R::STAGE;
-    const uint32_t* w = w0 + (size_t)g * (CH * 256);
-    const uint16_t* x = x0 + (size_t)g * GS;
-    const float* xs = xs0 + g;
+    const uint32_t* w = wg;
+    const uint16_t* x = xg;
+    const float* xs = xsg;
     settled(w, x, xs);
-#pragma unroll
-    for (int i = 0; i < CH; ++i) to_lds16(w + i * 256, lane * 16, lds + i * 1024);
-    lane_to_lds4(sb + (size_t)g * sb_stride, lds + R::AT_SB);
-#pragma unroll
-    for (int j = 0; j < RT * CH; ++j) to_lds16(x, xoff[j], lds + R::AT_X + j * 1024);
-    if (lane < 16 * RT) to_lds4(xs, xsoff, lds + R::AT_XS);
+    to_lds16(w, woff, lds);
+    lane_to_lds4(sb, lds + R::AT_SB);
+    to_lds16(x, xoff, lds + R::AT_X);
+    if constexpr (!OWN) {
+      if (lane < 16 * RT) to_lds4(xs, xsoff, lds + R::AT_XS);
+      xsg += 1;
+    }
+    wg += CH * 256;
+    xg += GS;
+    sb += sb_stride;
   };
 #pragma unroll
   for (int r = 0; r < RT; ++r)
@@ -321,7 +355,7 @@ __device__ __forceinline__ void qmm_ring_walk(const uint16_t* __restrict__ X, in
 #pragma unroll
       for (int i = 0; i < CH; ++i)
         x[r][i] = *reinterpret_cast<const uint4*>(stage + R::AT_X + (16 * r + c) * ROW + (((4 * i + kq) ^ turn(c)) * 16));
-      sums[r] = *reinterpret_cast<const float4*>(stage + R::AT_XS + (16 * r + 4 * kq) * 4);
+      if constexpr (!OWN) sums[r] = *reinterpret_cast<const float4*>(stage + R::AT_XS + (16 * r + 4 * kq) * 4);
     }
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -330,12 +364,15 @@ __device__ __forceinline__ void qmm_ring_walk(const uint16_t* __restrict__ X, in
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");          // the stage is read: its place is free
     if (g + RING_STAGES < g1) request(g + RING_STAGES);
-    f32x4_t p[RT][4];
+    f32x4_t p[RT][4], own[RT];
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
       bf16x8_t xa[RT];
 #pragma unroll
-      for (int r = 0; r < RT; ++r) xa[r] = __builtin_bit_cast(bf16x8_t, stage8_bf16(x[r][i]));
+      for (int r = 0; r < RT; ++r) {
+        xa[r] = __builtin_bit_cast(bf16x8_t, stage8_bf16(x[r][i]));
+        if constexpr (OWN) own[r] = i ? own[r] + ones_sum(xa[r]) : ones_sum(xa[r]);
+      }
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const bf16x8_t q = codes8(w[i][t]);
@@ -346,6 +383,7 @@ __device__ __forceinline__ void qmm_ring_walk(const uint16_t* __restrict__ X, in
     }
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
+      if constexpr (OWN) sums[r] = make_float4(own[r][0], own[r][1], own[r][2], own[r][3]);
       const float sc[4] = {sums[r].x, sums[r].y, sums[r].z, sums[r].w};
 #pragma unroll
       for (int t = 0; t < 4; ++t)
@@ -358,7 +396,7 @@ __device__ __forceinline__ void qmm_ring_walk(const uint16_t* __restrict__ X, in
 
 // grid (column tiles of 64 x row tiles of 16 RT, 1, SK).  Slice z takes groups [z * per, (z + 1) * per), its waves
 // split them again (added in wave order); SK > 1 leaves the slice's fp32 sums in part[z].
-template <int GS, int WAVES, int RT, int NI, bool COH = false, bool RING = false>
+template <int GS, int WAVES, int RT, int NI, bool COH, bool RING, bool OWN>
 __device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
                                           const uint32_t* __restrict__ W, const uint16_t* __restrict__ S,
                                           const uint16_t* __restrict__ B, int64_t sb_stride, void* __restrict__ out,
@@ -372,11 +410,11 @@ __device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_
   float acc[RT][4][NI];
   const int g0 = gs0 + (int)((long long)wave * per / WAVES), g1 = gs0 + (int)((long long)(wave + 1) * per / WAVES);
   if constexpr (RING) {
-    qmm_ring_walk<GS, RT>(X, ldx, XS, W, S, B, sb_stride, KG, tile, r0, valid, g0, g1, acc,
-                          reinterpret_cast<unsigned char*>(part) + wave * QmmRing<GS, RT>::WAVE);
+    qmm_ring_walk<GS, RT, OWN>(X, ldx, XS, W, S, B, sb_stride, KG, tile, r0, valid, g0, g1, acc,
+                               reinterpret_cast<unsigned char*>(part) + wave * QmmRing<GS, RT, OWN>::WAVE);
     __syncthreads();                                     // the rings are read: the sums take their place
   } else {
-    qmm_walk<GS, RT, NI>(X, ldx, XS, W, S, B, sb_stride, KG, tile, r0, valid, g0, g1, acc, [](int, float (&)[RT][4][NI]) {});
+    qmm_walk<GS, RT, NI, OWN>(X, ldx, XS, W, S, B, sb_stride, KG, tile, r0, valid, g0, g1, acc, [](int, float (&)[RT][4][NI]) {});
   }
 #pragma unroll
   for (int r = 0; r < RT; ++r)
@@ -401,15 +439,15 @@ __device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_
   }
 }
 
-template <int GS, int WAVES, int RT, int NI, bool RING = false>
-__global__ void __launch_bounds__(WAVES * 64)
+template <int GS, int WAVES, int RT, int NI, bool RING, bool OWN>
+__global__ void __launch_bounds__(WAVES * 64, 2)
     qmm_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
                const uint32_t* __restrict__ W, const uint16_t* __restrict__ S, const uint16_t* __restrict__ B,
                int64_t sb_stride, void* __restrict__ out, float* __restrict__ part_out, int M, int N, int KG, int SK,
                int f32) {
   extern __shared__ float lds[];
-  qmm_block<GS, WAVES, RT, NI, false, RING>(X, ldx, XS, W, S, B, sb_stride, out, part_out, M, N, KG, SK, f32, blockIdx.x, blockIdx.z,
-                               lds);
+  qmm_block<GS, WAVES, RT, NI, false, RING, OWN>(X, ldx, XS, W, S, B, sb_stride, out, part_out, M, N, KG, SK, f32, blockIdx.x,
+                                                 blockIdx.z, lds);
 }
 
 // The split matmul of a few rows and its reduce in one launch with no traffic between workgroups, for callers without
@@ -418,7 +456,7 @@ __global__ void __launch_bounds__(WAVES * 64)
 // take (slice z, wave w: run 4 z + w) keep their ends; a wave walks 4 SK / WAVES of them one after the other, parks each
 // one's sums in LDS, and the end adds a slice's four and then the slices in order: the bits of qmm_kernel and
 // qmm_reduce_kernel.
-template <int GS, int WAVES, int NI>
+template <int GS, int WAVES, int NI, bool OWN>
 __device__ __forceinline__ void qmm_whole_block(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
                                                 const uint32_t* __restrict__ W, const uint16_t* __restrict__ S,
                                                 const uint16_t* __restrict__ B, int64_t sb_stride,
@@ -453,7 +491,7 @@ __device__ __forceinline__ void qmm_whole_block(const uint16_t* __restrict__ X, 
     while (u < u1 && begin(u + 1) == begin(u)) ++u;
     end = u < u1 ? begin(u + 1) : -1;
   };
-  qmm_walk<GS, 1, NI>(X, ldx, XS, W, S, B, sb_stride, KG, tile, 0, M, begin(u0), begin(u1), acc, flush);
+  qmm_walk<GS, 1, NI, OWN>(X, ldx, XS, W, S, B, sb_stride, KG, tile, 0, M, begin(u0), begin(u1), acc, flush);
   __syncthreads();
   for (int o = tid; o < M * 64; o += WAVES * 64) {
     const int r = o >> 6, l = o & 63, cc = tile * 64 + l;
@@ -475,13 +513,13 @@ __device__ __forceinline__ void qmm_whole_block(const uint16_t* __restrict__ X, 
 // LDS bytes of a workgroup (at most 34 KB: eight slices come with NI = 1 only)
 constexpr size_t qmm_whole_lds(int sk, int ni) { return sizeof(float) * 4 * sk * 4 * ni * QPART; }
 
-template <int GS, int WAVES, int NI>
+template <int GS, int WAVES, int NI, bool OWN>
 __global__ void __launch_bounds__(WAVES * 64)
     qmm_whole_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
                      const uint32_t* __restrict__ W, const uint16_t* __restrict__ S, const uint16_t* __restrict__ B,
                      int64_t sb_stride, void* __restrict__ out, int M, int N, int KG, int SK, int f32) {
   extern __shared__ float lds[];
-  qmm_whole_block<GS, WAVES, NI>(X, ldx, XS, W, S, B, sb_stride, out, M, N, KG, SK, f32, blockIdx.x, lds);
+  qmm_whole_block<GS, WAVES, NI, OWN>(X, ldx, XS, W, S, B, sb_stride, out, M, N, KG, SK, f32, blockIdx.x, lds);
 }
 
 // What a slice's workgroup does once its sums are in part[z] (stored through to memory): wait for the stores'
@@ -522,16 +560,16 @@ __device__ __forceinline__ void qmm_arrive_tail(int* __restrict__ counter, const
 // part[z] with stores that go through to memory, waits for them to be acknowledged and counts itself in at the column
 // tile's counter; the workgroup that finds the others there adds the slices in slice order (qmm_reduce_kernel's
 // arithmetic) and puts the counter back to zero.
-template <int GS, int WAVES, int NI>
-__global__ void __launch_bounds__(WAVES * 64)
+template <int GS, int WAVES, int NI, bool OWN>
+__global__ void __launch_bounds__(WAVES * 64, 2)
     qmm_arrive_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
                       const uint32_t* __restrict__ W, const uint16_t* __restrict__ S, const uint16_t* __restrict__ B,
                       int64_t sb_stride, void* __restrict__ out, float* __restrict__ part_out, int* __restrict__ counters,
                       int M, int N, int KG, int SK, int f32) {
   extern __shared__ float lds[];
   __shared__ int last;
-  qmm_block<GS, WAVES, 1, NI, true>(X, ldx, XS, W, S, B, sb_stride, out, part_out, M, N, KG, SK, f32, blockIdx.x,
-                                    blockIdx.z, lds);
+  qmm_block<GS, WAVES, 1, NI, true, false, OWN>(X, ldx, XS, W, S, B, sb_stride, out, part_out, M, N, KG, SK, f32, blockIdx.x,
+                                                blockIdx.z, lds);
   qmm_arrive_tail<WAVES>(counters + (size_t)blockIdx.x * TF_QMM_COUNTER_STRIDE, part_out, out, M, N, SK, f32, blockIdx.x,
                          &last);
 }
@@ -553,7 +591,7 @@ struct GroupArgs {
 };
 
 template <int GS, int WAVES, int RT, int NI, bool RING = false>
-__global__ void __launch_bounds__(WAVES * 64)
+__global__ void __launch_bounds__(WAVES * 64, 2)
     qmm_group_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS, GroupArgs a, int M,
                      int KG, int f32) {
   extern __shared__ float lds[];
@@ -562,7 +600,7 @@ __global__ void __launch_bounds__(WAVES * 64)
   for (int i = 1; i < GROUP_MAX; ++i)
     if (i < a.count && (int)blockIdx.x >= a.first[i]) w = i;
   if ((int)blockIdx.z >= a.sk[w]) return;
-  qmm_block<GS, WAVES, RT, NI, false, RING>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], a.part[w], M, a.n[w], KG,
+  qmm_block<GS, WAVES, RT, NI, false, RING, false>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], a.part[w], M, a.n[w], KG,
                                a.sk[w], f32, blockIdx.x - a.first[w], blockIdx.z, lds);
 }
 
@@ -576,14 +614,14 @@ __global__ void __launch_bounds__(1024)
 #pragma unroll
   for (int i = 1; i < GROUP_MAX; ++i)
     if (i < a.count && (int)blockIdx.x >= a.first[i]) w = i;
-  qmm_whole_block<GS, 16, NI>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], M, a.n[w], KG, a.sk[w], f32,
+  qmm_whole_block<GS, 16, NI, false>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], M, a.n[w], KG, a.sk[w], f32,
                               blockIdx.x - a.first[w], lds);
 }
 
 // the grouped launch whose slices are added up by the last workgroup of a tile to finish (qmm_arrive_kernel's way);
 // a weight whose K is not split stores its rows itself
 template <int GS, int WAVES, int NI>
-__global__ void __launch_bounds__(WAVES * 64)
+__global__ void __launch_bounds__(WAVES * 64, 2)
     qmm_group_arrive_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS, GroupArgs a, int M,
                             int KG, int f32) {
   extern __shared__ float lds[];
@@ -594,7 +632,7 @@ __global__ void __launch_bounds__(WAVES * 64)
     if (i < a.count && (int)blockIdx.x >= a.first[i]) w = i;
   if ((int)blockIdx.z >= a.sk[w]) return;
   const int block = blockIdx.x - a.first[w];
-  qmm_block<GS, WAVES, 1, NI, true>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], a.part[w], M, a.n[w], KG,
+  qmm_block<GS, WAVES, 1, NI, true, false, false>(X, ldx, XS, a.w[w], a.s[w], a.b[w], a.sb_stride[w], a.out[w], a.part[w], M, a.n[w], KG,
                                     a.sk[w], f32, block, blockIdx.z, lds);
   if (a.sk[w] > 1)
     qmm_arrive_tail<WAVES>(a.counters[w] + (size_t)block * TF_QMM_COUNTER_STRIDE, a.part[w], a.out[w], M, a.n[w],
@@ -640,12 +678,31 @@ __global__ void qmm_reduce_kernel(const float* __restrict__ part, void* __restri
   else reinterpret_cast<uint16_t*>(out)[i] = (uint16_t)f32_bf16_bits(acc);
 }
 
+// A wave takes 16 rows' sums of 16 groups (`ones_sum`); four waves a workgroup along the groups.
 template <int GS>
 __global__ void __launch_bounds__(256)
     group_sums_kernel(const uint16_t* __restrict__ X, int64_t ldx, int M, int KG, float* __restrict__ XS) {
-  const int r = blockIdx.x;
-  const uint16_t* xrow[1] = {X + (size_t)r * ldx};
-  group_sums_block<GS>(xrow, 1, KG, XS + (size_t)r * KG, threadIdx.x, 256);
+  const int lane = threadIdx.x & 63, c = lane & 15, kq = lane >> 4;
+  const int runs = (KG - 1) / 64 + 1, rt = blockIdx.x / runs;
+  const int r0 = rt * 16, g0 = ((blockIdx.x - rt * runs) * 4 + (threadIdx.x >> 6)) * 16;
+  if (g0 >= KG) return;
+  const uint16_t* xl = X + (size_t)min(r0 + c, M - 1) * ldx + 8 * kq;
+  f32x4_t mine = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int j = 0; j < 16; ++j) {
+    const size_t at = (size_t)min(g0 + j, KG - 1) * GS;
+    f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < GS / 32; ++i) {
+      const uint4 v = *reinterpret_cast<const uint4*>(xl + at + 32 * i);
+      const f32x4_t t = ones_sum(__builtin_bit_cast(bf16x8_t, stage8_bf16(v)));
+      sum = i ? sum + t : t;
+    }
+    if (c == j) mine = sum;                       // every column holds the sums: lane c keeps group g0 + c's
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (r0 + 4 * kq + i < M && g0 + c < KG) XS[(size_t)(r0 + 4 * kq + i) * KG + g0 + c] = mine[i];
 }
 
 constexpr int QMM_WAVES = 4;
@@ -667,8 +724,10 @@ static bool ring_pays(int m, int gs, int kg, int sk, int least) {
   return m > 10 || gs != 64 || kg < 128 || kg < 6 * QMM_WAVES * sk;
 }
 // LDS of its workgroup: the waves' rings, and later their sums in the same place
+template <bool OWN>
 static size_t ring_lds(int gs, int rt) {
-  const int wave = gs == 64 ? (rt == 1 ? QmmRing<64, 1>::WAVE : QmmRing<64, 2>::WAVE) : rt == 1 ? QmmRing<32, 1>::WAVE : QmmRing<32, 2>::WAVE;
+  const int wave = gs == 64 ? (rt == 1 ? QmmRing<64, 1, OWN>::WAVE : QmmRing<64, 2, OWN>::WAVE)
+                            : (rt == 1 ? QmmRing<32, 1, OWN>::WAVE : QmmRing<32, 2, OWN>::WAVE);
   return std::max((size_t)QMM_WAVES * wave, sizeof(float) * qmm_lds_floats(QMM_WAVES, rt));
 }
 constexpr int ARRIVE_ROWS = 8;        // rows up to which, given arrival counters, the split launch adds its own slices
@@ -787,20 +846,25 @@ extern "C" int tf_group_sums(const uint16_t* x, int64_t ldx, int m, int k, int g
   TF_REQUIRE(gs == 32 || gs == 64, "group_sums: groups of 32 or 64 inputs, not %d", gs);
   TF_REQUIRE(x && xs && m >= 1 && k >= gs && k % gs == 0, "group_sums: x must be (M, K), K a multiple of the group");
   TF_REQUIRE(aligned16(x) && (m == 1 || ldx % 8 == 0), "x rows must start on 16-byte boundaries");
-  if (gs == 64) group_sums_kernel<64><<<m, 256, 0, as_stream(stream)>>>(x, ldx, m, k / gs, xs);
-  else group_sums_kernel<32><<<m, 256, 0, as_stream(stream)>>>(x, ldx, m, k / gs, xs);
+  const int kg = k / gs;
+  const int64_t blocks = (int64_t)((m - 1) / 16 + 1) * ((kg - 1) / 64 + 1);
+  TF_REQUIRE(blocks <= 0x7FFFFFFF, "group_sums: grid too large");
+  const unsigned grid = (unsigned)blocks;
+  if (gs == 64) group_sums_kernel<64><<<grid, 256, 0, as_stream(stream)>>>(x, ldx, m, kg, xs);
+  else group_sums_kernel<32><<<grid, 256, 0, as_stream(stream)>>>(x, ldx, m, kg, xs);
   TF_LAUNCH_OK("tf_group_sums");
   return 0;
 }
 
-// tf_qmm and tf_qmm_static: the checks and launches of the decode-form matmul; `part` holds the K slices.
+// tf_qmm, tf_qmm_own_sums (OWN: no xs) and tf_qmm_static: the checks and launches of the decode-form matmul; `part` holds the K slices.
+template <bool OWN>
 static int qmm_launch(const uint16_t* x, int64_t ldx, const float* xs, const uint32_t* weight, const uint16_t* scales,
                       const uint16_t* biases, int64_t sb_stride, void* out, float* part, int32_t* counters,
                       int n_counters, int m, int n, int k, int sk, int gs, int bm, int f32, int reduce,
                       tf_stream_t stream) {
   TF_REQUIRE(gs == 32 || gs == 64, "groups of 32 or 64");
   TF_REQUIRE(bm == 16 || bm == 32 || bm == 64, "row tile 16, 32 or 64");
-  TF_REQUIRE(x && xs && weight && scales && biases && out && m >= 1 && n >= 1, "qmm: null pointer or empty shape");
+  TF_REQUIRE(x && (OWN || xs) && weight && scales && biases && out && m >= 1 && n >= 1, "qmm: null pointer or empty shape");
   TF_REQUIRE(aligned16(x) && (m == 1 || ldx % 8 == 0), "x rows must start on 16-byte boundaries");
   TF_REQUIRE(ldx >= k || m == 1, "x: (M, K) bf16 with contiguous rows");
   const int kg = k / gs, npad = (n + 127) / 128 * 128;
@@ -813,13 +877,13 @@ static int qmm_launch(const uint16_t* x, int64_t ldx, const float* xs, const uin
   // tile: accepted, and no longer what decides)
   const int rt = m <= 16 ? 1 : 2, tiles = (n + 63) / 64, rts = (m + 16 * rt - 1) / (16 * rt);
   const bool ring = ring_pays(m, gs, kg, sk, 4) && ring_takes(ldx, sb_stride, scales, biases);
-  const size_t smem = ring ? ring_lds(gs, rt) : sizeof(float) * qmm_lds_floats(QMM_WAVES, rt);
+  const size_t smem = ring ? ring_lds<OWN>(gs, rt) : sizeof(float) * qmm_lds_floats(QMM_WAVES, rt);
   TF_REQUIRE((int64_t)tiles * rts <= 0x7FFFFFFF && sk <= 65535, "qmm: grid too large");
   const dim3 grid((unsigned)(tiles * rts), 1, (unsigned)sk);
   if (reduce && sk > 1 && counters && m <= ARRIVE_ROWS && tiles <= n_counters) {
     // few rows and arrival counters: the slices are added up by the last workgroup of a tile to finish
 #define TF_GO(GS_, NI_)                                                                                             \
-  qmm_arrive_kernel<GS_, QMM_WAVES, NI_><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, weight, scales, biases, sb_stride, \
+  qmm_arrive_kernel<GS_, QMM_WAVES, NI_, OWN><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, weight, scales, biases, sb_stride, \
                                                                             out, part, counters, m, n, kg, sk, f32)
     if (gs == 64) {
       if (m <= 4) TF_GO(64, 1);
@@ -835,7 +899,7 @@ static int qmm_launch(const uint16_t* x, int64_t ldx, const float* xs, const uin
   if (reduce && whole_takes(tiles, sk, m, k)) {
     const size_t whole = qmm_whole_lds(sk, m <= 4 ? 1 : 2);
 #define TF_GO(GS_, W_, NI_)                                                                                              \
-  qmm_whole_kernel<GS_, W_, NI_><<<(unsigned)tiles, W_ * 64, whole, s>>>(x, ldx, xs, weight, scales, biases, sb_stride, out, \
+  qmm_whole_kernel<GS_, W_, NI_, OWN><<<(unsigned)tiles, W_ * 64, whole, s>>>(x, ldx, xs, weight, scales, biases, sb_stride, out, \
                                                                          m, n, kg, sk, f32)
     if (gs == 64) {
       if (sk == 2 && m <= 4) TF_GO(64, 8, 1);
@@ -853,7 +917,7 @@ static int qmm_launch(const uint16_t* x, int64_t ldx, const float* xs, const uin
     return 0;
   }
 #define TF_GO(GS_, RT_, NI_, RING_)                                                                                      \
-  qmm_kernel<GS_, QMM_WAVES, RT_, NI_, RING_><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, weight, scales, biases,     \
+  qmm_kernel<GS_, QMM_WAVES, RT_, NI_, RING_, OWN><<<grid, QMM_WAVES * 64, smem, s>>>(x, ldx, xs, weight, scales, biases,     \
                                                                                  sb_stride, out, part, m, n, kg, sk, f32)
   if (gs == 64) {
     if (m <= 4) TF_GO(64, 1, 1, false);
@@ -886,8 +950,18 @@ extern "C" int tf_qmm(const uint16_t* x, int64_t ldx, const float* xs, const uin
                       tf_stream_t stream) {
   clear_error();
   TF_REQUIRE(!counters || n_counters >= 0, "qmm: a negative number of counters");
-  return qmm_launch(x, ldx, xs, weight, scales, biases, sb_stride, out, part, counters, n_counters, m, n, k, sk, gs, bm,
+  return qmm_launch<false>(x, ldx, xs, weight, scales, biases, sb_stride, out, part, counters, n_counters, m, n, k, sk, gs, bm,
                     f32, reduce, stream);
+}
+
+extern "C" int tf_qmm_own_sums(const uint16_t* x, int64_t ldx, const uint32_t* weight, const uint16_t* scales,
+                               const uint16_t* biases, int64_t sb_stride, void* out, float* part, int32_t* counters,
+                               int n_counters, int m, int n, int k, int sk, int gs, int bm, int f32, int reduce,
+                               tf_stream_t stream) {
+  clear_error();
+  TF_REQUIRE(!counters || n_counters >= 0, "qmm: a negative number of counters");
+  return qmm_launch<true>(x, ldx, nullptr, weight, scales, biases, sb_stride, out, part, counters, n_counters, m, n, k, sk, gs,
+                          bm, f32, reduce, stream);
 }
 
 // The K slices of tf_qmm_static: one array a GPU, part of the loaded code object, so no call ever allocates it.
@@ -936,7 +1010,7 @@ extern "C" int tf_qmm_static(const uint16_t* x, int64_t ldx, const float* xs, co
   float* part = nullptr;
   int32_t* counters = nullptr;
   if (sk > 1 && !static_scratch(&part, &counters)) return 1;
-  return qmm_launch(x, ldx, xs, weight, scales, biases, sb_stride, out, part, counters, TF_QMM_STATIC_COUNTERS, m, n, k,
+  return qmm_launch<false>(x, ldx, xs, weight, scales, biases, sb_stride, out, part, counters, TF_QMM_STATIC_COUNTERS, m, n, k,
                     sk, gs, bm, f32, 1, stream);
 }
 
@@ -1004,7 +1078,7 @@ extern "C" int tf_qmm_group(const uint16_t* x, int64_t ldx, const float* xs, int
   bool ring = false;                          // the weight that gains most decides
   for (int i = 0; i < count; ++i) ring = ring || ring_pays(m, gs, kg, sks[i], 5);
   for (int i = 0; i < count && ring; ++i) ring = ring_takes(ldx, sb_strides[i], scales[i], biases[i]);
-  const size_t smem = ring ? ring_lds(gs, rt) : sizeof(float) * qmm_lds_floats(QMM_WAVES, rt);
+  const size_t smem = ring ? ring_lds<false>(gs, rt) : sizeof(float) * qmm_lds_floats(QMM_WAVES, rt);
   const dim3 grid((unsigned)blocks, 1, (unsigned)max_sk);
   if (arrive) {
 #define TF_GO(GS_, NI_) \

@@ -186,8 +186,6 @@ def matmul(x: torch.Tensor, q: Q4, xs: torch.Tensor | None = None, *, sk: int | 
 
     x = _check_x(x, q, "matmul")
     m = int(x.shape[0])
-    own_xs = xs is None
-    xs = group_sums(x, q.gs) if own_xs else xs
     sk = split_k(q.n, q.k, q.gs) if not sk else sk
     if out is None:
         out = x.new_empty((m, q.n), dtype=torch.float32 if f32 else torch.bfloat16)
@@ -199,11 +197,13 @@ def matmul(x: torch.Tensor, q: Q4, xs: torch.Tensor | None = None, *, sk: int | 
     elif sk > 1 and (part.dtype != torch.float32 or part.numel() < sk * m * q.n or not part.is_contiguous()
                      or part.device != x.device):
         raise ValueError(f"matmul: part must hold {sk} x {m} x {q.n} fp32 values (split_k gives the slice count)")
-    if not own_xs and (xs.dtype != torch.float32 or tuple(xs.shape) != (m, q.k // q.gs) or not xs.is_contiguous()
-                       or xs.device != x.device):
+    if xs is not None and (xs.dtype != torch.float32 or tuple(xs.shape) != (m, q.k // q.gs) or not xs.is_contiguous()
+                           or xs.device != x.device):
         raise ValueError(f"matmul: xs must be contiguous fp32 ({m}, {q.k // q.gs}), the group sums of x")
     counters = q.counters if reduce and sk > 1 and m <= 8 else None
-    _lib.call("tf_qmm", _lib.ptr(x), x.stride(0), _lib.ptr(xs), _lib.ptr(q.weight), _lib.ptr(q.scales),
+    # without xs the launch takes the group sums itself
+    name, given = ("tf_qmm_own_sums", ()) if xs is None else ("tf_qmm", (_lib.ptr(xs),))
+    _lib.call(name, _lib.ptr(x), x.stride(0), *given, _lib.ptr(q.weight), _lib.ptr(q.scales),
               _lib.ptr(q.biases), q.scales.stride(0), _lib.ptr(out), _lib.ptr(part), _lib.ptr(counters),
               0 if counters is None else counters.numel() // COUNTER_STRIDE, m, q.n, q.k, sk, q.gs, bucket(m),
               int(f32), int(reduce))
