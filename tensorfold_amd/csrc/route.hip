@@ -1,6 +1,8 @@
 // MoE glue around the expert kernels: router logits, per-row top-k, the stable grouping of pairs by expert, and the
 // weighted combine.  All integer results (ids, members, items) are deterministic and independent of the row count.
 
+#include <type_traits>
+
 #include "routing.h"
 
 namespace tf {
@@ -14,7 +16,6 @@ namespace {
 // form spent its time on (11 us at 1 to 8 rows x 128 experts x 2688, 131 us at 4,096 x 513 x 2048).
 
 constexpr int ROUTER_SLICES = 8;
-constexpr int64_t ROUTER_ROUND = 512;      // workgroups of 32 x 64 that the chip holds at once: beyond, the wide kernel
 
 __device__ __forceinline__ int router_chunk(int s, int chunks) { return s * chunks / ROUTER_SLICES; }
 
@@ -23,14 +24,15 @@ __device__ __forceinline__ int router_chunk(int s, int chunks) { return s * chun
 // its last one again up to UNR made hidden sizes up to 896 slower than one chain a wave (32 rows x 128 experts x 512:
 // one chain 5.4 us, repeated 6.9, so 5.0) and cost up to a quarter where UNR does not divide a slice (8 x 128 x 4096
 // 12.1 -> 9.1 us, x 2688 7.7 -> 7.1; graph replays).
+template <int RM, int RN>
+using RouterParts = f32x4_t[ROUTER_SLICES][RM * RN][64];
+
 template <int RM, int RN, int UNR>
-__global__ void __launch_bounds__(64 * ROUTER_SLICES)
-    router_kernel(const uint16_t* __restrict__ X, int64_t ldx, const uint16_t* __restrict__ R, float* __restrict__ out,
-                  int M, int D, int NE) {
-  __shared__ f32x4_t part[ROUTER_SLICES][RM * RN][64];
+__device__ __forceinline__ void router_tile(const uint16_t* __restrict__ X, int64_t ldx, const uint16_t* __restrict__ R,
+                                            float* __restrict__ out, int M, int D, int NE, int m0, int e0,
+                                            RouterParts<RM, RN>& part) {
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, kq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int m0 = blockIdx.x * 16 * RM, e0 = blockIdx.y * 16 * RN;
   const uint16_t* xa[RM];
   const uint16_t* wb[RN];
 #pragma unroll
@@ -83,97 +85,134 @@ __global__ void __launch_bounds__(64 * ROUTER_SLICES)
   }
 }
 
-// Many tiles: four waves on 64 rows x 128 experts, both operands through LDS (whole 128-byte lines from memory, 64
-// inputs a step, two steps in flight in registers), a wave on 32 x 64 walking the slices itself.  Column tiles past the
-// last expert are not computed (a shared expert's gate leaves a workgroup with one of eight).
-constexpr int RW_M = 64, RW_N = 128, RW_STEP = 64, RW_ROW = RW_STEP * 2 + 16;      // bytes of an LDS row, padded
+template <int RM, int RN, int UNR>
+__global__ void __launch_bounds__(64 * ROUTER_SLICES)
+    router_kernel(const uint16_t* __restrict__ X, int64_t ldx, const uint16_t* __restrict__ R, float* __restrict__ out,
+                  int M, int D, int NE) {
+  __shared__ RouterParts<RM, RN> part;
+  router_tile<RM, RN, UNR>(X, ldx, R, out, M, D, NE, blockIdx.x * 16 * RM, blockIdx.y * 16 * RN, part);
+}
 
-__global__ void __launch_bounds__(256)
-    router_wide_kernel(const uint16_t* __restrict__ X, int64_t ldx, const uint16_t* __restrict__ R,
-                       float* __restrict__ out, int M, int D, int NE) {
-  __shared__ __align__(16) unsigned char lds[2][(RW_M + RW_N) * RW_ROW];
-  constexpr int PIECES = (RW_M + RW_N) * 8 / 256;
+// Many tiles: eight waves on 64 rows x 128 experts, both operands through LDS (whole 128-byte lines from memory, 64 inputs a
+// step), a wave on 32 x 32 walking the slices itself.  A step is a chain of LDS trips (the same inputs again and again from
+// the cache take as long), so it has as few as it can: both chunks' operands are read together, no condition between them, the
+// next step's go to the other stage under the matrix instructions, and two workgroups fit a compute unit.  Up to 16 experts past the last 128
+// (a shared expert's gate) are taken by workgroups of their own in router_kernel's way, 64 x 16.
+// 4,096 rows x 512 experts x 2048 28.6 us with four waves of 32 x 64, 21.2; x 513 30.4, 23.7.
+constexpr int RW_M = 64, RW_N = 128, RW_MORE = 16, RW_STEP = 64, RW_ROW = RW_STEP * 2 + 16;      // bytes of an LDS row, padded
+constexpr int RW_THREADS = 512, RW_SETS = 2, RW_LDS = 2 * (RW_M + RW_N) * RW_ROW;
+static_assert(RW_THREADS == 64 * ROUTER_SLICES && sizeof(RouterParts<RW_M / 16, 1>) <= RW_LDS, "the narrow tile's workgroup");
+
+__device__ __forceinline__ void router_wide_tile(const uint16_t* __restrict__ X, int64_t ldx, const uint16_t* __restrict__ R,
+                                                 float* __restrict__ out, int M, int D, int NE, unsigned char* lds) {
+  constexpr int PIECES = (RW_M + RW_N) * 8 / RW_THREADS;
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, kq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int m0 = blockIdx.x * RW_M, e0 = blockIdx.y * RW_N, wm = 32 * (wave & 1), we = 64 * (wave >> 1);
-  const int rn = min(4, (NE - e0 - we + 15) >> 4);          // column tiles this wave has
+  const int m0 = blockIdx.x * RW_M, e0 = blockIdx.y * RW_N, wm = 32 * (wave & 1), we = 32 * (wave >> 1);
+  // this thread's 16-byte pieces of the step's rows
   const uint16_t* src[PIECES];
+  int at[PIECES];
 #pragma unroll
   for (int j = 0; j < PIECES; ++j) {
-    const int row = (tid >> 3) + 32 * j, ch = tid & 7;
+    const int row = (tid >> 3) + 64 * j, ch = tid & 7;
     src[j] = (row < RW_M ? X + (size_t)min(m0 + row, M - 1) * ldx : R + (size_t)min(e0 + row - RW_M, NE - 1) * D) + ch * 8;
+    at[j] = row * RW_ROW + ch * 16;
   }
   const int chunks = D / 32, steps = (chunks + 1) / 2;
-  u32x4_t v0[PIECES], v1[PIECES];
-  // (D in whole chunks of 32: the last step's second half may lie past the row and is then not read)
-  auto load = [&](u32x4_t (&w)[PIECES], int step) {
-    const int k0 = RW_STEP * min(step, steps - 1) + ((tid & 7) * 8 + RW_STEP * min(step, steps - 1) < D ? 0 : -32);
+  u32x4_t v[RW_SETS][PIECES];
+  // (D in whole chunks of 32: the last step's second half may lie past the row; it is then the first again, and counts as zeros)
+  auto load = [&](u32x4_t (&w)[PIECES], int step) __attribute__((always_inline)) {
+    const int k0 = min(RW_STEP * step, D - 8 - (tid & 7) * 8);
 #pragma unroll
     for (int j = 0; j < PIECES; ++j) w[j] = *reinterpret_cast<const u32x4_t*>(src[j] + k0);
   };
-  auto store = [&](int u, const u32x4_t (&w)[PIECES]) {
+  auto store = [&](int step, int u, u32x4_t (&w)[PIECES]) __attribute__((always_inline)) {
+    const bool past = RW_STEP * step + (tid & 7) * 8 >= D;
 #pragma unroll
-    for (int j = 0; j < PIECES; ++j)
-      *reinterpret_cast<u32x4_t*>(&lds[u][((tid >> 3) + 32 * j) * RW_ROW + (tid & 7) * 16]) = w[j];
+    for (int j = 0; j < PIECES; ++j) {
+      if (past) w[j] = (u32x4_t){0u, 0u, 0u, 0u};
+      *reinterpret_cast<u32x4_t*>(lds + u * (RW_LDS / 2) + at[j]) = w[j];
+    }
   };
-  f32x4_t acc[2][4], sum[2][4];
+  f32x4_t acc[2][2], sum[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = sum[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < 2; ++j) acc[i][j] = sum[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  auto join = [](f32x4_t& total, f32x4_t& part) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) total[q] = __fadd_rn(total[q], part[q]);
+    part = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  };
   int slice = 0, end = router_chunk(1, chunks);
   while (end == 0) end = router_chunk(++slice + 1, chunks);
-  // one step from stage u: the next step's operands (in `next`) go to the other stage, those after it into `mine`
-  auto walk = [&](int u, int step, u32x4_t (&mine)[PIECES], const u32x4_t (&next)[PIECES]) __attribute__((always_inline)) {
-    load(mine, step + 2);
+  // one step from stage U & 1: set U takes the operands of four steps on, set U + 1 goes to the other stage
+  auto walk = [&](int step, auto U) __attribute__((always_inline)) {
+    constexpr int u = decltype(U)::value;
+    load(v[u], step + RW_SETS);
+    // both chunks' operands first, and no condition on the way: a branch between two reads would put a second trip to LDS
+    // into every step
+    auto operand = [&](int row, int h) {
+      return *reinterpret_cast<const bf16x8_t*>(lds + (u & 1) * (RW_LDS / 2) + row * RW_ROW + h * 64 + kq * 16);
+    };
+    bf16x8_t a[2][2], b[2][2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int c = 2 * step + h;
-      if (c >= chunks) break;
-      bf16x8_t a[2];
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
-        a[i] = *reinterpret_cast<const bf16x8_t*>(&lds[u][(wm + 16 * i + r) * RW_ROW + h * 64 + kq * 16]);
+      for (int i = 0; i < 2; ++i) {
+        a[h][i] = operand(wm + 16 * i + r, h);
+        b[h][i] = operand(RW_M + we + 16 * i + r, h);
+      }
+    }
+    // the other stage was last read before the barrier: its writes land under the matrix instructions
+    store(step + 1, 1 - (u & 1), v[(u + 1) % RW_SETS]);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (j < rn) {
-          const bf16x8_t b = *reinterpret_cast<const bf16x8_t*>(&lds[u][(RW_M + we + 16 * j + r) * RW_ROW + h * 64 + kq * 16]);
+    for (int h = 0; h < 2; ++h) {
 #pragma unroll
-          for (int i = 0; i < 2; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b, acc[i][j], 0, 0, 0);
-        }
-      if (c + 1 != end) continue;
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h][i], b[h][j], acc[i][j], 0, 0, 0);
+      if (2 * step + h + 1 != end) continue;
       // the slice that ends here joins the sum (slices without a chunk add nothing)
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) sum[i][j][q] = __fadd_rn(sum[i][j][q], acc[i][j][q]);
-          acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-        }
+        for (int j = 0; j < 2; ++j) join(sum[i][j], acc[i][j]);
       do end = router_chunk(++slice + 1, chunks);
       while (slice + 1 < ROUTER_SLICES && end == router_chunk(slice, chunks));
     }
-    store(1 - u, next);
     __syncthreads();
   };
-  load(v0, 0);
-  load(v1, 1);
-  store(0, v0);
+#pragma unroll
+  for (int u = 0; u < RW_SETS; ++u) load(v[u], u);
+  store(0, 0, v[0]);
   __syncthreads();
-  for (int step = 0; step < steps; step += 2) {
-    walk(0, step, v0, v1);
-    if (step + 1 < steps) walk(1, step + 1, v1, v0);
+  int step = 0;
+  static_assert(RW_SETS == 2, "the steps below");
+  for (; step + 1 < steps; step += 2) {
+    walk(step, std::integral_constant<int, 0>());
+    walk(step + 1, std::integral_constant<int, 1>());
   }
+  if (step < steps) walk(step, std::integral_constant<int, 0>());
+  auto put = [&](int row0, int col, const f32x4_t& s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (row0 + 4 * kq + q < M && col < NE) out[(size_t)(row0 + 4 * kq + q) * NE + col] = s[q];
+  };
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int row = m0 + wm + 16 * i + 4 * kq + q, col = e0 + we + 16 * j + r;
-        if (j < rn && row < M && col < NE) out[(size_t)row * NE + col] = sum[i][j][q];
-      }
+    for (int j = 0; j < 2; ++j)
+      put(m0 + wm + 16 * i, e0 + we + 16 * j + r, sum[i][j]);
+}
+
+__global__ void __launch_bounds__(RW_THREADS, 4)
+    router_wide_kernel(const uint16_t* __restrict__ X, int64_t ldx, const uint16_t* __restrict__ R,
+                       float* __restrict__ out, int M, int D, int NE) {
+  __shared__ __align__(16) unsigned char lds[RW_LDS];
+  if (NE - (int)blockIdx.y * RW_N > RW_MORE) router_wide_tile(X, ldx, R, out, M, D, NE, lds);
+  else router_tile<RW_M / 16, 1, 4>(X, ldx, R, out, M, D, NE, blockIdx.x * RW_M, blockIdx.y * RW_N,
+                                    *reinterpret_cast<RouterParts<RW_M / 16, 1>*>(lds));
 }
 
 __global__ void __launch_bounds__(64)
@@ -412,6 +451,52 @@ __global__ void __launch_bounds__(256)
   *reinterpret_cast<uint32_t*>(out + (size_t)r * D + d) = pack_bf16(a0, a1);
 }
 
+// 16-bit pair outputs, eight columns a thread (16-byte loads), rows side by side in a workgroup: 4,096 rows x 11 x 2048 36.2 us
+// with two columns a thread, 35.1 so (5.3 TB/s); 2,000 x 9 x 1024 11.2, 7.5; 777 x 8 x 2688 7.5, 5.9
+template <int YKIND>
+__global__ void __launch_bounds__(256)
+    combine8_kernel(const uint16_t* __restrict__ Y, const float* __restrict__ Wt, uint16_t* __restrict__ out, int rows, int S,
+                    int D8) {
+  const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
+  const long long r = t / D8;
+  if (r >= rows) return;
+  const int D = D8 * 8, d = (int)(t - r * D8) * 8;
+  const uint16_t* y = Y + (size_t)r * S * D + d;
+  float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < S; k0 += 8) {
+    float w[8];
+    u32x4_t v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int k = k0 + j < S ? k0 + j : S - 1;
+      w[j] = Wt[(size_t)r * S + k];
+      v[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(y + (size_t)k * D));
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (k0 + j < S) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float lo, hi;
+          if (YKIND == 1) {
+            lo = bf16_lo(v[j][i]);
+            hi = bf16_hi(v[j][i]);
+          } else {
+            typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+            const uint32_t u = v[j][i];
+            const half2_t h = __builtin_bit_cast(half2_t, u);
+            lo = (float)h[0];
+            hi = (float)h[1];
+          }
+          a[2 * i] = fmaf(w[j], lo, a[2 * i]);
+          a[2 * i + 1] = fmaf(w[j], hi, a[2 * i + 1]);
+        }
+      }
+  }
+  *reinterpret_cast<uint4*>(out + (size_t)r * D + d) =
+      make_uint4(pack_bf16(a[0], a[1]), pack_bf16(a[2], a[3]), pack_bf16(a[4], a[5]), pack_bf16(a[6], a[7]));
+}
+
 // fp32 pair outputs, four columns a thread (16-byte loads): the wide prompt chunks, where the combine is a 370 MB read
 __global__ void __launch_bounds__(256)
     combine4_kernel(const float* __restrict__ Y, const float* __restrict__ Wt, uint16_t* __restrict__ out, int S, int D) {
@@ -457,12 +542,14 @@ extern "C" int tf_moe_router(const uint16_t* x, int64_t ldx, const uint16_t* row
   // to itself and larger ones (operands read fewer times over) once they do not: 392 tiles x 2688 18.3 us as 16 x 16,
   // 13.3 as 32 x 32 (128 tiles 7.4 / 13).  Between the two, 32 x 16 while each has a unit to itself, all of a slice in
   // flight up to 3,072 inputs: 777 rows x 128 x 2688 11.3 us as 32 x 32 (100 units of the 256 at work), 9.6 so; 250 x 512 x 4096
-  // 16.8, 13.2; 8,000 x 16 x 512 3.6, 3.5; 1,617 x 2048 14.2 us as 32 x 64, 47 as one wave's 32 x 64; 8,448 x 2048
-  // 30.5 us wide.  The wide kernel takes what would be more than one round of 32 x 64, two workgroups a unit: below that its
-  // own 64 x 128 leave units idle (4,096 rows x 129 x 512 11.8 us on 128 workgroups, 8.6 as 32 x 64; x 2048 28.3, 21.3).
+  // 16.8, 13.2; 8,000 x 16 x 512 3.6, 3.5; 1,617 x 2048 14.2 us as 32 x 64, 47 as one wave's 32 x 64.  32 x 64 while each
+  // has a unit to itself (4,096 x 128 x 3072 19.3 us, wide 28.1); past that the wide kernel, whose workgroups take 20 us of 2048
+  // inputs however few they are (1,500 x 400 x 2048 26.2, 20.3; 2,000 x 512 x 4096 47.9, 36.4), but for a short D, which two rounds of the
+  // shorter tiles walk sooner (1,055 x 512 x 288 5.0, 6.5), and where most of the last 64 columns is padding, which costs them little
+  // (3,000 x 129 x 1024 9.9, 12.3; 4,100 x 72 x 2048 16.7, 20.1).
   // With up to 32 experts a column tile of 64 or 128 would be mostly padding: 32,768 rows x 8 x 2048 36 us as 32 x 64,
   // 24.7 as 64 x 16 (one wave a tile, the single chain: 27); 16,384 x 32 x 1024 13.1 as 32 x 64, 10.7 as 32 x 32.
-  const int64_t tiles = (int64_t)((m + 15) / 16) * ((ne + 15) / 16);
+  const int64_t tiles = (int64_t)((m + 15) / 16) * ((ne + 15) / 16), narrow = (int64_t)((m + 31) / 32) * ((ne + 63) / 64);
   if (tiles <= 256) {
     const dim3 grid((m + 15) / 16, (ne + 15) / 16);
     if (d <= 32 * 8 * ROUTER_SLICES) router_kernel<1, 1, 8><<<grid, 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
@@ -475,10 +562,10 @@ extern "C" int tf_moe_router(const uint16_t* x, int64_t ldx, const uint16_t* row
     router_kernel<4, 1, 4><<<dim3((m + 63) / 64), 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
   } else if (tiles <= 1024 || ne <= 32) {
     router_kernel<2, 2, 4><<<dim3((m + 31) / 32, (ne + 31) / 32), 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
-  } else if ((int64_t)((m + 31) / 32) * ((ne + 63) / 64) <= ROUTER_ROUND) {
+  } else if (narrow <= 256 || (narrow <= 512 && (int64_t)((m + 31) / 32) * ((ne + 15) / 16) <= 4 * (d < 512 ? 512 : 240))) {
     router_kernel<2, 4, 4><<<dim3((m + 31) / 32, (ne + 63) / 64), 64 * ROUTER_SLICES, 0, s>>>(x, ldx, rows, logits, m, d, ne);
   } else {
-    router_wide_kernel<<<dim3((m + 63) / 64, (ne + 127) / 128), 256, 0, s>>>(x, ldx, rows, logits, m, d, ne);
+    router_wide_kernel<<<dim3((m + RW_M - 1) / RW_M, (ne + RW_N - 1) / RW_N), RW_THREADS, 0, s>>>(x, ldx, rows, logits, m, d, ne);
   }
   TF_LAUNCH_OK("tf_moe_router");
   return 0;
@@ -554,6 +641,14 @@ extern "C" int tf_moe_combine(const void* y, int y_bf16, const float* wts, uint1
   if (!y_bf16 && d % 4 == 0 && aligned16(y) && rows >= 64) {
     combine4_kernel<<<dim3(rows, (d / 4 + 255) / 256), 256, 0, as_stream(stream)>>>(
         static_cast<const float*>(y), wts, out, slots, d);
+    TF_LAUNCH_OK("tf_moe_combine");
+    return 0;
+  }
+  // (a few rows have too few workgroups of eight columns a thread: 100 x 7 x 512 2.8 us, 3.1 so)
+  const int64_t wide = ((int64_t)rows * (d / 8) + 255) / 256;
+  if (y_bf16 && d % 8 == 0 && aligned16(y) && aligned16(out) && wide >= 128 && wide <= 0x7FFFFFFF) {
+    if (y_bf16 == 1) combine8_kernel<1><<<(unsigned)wide, 256, 0, as_stream(stream)>>>(static_cast<const uint16_t*>(y), wts, out, rows, slots, d / 8);
+    else combine8_kernel<2><<<(unsigned)wide, 256, 0, as_stream(stream)>>>(static_cast<const uint16_t*>(y), wts, out, rows, slots, d / 8);
     TF_LAUNCH_OK("tf_moe_combine");
     return 0;
   }
