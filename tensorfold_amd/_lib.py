@@ -125,13 +125,74 @@ def stream() -> int:
         return torch.cuda.current_stream().cuda_stream
 
 
-def call(name: str, *args) -> None:
-    """Run entry point ``name`` on the current stream; a non-zero status raises with the library's sentence."""
+_native: dict | None = None          # entry point -> its Python function of csrc/call.cpp; empty where that is not built
 
+
+def _bound() -> dict:
+    """The functions of ``tfmi_call.so``, bound to the library that ``lib`` has loaded."""
+
+    from importlib.machinery import ExtensionFileLoader
+    from importlib.util import module_from_spec, spec_from_loader
+
+    path = build.call_lib()
+    if path is None:
+        return {}
+    loader = ExtensionFileLoader("tfmi_call", str(path))
+    module = module_from_spec(spec_from_loader("tfmi_call", loader))
+    loader.exec_module(module)
+    module.bind(str(build.LIB))
+    return {name: getattr(module, name) for name in (*PROTOTYPES, "empties", *WHOLE) if hasattr(module, name)}
+
+
+def _start() -> dict:
+    global _native
     _ready()
-    so = _other or lib()
+    _native = _bound()
+    return _native
+
+
+def empties(x: torch.Tensor, sizes: list[tuple[int, int, bool]]) -> list[torch.Tensor]:
+    """Uninitialised tensors [rows, columns] on x's device, of its type or fp32, one for each (rows, columns, fp32?)."""
+
+    make = (_native if _native is not None else _start()).get("empties")
+    if make is not None:
+        return make(x, sizes)
+    return [x.new_empty((r, c), dtype=torch.float32) if wide else x.new_empty((r, c)) for r, c, wide in sizes]
+
+
+# calls that csrc/call.cpp makes as a whole where every argument is the ordinary one
+WHOLE = ("matmul", "matmul_group", "prefill_matmul", "add_rmsnorm")
+
+
+def whole(name: str, *args):
+    """What ``name`` of ``WHOLE`` returns, launch and all, or None: some argument wants the general way."""
+
+    if _native is None:
+        if not (isinstance(args[0], torch.Tensor) and args[0].is_cuda):
+            return None
+        _start()
+    make = _native.get(name)
+    return None if make is None or _other is not None else make(*args, stream())
+
+
+def call(name: str, *args) -> None:
+    """Run entry point ``name`` on the current stream; a non-zero status raises with the library's sentence.  A pointer
+    is a tensor, an address or None; where the entry point takes a table (of pointers, strides or counts) a list."""
+
+    entry = (_native if _native is not None else _start()).get(name)
+    if entry is not None and _other is None:
+        entry(*args, stream())
+        return
+    so, kinds = _other or lib(), TABLES.get(name, {})
+    plain = lambda a: a.data_ptr() if isinstance(a, torch.Tensor) else a
+    args = [(kinds[i] * len(a))(*map(plain, a)) if i in kinds and isinstance(a, list) else plain(a) for i, a in enumerate(args)]
     if getattr(so, name)(*args, stream()):
         raise RuntimeError(so.tf_last_error().decode())
+
+
+# the element types of an entry point's tables, by argument, for the ctypes path
+TABLES = {"tf_qmm_group": {4: c_void_p, 5: c_void_p, 6: c_void_p, 7: c_int64, 8: c_void_p, 9: c_void_p, 10: c_void_p,
+                           11: c_int, 12: c_int, 13: c_int}}
 
 
 def on_gpu(*tensors: torch.Tensor) -> None:

@@ -20,6 +20,7 @@ CSRC = HERE / "csrc"
 LIB = HERE / "libtfmi.so"
 TIMELINE_LIB = HERE / "libtfmi_timeline.so"      # the same kernels with per-workgroup timestamps (see compile)
 SOURCES = ("api.hip", "pack.hip", "decode.hip", "fused.hip", "route.hip", "norm.hip", "prefill.hip", "prefill8.hip", "exl3.hip", "exl3_experts.hip")
+CALL_LIB = HERE / "tfmi_call.so"                 # the entry points as Python functions (csrc/call.cpp); host code alone
 # packed-fp32 VALU forms are switched off for the device pass (the host pass warns that it does not know the feature)
 FLAGS = ("-O3", "-std=c++17", "-fPIC", "-shared", f"--offload-arch={ARCH}",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops")
@@ -45,12 +46,25 @@ def source_id() -> str:
     return h.hexdigest()[:16]
 
 
-def built_id(path: Path = LIB) -> str | None:
+def call_id() -> str:
+    """16 hex digits over what ``tfmi_call.so`` is built from and for."""
+
+    import hashlib
+
+    import torch
+
+    h = hashlib.sha256(f"{sys.version} {torch.__version__}".encode())
+    for path in (CSRC / "call.cpp", HERE.parent / "include" / "tfmi.h"):
+        h.update(path.read_bytes())
+    return h.hexdigest()[:16]
+
+
+def built_id(path: Path = LIB, mark: bytes = b"TFMI_BUILD_ID=") -> str | None:
     """The digest a library file carries (``tf_build_id``), read from the file without loading it."""
 
     if not path.exists():
         return None
-    blob, mark = path.read_bytes(), b"TFMI_BUILD_ID="
+    blob = path.read_bytes()
     at = blob.find(mark)
     return None if at < 0 else blob[at + len(mark):at + len(mark) + 16].decode(errors="replace")
 
@@ -111,7 +125,38 @@ def compile(verbose: bool = False, timeline: bool = False) -> Path:
         for text in logs:
             if text:
                 say(text)
+    if not timeline and compile_call() is None:
+        say("no C++ compiler, Python headers or torch headers: launches go through ctypes")
     return target
+
+
+def compile_call() -> Path | None:
+    """``tfmi_call.so`` with the host's C++ compiler; None where that, Python's headers or torch's are missing."""
+
+    import sysconfig
+
+    import torch
+
+    cc, python, root = shutil.which("g++") or shutil.which("c++"), Path(sysconfig.get_paths()["include"]), Path(torch.__file__).parent
+    if cc is None or not (python / "Python.h").exists() or not (root / "include/torch/csrc/autograd/python_variable.h").exists():
+        return None
+    done = subprocess.run([cc, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", f"-I{python}",
+                           f"-I{root / 'include'}", f"-I{root / 'include/torch/csrc/api/include'}",
+                           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DTF_CALL_ID="{call_id()}"',
+                           str(CSRC / "call.cpp"), "-o", str(CALL_LIB), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu",
+                           "-lc10", "-ldl"], capture_output=True, text=True)
+    if done.returncode:
+        raise RuntimeError(f"tensorfold-amd: {cc} failed:\n{done.stderr}")
+    return CALL_LIB
+
+
+def call_lib() -> Path | None:
+    """``tfmi_call.so`` for the sources beside it, built first if it is missing or out of date; None where it cannot be
+    (``_lib.call`` then goes through ctypes: the same launches, a few microseconds later)."""
+
+    if not (CSRC / "call.cpp").exists():
+        return CALL_LIB if CALL_LIB.exists() else None
+    return CALL_LIB if built_id(CALL_LIB, b"TFMI_CALL_ID=") == call_id() else compile_call()
 
 
 @lru_cache(maxsize=1)

@@ -227,36 +227,36 @@ def routed(x: torch.Tensor, pick: torch.Tensor, wts: torch.Tensor | None, ex: Ex
     _lib.on_gpu(x, pick, wts)
     plan = s.plan
     items = grouped.max_items(p, n_exp, grouped.TILE)
-    plan_args = (_lib.ptr(plan.items), _lib.ptr(plan.counts), _lib.ptr(plan.members))
-    rot_args = (_lib.ptr(x), _DTYPES[x.dtype], x.stride(0), _lib.ptr(pick), _lib.ptr(ex.suh[GATE]), _lib.ptr(ex.suh[UP]),
-                _lib.ptr(s.xg), _lib.ptr(s.xu), R, slots, d, n_exp)
+    plan_args = (plan.items, plan.counts, plan.members)
+    rot_args = (x, _DTYPES[x.dtype], x.stride(0), pick, ex.suh[GATE], ex.suh[UP],
+                s.xg, s.xu, R, slots, d, n_exp)
     if group and p <= grouped.SMALL:
         # one launch for the pair sort (it drops ids outside [0, E)) and the rotation: neither needs the other
         plan.tile = grouped.TILE
-        _lib.call("tf_exl3x_plan_rot_in", *rot_args, grouped.TILE, _lib.ptr(plan.members), _lib.ptr(plan.items),
-                  _lib.ptr(plan.counts))
+        _lib.call("tf_exl3x_plan_rot_in", *rot_args, grouped.TILE, plan.members, plan.items,
+                  plan.counts)
     else:
         if group:
             grouped.route(pick, plan)
         _lib.call("tf_exl3x_rot_in", *rot_args)
-    _lib.call("tf_exl3x_grouped", _lib.ptr(s.xg), _lib.ptr(s.xu), _lib.ptr(ex.ptr[GATE]), _lib.ptr(ex.ptr[UP]),
-              _lib.ptr(ex.k2[GATE]), _lib.ptr(ex.k2[UP]), *plan_args, _lib.ptr(s.z), 2, d, width, p, s.sk_gu, ex.cb,
+    _lib.call("tf_exl3x_grouped", s.xg, s.xu, ex.ptr[GATE], ex.ptr[UP],
+              ex.k2[GATE], ex.k2[UP], *plan_args, s.z, 2, d, width, p, s.sk_gu, ex.cb,
               n_exp, items)
-    _lib.call("tf_exl3x_gateup_epilogue", _lib.ptr(s.z), _lib.ptr(pick), _lib.ptr(ex.svh[GATE]), _lib.ptr(ex.svh[UP]),
-              _lib.ptr(ex.suh[DOWN]), _lib.ptr(s.xd), p, width, s.sk_gu, n_exp,
+    _lib.call("tf_exl3x_gateup_epilogue", s.z, pick, ex.svh[GATE], ex.svh[UP],
+              ex.suh[DOWN], s.xd, p, width, s.sk_gu, n_exp,
               float(min(limit, 3.0e38)), act_mode)
-    _lib.call("tf_exl3x_grouped", _lib.ptr(s.xd), None, _lib.ptr(ex.ptr[DOWN]), None, _lib.ptr(ex.k2[DOWN]), None,
-              *plan_args, _lib.ptr(s.z), 1, width, d, p, s.sk_d, ex.cb, n_exp, items)
+    _lib.call("tf_exl3x_grouped", s.xd, None, ex.ptr[DOWN], None, ex.k2[DOWN], None,
+              *plan_args, s.z, 1, width, d, p, s.sk_d, ex.cb, n_exp, items)
     if wts is None:
-        _lib.call("tf_exl3x_down_combine", _lib.ptr(s.z), _lib.ptr(pick), _lib.ptr(ex.svh[DOWN]), _lib.ptr(s.y), None, None,
+        _lib.call("tf_exl3x_down_combine", s.z, pick, ex.svh[DOWN], s.y, None, None,
                   R, slots, d, s.sk_d, n_exp)
         return s.y[:p]
     if out is None:
         out = torch.empty((R, d), dtype=torch.float32, device=x.device)
     elif out.dtype != torch.float32 or tuple(out.shape) != (R, d) or not out.is_contiguous():
         raise ValueError(f"out must be a contiguous fp32 [{R}, {d}]")
-    _lib.call("tf_exl3x_down_combine", _lib.ptr(s.z), _lib.ptr(pick), _lib.ptr(ex.svh[DOWN]), _lib.ptr(s.y), _lib.ptr(wts),
-              _lib.ptr(out), R, slots, d, s.sk_d, n_exp)
+    _lib.call("tf_exl3x_down_combine", s.z, pick, ex.svh[DOWN], s.y, wts,
+              out, R, slots, d, s.sk_d, n_exp)
     return out
 
 
@@ -271,5 +271,5 @@ def dequant(trellis: torch.Tensor, codebook: int | str) -> torch.Tensor:
     words = trellis.contiguous().view(torch.int32)
     out = torch.empty((k, n), dtype=torch.float16, device=trellis.device)
     tile = 4 * k2
-    _lib.call("tf_exl3_unpack", _lib.ptr(words), _lib.ptr(out), k, n, (n // 16) * tile, 8 * tile, k2, cb)
+    _lib.call("tf_exl3_unpack", words, out, k, n, (n // 16) * tile, 8 * tile, k2, cb)
     return out

@@ -92,7 +92,7 @@ def _decode(words: torch.Tensor, k: int, n: int, strides: tuple[int, int], k2: i
 
     if out is None:
         out = words.new_empty((k, n), dtype=torch.float16)
-    _lib.call("tf_exl3_unpack", _lib.ptr(words), _lib.ptr(out), k, n, *strides, k2, CODEBOOK_IDS[codebook])
+    _lib.call("tf_exl3_unpack", words, out, k, n, *strides, k2, CODEBOOK_IDS[codebook])
     return out
 
 
@@ -188,10 +188,10 @@ class Exl3Linear:
                          or z.device != x.device):
             raise ValueError(f"z must hold {sk} x {m} x {self.n} fp32 values on x's device")
         stride_k, stride_nb = self.strides
-        _lib.call("tf_exl3_rot_in", _lib.ptr(x), _DTYPES[x.dtype], _lib.ptr(self.suh), _lib.ptr(xh), m, self.k)
-        _lib.call("tf_exl3_linear", _lib.ptr(xh), _lib.ptr(self.words), stride_k, stride_nb, _lib.ptr(self.svh),
-                  _lib.ptr(self.bias), _lib.ptr(out), _DTYPES[out.dtype], _lib.ptr(z) if sk > 1 else None,
-                  _lib.ptr(self.counters), m, self.k, self.n, self.k2, CODEBOOK_IDS[self.codebook], sk, wk)
+        _lib.call("tf_exl3_rot_in", x, _DTYPES[x.dtype], self.suh, xh, m, self.k)
+        _lib.call("tf_exl3_linear", xh, self.words, stride_k, stride_nb, self.svh,
+                  self.bias, out, _DTYPES[out.dtype], z if sk > 1 else None,
+                  self.counters, m, self.k, self.n, self.k2, CODEBOOK_IDS[self.codebook], sk, wk)
         return out
 
     def unpack(self, out: torch.Tensor | None = None) -> torch.Tensor:
@@ -272,11 +272,11 @@ class Exl3Stack:
                          or z.device != x.device):
             raise ValueError(f"z must hold {count} x {sk} x {m} x {self.n} fp32 values on x's device")
         stride_k, stride_nb = self.layer(0).strides
-        _lib.call("tf_exl3_rot_in_stacked", _lib.ptr(x), _DTYPES[x.dtype], _lib.ptr(self.suh), _lib.ptr(xh), count, m,
+        _lib.call("tf_exl3_rot_in_stacked", x, _DTYPES[x.dtype], self.suh, xh, count, m,
                   self.k)
-        _lib.call("tf_exl3_linear_stacked", _lib.ptr(xh), _lib.ptr(self.words), stride_k, stride_nb,
-                  self.words.stride(0), _lib.ptr(self.svh), _lib.ptr(self.bias), _lib.ptr(out), _DTYPES[out.dtype],
-                  _lib.ptr(z) if sk > 1 else None, _lib.ptr(self.counters), count, m, self.k, self.n, k2_of(self.bits),
+        _lib.call("tf_exl3_linear_stacked", xh, self.words, stride_k, stride_nb,
+                  self.words.stride(0), self.svh, self.bias, out, _DTYPES[out.dtype],
+                  z if sk > 1 else None, self.counters, count, m, self.k, self.n, k2_of(self.bits),
                   CODEBOOK_IDS[self.codebook], sk, wk)
         return out
 
@@ -334,15 +334,15 @@ class Exl3MLP:
             raise ValueError(f"mid must be contiguous (2, {m}, {g.n}) {mid_dtype} on x's device")
         (sk, wk), (dsk, dwk) = g.split, d.split
         stride_k, stride_nb = g.layer(0).strides
-        _lib.call("tf_exl3_rot_in_stacked", _lib.ptr(x), _DTYPES[x.dtype], _lib.ptr(g.suh), _lib.ptr(s["xh"]), 2, m, g.k)
-        _lib.call("tf_exl3_gate_up", _lib.ptr(s["xh"]), _lib.ptr(g.words), stride_k, stride_nb, g.words.stride(0),
-                  _lib.ptr(g.svh), _lib.ptr(g.bias), _lib.ptr(mid), _DTYPES[mid_dtype], _lib.ptr(s["z"]),
-                  _lib.ptr(g.counters), _lib.ptr(d.suh), _lib.ptr(s["hh"]), m, g.k, g.n, k2_of(g.bits),
+        _lib.call("tf_exl3_rot_in_stacked", x, _DTYPES[x.dtype], g.suh, s["xh"], 2, m, g.k)
+        _lib.call("tf_exl3_gate_up", s["xh"], g.words, stride_k, stride_nb, g.words.stride(0),
+                  g.svh, g.bias, mid, _DTYPES[mid_dtype], s["z"],
+                  g.counters, d.suh, s["hh"], m, g.k, g.n, k2_of(g.bits),
                   CODEBOOK_IDS[g.codebook], sk, wk)
         stride_k, stride_nb = d.strides
-        _lib.call("tf_exl3_linear", _lib.ptr(s["hh"]), _lib.ptr(d.words), stride_k, stride_nb, _lib.ptr(d.svh),
-                  _lib.ptr(d.bias), _lib.ptr(out), _DTYPES[out.dtype], _lib.ptr(s["z"]) if dsk > 1 else None,
-                  _lib.ptr(d.counters), m, d.k, d.n, d.k2, CODEBOOK_IDS[d.codebook], dsk, dwk)
+        _lib.call("tf_exl3_linear", s["hh"], d.words, stride_k, stride_nb, d.svh,
+                  d.bias, out, _DTYPES[out.dtype], s["z"] if dsk > 1 else None,
+                  d.counters, m, d.k, d.n, d.k2, CODEBOOK_IDS[d.codebook], dsk, dwk)
         return out
 
 
@@ -360,7 +360,7 @@ def swiglu_rot_in(y: torch.Tensor, suh: torch.Tensor, xh: torch.Tensor | None = 
         xh = torch.empty((m, n), dtype=torch.float16, device=y.device)
     elif xh.dtype != torch.float16 or tuple(xh.shape) != (m, n) or not xh.is_contiguous() or xh.device != y.device:
         raise ValueError(f"xh must be a contiguous fp16 ({m}, {n}) on y's device")
-    _lib.call("tf_exl3_swiglu_rot_in", _lib.ptr(y), _DTYPES[y.dtype], _lib.ptr(suh), _lib.ptr(xh), m, n)
+    _lib.call("tf_exl3_swiglu_rot_in", y, _DTYPES[y.dtype], suh, xh, m, n)
     return xh
 
 

@@ -46,7 +46,7 @@ def decode(layer: Exl3Linear, ws: Workspace) -> torch.Tensor:
 
     k, n = layer.k, layer.n
     w8 = ws._grow("w", k * n, layer.words.device)[:k * n].view(k // 8, n, 8)
-    _lib.call("tf_exl3_unpack_k8", _lib.ptr(layer.words), _lib.ptr(w8), k, n, *layer.strides, layer.k2,
+    _lib.call("tf_exl3_unpack_k8", layer.words, w8, k, n, *layer.strides, layer.k2,
               CODEBOOK_IDS[layer.codebook])
     return w8
 
@@ -73,11 +73,11 @@ def matmul(layer: Exl3Linear, x: torch.Tensor, out: torch.Tensor, ws: Workspace,
     _lib.on_gpu(x, out)
     x = x.contiguous()
     xh = ws._grow("xh", m * k, x.device)[:m * k].view(m, k)
-    _lib.call("tf_exl3_rot_in", _lib.ptr(x), _DTYPES[x.dtype], _lib.ptr(layer.suh), _lib.ptr(xh), m, k)
+    _lib.call("tf_exl3_rot_in", x, _DTYPES[x.dtype], layer.suh, xh, m, k)
     if wt is None:
         wt = decode(layer, ws)
     elif wt.dtype != torch.float16 or tuple(wt.shape) != (k // 8, n, 8) or not wt.is_contiguous() or wt.device != x.device:
         raise ValueError(f"prefill matmul: wt must be the contiguous fp16 ({k // 8}, {n}, 8) that decode() returns")
-    _lib.call("tf_exl3_gemm", _lib.ptr(xh), _lib.ptr(wt), _lib.ptr(layer.svh), _lib.ptr(layer.bias), _lib.ptr(out),
+    _lib.call("tf_exl3_gemm", xh, wt, layer.svh, layer.bias, out,
               _DTYPES[out.dtype], out.stride(0), m, k, n)
     return out

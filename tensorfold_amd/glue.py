@@ -28,15 +28,14 @@ def add_rmsnorm(x: torch.Tensor, r: torch.Tensor | None, w: torch.Tensor, eps: f
     """h = x + r (bf16; x itself when r is None), y = rmsnorm(h) * w (bf16), xs = y's group sums (fp32).
     Returns (h, y, xs)."""
 
+    if r is not None and (made := _lib.whole("add_rmsnorm", x, r, w, eps, gs)) is not None:
+        return made
     rows, d = _check(x, w, gs)
     if r is not None and (r.dtype != torch.bfloat16 or r.shape != x.shape or not r.is_contiguous() or not r.is_cuda):
         raise ValueError("add_rmsnorm: r must be a contiguous bf16 GPU tensor of x's shape")
-    h = torch.empty_like(x) if r is not None else x
-    y = torch.empty_like(x)
-    xs = torch.empty((rows, d // gs), dtype=torch.float32, device=x.device)
-    _lib.call("tf_add_norm", _lib.ptr(x), _lib.ptr(r), 0 if r is None else 1, None, 0, 0, _lib.ptr(w), float(eps),
-              _lib.ptr(h) if r is not None else None, _lib.ptr(y), _lib.ptr(xs), rows, d, gs)
-    return h, y, xs
+    y, xs, *h = _lib.empties(x, [(rows, d, False), (rows, d // gs, True)] + [(rows, d, False)] * (r is not None))
+    _lib.call("tf_add_norm", x, r, 0 if r is None else 1, None, 0, 0, w, float(eps), h[0] if h else None, y, xs, rows, d, gs)
+    return h[0] if h else x, y, xs
 
 
 def add_moe_norm(h: torch.Tensor, y: torch.Tensor, wt: torch.Tensor, w: torch.Tensor, eps: float, top_k: int,
@@ -53,9 +52,7 @@ def add_moe_norm(h: torch.Tensor, y: torch.Tensor, wt: torch.Tensor, w: torch.Te
     if not 0 <= top_k <= slots:
         raise ValueError(f"add_moe_norm: top_k {top_k} outside 0..{slots}")
     _lib.on_gpu(y, wt)
-    hn = torch.empty_like(h)
-    out = torch.empty_like(h)
-    xs = torch.empty((rows, d // gs), dtype=torch.float32, device=h.device)
-    _lib.call("tf_add_norm", _lib.ptr(h), _lib.ptr(y), 3 if y.dtype == torch.bfloat16 else 2, _lib.ptr(wt), slots,
-              int(top_k), _lib.ptr(w), float(eps), _lib.ptr(hn), _lib.ptr(out), _lib.ptr(xs), rows, d, gs)
+    hn, out, xs = _lib.empties(h, [(rows, d, False), (rows, d, False), (rows, d // gs, True)])
+    _lib.call("tf_add_norm", h, y, 3 if y.dtype == torch.bfloat16 else 2, wt, slots, int(top_k), w, float(eps), hn, out, xs,
+              rows, d, gs)
     return hn, out, xs

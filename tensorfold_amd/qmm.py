@@ -8,7 +8,6 @@ do not depend on its neighbours.
 
 from __future__ import annotations
 
-import ctypes
 import dataclasses
 from functools import lru_cache
 
@@ -184,16 +183,18 @@ def matmul(x: torch.Tensor, q: Q4, xs: torch.Tensor | None = None, *, sk: int | 
     With ``reduce=False`` the fp32 K slices come back unadded as (sk, M, n); adding them in order and rounding once
     reproduces the reduced result bit for bit."""
 
+    sk = split_k(q.n, q.k, q.gs) if not sk else sk
+    if xs is None and out is None and part is None and reduce and (y := _lib.whole("matmul", x, q, sk, f32)) is not None:
+        return y
     x = _check_x(x, q, "matmul")
     m = int(x.shape[0])
-    sk = split_k(q.n, q.k, q.gs) if not sk else sk
     if out is None:
-        out = x.new_empty((m, q.n), dtype=torch.float32 if f32 else torch.bfloat16)
+        out, = _lib.empties(x, [(m, q.n, f32)])
     elif tuple(out.shape) != (m, q.n) or out.dtype != (torch.float32 if f32 else torch.bfloat16) \
             or not out.is_contiguous() or out.device != x.device:
         raise ValueError(f"matmul: out must be contiguous ({m}, {q.n}) {'fp32' if f32 else 'bf16'} on x's device")
     if sk > 1 and part is None:
-        part = x.new_empty((sk, m, q.n), dtype=torch.float32)
+        part, = _lib.empties(x, [(sk * m, q.n, True)])
     elif sk > 1 and (part.dtype != torch.float32 or part.numel() < sk * m * q.n or not part.is_contiguous()
                      or part.device != x.device):
         raise ValueError(f"matmul: part must hold {sk} x {m} x {q.n} fp32 values (split_k gives the slice count)")
@@ -202,9 +203,8 @@ def matmul(x: torch.Tensor, q: Q4, xs: torch.Tensor | None = None, *, sk: int | 
         raise ValueError(f"matmul: xs must be contiguous fp32 ({m}, {q.k // q.gs}), the group sums of x")
     counters = q.counters if reduce and sk > 1 and m <= 8 else None
     # without xs the launch takes the group sums itself
-    name, given = ("tf_qmm_own_sums", ()) if xs is None else ("tf_qmm", (_lib.ptr(xs),))
-    _lib.call(name, _lib.ptr(x), x.stride(0), *given, _lib.ptr(q.weight), _lib.ptr(q.scales),
-              _lib.ptr(q.biases), q.scales.stride(0), _lib.ptr(out), _lib.ptr(part), _lib.ptr(counters),
+    name, given = ("tf_qmm_own_sums", ()) if xs is None else ("tf_qmm", (xs,))
+    _lib.call(name, x, x.stride(0), *given, q.weight, q.scales, q.biases, q.scales.stride(0), out, part, counters,
               0 if counters is None else counters.numel() // COUNTER_STRIDE, m, q.n, q.k, sk, q.gs, bucket(m),
               int(f32), int(reduce))
     if reduce or sk == 1:
@@ -253,6 +253,10 @@ def matmul_group(x: torch.Tensor, qs: list[Q4], xs: torch.Tensor | None = None, 
     if not 1 <= n <= 4:
         raise ValueError("matmul_group: one to four weights")
     gs, k = qs[0].gs, qs[0].k
+    if xs is not None and not sks and outs is None and not parts:
+        ys = _lib.whole("matmul_group", x, xs, qs, [split_k(q.n, q.k, gs) for q in qs], f32)
+        if ys is not None:
+            return ys
     if x.dtype != torch.bfloat16 or x.dim() != 2:
         raise ValueError("matmul_group: x must be (M, K) bf16 with every weight's K")
     m, width = x.shape
@@ -274,7 +278,7 @@ def matmul_group(x: torch.Tensor, qs: list[Q4], xs: torch.Tensor | None = None, 
     dtype = torch.float32 if f32 else torch.bfloat16
     given = outs is not None
     if not given:
-        outs = [x.new_empty((m, q.n), dtype=dtype) for q in qs]
+        outs = _lib.empties(x, [(m, q.n, f32) for q in qs])
     parts = list(parts) if parts else [None] * n
     if len(sks) != n or len(outs) != n or len(parts) != n:
         raise ValueError("matmul_group: one slice count, output and part a weight")
@@ -294,25 +298,17 @@ def matmul_group(x: torch.Tensor, qs: list[Q4], xs: torch.Tensor | None = None, 
         else:
             part_at[i] = part.data_ptr()
     if own:
-        buffer = x.new_empty((own // 4,), dtype=torch.float32)
+        buffer, = _lib.empties(x, [(1, own // 4, True)])
         base = buffer.data_ptr()
         part_at = [at + base if part is None and at is not None else at for at, part in zip(part_at, parts)]
     if m > 8:
         counters = [None] * n
     else:
         counters = [c if sk > 1 else None for c, sk in zip(counters, sks)]
-    # The entry point's tables side by side in two arrays (addresses and strides, then counts) and one buffer for the
-    # parts: at a row the GPU needs 11 us for the norm and q, k and v (4096 + 1024 + 1024 columns) and the host bounds
-    # the pair of calls: 37 us, with nine arrays, a part a weight and a Stream object a launch; 26 so.
-    wide = (ctypes.c_int64 * (7 * n))(
-        *[q.weight.data_ptr() for q in qs], *[q.scales.data_ptr() for q in qs], *[q.biases.data_ptr() for q in qs],
-        *[q.scales.stride(0) for q in qs], *[out.data_ptr() for out in outs], *[at or 0 for at in part_at],
-        *[0 if c is None else c.data_ptr() for c in counters])
-    narrow = (ctypes.c_int * (3 * n))(*[0 if c is None else c.numel() // COUNTER_STRIDE for c in counters],
-                                      *[q.n for q in qs], *sks)
-    w, c = ctypes.addressof(wide), ctypes.addressof(narrow)
-    _lib.call("tf_qmm_group", x.data_ptr(), x.stride(0), xs.data_ptr(), n, w, w + 8 * n, w + 16 * n, w + 24 * n,
-              w + 32 * n, w + 40 * n, w + 48 * n, c, c + 4 * n, c + 8 * n, m, k, gs, bucket(m), int(f32))
+    _lib.call("tf_qmm_group", x, x.stride(0), xs, n, [q.weight for q in qs], [q.scales for q in qs], [q.biases for q in qs],
+              [q.scales.stride(0) for q in qs], outs, part_at, counters,
+              [0 if c is None else c.numel() // COUNTER_STRIDE for c in counters], [q.n for q in qs], sks, m, k, gs,
+              bucket(m), int(f32))
     return outs
 
 
@@ -336,16 +332,17 @@ def prefill_matmul(x: torch.Tensor, q: Q4, *, f32: bool = False, tile: int = 0,
 
     if tile not in (0, 1, 2, 3, 4, 5, 6, 8, 9):
         raise ValueError("prefill_matmul: tile 0 to 6, 8 or 9 (see prompt_tile)")
+    if out is None and arith is None and (y := _lib.whole("prefill_matmul", x, q, f32, tile)) is not None:
+        return y
     x = _check_x(x, q, "prefill_matmul")
     m = int(x.shape[0])
     if out is None:
-        out = x.new_empty((m, q.n), dtype=torch.float32 if f32 else torch.bfloat16)
+        out, = _lib.empties(x, [(m, q.n, f32)])
     elif tuple(out.shape) != (m, q.n) or out.dtype != (torch.float32 if f32 else torch.bfloat16) \
             or not out.is_contiguous() or out.device != x.device:
         raise ValueError(f"prefill_matmul: out must be contiguous ({m}, {q.n}) {'fp32' if f32 else 'bf16'}")
     s16, b16 = q.scales.contiguous(), q.biases.contiguous()
-    _lib.call("tf_qmm_prefill", _lib.ptr(x), x.stride(0), _lib.ptr(q.weight), _lib.ptr(s16), _lib.ptr(b16),
-              _lib.ptr(out), m, q.n, q.k, q.gs, int(f32), tile,
+    _lib.call("tf_qmm_prefill", x, x.stride(0), q.weight, s16, b16, out, m, q.n, q.k, q.gs, int(f32), tile,
               q.arith if arith is None else int(arith))
     return out
 

@@ -1,0 +1,80 @@
+"""The entry points as Python functions (csrc/call.cpp) against ctypes: the same names, argument counts, values and sentences,
+without a GPU (what the library refuses before it launches)."""
+
+import pytest
+import torch
+
+from tensorfold_amd import _lib, build
+
+NATIVE = _lib._bound() if build.call_lib() else None
+pytestmark = pytest.mark.skipif(NATIVE is None, reason="no C++ compiler, Python headers or torch headers")
+QUERIES = {"tf_qmm_prompt_tile", "tf_qmm_prompt_rows", "tf_exl3_gemm_tile"}          # launch nothing: called on the library itself
+
+
+def sentence(name, *args):
+    with pytest.raises(RuntimeError) as caught:
+        NATIVE[name](*args)
+    assert getattr(_lib.lib(), name)(*[a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args]) != 0
+    assert _lib.lib().tf_last_error().decode() == str(caught.value)
+    return str(caught.value)
+
+
+def test_every_launch_is_there_with_its_arguments():
+    assert set(NATIVE) - {"empties", *_lib.WHOLE} == set(_lib.PROTOTYPES) - QUERIES
+    for name, args in _lib.PROTOTYPES.items():
+        if name not in QUERIES:
+            for given in (0, len(args) - 1, len(args) + 1):
+                with pytest.raises(TypeError, match=f"takes {len(args)}"):
+                    NATIVE[name](*[0] * given)
+
+
+def test_values_arrive_as_ctypes_passes_them():
+    x = torch.zeros((2, 64), dtype=torch.bfloat16)
+    assert "not 48" in sentence("tf_group_sums", x, 64, 2, 64, 48, x, None)
+    assert "16-byte" in sentence("tf_group_sums", x.data_ptr() + 2, 64, 2, 64, 64, x, None)          # an address
+    assert "a multiple of the group" in sentence("tf_group_sums", None, 64, 2, 64, 64, x, None)      # no pointer
+    assert "not -3" in sentence("tf_moe_topk", x, 64, 1, 64, -3, True, x, x, None)                   # signs and truth values
+    # 64-bit strides, a float among the whole numbers, the last of many arguments
+    assert "exceed the grid limit" in sentence("tf_experts_prefill", 64, 1, x, 1 << 40, 0, x, 1, 1, x, x, x, x, 32, 0.5, 1 << 40,
+                                               64, 0, None)
+
+
+def test_tables_are_lists():
+    x = torch.zeros((2, 64), dtype=torch.bfloat16)
+    w = torch.zeros((64,), dtype=torch.int32)
+    group = lambda ws, sks, gs: NATIVE["tf_qmm_group"](x, 64, x, len(ws), ws, ws, ws, [128] * len(ws), ws, [None] * len(ws),
+                                                       [None] * len(ws), [0] * len(ws), [64] * len(ws), sks, 2, 64, gs, 16, 0, None)
+    for ws, sks, gs, text in (([w], [1], 48, "groups of 32 or 64"), ([w] * 5, [1] * 5, 64, "1 to 4 weights, not 5"),
+                              ([w, None], [1, 1], 64, "null pointer"), ([w, w], [1, 3], 64, "whole groups a slice"),
+                              ([w, w], [1, 70000], 64, "whole groups a slice")):
+        with pytest.raises(RuntimeError, match=text):
+            group(ws, sks, gs)
+    with pytest.raises(TypeError, match="longer list"):
+        group([w] * 9, [1] * 9, 64)
+
+
+@pytest.mark.parametrize("bad", [1.5, "1", (1,), object()])
+def test_what_is_no_number_and_no_tensor_is_refused(bad):
+    x = torch.zeros((2, 64), dtype=torch.bfloat16)
+    for args in ((bad, 64, 2, 64, 64, x, None), (x, bad, 2, 64, 64, x, None)):
+        with pytest.raises(TypeError):
+            NATIVE["tf_group_sums"](*args)
+
+
+def test_empties():
+    x = torch.zeros((2, 64), dtype=torch.bfloat16)
+    made = NATIVE["empties"](x, [(3, 5, False), (2, 7, True), (0, 4, 0)])
+    assert [(tuple(t.shape), t.dtype, t.is_contiguous(), t.requires_grad) for t in made] == \
+        [((3, 5), torch.bfloat16, True, False), ((2, 7), torch.float32, True, False), ((0, 4), torch.bfloat16, True, False)]
+    for bad in ((x, [(1, 2)]), (x, [(-1, 2, 0)]), (x, 3), (3, []), (x,)):
+        with pytest.raises((TypeError, RuntimeError)):
+            NATIVE["empties"](*bad)
+
+
+def test_a_tensor_without_storage_raises():
+    meta = torch.empty((2, 64), dtype=torch.bfloat16, device="meta")
+    x = torch.zeros((2, 64), dtype=torch.bfloat16)
+    try:
+        NATIVE["tf_group_sums"](meta, 64, 2, 64, 48, x, None)          # (torch hands out an address of 0, or refuses)
+    except RuntimeError:
+        pass
