@@ -21,6 +21,10 @@ LIB = HERE / "libtfmi.so"
 TIMELINE_LIB = HERE / "libtfmi_timeline.so"      # the same kernels with per-workgroup timestamps (see compile)
 SOURCES = ("api.hip", "pack.hip", "decode.hip", "fused.hip", "route.hip", "norm.hip", "prefill.hip", "prefill8.hip", "exl3.hip", "exl3_experts.hip")
 CALL_LIB = HERE / "tfmi_call.so"                 # the entry points as Python functions (csrc/call.cpp); host code alone
+# NDEBUG: without it pybind11 (under torch's headers) brings a thread-local counter, and a library with thread-local storage
+# that is loaded late and never touches its own puts every other library's access to theirs on glibc's slow path (before 2.39):
+# a torch.randint and a conversion take 22.7 us beside such a tfmi_call.so, 20.3 without
+CALL_FLAGS = ("-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden")
 # packed-fp32 VALU forms are switched off for the device pass (the host pass warns that it does not know the feature)
 FLAGS = ("-O3", "-std=c++17", "-fPIC", "-shared", f"--offload-arch={ARCH}",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops")
@@ -53,7 +57,7 @@ def call_id() -> str:
 
     import torch
 
-    h = hashlib.sha256(f"{sys.version} {torch.__version__}".encode())
+    h = hashlib.sha256(f"{sys.version} {torch.__version__} {CALL_FLAGS}".encode())
     for path in (CSRC / "call.cpp", HERE.parent / "include" / "tfmi.h"):
         h.update(path.read_bytes())
     return h.hexdigest()[:16]
@@ -140,7 +144,7 @@ def compile_call() -> Path | None:
     cc, python, root = shutil.which("g++") or shutil.which("c++"), Path(sysconfig.get_paths()["include"]), Path(torch.__file__).parent
     if cc is None or not (python / "Python.h").exists() or not (root / "include/torch/csrc/autograd/python_variable.h").exists():
         return None
-    done = subprocess.run([cc, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", f"-I{python}",
+    done = subprocess.run([cc, *CALL_FLAGS, f"-I{python}",
                            f"-I{root / 'include'}", f"-I{root / 'include/torch/csrc/api/include'}",
                            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DTF_CALL_ID="{call_id()}"',
                            str(CSRC / "call.cpp"), "-o", str(CALL_LIB), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu",

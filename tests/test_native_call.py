@@ -78,3 +78,12 @@ def test_a_tensor_without_storage_raises():
         NATIVE["tf_group_sums"](meta, 64, 2, 64, 48, x, None)          # (torch hands out an address of 0, or refuses)
     except RuntimeError:
         pass
+
+
+def test_the_module_has_no_thread_local_storage():
+    import struct
+
+    image = build.CALL_LIB.read_bytes()
+    at, size, count = struct.unpack_from("<Q", image, 0x20)[0], *struct.unpack_from("<HH", image, 0x36)          # ELF64 program headers
+    kinds = [struct.unpack_from("<I", image, at + i * size)[0] for i in range(count)]
+    assert 1 in kinds and 7 not in kinds          # PT_LOAD, PT_TLS
