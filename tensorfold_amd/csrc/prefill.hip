@@ -394,7 +394,7 @@ static_assert(BIG_LDS + 2 * 2 * BIG_ROWS * 4 + 16 <= 64 * 1024, "within what a l
 // LDS of one stage where a workgroup takes RT row tiles (the dense kernel's 9 are more rows than an item has)
 constexpr int big_stage(int rt) { return std::max(16 * rt, BIG_ROWS) * AROW; }
 
-// The pipeline for an item of at most 16 * RT rows (RT = 2, 4 or 8; the dense prompt matmul's tiles: 2 to 9).  K is a multiple of KSTEP and nothing inside a
+// The pipeline for an item of at most 16 * RT rows (RT = 1 to 8; the dense prompt matmul's tiles: 2 to 9).  K is a multiple of KSTEP and nothing inside a
 // step is conditional (prefetches past the end re-read the last step, rows past the item read its first row), so the
 // compiler is free to keep the LDS reads of the next row tile in flight under the MFMAs of this one.
 // Where a wave's weights come from.  A wave takes 64 weight columns (four operands of 16), and for loading them lane L
@@ -771,6 +771,19 @@ constexpr int expert_threads(int ar) { return 64 * expert_waves(ar); }
 // 32-column blocks a workgroup of the big kernel covers
 constexpr int big_blocks(int nm, int ar) { return nm == 2 ? expert_waves(ar) : 2 * expert_waves(ar); }
 
+// The row tiles an item of `cnt` rows runs with.  Most of a prompt's items are an expert's few rows or a full 128 (4,096 rows of
+// 10 of 512 experts, some popular: 253 items of at most 16 rows, 300 of more than 112, 110 between), and a short item is bound by its
+// weights' way through the vector unit, so what multiplies and stages rows that are not there is in its way: with 2, 4 and 8
+// row tiles alone 777 rows x 128 experts of 2688 x 1856 took 307 us, routing and all, with these 298; 4,096 rows x 512 experts of 2048 x 512
+// 530, now 521.
+#define TF_ITEM_ROWS(cnt)         \
+  if (cnt <= 16) TF_ROWS(1);      \
+  else if (cnt <= 32) TF_ROWS(2); \
+  else if (cnt <= 48) TF_ROWS(3); \
+  else if (cnt <= 64) TF_ROWS(4); \
+  else if (cnt <= 96) TF_ROWS(6); \
+  else TF_ROWS(8);
+
 template <int GS, int NM, int EPI, int AR>
 __global__ void __launch_bounds__(expert_threads(AR), expert_threads(AR) == 256 ? 2 : 1)
     experts_prefill_big_kernel(const uint16_t* __restrict__ X, int64_t x_stride, int slots,
@@ -820,9 +833,11 @@ __global__ void __launch_bounds__(expert_threads(AR), expert_threads(AR) == 256 
   const int K = KG * GS;
   const bool busy = cbt * NBW + (NM == 2 ? wave : 2 * wave) < NB;          // the wave has a column
   constexpr bool SKIP = AR == TF_ARITH_BF16;          // (the fp16 form's loop came out 1 % slower for it)
-  if (cnt <= 32) big_body<GS, NM, EPI, 2, AR, OUT_LINES, ExpertSource<GS, NM>, 4, expert_threads(AR), OUT_LINES, NoStaged, SKIP>(X, x_stride, ws, ocol, jok, K, src_rows, dst_rows, cnt, out, N, limit, smem, NoStaged(), tid, busy);
-  else if (cnt <= 64) big_body<GS, NM, EPI, 4, AR, OUT_LINES, ExpertSource<GS, NM>, 4, expert_threads(AR), OUT_LINES, NoStaged, SKIP>(X, x_stride, ws, ocol, jok, K, src_rows, dst_rows, cnt, out, N, limit, smem, NoStaged(), tid, busy);
-  else big_body<GS, NM, EPI, 8, AR, OUT_LINES, ExpertSource<GS, NM>, 4, expert_threads(AR), OUT_LINES, NoStaged, SKIP>(X, x_stride, ws, ocol, jok, K, src_rows, dst_rows, cnt, out, N, limit, smem, NoStaged(), tid, busy);
+#define TF_ROWS(RT_)                                                                                                          \
+  big_body<GS, NM, EPI, RT_, AR, OUT_LINES, ExpertSource<GS, NM>, 4, expert_threads(AR), OUT_LINES, NoStaged, SKIP>(          \
+      X, x_stride, ws, ocol, jok, K, src_rows, dst_rows, cnt, out, N, limit, smem, NoStaged(), tid, busy)
+  TF_ITEM_ROWS(cnt)
+#undef TF_ROWS
   TF_MARK(4);
 #ifdef TF_TIMELINE
   __builtin_amdgcn_s_waitcnt(0);         // mark 5 is the results written, not only issued
@@ -957,9 +972,9 @@ __global__ void __launch_bounds__(expert_threads(AR), expert_threads(AR) == 256 
       }
     };
     const uint32_t* We = W + (size_t)e * NB * KG * (size_t)(NM * BW);
-    if (cnt <= 32) resident_unit<GS, NM, EPI, AR, 2>(X, x_stride, We, KG, NB, cbt, cnt, out, N, limit, k & 1, tid, staged);
-    else if (cnt <= 64) resident_unit<GS, NM, EPI, AR, 4>(X, x_stride, We, KG, NB, cbt, cnt, out, N, limit, k & 1, tid, staged);
-    else resident_unit<GS, NM, EPI, AR, 8>(X, x_stride, We, KG, NB, cbt, cnt, out, N, limit, k & 1, tid, staged);
+#define TF_ROWS(RT_) resident_unit<GS, NM, EPI, AR, RT_>(X, x_stride, We, KG, NB, cbt, cnt, out, N, limit, k & 1, tid, staged)
+    TF_ITEM_ROWS(cnt)
+#undef TF_ROWS
     TF_MARK(4);
 #ifdef TF_TIMELINE
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
