@@ -1117,6 +1117,12 @@ __global__ void __launch_bounds__(64 * WR * WC)
   constexpr int CPS = STEP / 32, GPS = STEP / GS, PPR = STEP / 8;        // chunks, groups, 16-byte pieces of a row a step
   constexpr int PPT = T::BM * PPR / T::THREADS;
   constexpr int WSETS = 4;
+  // A chunk's operands are read AHEAD chunks before their use; OVER the ends of steps, with the barrier inside the step, or within
+  // a step between its two barriers.  Over the ends: 64 x 128 35.1 -> 28.9 us a round of K = 4096 (300 rows x 12288 49.2 -> 45.7,
+  // 1,000 x 4096 49.6 -> 47.1), 32 x 128 19.0 -> 18.3, 16 x 64 14.3 -> 13.6 (40 rows x 1024 x 5120); but 32 x 64, of which a compute unit
+  // holds three or four, 20.3 -> 21.7 where it has two (200 rows x 4096 x 4096).
+  constexpr bool OVER = !(RT == 2 && WC == 4);
+  constexpr int AHEAD = OVER ? 3 : 1;
   static_assert(T::BM * PPR % T::THREADS == 0 && T::THREADS % PPR == 0 && 128 % T::BN == 0, "whole pieces a thread");
   extern __shared__ __align__(16) unsigned char smem[];
   const int ct = short_tiles(N, T::BN), mt = short_tiles(M, T::BM);
@@ -1175,7 +1181,7 @@ __global__ void __launch_bounds__(64 * WR * WC)
 #pragma unroll
     for (int j = 0; j < PPT; ++j) v[j] = *reinterpret_cast<const uint4*>(asrc[j] + k);
   };
-  auto store_a = [&](int step, int buf, uint4 (&v)[PPT]) {
+  auto store_a = [&](int step, int stage, uint4 (&v)[PPT]) {
     if ((step + 1) * STEP > K) {                                 // inputs past a ragged end count as zeros
 #pragma unroll
       for (int j = 0; j < PPT; ++j)
@@ -1183,7 +1189,7 @@ __global__ void __launch_bounds__(64 * WR * WC)
     }
 #pragma unroll
     for (int j = 0; j < PPT; ++j)
-      *reinterpret_cast<uint4*>(smem + buf * (T::BM * T::ROW) + (arow + j * (T::THREADS / PPR)) * T::ROW + ach * 2) =
+      *reinterpret_cast<uint4*>(smem + stage + (arow + j * (T::THREADS / PPR)) * T::ROW + ach * 2) =
           AR ? stage8_bf16(v[j]) : stage8(v[j]);
   };
 
@@ -1200,22 +1206,40 @@ __global__ void __launch_bounds__(64 * WR * WC)
 #pragma unroll
   for (int u = 1; u < WSETS; ++u) load_w(u, w[u]);
   store_a(0, 0, a[0]);
+  if constexpr (OVER) load_a(2, a[0]);
   __syncthreads();
-  // one step from landing set U and LDS stage U & 1
-  auto walk = [&](int step, auto U) __attribute__((always_inline)) {
-    constexpr int u = decltype(U)::value;
-    load_a(step + 2, a[u & 1]);
-    const unsigned char* at = smem + (u & 1) * (T::BM * T::ROW) + (wr * 16 * RT + c) * T::ROW + kq * 16;
-    uint32_t q[CT][4], sb[CT][4];
-    u32x4_t av[2][RT];
+  static_assert(CPS % (AHEAD + 1) == 0, "a step begins with the first of the operand sets");
+  u32x4_t av[AHEAD + 1][RT];
+  const int mine_at = (wr * 16 * RT + c) * T::ROW + kq * 16;
+  auto read_a = [&](int stage, int i) {
 #pragma unroll
-    for (int r = 0; r < RT; ++r) av[0][r] = *reinterpret_cast<const u32x4_t*>(at + 16 * r * T::ROW);
+    for (int r = 0; r < RT; ++r)
+      av[i % (AHEAD + 1)][r] = *reinterpret_cast<const u32x4_t*>(smem + stage + mine_at + 16 * r * T::ROW + i * 64);
+  };
+  if constexpr (OVER) {
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) read_a(0, i);
+  }
+  // One step from landing set U and LDS stage U & 1.  OVER: the next step's inputs are put away at its top, where that stage has
+  // been read by all (its last chunk is read ahead of the barrier before), and may be read behind its own barrier.
+  auto walk = [&](int step, auto U) __attribute__((always_inline)) {
+    constexpr int u = decltype(U)::value, stage = (u & 1) * (T::BM * T::ROW), next = T::BM * T::ROW - stage;
+    if constexpr (OVER) {
+      store_a(step + 1, next, a[1 - (u & 1)]);
+      load_a(step + 3, a[1 - (u & 1)]);
+    } else {
+      load_a(step + 2, a[u & 1]);
+      read_a(stage, 0);
+    }
+    uint32_t q[CT][4], sb[CT][4];
 #pragma unroll
     for (int i = 0; i < CPS; ++i) {
-      if (i + 1 < CPS) {
-#pragma unroll
-        for (int r = 0; r < RT; ++r)
-          av[(i + 1) & 1][r] = *reinterpret_cast<const u32x4_t*>(at + 16 * r * T::ROW + (i + 1) * 64);
+      if constexpr (OVER) {
+        if (i == CPS - AHEAD) __syncthreads();
+        read_a(i + AHEAD < CPS ? stage : next, (i + AHEAD) % CPS);
+        __builtin_amdgcn_sched_barrier(0x7F);                    // all but LDS operations may pass
+      } else if (i + AHEAD < CPS) {
+        read_a(stage, i + AHEAD);
       }
       u32x4_t bw[CT];
 #pragma unroll
@@ -1243,17 +1267,20 @@ __global__ void __launch_bounds__(64 * WR * WC)
       for (int r = 0; r < RT; ++r)
 #pragma unroll
         for (int t = 0; t < CT; ++t) {
+          const u32x4_t& xa = av[i % (AHEAD + 1)][r];
           if constexpr (AR)
             acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, bw[t]),
-                                                                __builtin_bit_cast(bf16x8_t, av[i & 1][r]), acc[r][t], 0, 0, 0);
+                                                                __builtin_bit_cast(bf16x8_t, xa), acc[r][t], 0, 0, 0);
           else
             acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, bw[t]),
-                                                               __builtin_bit_cast(f16x8_t, av[i & 1][r]), acc[r][t], 0, 0, 0);
+                                                               __builtin_bit_cast(f16x8_t, xa), acc[r][t], 0, 0, 0);
         }
     }
     load_w(step + WSETS, w[u]);
-    store_a(step + 1, 1 - (u & 1), a[1 - (u & 1)]);
-    __syncthreads();
+    if constexpr (!OVER) {
+      store_a(step + 1, next, a[1 - (u & 1)]);
+      __syncthreads();
+    }
   };
   int step = 0;
   for (; step + WSETS <= steps; step += WSETS) {
@@ -1358,7 +1385,7 @@ static bool big_takes(int64_t n, int64_t k) {
 // What code 0 stands for.  A call's time is about a start plus a cost a round of 256 workgroups, in the same unit per
 // input of K (half microseconds at K = 4096; measured on 17 to 4,096 rows x 512 to 17,408 columns): the least of them is
 // taken.  17 rows x 4096 x 4096 82.9 -> 12.9 us, 100 rows 86.3 -> 14.4 (32 x 64), 512 rows 89 -> 33 (32 x 128),
-// 1,000 rows 89 -> 53 (64 x 128); at 2,000 rows the eight-wave kernel's 95.7 is the best again (64 x 128 98.5).
+// 1,000 rows 89 -> 47 (64 x 128); at 2,000 rows the eight-wave kernel's 95.7 is the best again (64 x 128 98.5).
 constexpr int SHORT_K = 192;
 
 // The eight-wave kernel's row tiles.  Where all are 128 rows the last round of 256 workgroups is seldom full and costs what a
