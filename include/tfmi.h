@@ -326,6 +326,10 @@ int tf_exl3_unpack(const uint32_t* T, uint16_t* W, int k, int n, int64_t stride_
  * The reference decodes W_q [K, N] with `unpack` once a chunk (exl3/prefill.py:88-89). */
 int tf_exl3_unpack_k8(const uint32_t* T, uint16_t* W8, int k, int n, int64_t stride_k, int64_t stride_nb, int k2,
                       int cb, tf_stream_t stream);
+/* tf_exl3_rot_in of x [m, k] and tf_exl3_unpack_k8 of the layer's weight, in one launch: what a prompt's product starts from. */
+int tf_exl3_rot_in_unpack_k8(const void* x, int x_dtype, const uint16_t* suh, uint16_t* xh, int m, const uint32_t* T,
+                             uint16_t* W8, int k, int n, int64_t stride_k, int64_t stride_nb, int k2, int cb,
+                             tf_stream_t stream);
 /* y[m, block] = ((xh[m] @ W_q[:, block]) H / sqrt(128)) * svh + bias for any m: xh fp16 [m, k] from tf_exl3_rot_in,
  * w8 from tf_exl3_unpack_k8 (k * n < 2^31), K added in order in fp32 (a row's bits do not depend on m or on the
  * rows beside it), the rotation exact in fp32.  y rows are y_stride elements apart.  Replaces exl3/prefill.py:16-44

@@ -56,6 +56,7 @@ PROTOTYPES = {
     "tf_exl3_swiglu_rot_in": [P, I, P, P, I, I, P],
     "tf_exl3_unpack": [P, P, I, I, L, L, I, I, P],
     "tf_exl3_unpack_k8": [P, P, I, I, L, L, I, I, P],
+    "tf_exl3_rot_in_unpack_k8": [P, I, P, P, I, P, P, I, I, L, L, I, I, P],
     "tf_exl3_gemm_tile": [I, I],
     "tf_exl3_gemm": [P, P, P, P, P, I, L, I, I, I, P],
 }

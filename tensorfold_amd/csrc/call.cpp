@@ -32,7 +32,8 @@ namespace {
   X(tf_moe_decode_sliced) X(tf_moe_route_decode) X(tf_moe_decode_experts) X(tf_moe_router) X(tf_moe_topk) X(tf_moe_combine) \
   X(tf_exl3x_rot_in) X(tf_exl3x_grouped) X(tf_exl3x_gateup_epilogue) X(tf_exl3x_down_combine) X(tf_exl3x_plan_rot_in)       \
   X(tf_add_norm) X(tf_exl3_rot_in) X(tf_exl3_linear) X(tf_exl3_rot_in_stacked) X(tf_exl3_linear_stacked) X(tf_exl3_gate_up) \
-  X(tf_exl3_swiglu_rot_in) X(tf_exl3_unpack) X(tf_exl3_unpack_k8) X(tf_exl3_gemm)
+  X(tf_exl3_swiglu_rot_in) X(tf_exl3_unpack) X(tf_exl3_unpack_k8) X(tf_exl3_rot_in_unpack_k8) \
+  X(tf_exl3_gemm)
 
 struct Library {
   decltype(&::tf_last_error) tf_last_error;

@@ -14,14 +14,12 @@ namespace {
 // blocks of x as they lie in memory, two at a time.  blockIdx.y is the layer of a stack: its own suh [K] and xh [M, K] over the one
 // x.  Bound by memory once the butterflies stay in registers (1,000 rows x 5120: 11.2 us with a wave a block and
 // ds_bpermute, 6.5 now).
-__global__ void __launch_bounds__(256)
-    rot_in_kernel(const void* __restrict__ x, int x_dtype, const uint16_t* __restrict__ suh, uint16_t* __restrict__ xh,
-                  uint32_t blocks, int K) {
+__device__ __forceinline__ void rot_in_walk(const void* __restrict__ x, int x_dtype, const uint16_t* __restrict__ suh,
+                                            uint16_t* __restrict__ xh, uint32_t blocks, int K, uint32_t workgroup,
+                                            uint32_t workgroups) {
   const int lane = threadIdx.x & 63, sub = lane & 15;
-  suh += (size_t)blockIdx.y * K;
-  xh += (size_t)blockIdx.y * blocks * 128;
-  const uint32_t groups = gridDim.x * 16, kb = (uint32_t)K >> 7;
-  for (uint32_t u = blockIdx.x * 16 + (threadIdx.x >> 4); u < blocks; u += 2 * groups) {
+  const uint32_t groups = workgroups * 16, kb = (uint32_t)K >> 7;
+  for (uint32_t u = workgroup * 16 + (threadIdx.x >> 4); u < blocks; u += 2 * groups) {
     const uint32_t u1 = u + groups;                                           // the second block of the two
     const bool two = u1 < blocks;
     float s[8], s1[8], v[8], v1[8];
@@ -42,6 +40,12 @@ __global__ void __launch_bounds__(256)
     finish(u, v, s);
     if (two) finish(u1, v1, s1);
   }
+}
+
+__global__ void __launch_bounds__(256)
+    rot_in_kernel(const void* __restrict__ x, int x_dtype, const uint16_t* __restrict__ suh, uint16_t* __restrict__ xh,
+                  uint32_t blocks, int K) {
+  rot_in_walk(x, x_dtype, suh + (size_t)blockIdx.y * K, xh + (size_t)blockIdx.y * blocks * 128, blocks, K, blockIdx.x, gridDim.x);
 }
 
 // The SwiGLU of a stack's two outputs (gate y[0], up y[1], each [M, N]) and the next layer's input rotation in a
@@ -225,14 +229,30 @@ __global__ void __launch_bounds__(64)
 // back through it and leave as four stores of 16 bytes a lane, runs of 2 KB.  (With a lane loading its own words and
 // storing its own pairs, 32 memory instructions of 4 bytes a wave, the address unit's 16 cycles an instruction were the whole
 // time: 5120 x 17408 at 3 bits 43 us, now 34.)
+// The first rot.rows rows of the grid rotate a prompt's inputs instead (none where the weight alone is asked for): neither work
+// needs the other, and a launch of its own for the smaller one is mostly its start and its end (1,000 rows x 5120 -> 17408 at 3 bits,
+// product and all: 197.3 us in three launches, 193.8 in two).
+struct Rotation {
+  const void* x;
+  const uint16_t* suh;
+  uint16_t* xh;
+  uint32_t blocks;
+  int x_dtype, k, rows;
+};
+
 template <int K2, int CB>
 __global__ void __launch_bounds__(256)
     unpack_k8_kernel(const uint32_t* __restrict__ T, uint16_t* __restrict__ W8, int N, int64_t stride_k,
-                     int64_t stride_nb) {
+                     int64_t stride_nb, Rotation rot) {
+  const int by = (int)blockIdx.y - rot.rows;
+  if (by < 0) {
+    rot_in_walk(rot.x, rot.x_dtype, rot.suh, rot.xh, rot.blocks, rot.k, blockIdx.y * gridDim.x + blockIdx.x, rot.rows * gridDim.x);
+    return;
+  }
   constexpr int TW = tile_words<K2>(), PIECES = 2 * TW;                    // a run of eight tiles in 16-byte pieces
   static_assert(8 * TW <= 1024, "the run fits where the values go");
   __shared__ __align__(16) uint32_t stage[4][1024];                        // [octet of two][column][4 pairs of inputs]
-  const int wave = threadIdx.x >> 6, kt = 4 * blockIdx.y + wave, nb = blockIdx.x, lane = threadIdx.x & 63, L = lane & 31, h = lane >> 5;
+  const int wave = threadIdx.x >> 6, kt = 4 * by + wave, nb = blockIdx.x, lane = threadIdx.x & 63, L = lane & 31, h = lane >> 5;
   const uint32_t* run = T + (size_t)kt * stride_k + (size_t)nb * stride_nb;
   uint32_t* own = stage[wave];
 #pragma unroll
@@ -445,18 +465,28 @@ __global__ void __launch_bounds__(64 * GEMM_WAVES, 2)
 
 using namespace tf;
 
-static int rot_in_launch(const char* who, const void* x, int x_dtype, const uint16_t* suh, uint16_t* xh, int layers,
-                         int m, int k, tf_stream_t stream) {
-  clear_error();
+// what a rotation asks of its arguments, and the workgroups it takes
+static int rot_in_plan(const char* who, const void* x, int x_dtype, const uint16_t* suh, const uint16_t* xh, int layers, int m, int k,
+                       uint32_t& blocks, unsigned& workgroups) {
   TF_REQUIRE(x && suh && xh, "%s: null pointer argument", who);
   TF_REQUIRE(x_dtype == TF_F16 || x_dtype == TF_BF16 || x_dtype == TF_F32, "x: expected fp16, bf16 or fp32");
   TF_REQUIRE(m >= 1 && k >= 128 && k % 128 == 0, "x and xh must be [M, K], K a multiple of 128, suh [K]");
   TF_REQUIRE(layers >= 1 && layers <= 64, "%s: 1 to 64 layers a stack", who);
   TF_REQUIRE(aligned16(x) && aligned16(xh), "x: must be 16-byte aligned");
   // sixteen blocks a workgroup, thirty-two once that fills the chip; past 4,096 workgroups they walk
-  const int64_t blocks = (int64_t)m * (k / 128), groups = blocks < 16384 ? (blocks + 15) / 16 : (blocks + 31) / 32;
-  TF_REQUIRE(blocks < (1LL << 31), "%s: %lld blocks of 128 are more than a launch counts", who, (long long)blocks);
-  rot_in_kernel<<<dim3((unsigned)(groups < 4096 ? groups : 4096), layers), 256, 0, as_stream(stream)>>>(x, x_dtype, suh, xh, (uint32_t)blocks, k);
+  const int64_t all = (int64_t)m * (k / 128), groups = all < 16384 ? (all + 15) / 16 : (all + 31) / 32;
+  TF_REQUIRE(all < (1LL << 31), "%s: %lld blocks of 128 are more than a launch counts", who, (long long)all);
+  blocks = (uint32_t)all, workgroups = (unsigned)(groups < 4096 ? groups : 4096);
+  return 0;
+}
+
+static int rot_in_launch(const char* who, const void* x, int x_dtype, const uint16_t* suh, uint16_t* xh, int layers,
+                         int m, int k, tf_stream_t stream) {
+  clear_error();
+  uint32_t blocks;
+  unsigned workgroups;
+  if (rot_in_plan(who, x, x_dtype, suh, xh, layers, m, k, blocks, workgroups)) return 1;
+  rot_in_kernel<<<dim3(workgroups, layers), 256, 0, as_stream(stream)>>>(x, x_dtype, suh, xh, blocks, k);
   TF_LAUNCH_OK(who);
   return 0;
 }
@@ -567,24 +597,45 @@ extern "C" int tf_exl3_unpack(const uint32_t* T, uint16_t* W, int k, int n, int6
   return 1;
 }
 
-extern "C" int tf_exl3_unpack_k8(const uint32_t* T, uint16_t* W8, int k, int n, int64_t stride_k, int64_t stride_nb,
-                                 int k2, int cb, tf_stream_t stream) {
-  clear_error();
+static int unpack_k8_launch(const char* who, const uint32_t* T, uint16_t* W8, int k, int n, int64_t stride_k, int64_t stride_nb,
+                            int k2, int cb, const Rotation& rot, hipStream_t s) {
   TF_REQUIRE(T && W8 && aligned16(W8), "unpack_k8: null or unaligned pointer argument");
   TF_REQUIRE(k >= 128 && n >= 128 && k % 128 == 0 && n % 128 == 0, "W must be [K, N], multiples of 128");
-  TF_REQUIRE(k / 64 <= 65535, "unpack_k8: K too large for one launch");
-  const dim3 grid((unsigned)(n / 128), (unsigned)(k / 64));
-  hipStream_t s = as_stream(stream);
-#define TF_LAUNCH(K2_, CB_)                                                            \
-  if (k2 == K2_ && cb == CB_) {                                                        \
-    unpack_k8_kernel<K2_, CB_><<<grid, 256, 0, s>>>(T, W8, n, stride_k, stride_nb);    \
-    TF_LAUNCH_OK("tf_exl3_unpack_k8");                                                 \
-    return 0;                                                                          \
+  TF_REQUIRE(k / 64 + rot.rows <= 65535, "unpack_k8: K too large for one launch");
+  const dim3 grid((unsigned)(n / 128), (unsigned)(k / 64 + rot.rows));
+#define TF_LAUNCH(K2_, CB_)                                                               \
+  if (k2 == K2_ && cb == CB_) {                                                           \
+    unpack_k8_kernel<K2_, CB_><<<grid, 256, 0, s>>>(T, W8, n, stride_k, stride_nb, rot);  \
+    TF_LAUNCH_OK(who);                                                                    \
+    return 0;                                                                             \
   }
   TF_EXL3_ALL(TF_LAUNCH)
 #undef TF_LAUNCH
   set_error("unsupported EXL3 width/codebook: K2=%d codebook=%d", k2, cb);
   return 1;
+}
+
+extern "C" int tf_exl3_unpack_k8(const uint32_t* T, uint16_t* W8, int k, int n, int64_t stride_k, int64_t stride_nb,
+                                 int k2, int cb, tf_stream_t stream) {
+  clear_error();
+  return unpack_k8_launch("tf_exl3_unpack_k8", T, W8, k, n, stride_k, stride_nb, k2, cb, Rotation{}, as_stream(stream));
+}
+
+extern "C" int tf_exl3_rot_in_unpack_k8(const void* x, int x_dtype, const uint16_t* suh, uint16_t* xh, int m, const uint32_t* T,
+                                        uint16_t* W8, int k, int n, int64_t stride_k, int64_t stride_nb, int k2, int cb,
+                                        tf_stream_t stream) {
+  clear_error();
+  Rotation rot = {x, suh, xh, 0, x_dtype, k, 0};
+  unsigned workgroups;
+  if (rot_in_plan("tf_exl3_rot_in", x, x_dtype, suh, xh, 1, m, k, rot.blocks, workgroups)) return 1;
+  TF_REQUIRE(n >= 128 && n % 128 == 0, "W must be [K, N], multiples of 128");
+  rot.rows = (int)((workgroups + n / 128 - 1) / (n / 128));
+  if (k / 64 + rot.rows <= 65535)
+    return unpack_k8_launch("tf_exl3_rot_in_unpack_k8", T, W8, k, n, stride_k, stride_nb, k2, cb, rot, as_stream(stream));
+  // more rows than a grid has: one launch after the other
+  rot.rows = 0;
+  if (rot_in_launch("tf_exl3_rot_in", x, x_dtype, suh, xh, 1, m, k, stream)) return 1;
+  return unpack_k8_launch("tf_exl3_unpack_k8", T, W8, k, n, stride_k, stride_nb, k2, cb, rot, as_stream(stream));
 }
 
 // Row tiles (of 16) a workgroup, 2 to 9.  Estimated time: the tiles a compute unit gets, times what a tile takes there,

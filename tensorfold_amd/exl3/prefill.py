@@ -44,11 +44,14 @@ def decode(layer: Exl3Linear, ws: Workspace) -> torch.Tensor:
     """W_q as fp16 [K / 8, N, 8] (``w8[o, c, i] = W_q[8 * o + i, c]``) into the workspace: once a chunk, or once for
     several calls on one layer."""
 
-    k, n = layer.k, layer.n
-    w8 = ws._grow("w", k * n, layer.words.device)[:k * n].view(k // 8, n, 8)
-    _lib.call("tf_exl3_unpack_k8", layer.words, w8, k, n, *layer.strides, layer.k2,
-              CODEBOOK_IDS[layer.codebook])
+    w8 = _decoded(layer, ws)
+    _lib.call("tf_exl3_unpack_k8", layer.words, w8, layer.k, layer.n, *layer.strides, layer.k2, CODEBOOK_IDS[layer.codebook])
     return w8
+
+
+def _decoded(layer: Exl3Linear, ws: Workspace) -> torch.Tensor:
+    k, n = layer.k, layer.n
+    return ws._grow("w", k * n, layer.words.device)[:k * n].view(k // 8, n, 8)
 
 
 def row_tiles(m: int, n: int) -> int:
@@ -73,11 +76,14 @@ def matmul(layer: Exl3Linear, x: torch.Tensor, out: torch.Tensor, ws: Workspace,
     _lib.on_gpu(x, out)
     x = x.contiguous()
     xh = ws._grow("xh", m * k, x.device)[:m * k].view(m, k)
-    _lib.call("tf_exl3_rot_in", x, _DTYPES[x.dtype], layer.suh, xh, m, k)
     if wt is None:
-        wt = decode(layer, ws)
+        wt = _decoded(layer, ws)
+        _lib.call("tf_exl3_rot_in_unpack_k8", x, _DTYPES[x.dtype], layer.suh, xh, m, layer.words, wt, k, n, *layer.strides,
+                  layer.k2, CODEBOOK_IDS[layer.codebook])
     elif wt.dtype != torch.float16 or tuple(wt.shape) != (k // 8, n, 8) or not wt.is_contiguous() or wt.device != x.device:
         raise ValueError(f"prefill matmul: wt must be the contiguous fp16 ({k // 8}, {n}, 8) that decode() returns")
+    else:
+        _lib.call("tf_exl3_rot_in", x, _DTYPES[x.dtype], layer.suh, xh, m, k)
     _lib.call("tf_exl3_gemm", xh, wt, layer.svh, layer.bias, out,
               _DTYPES[out.dtype], out.stride(0), m, k, n)
     return out
