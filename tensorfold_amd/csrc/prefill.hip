@@ -1117,11 +1117,12 @@ __global__ void __launch_bounds__(64 * WR * WC)
   constexpr int CPS = STEP / 32, GPS = STEP / GS, PPR = STEP / 8;        // chunks, groups, 16-byte pieces of a row a step
   constexpr int PPT = T::BM * PPR / T::THREADS;
   constexpr int WSETS = 4;
-  // A chunk's operands are read AHEAD chunks before their use; OVER the ends of steps, with the barrier inside the step, or within
-  // a step between its two barriers.  Over the ends: 64 x 128 35.1 -> 28.9 us a round of K = 4096 (300 rows x 12288 49.2 -> 45.7,
-  // 1,000 x 4096 49.6 -> 47.1), 32 x 128 19.0 -> 18.3, 16 x 64 14.3 -> 13.6 (40 rows x 1024 x 5120); but 32 x 64, of which a compute unit
-  // holds three or four, 20.3 -> 21.7 where it has two (200 rows x 4096 x 4096).
-  constexpr bool OVER = !(RT == 2 && WC == 4);
+  // A chunk's operands are read AHEAD chunks before their use: OVER the ends of steps, with the barrier inside the step, or within
+  // a step between its two barriers.  Over the ends 64 x 128 takes 28.9 us a round of K = 4096 where it took 35.1 (300 rows x
+  // 12288 49.2 -> 46.2, 1,000 x 4096 49.6 -> 47.1).  The smaller tiles, whose workgroups share compute units, gain 2 to 5 % in a call of
+  // one round (16 x 64, 40 rows x 1024 x 5120 14.3 -> 13.6) and lose 1 to 5 % in the others (16 x 64, 512 rows x 4096 49.1 -> 49.8; 32 x 64, 200
+  // rows 20.3 -> 21.7), and 32 x 128 with groups of 32 loses 14 % (140 rows x 10310 x 3488 32.0 -> 37.5): they read within a step.
+  constexpr bool OVER = CT > 1;
   constexpr int AHEAD = OVER ? 3 : 1;
   static_assert(T::BM * PPR % T::THREADS == 0 && T::THREADS % PPR == 0 && 128 % T::BN == 0, "whole pieces a thread");
   extern __shared__ __align__(16) unsigned char smem[];
