@@ -1210,37 +1210,39 @@ __global__ void __launch_bounds__(64 * WR * WC)
   if constexpr (OVER) load_a(2, a[0]);
   __syncthreads();
   static_assert(CPS % (AHEAD + 1) == 0, "a step begins with the first of the operand sets");
-  u32x4_t av[AHEAD + 1][RT];
-  const int mine_at = (wr * 16 * RT + c) * T::ROW + kq * 16;
-  auto read_a = [&](int stage, int i) {
+  typedef u32x4_t Operands[AHEAD + 1][RT];
+  auto read_a = [&](int stage, int i, Operands& av) {
+    const unsigned char* at = smem + stage + (wr * 16 * RT + c) * T::ROW + kq * 16;
 #pragma unroll
-    for (int r = 0; r < RT; ++r)
-      av[i % (AHEAD + 1)][r] = *reinterpret_cast<const u32x4_t*>(smem + stage + mine_at + 16 * r * T::ROW + i * 64);
+    for (int r = 0; r < RT; ++r) av[i % (AHEAD + 1)][r] = *reinterpret_cast<const u32x4_t*>(at + 16 * r * T::ROW + i * 64);
   };
+  Operands kept;                                                 // OVER: from step to step
   if constexpr (OVER) {
 #pragma unroll
-    for (int i = 0; i < AHEAD; ++i) read_a(0, i);
+    for (int i = 0; i < AHEAD; ++i) read_a(0, i, kept);
   }
   // One step from landing set U and LDS stage U & 1.  OVER: the next step's inputs are put away at its top, where that stage has
   // been read by all (its last chunk is read ahead of the barrier before), and may be read behind its own barrier.
   auto walk = [&](int step, auto U) __attribute__((always_inline)) {
     constexpr int u = decltype(U)::value, stage = (u & 1) * (T::BM * T::ROW), next = T::BM * T::ROW - stage;
+    Operands within;
+    Operands& av = OVER ? kept : within;
     if constexpr (OVER) {
       store_a(step + 1, next, a[1 - (u & 1)]);
       load_a(step + 3, a[1 - (u & 1)]);
     } else {
       load_a(step + 2, a[u & 1]);
-      read_a(stage, 0);
+      read_a(stage, 0, av);
     }
     uint32_t q[CT][4], sb[CT][4];
 #pragma unroll
     for (int i = 0; i < CPS; ++i) {
       if constexpr (OVER) {
         if (i == CPS - AHEAD) __syncthreads();
-        read_a(i + AHEAD < CPS ? stage : next, (i + AHEAD) % CPS);
+        read_a(i + AHEAD < CPS ? stage : next, (i + AHEAD) % CPS, av);
         __builtin_amdgcn_sched_barrier(0x7F);                    // all but LDS operations may pass
       } else if (i + AHEAD < CPS) {
-        read_a(stage, i + AHEAD);
+        read_a(stage, i + AHEAD, av);
       }
       u32x4_t bw[CT];
 #pragma unroll
@@ -1268,7 +1270,7 @@ __global__ void __launch_bounds__(64 * WR * WC)
       for (int r = 0; r < RT; ++r)
 #pragma unroll
         for (int t = 0; t < CT; ++t) {
-          const u32x4_t& xa = av[i % (AHEAD + 1)][r];
+          const u32x4_t xa = av[i % (AHEAD + 1)][r];
           if constexpr (AR)
             acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, bw[t]),
                                                                 __builtin_bit_cast(bf16x8_t, xa), acc[r][t], 0, 0, 0);
