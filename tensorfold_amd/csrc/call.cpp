@@ -174,7 +174,7 @@ PyObject* empties(PyObject*, PyObject* const* args, Py_ssize_t given) {
 // qmm.matmul, qmm.matmul_group, qmm.prefill_matmul and glue.add_rmsnorm where every argument is the ordinary one: results made here,
 // then the launch.  What is not (a row layout that wants a copy, a buffer of the caller's, a wrong type) returns None and
 // takes the caller's general way, which copies or raises.  The norm with q, k and v at one row: 26.2 us in Python with ctypes, 21.6
-// with the launches above, 14.8 so (10 us on the GPU); a matmul of a few rows 15.9, 6.1.
+// with the launches above, 12.9 so (10 us on the GPU); a matmul of a few rows 15.9, 6.1.
 
 PyObject *s_weight, *s_scales, *s_biases, *s_n, *s_k, *s_gs, *s_arith, *s_counters;          // attribute names, interned by bind
 
