@@ -1,13 +1,15 @@
 // The launching entry points of include/tfmi.h as Python functions, for _lib.call: the arguments go from the interpreter to the
 // library without ctypes, which converted each of a launch's 8 to 24 through an object of its own (2 to 3 us a launch; the decode
 // layer of one row and the norm with q, k and v are bound by the host).  A pointer is a tensor, a whole number or None, a table of
-// them a list.  Raises what ctypes' caller raised: RuntimeError with the library's sentence.
+// them a list.  Raises what ctypes' caller raised: RuntimeError with the library's sentence; and what torch raises for the results that
+// are made here: torch.OutOfMemoryError where a device is full.
 
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <dlfcn.h>
 
 #include <ATen/ops/empty.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdint>
@@ -115,13 +117,14 @@ PyObject* run(int (*entry)(A...), PyObject* const* args, Py_ssize_t given, std::
   return nullptr;
 }
 
-// no C++ exception (a tensor without storage) leaves through the interpreter
+// no C++ exception (a tensor without storage, an allocation refused) leaves through the interpreter: it is raised as the type that
+// torch's own functions raise it as
 template <class F>
 PyObject* caught(F&& f) {
   try {
     return f();
-  } catch (const std::exception& e) {
-    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+  } catch (...) {
+    torch::translate_exception_to_python(std::current_exception());
     return nullptr;
   }
 }

@@ -113,3 +113,12 @@ def test_under_capture_and_on_another_stream():
         y = qmm.matmul(x, q)
     torch.cuda.current_stream().wait_stream(side)
     assert torch.equal(y, want)
+
+
+def test_a_full_device_raises_torch_s_own_error():
+    x = torch.zeros((1, 64), dtype=torch.bfloat16, device=DEV)
+    assert "empties" in _lib._start()
+    with pytest.raises(torch.OutOfMemoryError):                            # 4 PiB: refused as it is asked for
+        _lib.empties(x, [(1 << 20, 1 << 30, True)])
+    with pytest.raises(torch.OutOfMemoryError):
+        qmm.matmul(x, weight(130, 64, 64), sk=1 << 30)

@@ -80,6 +80,18 @@ def test_a_tensor_without_storage_raises():
         pass
 
 
+def test_what_an_allocation_raises_keeps_its_type():
+    class Elsewhere(torch.Tensor):
+        __torch_dispatch__ = classmethod(lambda *_: None)
+
+    # a device that this torch has no allocator for: torch.empty raises NotImplementedError, a type of torch's own in C++
+    x = torch.Tensor._make_wrapper_subclass(Elsewhere, (2, 64), dtype=torch.bfloat16, device="vulkan")
+    with pytest.raises(NotImplementedError):
+        torch.empty((2, 64), device="vulkan")
+    with pytest.raises(NotImplementedError):
+        NATIVE["empties"](x, [(2, 64, False)])
+
+
 def test_the_module_has_no_thread_local_storage():
     import struct
 
