@@ -18,6 +18,7 @@
 #include <tuple>
 #include <type_traits>
 #include <utility>
+#include <vector>
 
 #include "../../include/tfmi.h"
 
@@ -129,6 +130,16 @@ PyObject* caught(F&& f) {
   }
 }
 
+// The interpreter's lock let go for a scope: an allocation may wait for the device, and other threads go on meanwhile, as under
+// torch's own functions.
+struct Released {
+  PyThreadState* state = PyEval_SaveThread();
+  Released() = default;
+  ~Released() { PyEval_RestoreThread(state); }
+  Released(const Released&) = delete;
+  Released& operator=(const Released&) = delete;
+};
+
 template <class... A>
 PyObject* call(int (*entry)(A...), PyObject* const* args, Py_ssize_t given) {
   return run(entry, args, given, std::index_sequence_for<A...>());
@@ -139,6 +150,19 @@ PyObject* call(int (*entry)(A...), PyObject* const* args, Py_ssize_t given) {
 TF_ENTRIES(TF_WRAP)
 #undef TF_WRAP
 
+PyObject* listed(at::Tensor* tensors, size_t count) {
+  PyObject* list = PyList_New(count);
+  for (size_t i = 0; list && i < count; ++i) {
+    PyObject* t = THPVariable_Wrap(std::move(tensors[i]));
+    if (!t) {
+      Py_DECREF(list);
+      return nullptr;
+    }
+    PyList_SET_ITEM(list, i, t);
+  }
+  return list;
+}
+
 // empties(x, [(rows, columns, fp32?), ...]): uninitialised contiguous tensors on x's device, of its type or fp32
 PyObject* empties(PyObject*, PyObject* const* args, Py_ssize_t given) {
   if (given != 2 || !THPVariable_Check(args[0]) || !PyList_Check(args[1])) {
@@ -148,27 +172,20 @@ PyObject* empties(PyObject*, PyObject* const* args, Py_ssize_t given) {
   return caught([&]() -> PyObject* {
     const auto same = at::TensorOptions().dtype(THPVariable_Unpack(args[0]).dtype()).device(THPVariable_Unpack(args[0]).device());
     const auto f32 = same.dtype(at::kFloat);
-    const Py_ssize_t n = PyList_GET_SIZE(args[1]);
-    PyObject* made = PyList_New(n);
-    if (!made) return nullptr;
-    for (Py_ssize_t i = 0; i < n; ++i) {
+    struct Size {
       long long rows, columns;
       int wide;
-      PyObject* t = nullptr;
-      try {
-        if (PyArg_ParseTuple(PyList_GET_ITEM(args[1], i), "LLp", &rows, &columns, &wide))
-          t = THPVariable_Wrap(at::empty({rows, columns}, wide ? f32 : same));
-      } catch (...) {
-        Py_DECREF(made);
-        throw;
-      }
-      if (!t) {
-        Py_DECREF(made);
-        return nullptr;
-      }
-      PyList_SET_ITEM(made, i, t);
+    };
+    std::vector<Size> sizes(PyList_GET_SIZE(args[1]));
+    for (size_t i = 0; i < sizes.size(); ++i)
+      if (!PyArg_ParseTuple(PyList_GET_ITEM(args[1], i), "LLp", &sizes[i].rows, &sizes[i].columns, &sizes[i].wide)) return nullptr;
+    std::vector<at::Tensor> made;
+    made.reserve(sizes.size());
+    {
+      const Released released;
+      for (const Size& s : sizes) made.push_back(at::empty({s.rows, s.columns}, s.wide ? f32 : same));
     }
-    return made;
+    return listed(made.data(), made.size());
   });
 }
 
@@ -231,12 +248,7 @@ at::Tensor made(const at::Tensor& x, int64_t rows, int64_t columns, bool f32) {
   return at::empty({rows, columns}, at::TensorOptions().dtype(f32 ? at::kFloat : at::kBFloat16).device(x.device()));
 }
 
-template <class... A>
-bool launched(int (*entry)(A...), A... args) {
-  int status;
-  Py_BEGIN_ALLOW_THREADS;
-  status = entry(args...);
-  Py_END_ALLOW_THREADS;
+bool launched(int status) {
   if (status) PyErr_SetString(PyExc_RuntimeError, library.tf_last_error());
   return !status;
 }
@@ -264,15 +276,20 @@ PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t given) {
     const int64_t m = x.size(0);
     const bool arrive = sk > 1 && m <= COUNTER_ROWS;
     if (sk < 1 || (arrive && !q.counters_ok())) Py_RETURN_NONE;
-    at::Tensor out = made(x, m, q.n, f32), part;
-    if (sk > 1) part = made(x, sk * m, q.n, true);
-    if (!launched(library.tf_qmm_own_sums, (const uint16_t*)bits(x), x.stride(0), (const uint32_t*)q.weight().data_ptr(),
-                  (const uint16_t*)bits(q.scales()), (const uint16_t*)bits(q.biases()), q.scales().stride(0), out.data_ptr(),
-                  sk > 1 ? (float*)part.data_ptr() : nullptr, arrive ? (int32_t*)q.counters().data_ptr() : nullptr,
-                  arrive ? (int)(q.counters().numel() / TF_QMM_COUNTER_STRIDE) : 0, (int)m, (int)q.n, (int)q.k, sk, (int)q.gs,
-                  row_tile(m), f32, 1, (tf_stream_t)PyLong_AsVoidPtr(args[4])))
-      return nullptr;
-    return THPVariable_Wrap(std::move(out));
+    const tf_stream_t stream = PyLong_AsVoidPtr(args[4]);
+    at::Tensor out, part;
+    int status;
+    {
+      const Released released;
+      out = made(x, m, q.n, f32);
+      if (sk > 1) part = made(x, sk * m, q.n, true);
+      status = library.tf_qmm_own_sums(bits(x), x.stride(0), (const uint32_t*)q.weight().data_ptr(), bits(q.scales()), bits(q.biases()),
+                                       q.scales().stride(0), out.data_ptr(), sk > 1 ? (float*)part.data_ptr() : nullptr,
+                                       arrive ? (int32_t*)q.counters().data_ptr() : nullptr,
+                                       arrive ? (int)(q.counters().numel() / TF_QMM_COUNTER_STRIDE) : 0, (int)m, (int)q.n, (int)q.k,
+                                       sk, (int)q.gs, row_tile(m), f32, 1, stream);
+    }
+    return launched(status) ? THPVariable_Wrap(std::move(out)) : nullptr;
   });
 }
 
@@ -284,12 +301,16 @@ PyObject* prefill_matmul(PyObject*, PyObject* const* args, Py_ssize_t given) {
     if (!q.ok || !ordinary_rows(args[0], q.k) || !q.scales().is_contiguous() || !q.biases().is_contiguous()) Py_RETURN_NONE;
     const at::Tensor& x = THPVariable_Unpack(args[0]);
     const int f32 = PyLong_AsLong(args[2]) != 0, tile = (int)PyLong_AsLong(args[3]);
-    at::Tensor out = made(x, x.size(0), q.n, f32);
-    if (!launched(library.tf_qmm_prefill, (const uint16_t*)bits(x), x.stride(0), (const uint32_t*)q.weight().data_ptr(),
-                  (const uint16_t*)bits(q.scales()), (const uint16_t*)bits(q.biases()), out.data_ptr(), (int)x.size(0), (int)q.n,
-                  (int)q.k, (int)q.gs, f32, tile, (int)q.arith, (tf_stream_t)PyLong_AsVoidPtr(args[4])))
-      return nullptr;
-    return THPVariable_Wrap(std::move(out));
+    const tf_stream_t stream = PyLong_AsVoidPtr(args[4]);
+    at::Tensor out;
+    int status;
+    {
+      const Released released;
+      out = made(x, x.size(0), q.n, f32);
+      status = library.tf_qmm_prefill(bits(x), x.stride(0), (const uint32_t*)q.weight().data_ptr(), bits(q.scales()), bits(q.biases()),
+                                      out.data_ptr(), (int)x.size(0), (int)q.n, (int)q.k, (int)q.gs, f32, tile, (int)q.arith, stream);
+    }
+    return launched(status) ? THPVariable_Wrap(std::move(out)) : nullptr;
   });
 }
 
@@ -325,34 +346,27 @@ PyObject* matmul_group(PyObject*, PyObject* const* args, Py_ssize_t given) {
     int32_t* counters[MOST];
     void* to[MOST];
     at::Tensor out[MOST], parts;
-    for (int i = 0; i < count; ++i) {
-      w[i] = (const uint32_t*)q[i]->weight().data_ptr(), s[i] = bits(q[i]->scales()), b[i] = bits(q[i]->biases());
-      stride[i] = q[i]->scales().stride(0);
-      out[i] = made(x, m, n[i], f32);
-      to[i] = out[i].data_ptr();
-      place[i] = own;                                        // the parts lie in one buffer, each on 256 bytes
-      if (sk[i] > 1) own += (sk[i] * m * n[i] + 63) / 64 * 64;
-      const bool arrive = sk[i] > 1 && m <= COUNTER_ROWS;
-      counters[i] = arrive ? (int32_t*)q[i]->counters().data_ptr() : nullptr;
-      n_counters[i] = arrive ? (int)(q[i]->counters().numel() / TF_QMM_COUNTER_STRIDE) : 0;
-    }
-    if (own) parts = made(x, 1, own, true);
-    for (int i = 0; i < count; ++i) part[i] = sk[i] > 1 ? (float*)parts.data_ptr() + place[i] : nullptr;
-    if (!launched(library.tf_qmm_group, (const uint16_t*)bits(x), x.stride(0), (const float*)xs.data_ptr(), count,
-                  (const uint32_t* const*)w, (const uint16_t* const*)s, (const uint16_t* const*)b, (const int64_t*)stride,
-                  (void* const*)to, (float* const*)part, (int32_t* const*)counters, (const int*)n_counters, (const int*)n,
-                  (const int*)sk, (int)m, (int)k, (int)gs, row_tile(m), f32, (tf_stream_t)PyLong_AsVoidPtr(args[5])))
-      return nullptr;
-    PyObject* list = PyList_New(count);
-    for (int i = 0; list && i < count; ++i) {
-      PyObject* t = THPVariable_Wrap(std::move(out[i]));
-      if (!t) {
-        Py_DECREF(list);
-        return nullptr;
+    const tf_stream_t stream = PyLong_AsVoidPtr(args[5]);
+    int status;
+    {
+      const Released released;
+      for (int i = 0; i < count; ++i) {
+        w[i] = (const uint32_t*)q[i]->weight().data_ptr(), s[i] = bits(q[i]->scales()), b[i] = bits(q[i]->biases());
+        stride[i] = q[i]->scales().stride(0);
+        out[i] = made(x, m, n[i], f32);
+        to[i] = out[i].data_ptr();
+        place[i] = own;                                      // the parts lie in one buffer, each on 256 bytes
+        if (sk[i] > 1) own += (sk[i] * m * n[i] + 63) / 64 * 64;
+        const bool arrive = sk[i] > 1 && m <= COUNTER_ROWS;
+        counters[i] = arrive ? (int32_t*)q[i]->counters().data_ptr() : nullptr;
+        n_counters[i] = arrive ? (int)(q[i]->counters().numel() / TF_QMM_COUNTER_STRIDE) : 0;
       }
-      PyList_SET_ITEM(list, i, t);
+      if (own) parts = made(x, 1, own, true);
+      for (int i = 0; i < count; ++i) part[i] = sk[i] > 1 ? (float*)parts.data_ptr() + place[i] : nullptr;
+      status = library.tf_qmm_group(bits(x), x.stride(0), (const float*)xs.data_ptr(), count, w, s, b, stride, to, part, counters,
+                                    n_counters, n, sk, (int)m, (int)k, (int)gs, row_tile(m), f32, stream);
     }
-    return list;
+    return launched(status) ? listed(out, count) : nullptr;
   });
 }
 
@@ -372,11 +386,17 @@ PyObject* add_rmsnorm(PyObject*, PyObject* const* args, Py_ssize_t given) {
       Py_RETURN_NONE;
     const int64_t rows = x.size(0), d = x.size(1);
     if (rows < 1 || rows > INT32_MAX || d < gs || d > 16384 || d % gs) Py_RETURN_NONE;
-    at::Tensor h = made(x, rows, d, false), y = made(x, rows, d, false), xs = made(x, rows, d / gs, true);
-    if (!launched(library.tf_add_norm, (const uint16_t*)bits(x), (const void*)r.data_ptr(), 1, (const float*)nullptr, 0, 0,
-                  (const uint16_t*)bits(w), (float)PyFloat_AS_DOUBLE(args[3]), bits(h), bits(y), (float*)xs.data_ptr(), (int)rows,
-                  (int)d, (int)gs, (tf_stream_t)PyLong_AsVoidPtr(args[5])))
-      return nullptr;
+    const tf_stream_t stream = PyLong_AsVoidPtr(args[5]);
+    const float eps = (float)PyFloat_AS_DOUBLE(args[3]);
+    at::Tensor h, y, xs;
+    int status;
+    {
+      const Released released;
+      h = made(x, rows, d, false), y = made(x, rows, d, false), xs = made(x, rows, d / gs, true);
+      status = library.tf_add_norm(bits(x), r.data_ptr(), 1, nullptr, 0, 0, bits(w), eps, bits(h), bits(y), (float*)xs.data_ptr(),
+                                   (int)rows, (int)d, (int)gs, stream);
+    }
+    if (!launched(status)) return nullptr;
     Owned a(THPVariable_Wrap(std::move(h))), b(THPVariable_Wrap(std::move(y))), c(THPVariable_Wrap(std::move(xs)));
     if (!a.o || !b.o || !c.o) return nullptr;
     return PyTuple_Pack(3, a.o, b.o, c.o);

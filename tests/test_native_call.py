@@ -1,6 +1,8 @@
 """The entry points as Python functions (csrc/call.cpp) against ctypes: the same names, argument counts, values and sentences,
 without a GPU (what the library refuses before it launches)."""
 
+import shutil
+
 import pytest
 import torch
 
@@ -90,6 +92,44 @@ def test_what_an_allocation_raises_keeps_its_type():
         torch.empty((2, 64), device="vulkan")
     with pytest.raises(NotImplementedError):
         NATIVE["empties"](x, [(2, 64, False)])
+
+
+WATCH = """
+#include <Python.h>
+#include <c10/core/CPUAllocator.h>
+struct Watch : c10::Allocator {
+  c10::Allocator* inner = c10::GetCPUAllocator();
+  int held = 0, calls = 0;
+  c10::DataPtr allocate(size_t n) override { return ++calls, held += PyGILState_Check(), inner->allocate(n); }
+  void copy_data(void* to, const void* from, size_t n) const override { inner->copy_data(to, from, n); }
+};
+static Watch watch;
+extern "C" void begin() { c10::SetCPUAllocator(&watch, 100); }
+extern "C" int calls() { return watch.calls; }
+extern "C" int held() { c10::SetCPUAllocator(watch.inner, 100); return watch.held; }
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no C++ compiler")
+def test_other_threads_go_on_while_memory_is_allocated(tmp_path):
+    import ctypes
+    import subprocess
+    import sysconfig
+    from pathlib import Path
+
+    root = Path(torch.__file__).parent
+    (tmp_path / "watch.cpp").write_text(WATCH)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+                    f"-I{sysconfig.get_paths()['include']}", f"-I{root / 'include'}", str(tmp_path / "watch.cpp"), "-o",
+                    str(tmp_path / "watch.so"), f"-L{root / 'lib'}", "-lc10"], check=True, capture_output=True)
+    watch, x = ctypes.PyDLL(str(tmp_path / "watch.so")), torch.zeros((2, 64), dtype=torch.bfloat16)
+    watch.begin()
+    try:
+        made = NATIVE["empties"](x, [(3, 64, False), (2, 5, True)])
+        calls = watch.calls()
+    finally:
+        held = watch.held()
+    assert len(made) == calls == 2 and held == 0
 
 
 def test_the_module_has_no_thread_local_storage():
