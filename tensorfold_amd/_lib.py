@@ -185,9 +185,11 @@ def call(name: str, *args) -> None:
         entry(*args, stream())
         return
     so, kinds = _other or lib(), TABLES.get(name, {})
-    plain = lambda a: a.data_ptr() if isinstance(a, torch.Tensor) else a
-    args = [(kinds[i] * len(a))(*map(plain, a)) if i in kinds and isinstance(a, list) else plain(a) for i, a in enumerate(args)]
-    if getattr(so, name)(*args, stream()):
+    # (a tensor of one number may stand for a whole number: only where a pointer belongs is it an address)
+    plain = lambda a, kind: a.data_ptr() if kind is P and isinstance(a, torch.Tensor) else a
+    args = [(kinds[i] * len(a))(*(plain(t, kinds[i]) for t in a)) if i in kinds and isinstance(a, list) else plain(a, kind)
+            for i, (a, kind) in enumerate(zip((*args, stream()), PROTOTYPES[name], strict=True))]
+    if getattr(so, name)(*args):
         raise RuntimeError(so.tf_last_error().decode())
 
 

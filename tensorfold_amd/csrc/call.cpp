@@ -1,7 +1,7 @@
 // The launching entry points of include/tfmi.h as Python functions, for _lib.call: the arguments go from the interpreter to the
 // library without ctypes, which converted each of a launch's 8 to 24 through an object of its own (2 to 3 us a launch; the decode
-// layer of one row and the norm with q, k and v are bound by the host).  A pointer is a tensor, a whole number or None, a table of
-// them a list.  Raises what ctypes' caller raised: RuntimeError with the library's sentence; and what torch raises for the results that
+// layer of one row and the norm with q, k and v are bound by the host).  A pointer is a tensor, an int or None, a table of
+// them a list, a whole number whatever has an __index__.  Raises what ctypes' caller raised: RuntimeError with the library's sentence; and what torch raises for the results that
 // are made here: torch.OutOfMemoryError where a device is full.
 
 #define PY_SSIZE_T_CLEAN
@@ -53,10 +53,14 @@ struct Tables {
   int used = 0;
 };
 
+// whatever stands for a whole number (an int, numpy's, a tensor's one), as ctypes takes it
 uint64_t whole(PyObject* o) {
   if (PyLong_Check(o)) return PyLong_AsUnsignedLongLongMask(o);
-  PyErr_SetString(PyExc_TypeError, "expected a whole number");
-  return 0;
+  PyObject* index = PyNumber_Index(o);
+  if (!index) return 0;
+  const uint64_t value = PyLong_AsUnsignedLongLongMask(index);
+  Py_DECREF(index);
+  return value;
 }
 
 uint64_t address(PyObject* o) {

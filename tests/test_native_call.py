@@ -3,6 +3,7 @@ without a GPU (what the library refuses before it launches)."""
 
 import shutil
 
+import numpy as np
 import pytest
 import torch
 
@@ -39,6 +40,19 @@ def test_values_arrive_as_ctypes_passes_them():
     # 64-bit strides, a float among the whole numbers, the last of many arguments
     assert "exceed the grid limit" in sentence("tf_experts_prefill", 64, 1, x, 1 << 40, 0, x, 1, 1, x, x, x, x, 32, 0.5, 1 << 40,
                                                64, 0, None)
+
+
+@pytest.mark.parametrize("number", [np.int32, np.int64, np.uint16, torch.tensor])
+@pytest.mark.parametrize("native", [True, False])
+def test_whole_numbers_of_other_types_are_taken_as_ctypes_takes_them(monkeypatch, number, native):
+    monkeypatch.setattr(_lib, "_native", NATIVE if native else {})
+    monkeypatch.setattr(_lib, "stream", lambda: 0)
+    x, w = torch.zeros((2, 64), dtype=torch.bfloat16), torch.zeros((64,), dtype=torch.int32)
+    with pytest.raises(RuntimeError, match="not 48"):
+        _lib.call("tf_group_sums", x, number(64), number(2), number(64), number(48), x)
+    with pytest.raises(RuntimeError, match="whole groups a slice"):
+        _lib.call("tf_qmm_group", x, 64, x, 1, [w], [w], [w], [number(128)], [w], [None], [None], [number(0)], [number(64)], [number(3)],
+                  number(2), number(64), 64, 16, 0)
 
 
 def test_tables_are_lists():
