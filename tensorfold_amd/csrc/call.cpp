@@ -260,10 +260,19 @@ bool launched(int status) {
 int row_tile(int64_t m) { return m <= 16 ? 16 : m <= 32 ? 32 : 64; }
 uint16_t* bits(const at::Tensor& t) { return static_cast<uint16_t*>(t.data_ptr()); }
 
+// an int that a C int holds: what does not fit one is not cut down to it here
+bool small(PyObject* o) {
+  int over = 0;
+  if (!PyLong_Check(o)) return false;
+  const long value = PyLong_AsLongAndOverflow(o, &over);
+  return !over && value >= INT32_MIN && value <= INT32_MAX;
+}
+
+// args[first ..]: small numbers, and the stream last
 bool numbers(PyObject* const* args, Py_ssize_t given, Py_ssize_t wanted, Py_ssize_t first) {
-  if (!library.tf_last_error || given != wanted) return false;
-  for (Py_ssize_t i = first; i < given; ++i)
-    if (!PyLong_Check(args[i])) return false;
+  if (!library.tf_last_error || given != wanted || !PyLong_Check(args[given - 1])) return false;
+  for (Py_ssize_t i = first; i < given - 1; ++i)
+    if (!small(args[i])) return false;
   return true;
 }
 
@@ -329,8 +338,7 @@ PyObject* matmul_group(PyObject*, PyObject* const* args, Py_ssize_t given) {
     int sk[MOST], n[MOST], n_counters[MOST];
     for (int i = 0; i < count; ++i) {
       q[i].emplace(PyList_GET_ITEM(args[2], i));
-      if (!q[i]->ok || q[i]->k != q[0]->k || q[i]->gs != q[0]->gs || !q[i]->counters_ok() ||
-          !PyLong_Check(PyList_GET_ITEM(args[3], i)))
+      if (!q[i]->ok || q[i]->k != q[0]->k || q[i]->gs != q[0]->gs || !q[i]->counters_ok() || !small(PyList_GET_ITEM(args[3], i)))
         Py_RETURN_NONE;
       sk[i] = (int)PyLong_AsLong(PyList_GET_ITEM(args[3], i)), n[i] = (int)q[i]->n;
       if (sk[i] < 1) Py_RETURN_NONE;

@@ -122,3 +122,15 @@ def test_a_full_device_raises_torch_s_own_error():
         _lib.empties(x, [(1 << 20, 1 << 30, True)])
     with pytest.raises(torch.OutOfMemoryError):
         qmm.matmul(x, weight(130, 64, 64), sk=1 << 30)
+
+
+def test_numbers_past_32_bits_are_not_cut_down():
+    q, x = weight(130, 512, 64), synthetic.activations(3, 512, 1).to(DEV)
+    for sk in (2 ** 32 + 1, 2 ** 32 + 2):
+        assert _lib.whole("matmul", x, q, sk, False) is None
+        with pytest.raises(RuntimeError):                                  # a workspace of some terabytes, refused
+            qmm.matmul(x, q, sk=sk)
+    r, w = synthetic.activations(3, 512, 2).to(DEV), synthetic.activations(1, 512, 3).to(DEV)[0].contiguous()
+    for gs in (2 ** 32 + 64, 2 ** 70):
+        with pytest.raises(ValueError, match="whole groups"):
+            glue.add_rmsnorm(x, r, w, 1e-6, gs)

@@ -108,6 +108,12 @@ def test_what_an_allocation_raises_keeps_its_type():
         NATIVE["empties"](x, [(2, 64, False)])
 
 
+@pytest.mark.parametrize("gs", [2 ** 70, -2 ** 70, 2 ** 40])
+def test_a_whole_call_leaves_numbers_past_32_bits_to_the_general_way(gs):
+    x, w = torch.zeros((2, 64), dtype=torch.bfloat16), torch.zeros((64,), dtype=torch.bfloat16)
+    assert NATIVE["add_rmsnorm"](x, x, w, 1e-6, gs, 0) is None
+
+
 WATCH = """
 #include <Python.h>
 #include <c10/core/CPUAllocator.h>
