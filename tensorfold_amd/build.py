@@ -7,10 +7,13 @@ time, in the tree, for the one target this package supports, and a GPU that is n
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import os
 import shutil
 import subprocess
 import sys
+import tempfile
 from functools import lru_cache
 from pathlib import Path
 
@@ -73,6 +76,17 @@ def built_id(path: Path = LIB, mark: bytes = b"TFMI_BUILD_ID=") -> str | None:
     return None if at < 0 else blob[at + len(mark):at + len(mark) + 16].decode(errors="replace")
 
 
+@contextlib.contextmanager
+def beside(target: Path):
+    """Where to write ``target``'s next version: it takes the old one's place in one step at the block's end, so that other
+    processes (ranks that find it out of date all build it) load the whole old file or the whole new one."""
+
+    with tempfile.TemporaryDirectory(dir=target.parent, prefix=".tfmi-build-") as tmp:
+        made = Path(tmp) / target.name
+        yield made
+        os.replace(made, target)
+
+
 def stale() -> bool:
     """Whether the library is missing or was built from other sources than the ones beside it."""
 
@@ -99,7 +113,6 @@ def compile(verbose: bool = False, timeline: bool = False) -> Path:
     side by side, then a link.  ``timeline``: the same sources with -DTF_TIMELINE into ``libtfmi_timeline.so``, whose
     decode expert kernels note per-workgroup timestamps (an instrument: only ``timeline_lib`` builds it)."""
 
-    import tempfile
     from concurrent.futures import ThreadPoolExecutor
 
     cc = hipcc()
@@ -124,7 +137,8 @@ def compile(verbose: bool = False, timeline: bool = False) -> Path:
         with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
             logs = list(pool.map(lambda so: run([cc, *compile_flags, "-c", str(CSRC / so[0]), "-o", so[1]]),
                                  zip(SOURCES, objects)))
-        logs.append(run([cc, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", str(target), *objects]))
+        with beside(target) as made:
+            logs.append(run([cc, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", str(made), *objects]))
     if verbose:
         for text in logs:
             if text:
@@ -144,13 +158,14 @@ def compile_call() -> Path | None:
     cc, python, root = shutil.which("g++") or shutil.which("c++"), Path(sysconfig.get_paths()["include"]), Path(torch.__file__).parent
     if cc is None or not (python / "Python.h").exists() or not (root / "include/torch/csrc/autograd/python_variable.h").exists():
         return None
-    done = subprocess.run([cc, *CALL_FLAGS, f"-I{python}",
-                           f"-I{root / 'include'}", f"-I{root / 'include/torch/csrc/api/include'}",
-                           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DTF_CALL_ID="{call_id()}"',
-                           str(CSRC / "call.cpp"), "-o", str(CALL_LIB), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu",
-                           "-lc10", "-ldl"], capture_output=True, text=True)
-    if done.returncode:
-        raise RuntimeError(f"tensorfold-amd: {cc} failed:\n{done.stderr}")
+    with beside(CALL_LIB) as made:
+        done = subprocess.run([cc, *CALL_FLAGS, f"-I{python}",
+                               f"-I{root / 'include'}", f"-I{root / 'include/torch/csrc/api/include'}",
+                               f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DTF_CALL_ID="{call_id()}"',
+                               str(CSRC / "call.cpp"), "-o", str(made), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu",
+                               "-lc10", "-ldl"], capture_output=True, text=True)
+        if done.returncode:
+            raise RuntimeError(f"tensorfold-amd: {cc} failed:\n{done.stderr}")
     return CALL_LIB
 
 
