@@ -130,7 +130,7 @@ _native: dict | None = None          # entry point -> its Python function of csr
 
 
 def _bound() -> dict:
-    """The functions of ``tfmi_call.so``, bound to the library that ``lib`` has loaded."""
+    """The functions of ``tfmi_call.so``, bound to the library that ``lib`` has loaded; none where it cannot be had."""
 
     from importlib.machinery import ExtensionFileLoader
     from importlib.util import module_from_spec, spec_from_loader
@@ -139,9 +139,13 @@ def _bound() -> dict:
     if path is None:
         return {}
     loader = ExtensionFileLoader("tfmi_call", str(path))
-    module = module_from_spec(spec_from_loader("tfmi_call", loader))
-    loader.exec_module(module)
-    module.bind(str(build.LIB))
+    try:
+        module = module_from_spec(spec_from_loader("tfmi_call", loader))
+        loader.exec_module(module)
+        module.bind(str(build.LIB))
+    except (ImportError, RuntimeError) as e:          # not loadable here: the kernels do not need it
+        build.say(f"{e}: launches go through ctypes, a few microseconds slower")
+        return {}
     return {name: getattr(module, name) for name in (*PROTOTYPES, "empties", *WHOLE) if hasattr(module, name)}
 
 

@@ -143,8 +143,8 @@ def compile(verbose: bool = False, timeline: bool = False) -> Path:
         for text in logs:
             if text:
                 say(text)
-    if not timeline and compile_call() is None:
-        say("no C++ compiler, Python headers or torch headers: launches go through ctypes")
+    if not timeline:
+        _try_call()
     return target
 
 
@@ -169,13 +169,26 @@ def compile_call() -> Path | None:
     return CALL_LIB
 
 
+def _try_call() -> Path | None:
+    """``compile_call`` where a failure (a compiler that cannot, a folder that is not written to) is said and not raised: the
+    kernels do not need this library."""
+
+    try:
+        made, why = compile_call(), "no C++ compiler, Python headers or torch headers"
+    except (RuntimeError, OSError) as e:
+        made, why = None, str(e)
+    if made is None:
+        say(f"{why}: launches go through ctypes, a few microseconds slower")
+    return made
+
+
 def call_lib() -> Path | None:
     """``tfmi_call.so`` for the sources beside it, built first if it is missing or out of date; None where it cannot be
     (``_lib.call`` then goes through ctypes: the same launches, a few microseconds later)."""
 
     if not (CSRC / "call.cpp").exists():
         return CALL_LIB if CALL_LIB.exists() else None
-    return CALL_LIB if built_id(CALL_LIB, b"TFMI_CALL_ID=") == call_id() else compile_call()
+    return CALL_LIB if built_id(CALL_LIB, b"TFMI_CALL_ID=") == call_id() else _try_call()
 
 
 @lru_cache(maxsize=1)

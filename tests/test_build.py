@@ -5,7 +5,7 @@ from pathlib import Path
 
 import pytest
 
-from tensorfold_amd import build
+from tensorfold_amd import _lib, build
 
 
 @pytest.fixture
@@ -24,7 +24,7 @@ def tree(tmp_path, monkeypatch):
             output.write_bytes(b"new")
         return subprocess.CompletedProcess(cmd, Tree.status, "", "no such luck")
 
-    Tree.ran = []
+    _lib.lib()                                               # the built kernels, as the calls below find them
     for path in (Tree.kernels, Tree.call):
         path.write_bytes(b"old")
     monkeypatch.setattr(build, "LIB", Tree.kernels)
@@ -47,3 +47,47 @@ def test_a_library_takes_its_place_whole(tree):
     with pytest.raises(RuntimeError, match="no such luck"):
         build.compile_call()
     assert tree.call.read_bytes() == b"new" and {p.name for p in tree.call.parent.iterdir()} == {"libtfmi.so", "tfmi_call.so"}
+
+
+def _says(capfd, *texts):
+    err = capfd.readouterr().err
+    return all(t in err for t in (*texts, "launches go through ctypes")) and err.count("ctypes") == 1
+
+
+def test_without_a_call_library_launches_go_through_ctypes(tree, monkeypatch, capfd):
+    """A compiler that fails, a folder that is not there to write to, a file that does not load: said once, and the kernels
+    run."""
+
+    monkeypatch.setattr(_lib, "_ready", lambda: True)
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.setattr(_lib, "stream", lambda: 0)
+    x = __import__("torch").zeros((2, 64)).bfloat16()
+
+    def refused():
+        for _ in range(2):
+            with pytest.raises(RuntimeError, match="not 48"):
+                _lib.call("tf_group_sums", x, 64, 2, 64, 48, x)
+        assert _lib._native == {}
+        _lib._native = None
+
+    tree.status = 1
+    refused()
+    assert len(tree.ran) == 1 and _says(capfd, "no such luck") and tree.call.read_bytes() == b"old"
+    tree.status = 0
+    refused()                                                # "new" is no library
+    assert tree.call.read_bytes() == b"new" and _says(capfd, "tfmi_call.so")
+    monkeypatch.setattr(build, "CALL_LIB", tree.call / "below" / "tfmi_call.so")
+    refused()
+    assert _says(capfd, "Not a directory")
+    monkeypatch.setattr(build.shutil, "which", lambda name: None)
+    refused()
+    assert _says(capfd, "no C++ compiler")
+
+
+def test_a_build_of_the_kernels_does_without_it(tree, capfd):
+    def run(output):
+        tree.status = int(output.name == "tfmi_call.so")
+
+    tree.during = run
+    assert build.compile() == tree.kernels and tree.kernels.read_bytes() == b"new" and tree.call.read_bytes() == b"old"
+    assert _says(capfd, "no such luck")
