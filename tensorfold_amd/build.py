@@ -53,14 +53,22 @@ def source_id() -> str:
     return h.hexdigest()[:16]
 
 
-def call_id() -> str:
-    """16 hex digits over what ``tfmi_call.so`` is built from and for."""
+def call_for() -> str:
+    """16 hex digits over what ``tfmi_call.so`` is built for: another Python or torch may lay out its objects otherwise."""
 
     import hashlib
 
     import torch
 
-    h = hashlib.sha256(f"{sys.version} {torch.__version__} {CALL_FLAGS}".encode())
+    return hashlib.sha256(f"{sys.version} {torch.__version__}".encode()).hexdigest()[:16]
+
+
+def call_id() -> str:
+    """16 hex digits over what ``tfmi_call.so`` is built from and for."""
+
+    import hashlib
+
+    h = hashlib.sha256(f"{call_for()} {CALL_FLAGS}".encode())
     for path in (CSRC / "call.cpp", HERE.parent / "include" / "tfmi.h"):
         h.update(path.read_bytes())
     return h.hexdigest()[:16]
@@ -162,6 +170,7 @@ def compile_call() -> Path | None:
         done = subprocess.run([cc, *CALL_FLAGS, f"-I{python}",
                                f"-I{root / 'include'}", f"-I{root / 'include/torch/csrc/api/include'}",
                                f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DTF_CALL_ID="{call_id()}"',
+                               f'-DTF_CALL_FOR="{call_for()}"',
                                str(CSRC / "call.cpp"), "-o", str(made), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu",
                                "-lc10", "-ldl"], capture_output=True, text=True)
         if done.returncode:
@@ -186,8 +195,8 @@ def call_lib() -> Path | None:
     """``tfmi_call.so`` for the sources beside it, built first if it is missing or out of date; None where it cannot be
     (``_lib.call`` then goes through ctypes: the same launches, a few microseconds later)."""
 
-    if not (CSRC / "call.cpp").exists():
-        return CALL_LIB if CALL_LIB.exists() else None
+    if not (CSRC / "call.cpp").exists():          # shipped without its sources: taken where it was built for this Python and torch
+        return CALL_LIB if built_id(CALL_LIB, b"TFMI_CALL_FOR=") == call_for() else None
     return CALL_LIB if built_id(CALL_LIB, b"TFMI_CALL_ID=") == call_id() else _try_call()
 
 

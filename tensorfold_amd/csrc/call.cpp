@@ -25,6 +25,9 @@
 #ifndef TF_CALL_ID
 #define TF_CALL_ID "unknown"
 #endif
+#ifndef TF_CALL_FOR
+#define TF_CALL_FOR "unknown"
+#endif
 
 namespace {
 
@@ -454,6 +457,6 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "tfmi_call", nullptr, -1, methods, 
 
 }  // namespace
 
-extern "C" __attribute__((used)) const char tf_call_id[] = "TFMI_CALL_ID=" TF_CALL_ID;
+extern "C" __attribute__((used)) const char tf_call_id[] = "TFMI_CALL_ID=" TF_CALL_ID " TFMI_CALL_FOR=" TF_CALL_FOR;
 
 PyMODINIT_FUNC PyInit_tfmi_call() { return PyModule_Create(&module); }

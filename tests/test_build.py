@@ -91,3 +91,18 @@ def test_a_build_of_the_kernels_does_without_it(tree, capfd):
     tree.during = run
     assert build.compile() == tree.kernels and tree.kernels.read_bytes() == b"new" and tree.call.read_bytes() == b"old"
     assert _says(capfd, "no such luck")
+
+
+def test_a_call_library_without_sources_is_taken_for_its_python_and_torch_alone(tree, monkeypatch):
+    monkeypatch.setattr(build, "CSRC", tree.call.parent)
+    for text, taken in ((b"TFMI_CALL_ID=0123456789abcdef TFMI_CALL_FOR=" + build.call_for().encode(), tree.call),
+                        (b"TFMI_CALL_ID=0123456789abcdef TFMI_CALL_FOR=0123456789abcdef", None), (b"an older build's", None)):
+        tree.call.write_bytes(text)
+        assert build.call_lib() == taken and not tree.ran
+
+
+def test_the_built_call_library_names_both():
+    if build.call_lib() is None:
+        pytest.skip("no C++ compiler, Python headers or torch headers")
+    assert build.built_id(build.CALL_LIB, b"TFMI_CALL_ID=") == build.call_id()
+    assert build.built_id(build.CALL_LIB, b"TFMI_CALL_FOR=") == build.call_for()
