@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import threading
 from ctypes import c_float, c_int, c_int64, c_void_p
 from functools import lru_cache
 from pathlib import Path
@@ -149,11 +150,18 @@ def _bound() -> dict:
     return {name: getattr(module, name) for name in (*PROTOTYPES, "empties", *WHOLE) if hasattr(module, name)}
 
 
+_starting = threading.Lock()
+
+
 def _start() -> dict:
+    """The first call's part: the device looked at and the native functions bound, once whatever threads ask."""
+
     global _native
-    _ready()
-    _native = _bound()
-    return _native
+    with _starting:
+        if _native is None:
+            _ready()
+            _native = _bound()
+        return _native
 
 
 def empties(x: torch.Tensor, sizes: list[tuple[int, int, bool]]) -> list[torch.Tensor]:

@@ -159,3 +159,20 @@ def test_the_module_has_no_thread_local_storage():
     at, size, count = struct.unpack_from("<Q", image, 0x20)[0], *struct.unpack_from("<HH", image, 0x36)          # ELF64 program headers
     kinds = [struct.unpack_from("<I", image, at + i * size)[0] for i in range(count)]
     assert 1 in kinds and 7 not in kinds          # PT_LOAD, PT_TLS
+
+
+def test_threads_that_start_together_bind_it_once(monkeypatch):
+    import threading
+    import time
+
+    bound = []
+    monkeypatch.setattr(_lib, "_ready", lambda: True)
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.setattr(_lib, "_bound", lambda: (bound.append(1), time.sleep(0.05), dict(NATIVE))[2])
+    got = []
+    threads = [threading.Thread(target=lambda: got.append(_lib._start())) for _ in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(bound) == 1 and len(got) == 6 and all(g is got[0] for g in got)
