@@ -165,10 +165,11 @@ def _start() -> dict:
 
 
 def empties(x: torch.Tensor, sizes: list[tuple[int, int, bool]]) -> list[torch.Tensor]:
-    """Uninitialised tensors [rows, columns] on x's device, of its type or fp32, one for each (rows, columns, fp32?)."""
+    """Uninitialised tensors [rows, columns] on x's device, of its type or fp32, one for each (rows, columns, fp32?); of
+    x's class where that is a subclass."""
 
     make = (_native if _native is not None else _start()).get("empties")
-    if make is not None:
+    if make is not None and type(x) in (torch.Tensor, torch.nn.Parameter):
         return make(x, sizes)
     return [x.new_empty((r, c), dtype=torch.float32) if wide else x.new_empty((r, c)) for r, c, wide in sizes]
 

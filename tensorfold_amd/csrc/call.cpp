@@ -243,9 +243,9 @@ struct Weight {
   const at::Tensor& counters() const { return THPVariable_Unpack(c.o); }
 };
 
-// x: bf16 [m, k] on the GPU in rows the kernels read as they lie
+// x: bf16 [m, k] on the GPU in rows the kernels read as they lie (a subclass's results are of its type: torch makes those)
 bool ordinary_rows(PyObject* o, long k) {
-  if (!THPVariable_Check(o)) return false;
+  if (!THPVariable_CheckExact(o)) return false;
   const at::Tensor& x = THPVariable_Unpack(o);
   return x.dim() == 2 && x.scalar_type() == at::kBFloat16 && x.is_cuda() && x.size(1) == k && x.size(0) >= 1 &&
          x.size(0) <= INT32_MAX && x.stride(1) == 1 && (uintptr_t)x.data_ptr() % 16 == 0 && (x.size(0) == 1 || x.stride(0) % 8 == 0);
@@ -388,7 +388,7 @@ PyObject* matmul_group(PyObject*, PyObject* const* args, Py_ssize_t given) {
 // add_rmsnorm(x, r, w, eps, gs, stream) with a residual
 PyObject* add_rmsnorm(PyObject*, PyObject* const* args, Py_ssize_t given) {
   return caught([&]() -> PyObject* {
-    if (!numbers(args, given, 6, 4) || !PyFloat_Check(args[3]) || !THPVariable_Check(args[0]) || !THPVariable_Check(args[1]) ||
+    if (!numbers(args, given, 6, 4) || !PyFloat_Check(args[3]) || !THPVariable_CheckExact(args[0]) || !THPVariable_Check(args[1]) ||
         !THPVariable_Check(args[2]))
       Py_RETURN_NONE;
     const at::Tensor &x = THPVariable_Unpack(args[0]), &r = THPVariable_Unpack(args[1]), &w = THPVariable_Unpack(args[2]);

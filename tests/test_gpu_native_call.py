@@ -97,6 +97,19 @@ def test_what_is_not_ordinary_goes_the_general_way(general):
         qmm.matmul(x, q, sk=3)
 
 
+def test_results_of_a_subclass_are_of_its_class():
+    class Named(torch.Tensor):
+        pass
+
+    qs, x = [weight(130, 512, 64), weight(64, 512, 64)], synthetic.activations(3, 512, 1).to(DEV)
+    r, w = synthetic.activations(3, 512, 2).to(DEV), synthetic.activations(1, 512, 3).to(DEV)[0].contiguous()
+    named, xs = x.as_subclass(Named), qmm.group_sums(x, 64)
+    for f in (lambda t: [qmm.matmul(t, qs[0])], lambda t: [qmm.prefill_matmul(t, qs[0])], lambda t: qmm.matmul_group(t, qs, xs),
+              lambda t: list(glue.add_rmsnorm(t, r, w, 1e-6))[:2]):
+        for got, want in zip(f(named), f(x), strict=True):
+            assert type(got) is Named and type(want) is torch.Tensor and torch.equal(got.as_subclass(torch.Tensor), want)
+
+
 def test_under_capture_and_on_another_stream():
     q, x = weight(640, 2048, 64), synthetic.activations(3, 2048, 4).to(DEV)
     want = qmm.matmul(x, q)

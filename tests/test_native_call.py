@@ -87,6 +87,17 @@ def test_empties():
             NATIVE["empties"](*bad)
 
 
+def test_results_of_a_subclass_are_of_its_class(monkeypatch):
+    class Named(torch.Tensor):
+        pass
+
+    monkeypatch.setattr(_lib, "_native", NATIVE)
+    x = torch.zeros((2, 64), dtype=torch.bfloat16)
+    for given, kind in ((x, torch.Tensor), (torch.nn.Parameter(x), torch.Tensor), (x.as_subclass(Named), Named)):
+        for made, dtype in zip(_lib.empties(given, [(3, 5, False), (2, 7, True)]), (torch.bfloat16, torch.float32)):
+            assert type(made) is kind and made.dtype == dtype and not made.requires_grad
+
+
 def test_a_tensor_without_storage_raises():
     meta = torch.empty((2, 64), dtype=torch.bfloat16, device="meta")
     x = torch.zeros((2, 64), dtype=torch.bfloat16)
