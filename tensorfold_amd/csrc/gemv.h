@@ -40,31 +40,6 @@ constexpr int SLICES = 16;      // K slices of the expert GEMV
 constexpr int DEPTH = 2;        // groups of weights a wave keeps in flight
 constexpr int RBMAX = 2;        // rows a pass
 
-// fp32 sums of each group of GS inputs of `rows` rows, for groups [0, KG), into xs[r * KG + g].
-// LPG lanes share a group (8 inputs each, in order), then a fixed xor tree over them.
-template <int GS>
-__device__ __forceinline__ void group_sums_block(const uint16_t* const* xrow, int rows, int KG, float* xs, int tid,
-                                                 int threads) {
-  constexpr int LPG = GS / 8;
-  const int part = tid % LPG;
-  for (int r = 0; r < rows; ++r) {
-    for (int g = tid / LPG; g < KG; g += threads / LPG) {
-      const uint4 v = *reinterpret_cast<const uint4*>(xrow[r] + (size_t)g * GS + part * 8);
-      float s = bf16_lo(v.x);
-      s += bf16_hi(v.x);
-      s += bf16_lo(v.y);
-      s += bf16_hi(v.y);
-      s += bf16_lo(v.z);
-      s += bf16_hi(v.z);
-      s += bf16_lo(v.w);
-      s += bf16_hi(v.w);
-#pragma unroll
-      for (int m = 1; m < LPG; m <<= 1) s += __shfl_xor(s, m);
-      if (part == 0) xs[r * KG + g] = s;
-    }
-  }
-}
-
 // dot2c with its first operand taken from lane J of the reader's row of 16 lanes
 template <int J>
 __device__ __forceinline__ float dot2_bcast(float acc, uint32_t x, uint32_t q) {
