@@ -451,8 +451,11 @@ __global__ void __launch_bounds__(256)
   *reinterpret_cast<uint32_t*>(out + (size_t)r * D + d) = pack_bf16(a0, a1);
 }
 
-// 16-bit pair outputs, eight columns a thread (16-byte loads), rows side by side in a workgroup: 4,096 rows x 11 x 2048 36.2 us
-// with two columns a thread, 35.1 so (5.3 TB/s); 2,000 x 9 x 1024 11.2, 7.5; 777 x 8 x 2688 7.5, 5.9
+// 16-bit pair outputs, eight columns a thread (16-byte loads), rows side by side in a workgroup, eight slots a trip to memory and
+// then what is left of them: 4,096 rows x 11 x 2048 36.3 us with two columns a thread, 33.0 so (5.7 TB/s); 2,000 x 9 x 1024 10.6, 5.9;
+// 777 x 8 x 2688 7.0, 5.2.  A trip's loads are as many as it has slots and none waits for another: with eight in any case, the last slot
+// again for those that are not there, the compiler put a slot's loads behind the question whether there is such a slot, and few
+// rows were slower than two columns a thread (bf16, 261 x 11 x 1024 4.6 us, 3.2 with two columns, 3.2 so; 456 x 11 x 1216 5.7, 4.9, 3.8).
 template <int YKIND>
 __global__ void __launch_bounds__(256)
     combine8_kernel(const uint16_t* __restrict__ Y, const float* __restrict__ Wt, uint16_t* __restrict__ out, int rows, int S,
@@ -463,35 +466,44 @@ __global__ void __launch_bounds__(256)
   const int D = D8 * 8, d = (int)(t - r * D8) * 8;
   const uint16_t* y = Y + (size_t)r * S * D + d;
   float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < S; k0 += 8) {
-    float w[8];
-    u32x4_t v[8];
+  // N slots from k0 on
+  auto take = [&](int k0, auto N) __attribute__((always_inline)) {
+    float w[N];
+    u32x4_t v[N];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int k = k0 + j < S ? k0 + j : S - 1;
-      w[j] = Wt[(size_t)r * S + k];
-      v[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(y + (size_t)k * D));
+    for (int j = 0; j < N; ++j) {
+      w[j] = Wt[(size_t)r * S + k0 + j];
+      v[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(y + (size_t)(k0 + j) * D));
     }
+    // (nothing is converted before all of them are on their way)
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (k0 + j < S) {
+    for (int j = 0; j < N; ++j) asm volatile("" : "+v"(w[j]), "+v"(v[j]));
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float lo, hi;
-          if (YKIND == 1) {
-            lo = bf16_lo(v[j][i]);
-            hi = bf16_hi(v[j][i]);
-          } else {
-            typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-            const uint32_t u = v[j][i];
-            const half2_t h = __builtin_bit_cast(half2_t, u);
-            lo = (float)h[0];
-            hi = (float)h[1];
-          }
-          a[2 * i] = fmaf(w[j], lo, a[2 * i]);
-          a[2 * i + 1] = fmaf(w[j], hi, a[2 * i + 1]);
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float lo, hi;
+        if (YKIND == 1) {
+          lo = bf16_lo(v[j][i]);
+          hi = bf16_hi(v[j][i]);
+        } else {
+          typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+          const uint32_t u = v[j][i];
+          const half2_t h = __builtin_bit_cast(half2_t, u);
+          lo = (float)h[0];
+          hi = (float)h[1];
         }
+        a[2 * i] = fmaf(w[j], lo, a[2 * i]);
+        a[2 * i + 1] = fmaf(w[j], hi, a[2 * i + 1]);
       }
+  };
+  int k0 = 0;
+  for (; k0 + 8 <= S; k0 += 8) take(k0, std::integral_constant<int, 8>());
+  switch (S - k0) {
+#define TF_SLOTS(N_) \
+  case N_: take(k0, std::integral_constant<int, N_>()); break;
+    TF_SLOTS(1) TF_SLOTS(2) TF_SLOTS(3) TF_SLOTS(4) TF_SLOTS(5) TF_SLOTS(6) TF_SLOTS(7)
+#undef TF_SLOTS
   }
   *reinterpret_cast<uint4*>(out + (size_t)r * D + d) =
       make_uint4(pack_bf16(a[0], a[1]), pack_bf16(a[2], a[3]), pack_bf16(a[4], a[5]), pack_bf16(a[6], a[7]));
@@ -644,7 +656,7 @@ extern "C" int tf_moe_combine(const void* y, int y_bf16, const float* wts, uint1
     TF_LAUNCH_OK("tf_moe_combine");
     return 0;
   }
-  // (a few rows have too few workgroups of eight columns a thread: 100 x 7 x 512 2.8 us, 3.1 so)
+  // (a few rows have too few workgroups of eight columns a thread: 100 x 7 x 512 2.8 us, 3.1 so; at 131 of them both take 3.2)
   const int64_t wide = ((int64_t)rows * (d / 8) + 255) / 256;
   if (y_bf16 && d % 8 == 0 && aligned16(y) && aligned16(out) && wide >= 128 && wide <= 0x7FFFFFFF) {
     if (y_bf16 == 1) combine8_kernel<1><<<(unsigned)wide, 256, 0, as_stream(stream)>>>(static_cast<const uint16_t*>(y), wts, out, rows, slots, d / 8);
