@@ -98,6 +98,13 @@ __device__ __forceinline__ float row16_lane(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + I, 0xF, 0xF, true));
 }
 
+// Workgroups a compute unit that a launch's registers leave room for.  Told of two, the compiler keeps the accumulators among the
+// ordinary registers, which is up to 15 % faster (30 rows x 4745 x 1984 8.8 us, 8.2; 7 rows x 1869 x 1728 in groups of 32 7.9, 7.1),
+// but for the register walk of 5 to 8 rows of one weight in groups of 64: 6 rows x 644 x 1984 5.1 us, 5.4; 7 rows x 1000 x 5056
+// 11.4, 11.8, with its own group sums 11.3, 12.2; 8 rows x 7073 x 3392 10.1, 10.3, 10.0, 10.6.  (Of several weights it is not: 5 rows
+// x 7360 + 512 + 512 x 1024 5.4, 5.0.)
+constexpr int qmm_groups(int gs, int ni, bool ring) { return gs == 64 && ni == 2 && !ring ? 1 : 2; }
+
 constexpr int QPART = 68;          // floats of a row of a wave's 64 parked sums: padded against bank conflicts
 
 // LDS floats of a workgroup
@@ -455,7 +462,7 @@ __device__ __forceinline__ void qmm_block(const uint16_t* __restrict__ X, int64_
 }
 
 template <int GS, int WAVES, int RT, int NI, bool RING, bool OWN>
-__global__ void __launch_bounds__(WAVES * 64, 2)
+__global__ void __launch_bounds__(WAVES * 64, qmm_groups(GS, NI, RING))
     qmm_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
                const uint32_t* __restrict__ W, const uint16_t* __restrict__ S, const uint16_t* __restrict__ B,
                int64_t sb_stride, void* __restrict__ out, float* __restrict__ part_out, int M, int N, int KG, int SK,
@@ -576,7 +583,7 @@ __device__ __forceinline__ void qmm_arrive_tail(int* __restrict__ counter, const
 // tile's counter; the workgroup that finds the others there adds the slices in slice order (qmm_reduce_kernel's
 // arithmetic) and puts the counter back to zero.
 template <int GS, int WAVES, int NI, bool OWN>
-__global__ void __launch_bounds__(WAVES * 64, 2)
+__global__ void __launch_bounds__(WAVES * 64, qmm_groups(GS, NI, false))
     qmm_arrive_kernel(const uint16_t* __restrict__ X, int64_t ldx, const float* __restrict__ XS,
                       const uint32_t* __restrict__ W, const uint16_t* __restrict__ S, const uint16_t* __restrict__ B,
                       int64_t sb_stride, void* __restrict__ out, float* __restrict__ part_out, int* __restrict__ counters,
