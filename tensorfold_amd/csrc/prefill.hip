@@ -1387,8 +1387,15 @@ static bool big_takes(int64_t n, int64_t k) {
 //
 // What code 0 stands for.  A call's time is about a start plus a cost a round of 256 workgroups, in the same unit per
 // input of K (half microseconds at K = 4096; measured on 17 to 4,096 rows x 512 to 17,408 columns): the least of them is
-// taken.  17 rows x 4096 x 4096 82.9 -> 12.9 us, 100 rows 86.3 -> 14.4 (32 x 64), 512 rows 89 -> 33 (32 x 128),
+// taken.  17 rows x 4096 x 4096 82.9 -> 12.9 us, 100 rows 86.3 -> 14.4 (32 x 64), 512 rows 89 -> 31 (64 x 128),
 // 1,000 rows 89 -> 47 (64 x 128); at 2,000 rows the eight-wave kernel's 95.7 is the best again (64 x 128 98.5).
+//
+// 64 x 128 has a price of its own for one round, from 512 inputs on: 400 rows x 4096 x 4096 are one of it, 29.2 us, and two of
+// 32 x 128, 31.2 (512 rows 31.0, 33.4; 300 x 6144 x 4096 29.3, 31.6).  Its grid is rounded up to whole eights along the faster
+// index and workgroups go to the XCDs in turn, so it is one round where an XCD's share fits the XCD (576 rows x 3584 are 252
+// workgroups, but 36 on an XCD).  All of 71 calls that it moved from 32 x 128 are faster, by 1 to 21 %.  A price for more rounds
+// to match (two took 47 us, 56 here) slowed 37 of 698 by up to 31 %, and under 512 inputs one of those moved was slower
+// (112 x 12417 x 256 7.3 us, 64 x 128 7.6).
 constexpr int SHORT_K = 192;
 
 // The eight-wave kernel's row tiles.  Where all are 128 rows the last round of 256 workgroups is seldom full and costs what a
@@ -1426,11 +1433,19 @@ static BigTiles big_tiles(int64_t m, int64_t n) {
   return best;
 }
 
+// a call that is one round of 64 x 128 tiles: the XCD with the most of them has a compute unit for each
+static bool short64_once(int64_t m, int64_t n) {
+  const int64_t rows = (m + Short64::BM - 1) / Short64::BM, cols = (n + Short64::BN - 1) / Short64::BN;
+  if (rows * cols > 256) return false;          // (also what keeps the counts within an int)
+  const int64_t fast = short_by_col((int)m, (int)n) ? cols : rows, slow = short_by_col((int)m, (int)n) ? rows : cols;
+  return fast < 8 || (fast + 7) / 8 * slow <= 32;
+}
+
 static int prompt_tile(int64_t m, int64_t n, int64_t k) {
   auto rounds = [](int64_t workgroups) { return (workgroups + 255) / 256; };
   const int64_t t16 = 12 + 12 * rounds(Short16::workgroups(m, n)), t32 = 14 + 17 * rounds(Short32::workgroups(m, n)),
                 t32w = 16 + 26 * rounds(Short32Wide::workgroups(m, n)),
-                t64 = 32 + 40 * rounds(Short64::workgroups(m, n));
+                t64 = k >= 512 && short64_once(m, n) ? 66 : 32 + 40 * rounds(Short64::workgroups(m, n));
   const int64_t least = std::min(std::min(t16, t32), std::min(t32w, t64));
   const int64_t big = 10 + 10240 / std::max<int64_t>(k, 64) + big_tiles(m, n).cost;
   if (big_takes(n, k) && big <= least) return 9;

@@ -9,7 +9,7 @@ CODES = {1, 2, 3, 4, 5, 6, 8, 9}
 
 def test_the_rule_looks_at_rows_and_columns():
     assert qmm.prompt_tile(100, 4096, 4096) == 3           # 128 x 512 tiles would be 8 workgroups
-    assert qmm.prompt_tile(512, 4096, 4096) == 5
+    assert qmm.prompt_tile(512, 4096, 4096) == 6           # 31.0 us; 32 x 128 33.4
     assert qmm.prompt_tile(1000, 4096, 4096) == 6
     assert qmm.prompt_tile(2000, 4096, 4096) == 9
     assert qmm.prompt_tile(4096, 17408, 5120) == 9
@@ -25,6 +25,18 @@ def test_a_short_k_keeps_the_tiles_that_start_quickly():
     assert qmm.prompt_tile(8, 17408, 64) == 1              # 3.6 us; 16 x 64 4.1
     assert qmm.prompt_tile(33, 8192, 64) == 3              # 4.2 us; four-wave 4.5
     assert qmm.prompt_tile(4096, 8192, 224) == 6           # from 192 inputs on the other rule
+
+
+@pytest.mark.parametrize("m,n,k", [(400, 4096, 4096), (300, 6144, 4096), (256, 8192, 4096), (500, 4096, 5120), (98, 13184, 800),
+                                   (2264, 730, 2272)])
+def test_one_round_of_64_x_128_is_taken_where_32_x_128_takes_two(m, n, k):
+    assert qmm.prompt_tile(m, n, k) == 6
+
+
+def test_a_grid_that_an_xcd_takes_in_two_rounds_is_not_one():
+    assert qmm.prompt_tile(512, 4000, 4096) == 6           # 32 tiles of columns, the faster index, x 8: 32 on each XCD
+    assert qmm.prompt_tile(576, 3584, 4096) == 5           # 28, a grid of 32 x 9: 36 on the first
+    assert qmm.prompt_tile(1000, 2047, 448) == 5           # (fewer than 512 inputs)
 
 
 @pytest.mark.parametrize("k", [32, 64, 96, 4096, 4128, 5120])
