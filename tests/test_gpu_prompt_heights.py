@@ -32,3 +32,16 @@ def test_rounds_of_two_heights(m, n, k):
     x = synthetic.activations(m, k, n).to(DEV)
     for f32 in (False, True):
         assert torch.equal(qmm.prefill_matmul(x, q, f32=f32, tile=9), qmm.prefill_matmul(x, q, f32=f32, tile=8)), f32
+
+
+# tiles of 128 rows throughout: the last has 64 rows or less, 32 or less
+@pytest.mark.parametrize("m,n", [(1472, 10240), (1457, 10230), (1712, 9216), (2080, 7680), (2065, 7675)])
+@pytest.mark.parametrize("gs,k", [(64, 64), (32, 192)])
+def test_a_short_last_tile(m, n, gs, k):
+    assert _lib.lib().tf_qmm_prompt_rows(m, n) == 128
+    q = qmm.pack(*(t.to(DEV) for t in synthetic.affine_general(n, k, gs, m)), gs)
+    x = synthetic.activations(m, k, n).to(DEV)
+    for arith in (0, 1):
+        for f32 in (False, True):
+            assert torch.equal(qmm.prefill_matmul(x, q, f32=f32, arith=arith, tile=9),
+                               qmm.prefill_matmul(x, q, f32=f32, arith=arith, tile=8)), (arith, f32)
