@@ -112,12 +112,13 @@ enum { TF_ARITH_F16 = 0, TF_ARITH_BF16 = 1 };
 /* Prompt-form matmul on MFMA: each weight rounded once (see TF_ARITH_*), one fp32 chain over K.
  * tile: 1, 4, 8 = the four-wave kernel on 16, 64 or 128 rows x 128 columns a workgroup; 2, 3, 5, 6 = 16 x 64, 32 x 64,
  * 32 x 128 or 64 x 128, for what would leave compute units idle at larger ones; 9 = the eight-wave kernel (32 to 144 rows x
- * 512 columns, at most tf_qmm_prompt_rows rows, by how the call's tiles fill the chip; K in whole steps of 64 only); 0 = what tf_qmm_prompt_tile gives for the call's rows, columns and K (what
+ * 512 columns, tf_qmm_prompt_row_tiles tiles of at most tf_qmm_prompt_rows rows, by how the call's tiles fill the chip; K in whole steps of 64 only); 0 = what tf_qmm_prompt_tile gives for the call's rows, columns and K (what
  * kernels/qmm.py:202-205 `prompt_tile` stands for; host arithmetic alone, no GPU, returns the code).  A row's bits are
  * the same whatever the tile.
  * Replaces kernels/qmm.cpp:83-102 `qmm_prefill`. */
 int tf_qmm_prompt_tile(int m, int n, int k);
 int tf_qmm_prompt_rows(int m, int n);
+int tf_qmm_prompt_row_tiles(int m, int n);
 int tf_qmm_prefill(const uint16_t* x, int64_t ldx, const uint32_t* weight, const uint16_t* scales,
                    const uint16_t* biases, void* out, int m, int n, int k, int gs, int f32, int tile, int arith,
                    tf_stream_t stream);

@@ -26,6 +26,7 @@ PROTOTYPES = {
     "tf_qmm_group": [P, L, P, I, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, P],
     "tf_qmm_prompt_tile": [I, I, I],
     "tf_qmm_prompt_rows": [I, I],
+    "tf_qmm_prompt_row_tiles": [I, I],
     "tf_qmm_prefill": [P, L, P, P, P, P, I, I, I, I, I, I, I, P],
     "tf_quantize_rows": [P, L, I, I, I, P, P, P, P],
     "tf_qmm_prefill8": [P, P, P, P, P, P, P, I, I, I, I, I, I, P],

@@ -11,7 +11,7 @@ from tensorfold_amd import _lib, build
 
 NATIVE = _lib._bound() if build.call_lib() else None
 pytestmark = pytest.mark.skipif(NATIVE is None, reason="no C++ compiler, Python headers or torch headers")
-QUERIES = {"tf_qmm_prompt_tile", "tf_qmm_prompt_rows", "tf_exl3_gemm_tile"}          # launch nothing: called on the library itself
+QUERIES = {"tf_qmm_prompt_tile", "tf_qmm_prompt_rows", "tf_qmm_prompt_row_tiles", "tf_exl3_gemm_tile"}          # launch nothing: called on the library itself
 
 
 def sentence(name, *args):

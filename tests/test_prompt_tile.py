@@ -2,7 +2,7 @@
 
 import pytest
 
-from tensorfold_amd import qmm
+from tensorfold_amd import _lib, qmm
 
 CODES = {1, 2, 3, 4, 5, 6, 8, 9}
 
@@ -45,6 +45,14 @@ def test_every_size_has_a_tile(k):
         for n in (1, 64, 130, 4096, 17408, 248320):
             tile = qmm.prompt_tile(m, n, k)
             assert tile in CODES and (tile != 9 or k % 64 == 0), (m, n)
+
+
+@pytest.mark.parametrize("m,n,tiles,rows", [
+    (2471, 5739, 20, 128), (1166, 12301, 10, 128), (1181, 12342, 10, 128), (2193, 6202, 18, 128), (953, 15629, 8, 128),      # of 128 rows
+    (1858, 4352, 28, 80), (1329, 8768, 14, 96), (1362, 7808, 16, 96), (1554, 8372, 15, 112), (1300, 4096, 32, 48),          # dealt out
+    (2543, 5248, 23, 112), (1000, 17408, 7, 144), (4096, 17408, 30, 144)])
+def test_one_round_of_eight_wave_tiles_is_dealt_out_where_its_tallest_tile_is_shorter_for_it(m, n, tiles, rows):
+    assert (_lib.lib().tf_qmm_prompt_row_tiles(m, n), _lib.lib().tf_qmm_prompt_rows(m, n)) == (tiles, rows)
 
 
 def test_a_weight_past_a_32_bit_offset_keeps_off_the_eight_wave_tile():
