@@ -99,12 +99,13 @@ def test_results_of_a_subclass_are_of_its_class(monkeypatch):
 
 
 def test_a_tensor_without_storage_raises():
-    meta = torch.empty((2, 64), dtype=torch.bfloat16, device="meta")
     x = torch.zeros((2, 64), dtype=torch.bfloat16)
-    try:
-        NATIVE["tf_group_sums"](meta, 64, 2, 64, 48, x, None)          # (torch hands out an address of 0, or refuses)
-    except RuntimeError:
-        pass
+    nowhere = torch.empty((2, 64), dtype=torch.bfloat16, device="meta")          # torch hands out an address of 0
+    for args in ((nowhere, 64, 2, 64, 64, x, None), (x, 64, 2, 64, 64, nowhere, None)):
+        assert "x must be" in sentence("tf_group_sums", *args)
+    for args in ((x.to_sparse(), 64, 2, 64, 64, x, None), (x, 64, 2, 64, 64, x.to_sparse(), None)):
+        with pytest.raises(RuntimeError, match="storage"):
+            NATIVE["tf_group_sums"](*args)
 
 
 def test_what_an_allocation_raises_keeps_its_type():
