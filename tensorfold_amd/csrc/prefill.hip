@@ -410,7 +410,7 @@ constexpr int big_stage(int rt) { return std::max(16 * rt, BIG_ROWS) * AROW; }
 template <int GS, int NM>
 struct ExpertSource {
   static constexpr int CPS = KSTEP / 32, GPS = KSTEP / GS;
-  static constexpr bool KEEPS_GROUP_WORDS = false;
+  static constexpr bool KEEPS_GROUP_WORDS = false, SPARE_AGAIN = true;
   static constexpr uint32_t GSTRIDE = NM * block_words(GS);      // words from one group to the next
   struct Raw {
     u32x4_t q[CPS];
@@ -435,7 +435,7 @@ struct ExpertSource {
 template <int GS>
 struct DenseSource {
   static constexpr int CPS = KSTEP / 32, GPS = KSTEP / GS;
-  static constexpr bool KEEPS_GROUP_WORDS = true;
+  static constexpr bool KEEPS_GROUP_WORDS = true, SPARE_AGAIN = false;
   struct Raw {
     u32x4_t q[CPS];
     uint32_t s[GPS], b[GPS];          // each a bf16 in the low half, joined when a chunk is taken (not when they
@@ -506,30 +506,36 @@ __device__ __forceinline__ void big_body(const uint16_t* __restrict__ X, int64_t
     for (int j = 0; j < TJ; ++j) sb[j] = mine;
     across(sb);
   };
-  // this thread's pieces of the activation tile: piece q = (row q / 8, 16 bytes q % 8).  A thread past the last piece takes its
-  // first one again: requests under a condition would make the wait for the weights ahead of them one for everything (7
-  // row tiles of 8 waves: 129 -> 101 us a tile of K = 5120)
-  constexpr bool PAST = PIECES > NTHREADS && PIECES % NTHREADS != 0;
+  // this thread's pieces of the activation tile: piece q = (row q / 8, 16 bytes q % 8).  A thread past the last piece takes one
+  // again: requests under a condition would make the wait for the weights ahead of them one for everything (7 row tiles of 8
+  // waves: 129 -> 101 us a tile of K = 5120).  Where there are fewer pieces than threads, experts' items of one row tile on four
+  // waves and of three on eight do so too (355 rows x 26 experts of 2112 x 1344, bf16: down 19.5 -> 17.8 us; 1,428 rows x
+  // 341 experts of 576 x 704, 8 picks, fp16: up 61.9 -> 60.1, down 45.7 -> 42.6).  Not one or two on eight waves, which would ask
+  // four times or twice for what they need (777 rows x 128 experts of 2688 x 1856, 2 picks, up 86 us, 91 with two so), nor the
+  // dense tiles (850 x 6487 x 1920 in tiles of 48 rows 39.2 us, 41.4 so).
+  constexpr bool PAST = PIECES % NTHREADS != 0 &&
+                        (PIECES > NTHREADS || (WS::SPARE_AGAIN && (NTHREADS == 256 || 4 * PIECES >= 3 * NTHREADS)));
+  static_assert(!PAST || PIECES > NTHREADS || 2 * PIECES >= NTHREADS, "a spare thread's piece is there");
   const uint16_t* asrc[PPT];
 #pragma unroll
   for (int j = 0; j < PPT; ++j) {
     int q = tid + j * NTHREADS;
-    if (PAST && q >= PIECES) q = tid;
+    if (PAST && q >= PIECES) q = PIECES > NTHREADS ? tid : tid - PIECES;
     const int r = q >> 3, ch = q & 7;
     asrc[j] = X + (size_t)src_rows[r < cnt ? r : 0] * x_stride + ch * 8;
   }
   auto load_a = [&](int step, uint4 (&v)[PPT]) {
 #pragma unroll
     for (int j = 0; j < PPT; ++j)
-      if (PIECES >= NTHREADS || tid < PIECES)
+      if (PIECES >= NTHREADS || PAST || tid < PIECES)
         v[j] = *reinterpret_cast<const uint4*>(asrc[j] + (size_t)step * KSTEP);
   };
   auto store_a = [&](int buf, const uint4 (&v)[PPT]) {
 #pragma unroll
     for (int j = 0; j < PPT; ++j) {
       int q = tid + j * NTHREADS;
-      if (PAST && q >= PIECES) q = tid;
-      if (PIECES >= NTHREADS || q < PIECES)
+      if (PAST && q >= PIECES) q = PIECES > NTHREADS ? tid : tid - PIECES;
+      if (PIECES >= NTHREADS || PAST || q < PIECES)
         *reinterpret_cast<uint4*>(smem + buf * STAGE + (q >> 3) * AROW + (q & 7) * 16) =
             AR ? stage8_bf16(v[j]) : stage8(v[j]);
     }
