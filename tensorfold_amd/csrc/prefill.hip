@@ -1421,8 +1421,8 @@ constexpr int SHORT_K = 192;
 // those have room for, its 16-row units dealt out over them evenly: `tall` tiles of `rt` units, then tiles of one unit less.
 // `cost`: half microseconds at K = 4096 by the most units a tile has, for a round whose workgroups leave half the chip idle
 // and for a full one, where the clock is lower (17408 x 5120: 34 tiles of 128 rows 110 us, 238 tiles 139).  The rounds
-// whose cost is least are taken.  17408 x 5120, 1,000 rows: 239 -> 156 us (63 units on 7 row tiles), 512 rows 112 -> 101, 2,000 rows 380 ->
-// 305, 4,096 rows 656 -> 625; 12288 x 4096, 1,500 rows 200 -> 155; 4096 x 4096, 1,300 rows 78 -> 62.
+// whose cost is least are taken.  17408 x 5120, 1,000 rows: 239 -> 149 us (63 units on 7 row tiles), 512 rows 110 -> 95, 2,000 rows
+// 372 -> 283, 4,096 rows 630 -> 573; 12288 x 4096, 1,500 rows 196 -> 149; 4096 x 4096, 1,300 rows 77 -> 60.
 struct BigTiles {
   int64_t tiles, tall;
   int rt;
